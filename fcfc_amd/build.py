@@ -73,7 +73,7 @@ def build_oracle():
     reference binaries when the upstream sources are present."""
     od = os.path.join(ROOT, "oracle")
     _run(["make", "-C", od, "-j4"])
-    if os.path.isdir(os.environ.get("FCFC_REFDIR", "/root/reference")):
+    if os.path.isdir(os.path.join(os.environ.get("FCFC_REFDIR", "/root/reference"), "src")):
         _run(["make", "-C", od, "ref", "-j6"])
 
 
