@@ -144,102 +144,103 @@ __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ s
   }
 }
 
-/* Work items of the tile list: tile ti becomes S items (each a share of the
+/* Work items of the run list: run ti becomes S items (each a share of the
  * strip list) for ti < tt and St > S finer items from tt on, so that the
- * items the persistent workgroups take last are short and the launch ends
- * evenly.  ncap tiles in all: of each group of G consecutive tiles of the
- * tiling, its first `run` tiles.  A full count has one group (G = run =
- * the tile count); the autotuner's samples take runs spread over the whole
+ * items the wavefronts take last are short and the launch ends evenly.
+ * ncap runs in all: of each group of G consecutive runs of the list, its
+ * first `run` runs.  A full count has one group (G = run = the number of
+ * runs); the autotuner's samples take stretches spread over the whole
  * catalogue, each keeping the neighbourhood, and so the cache reuse, of a
  * full count. */
 struct FkSplit { int S, tt, St, ncap, G, run; };
-
-/* list position of tile ti of the tiling, or -1 when it is not sampled */
-__host__ __device__ inline int split_sample(const FkSplit &s, int ti) {
-  const int g = ti / s.G, p = ti - g * s.G;
-  return p < s.run ? g * s.run + p : -1;
-}
 
 __host__ __device__ inline long long split_pos(const FkSplit &s, int ti) {
   return ti < s.tt ? (long long) s.S * ti
                    : (long long) s.S * s.tt + (long long) s.St * (ti - s.tt);
 }
 
-/* Tiles of one row: consecutive cells, at most T objects, at most zmaxc
- * z-cells; a cell with more than T objects is split into T-sized tiles.
- * t0: index of the row's first tile in the tile list. */
-__device__ int row_tiles(const int *__restrict__ cs, int ncz, int T, int zmaxc,
-    int row, int job, int nstrips, const FkSplit &sp, int t0, FkTile *out) {
-  int nt = 0, open = 0, tp0 = 0, tcnt = 0, tz0 = 0, tz1 = 0;
-  /* emit tile (p0, p1, iz0, iz1) as items over the strip list */
-  auto emit = [&](int p0, int p1, int iz0, int iz1) {
-    const int ti = t0 + nt;
-    const int si = out ? split_sample(sp, ti) : -1;
-    if (si >= 0 && si < sp.ncap) {
-      const int S = si < sp.tt ? sp.S : sp.St;
-      FkTile *o = out + split_pos(sp, si);
-      for (int q = 0; q < S; q++)
-        o[q] = FkTile{row, p0, p1, iz0, iz1, job,
-                      (int) ((long long) nstrips * q / S),
-                      (int) ((long long) nstrips * (q + 1) / S)};
-    }
-    nt++;
-  };
-  for (int iz = 0; iz < ncz; iz++) {
-    const int c = cs[iz + 1] - cs[iz];
-    if (c == 0) continue;
-    if (open && (tcnt + c > T || iz - tz0 + 1 > zmaxc)) {
-      emit(tp0, tp0 + tcnt, tz0, tz1);
-      open = 0;
-    }
-    if (c > T) {
-      for (int k = 0; k < c; k += T) emit(cs[iz] + k, cs[iz] + min(k + T, c), iz, iz);
-      continue;
-    }
-    if (!open) { open = 1; tp0 = cs[iz]; tcnt = 0; tz0 = iz; }
-    tcnt += c; tz1 = iz;
-  }
-  if (open) emit(tp0, tp0 + tcnt, tz0, tz1);
-  return nt;
-}
+/* Runs of all jobs of a launch: job k owns the units unit0 .. unit0 + nrow
+ * nblk - 1 (unit0 ascending); a unit is one block of zm z-cells of one row,
+ * cut into runs of T consecutive objects. */
+struct FkTileJob { int unit0, nblk, zm, ncz, T; const int *cs; };
 
-/* Tiling of all jobs of a launch in one pass: job k owns rows row0 ..
- * row0 + ncx ncy - 1 of the launch's row space (row0 ascending). */
-struct FkTileJob { int row0, ncz, T, zmaxc, nstrips; const int *cs; };
-
-__device__ __forceinline__ int fk_tile_job(const FkTileJob *__restrict__ tj, int njob, int gr) {
-  int lo = 0, hi = njob - 1;                  /* last job with row0 <= gr */
+__device__ __forceinline__ int fk_tile_job(const FkTileJob *__restrict__ tj, int njob, int u) {
+  int lo = 0, hi = njob - 1;                  /* last job with unit0 <= u */
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (tj[mid].row0 <= gr) lo = mid; else hi = mid - 1;
+    if (tj[mid].unit0 <= u) lo = mid; else hi = mid - 1;
   }
   return lo;
 }
 
-__global__ void k_tile_count(int nrow, int njob, const FkTileJob *__restrict__ tj,
-    int *__restrict__ ntile) {
-  for (int gr = blockIdx.x * blockDim.x + threadIdx.x; gr < nrow; gr += gridDim.x * blockDim.x) {
-    const FkTileJob t = tj[fk_tile_job(tj, njob, gr)];
-    const int r = gr - t.row0;
-    ntile[gr] = row_tiles(t.cs + (size_t) r * t.ncz, t.ncz, t.T, t.zmaxc, r, 0, 0,
-                          FkSplit{1, 0, 1, 0, 1, 1}, 0, nullptr);
+/* objects [p0, p1) and row of a unit */
+__device__ __forceinline__ int fk_unit(const FkTileJob &t, int u, int &p0, int &p1) {
+  const int v = u - t.unit0, row = v / t.nblk, c0 = (v - row * t.nblk) * t.zm;
+  const int *cs = t.cs + (size_t) row * t.ncz;
+  p0 = cs[c0]; p1 = cs[min(c0 + t.zm, t.ncz)];
+  return row;
+}
+
+__global__ void k_run_count(int nunit, int njob, const FkTileJob *__restrict__ tj,
+    int *__restrict__ nrun) {
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nunit; u += gridDim.x * blockDim.x) {
+    const FkTileJob t = tj[fk_tile_job(tj, njob, u)];
+    int p0, p1;
+    fk_unit(t, u, p0, p1);
+    nrun[u] = (p1 - p0 + t.T - 1) / t.T;
   }
 }
-/* the tiles of row gr are numbered from toff[gr] */
-__global__ void k_tile_emit(int nrow, int njob, const FkTileJob *__restrict__ tj,
-    const int *__restrict__ toff, FkSplit sp, FkTile *__restrict__ tiles) {
-  for (int gr = blockIdx.x * blockDim.x + threadIdx.x; gr < nrow; gr += gridDim.x * blockDim.x) {
-    const int k = fk_tile_job(tj, njob, gr);
+/* the runs of unit u are numbered from roff[u] */
+__global__ void k_run_emit(int nunit, int njob, const FkTileJob *__restrict__ tj,
+    const int *__restrict__ roff, FkRun *__restrict__ runs) {
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nunit; u += gridDim.x * blockDim.x) {
+    const int k = fk_tile_job(tj, njob, u);
     const FkTileJob t = tj[k];
-    const int r = gr - t.row0;
-    row_tiles(t.cs + (size_t) r * t.ncz, t.ncz, t.T, t.zmaxc, r, k, t.nstrips, sp,
-              toff[gr], tiles);
+    int p0, p1;
+    const int row = fk_unit(t, u, p0, p1);
+    FkRun *o = runs + roff[u];
+    for (int p = p0; p < p1; p += t.T) *o++ = FkRun{row, p, min(p + t.T, p1), k};
   }
 }
 
 /* ======================================================================== */
 /*                             count kernel                                 */
 /* ======================================================================== */
+
+/* Loads through explicit address spaces: pointers that come out of the job
+ * descriptors are generic to the compiler, which would use flat loads. */
+template <class T>
+__device__ __forceinline__ T fk_gld(const T *p, int i) {
+  return ((const __attribute__((address_space(1))) T *) p)[i];
+}
+/* a descriptor at a uniform address, read with scalar loads (only the fields
+ * in use are kept) */
+template <class T>
+__device__ __forceinline__ T fk_cld(const T *p) {
+  struct Raw { int v[sizeof(T) / 4]; } r;
+  const __attribute__((address_space(4))) int *q = (const __attribute__((address_space(4))) int *) p;
+#pragma unroll
+  for (int i = 0; i < (int) (sizeof(T) / 4); i++) r.v[i] = q[i];
+  return __builtin_bit_cast(T, r);
+}
+/* element i of p at an address that the compiler cannot take for one it has
+ * read before: descriptors read through it are read again where they are used
+ * instead of being held in (and spilled from) scalar registers */
+template <class T>
+__device__ __forceinline__ const T *fk_again(const T *p, int i) {
+  i = __builtin_amdgcn_readfirstlane(i);
+  asm volatile("" : "+s"(i));
+  return p + i;
+}
+/* order LDS writes and reads of one wavefront (its LDS operations execute in
+ * order: only the compiler has to be held) */
+__device__ __forceinline__ void fk_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ int fk_lane_of(int v, int lane) {
+  return __builtin_amdgcn_readlane(v, lane);
+}
 
 /* v of lane (lane with the DPP pattern CTRL applied), both halves moved */
 template <int CTRL>
@@ -262,6 +263,27 @@ __device__ __forceinline__ double fk_row_sum(double v) {
   return v;
 }
 
+/* smallest v of the wavefront, in a scalar register; every lane active */
+__device__ __forceinline__ double fk_wave_min(double v) {
+  v = __builtin_fmin(v, fk_dpp<0xB1>(v));
+  v = __builtin_fmin(v, fk_dpp<0x4E>(v));
+  v = __builtin_fmin(v, fk_dpp<0x141>(v));
+  v = __builtin_fmin(v, fk_dpp<0x140>(v));
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  double m = 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const unsigned lo = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) u, 16 * r);
+    const unsigned hi = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) (u >> 32), 16 * r);
+    const double w = __builtin_bit_cast(double, ((unsigned long long) hi << 32) | lo);
+    m = r ? __builtin_fmin(m, w) : w;
+  }
+  const unsigned long long um = __builtin_bit_cast(unsigned long long, m);
+  const unsigned lo = (unsigned) __builtin_amdgcn_readfirstlane((int) (unsigned) um);
+  const unsigned hi = (unsigned) __builtin_amdgcn_readfirstlane((int) (unsigned) (um >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long) hi << 32) | lo);
+}
+
 /* FP32 exactness windows (see fp32_windows on the host). */
 struct FkWin {
   float e_s2, e_s2x2;         /* absolute window on s^2 (or s_perp^2), 2 e_s2 */
@@ -275,24 +297,6 @@ struct FkWin {
   float m2_floor;             /* survey: pairs with |a + b|^2 below this    */
 };                            /* are re-evaluated                          */
 
-/* A value that is the same in every lane (read from the job or tile held in
- * LDS), moved to a scalar register: the compiler cannot tell that it is
- * uniform and would otherwise keep it in a vector register. */
-__device__ __forceinline__ float fk_uni(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ FkWin fk_uni(const FkWin &w) {
-  FkWin u;
-  u.e_s2 = fk_uni(w.e_s2); u.e_s2x2 = fk_uni(w.e_s2x2);
-  u.e_pi = fk_uni(w.e_pi); u.e_pix2 = fk_uni(w.e_pix2);
-  u.idle_x = fk_uni(w.idle_x); u.idle_z = fk_uni(w.idle_z);
-  u.mu_sh = fk_uni(w.mu_sh); u.mu_c = fk_uni(w.mu_c);
-  u.mu_t16 = (unsigned) __builtin_amdgcn_readfirstlane((int) w.mu_t16);
-  u.s2_floor = fk_uni(w.s2_floor); u.nmu_f = fk_uni(w.nmu_f);
-  u.m2_floor = fk_uni(w.m2_floor);
-  return u;
-}
-
 /* Flags of the integer cells of the FP32 tables, set while they are staged
  * (the LDS cells then carry a float threshold in place of the flags). */
 #define FK_F_EDGE 0x10000u    /* a bin edge at the lower end of the integer cell */
@@ -301,7 +305,7 @@ __device__ __forceinline__ FkWin fk_uni(const FkWin &w) {
 #define FK_F_NEVER  0xBF80u   /* ... of cells without flags: -1                  */
 
 /* One counting job: a catalogue pair and its histogram.  A launch counts the
- * tiles of one or many jobs (batched mocks); tiles carry their job index. */
+ * runs of one or many jobs (batched mocks); runs carry their job index. */
 struct FkJob {
   FkCat A, B;
   FkGrid g;
@@ -321,36 +325,31 @@ struct FkArgs {
   const FkJob *jobs;
   int njobs;
   FkBins bins;
-  const FkTile *tiles;
-  int ntiles;
+  const FkRun *runs;
+  FkSplit sp;                 /* work items of the runs              */
+  int nitems;
   unsigned int *queue;
   unsigned long long *gcnt_u;
   double *gcnt_d;
   unsigned long long *stats;  /* evals, rechecked, census */
   int nh;                     /* LDS histogram copies */
   /* LDS byte offsets */
-  int off_hist, off_stab, off_ptab, off_edges, off_strip, off_chunk, off_queue;
+  int off_hist, off_stab, off_ptab, off_edges, off_chunk, off_queue;
   int stab_c0, ptab_c0;       /* table entries before cell 0 */
   int census;
   const double *G;            /* GRAD: dL/dcnt */
 };
 
-/* LDS strip table */
-struct FkStripLds {
-  int off[FK_NSB + 1];
-  int b0[FK_NSB * FK_MAXSEG];
-  int len[FK_NSB * FK_MAXSEG];
-  int code[FK_NSB * FK_MAXSEG];
-};
-
-/* Compute the (up to three) B segments of one strip for tile t. */
-__device__ void fk_strip_segments(const FkJob &J, const FkTile &t, int dx,
-    int dy, int diag, int *b0, int *len, int *code) {
-  const FkGrid &g = J.g;
+/* The (up to three) B segments of one strip for a run of row t.row whose
+ * objects span [zlo, zhi]: the objects of the strip's row within the z window
+ * of that span, unwrapped (main), and its images at -Lz and +Lz. */
+__device__ __forceinline__ void fk_strip_segments(const FkGrid &g, const int *cell_start,
+    const FkRun &t, double zlo, double zhi, int dx, int dy, int diag, int *b0, int *len,
+    int *code) {
   b0[0] = b0[1] = b0[2] = 0;
   len[0] = len[1] = len[2] = 0;
   code[0] = code[1] = code[2] = 13;
-  const int ix = t.row / g.ncy, iy = t.row - (t.row / g.ncy) * g.ncy;
+  const int ix = t.row / g.ncy, iy = t.row - ix * g.ncy;
   int bx = ix + dx, by = iy + dy, cx = 0, cy = 0;
   if (g.periodic) {
     if (bx < 0) { bx += g.ncx; cx = -1; } else if (bx >= g.ncx) { bx -= g.ncx; cx = 1; }
@@ -362,40 +361,31 @@ __device__ void fk_strip_segments(const FkJob &J, const FkTile &t, int dx,
   const double d2 = gx * gx + gy * gy;
   if (d2 >= g.Rxy2) return;
   const double hz = (g.hz_const >= 0) ? g.hz_const : sqrt(fmax(g.R2 - d2, 0.0));
-  const double zc0 = (double) t.iz0 - hz / g.wz - 1e-6;
-  const double zc1 = (double) (t.iz1 + 1) + hz / g.wz + 1e-6;
-  int izlo = (int) floor(zc0), izhi = (int) floor(zc1);
-  const int *cs = J.B.cell_start + (size_t) (bx * g.ncy + by) * g.ncz;
+  const int izlo = (int) floor((zlo - hz - g.oz) / g.wz - 1e-6);
+  const int izhi = (int) floor((zhi + hz - g.oz) / g.wz + 1e-6);
+  const int base = (bx * g.ncy + by) * g.ncz;
   const int cxy = (cx + 1) + 3 * (cy + 1);
-  if (g.periodic) {
-    if (izhi - izlo + 1 > g.ncz) {   /* cannot happen with the tile limits */
-      izlo = 0; izhi = g.ncz - 1;
-    }
-    if (izlo < 0) {                  /* image below z = 0: B shifted by -Lz */
-      int c0 = izlo + g.ncz, c1 = g.ncz - 1;
-      b0[0] = cs[c0]; len[0] = cs[c1 + 1] - cs[c0]; code[0] = cxy + 9 * 0;
-    }
-    {
-      int c0 = max(izlo, 0), c1 = min(izhi, g.ncz - 1);
-      if (diag) {
-        /* auto counts, same row: only objects after the tile (j > i) */
-        int e = cs[c1 + 1];
-        b0[1] = t.p1; len[1] = max(e - t.p1, 0); code[1] = cxy + 9 * 1;
-      }
-      else if (c1 >= c0) { b0[1] = cs[c0]; len[1] = cs[c1 + 1] - cs[c0]; code[1] = cxy + 9 * 1; }
-    }
-    if (izhi >= g.ncz && !diag) {    /* image above: B shifted by +Lz */
-      int c0 = 0, c1 = izhi - g.ncz;
-      b0[2] = cs[c0]; len[2] = cs[c1 + 1] - cs[c0]; code[2] = cxy + 9 * 2;
-    }
+  const int c0 = max(izlo, 0), c1 = min(izhi, g.ncz - 1);
+  code[1] = cxy + 9 * 1;
+  if (c1 >= c0) {
+    const int e = fk_gld(cell_start, base + c1 + 1);
+    /* auto counts, same row: only objects after the run (j > i) */
+    b0[1] = diag ? t.p1 : fk_gld(cell_start, base + c0);
+    len[1] = max(e - b0[1], 0);
   }
-  else {
-    int c0 = max(izlo, 0), c1 = min(izhi, g.ncz - 1);
-    if (diag) {
-      int e = (c1 >= 0) ? cs[c1 + 1] : t.p1;
-      b0[0] = t.p1; len[0] = max(e - t.p1, 0); code[0] = 13;
+  if (g.periodic) {
+    if (izlo < 0) {                    /* image below z = 0: B shifted by -Lz */
+      const int l0 = max(izlo + g.ncz, 0);
+      b0[0] = fk_gld(cell_start, base + l0);
+      len[0] = fk_gld(cell_start, base + g.ncz) - b0[0];
+      code[0] = cxy + 9 * 0;
     }
-    else if (c1 >= c0) { b0[0] = cs[c0]; len[0] = cs[c1 + 1] - cs[c0]; code[0] = 13; }
+    if (izhi >= g.ncz && !diag) {      /* image above: B shifted by +Lz */
+      const int l1 = min(izhi - g.ncz, g.ncz - 1);
+      b0[2] = fk_gld(cell_start, base);
+      len[2] = fk_gld(cell_start, base + l1 + 1) - b0[2];
+      code[2] = cxy + 9 * 2;
+    }
   }
 }
 
@@ -592,7 +582,7 @@ __device__ __forceinline__ unsigned fk_smu_index(double anmu, double r, FA fa, d
   unsigned idx = fk_mad_hi16(v, (unsigned) bn.nsh, sb);
   const bool exact = MUT ? !((v & 0xFFFFu) < (sb >> 16))
                          : (!((v & 0xFFFFu) < bn.mu_t16) || s2 < bn.s2_exact);
-  if (exact)
+  if (__builtin_expect(exact, 0))
     idx = (sb & 0xFFFFu) + __umul24((unsigned) bn.nsh, fk_mu_exact(fa(), s2, tm - FK_MU_C0, bn) + 1u)
           + (MUT ? bn.mu_t16 << 16 : 0u);
   return idx;
@@ -680,7 +670,7 @@ __device__ __forceinline__ unsigned fk_sv64(double ax, double ay, double az,
     unsigned idx = fk_mad_lo16(eq, (unsigned) bn.nsh, es & 0xFFFFu);
     const bool clear = (bb >= bn.q_bmin) & ((vq & 0xFFFFu) <= (eq >> 16)) &
                        ((vs & 0xFFFFu) <= (es >> 16));
-    if (!clear) {
+    if (__builtin_expect(!clear, 0)) {
       const double p2 = n / bb;
       const double sp2 = (s - t) - p2;
       const unsigned ks = min((unsigned) (int) sp2, (unsigned) (bn.soff + bn.stab_len)) + 2u;
@@ -889,7 +879,7 @@ __device__ __forceinline__ unsigned fk_recheck(const FkBins &bn, const FkJob &J,
     double ax, double ay, double az, int jg, int code, const unsigned *stab,
     const unsigned *ptab, const double *s2e, const double *pe, unsigned int *ncensus) {
   const int c3[3] = {code % 3 - 1, (code / 3) % 3 - 1, code / 9 - 1};
-  const double bo[3] = {J.B.x[jg], J.B.y[jg], J.B.z[jg]};
+  const double bo[3] = {fk_gld(J.B.x, jg), fk_gld(J.B.y, jg), fk_gld(J.B.z, jg)};
   const double ex = bo[0] + c3[0] * J.g.Lx;
   const double ey = bo[1] + c3[1] * J.g.Ly;
   const double ez = bo[2] + c3[2] * J.g.Lz;
@@ -906,15 +896,22 @@ __device__ __forceinline__ unsigned fk_recheck(const FkBins &bn, const FkJob &J,
 template <int BIN, bool HYB>
 __device__ __forceinline__ unsigned fk_recheck_sv(const FkBins &bn, const FkJob &J, int p,
     int jg, const unsigned *stab, const unsigned *ptab, const double *s2e, const double *pe) {
-  const double as = (BIN == FCFC_BIN_ISO) ? 0.0 : J.A.s[p];
-  const double bs = (BIN == FCFC_BIN_ISO) ? 0.0 : J.B.s[jg];
-  unsigned idx = fk_sv64<BIN, HYB, false, true>(J.A.x[p], J.A.y[p], J.A.z[p], as, J.B.x[jg],
-                                                J.B.y[jg], J.B.z[jg], bs, bn, stab, ptab, s2e, pe);
+  const double as = (BIN == FCFC_BIN_ISO) ? 0.0 : fk_gld(J.A.s, p);
+  const double bs = (BIN == FCFC_BIN_ISO) ? 0.0 : fk_gld(J.B.s, jg);
+  unsigned idx = fk_sv64<BIN, HYB, false, true>(fk_gld(J.A.x, p), fk_gld(J.A.y, p), fk_gld(J.A.z, p),
+                                                as, fk_gld(J.B.x, jg), fk_gld(J.B.y, jg),
+                                                fk_gld(J.B.z, jg), bs, bn, stab, ptab, s2e, pe);
   if (BIN == FCFC_BIN_SMU) idx -= (unsigned) bn.nsh;
   return idx >= (unsigned) bn.ntoh ? FK_NONE : idx;
 }
 
 /* ---------------------------- the kernel --------------------------------- */
+
+/* LDS bytes of one staged B object: coordinates (relative to the run's
+ * centre in FP32), |r|^2, weight, gradient share, sorted index */
+__host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool need_s, bool need_w, bool grad) {
+  return (f32 ? 12 : 24) + (need_s ? 8 : 0) + (need_w ? 8 : 0) + (grad ? 8 : 0) + 4;
+}
 
 /* One persistent kernel for counts (FP64 or FP32 + recheck) and for the
  * weight gradient.  Template parameters: binning, geometry, weighted
@@ -922,7 +919,17 @@ __device__ __forceinline__ unsigned fk_recheck_sv(const FkBins &bn, const FkJob 
  * kernels are held to 64 VGPRs (8 waves per SIMD, 4 workgroups per CU):
  * occupancy pays more than the FP32 form's spills, which sit in its rare
  * re-evaluation paths.  Weighted ones get 80 (6 waves per SIMD), as their
- * FP64 LDS histograms limit them to 3 workgroups per CU anyway. */
+ * FP64 LDS histograms limit them to 3 workgroups per CU anyway.
+ *
+ * The kernel is bound by the VALU instructions of the evaluated pairs, so the
+ * split is chosen to evaluate few: a wavefront takes 64 R objects on its own
+ * (a compact box, no lanes idle because a tile of 8 wavefronts is not full,
+ * no barrier in the loop), and a B object that is beyond the separation from
+ * that box costs one lane's share of a test instead of 64 R distances.
+ * Against tiles of 512 R objects that shared their B chunks (same data, ms of
+ * the whole call): (s, mu) RR of 4e6 objects 331 -> 232, weighted DD of 5e5
+ * 16.9 -> 9.1, w_p of 1e6 to 40 Mpc/h (128 objects in tiles of 1024) 11.8 ->
+ * 4.6, survey (s, mu) RR of 1.2e6 27.1 -> 16.1. */
 template <int BIN, int GEOM, bool WT, int MODE, bool HYB, int R>
 __global__ void __launch_bounds__(FK_NT, WT ? 6 : 8)
 k_count(const FkArgs a) {
@@ -969,26 +976,27 @@ k_count(const FkArgs a) {
   const unsigned *stab = HYB ? stab_raw + a.stab_c0 : stab_raw;
   const unsigned *ptab = HYB ? ptab_raw + a.ptab_c0 : ptab_raw;
   const unsigned os_lds = fk_lds_addr(stab_raw), op_lds = fk_lds_addr(ptab_raw);
-  /* FP32 re-evaluation queue of this wavefront: (A slot in the wavefront
-   * << 8) | chunk index */
-  uint16_t *wq = (uint16_t *) (lds + a.off_queue) + wave * FK_QCAP;
   double *s2e = (double *) (lds + a.off_edges);
   double *pe = s2e + (bn.ns + 1);
-  FkStripLds *st = (FkStripLds *) (lds + a.off_strip);
-  char *cp = lds + a.off_chunk;
-  double *cx = (double *) cp, *cy = cx + FK_CH, *cz = cy + FK_CH;
-  float *fx = (float *) cp, *fy = fx + FK_CH, *fz = fy + FK_CH;
-  cp += (F32 ? 12 : 24) * FK_CH;
+  /* the wavefront's chunk of B objects */
+  char *cp = lds + a.off_chunk + wave * (FK_CH * fk_chunk_bytes(F32, NEED_S, NEED_W, GRAD));
   double *cs_ = (double *) cp;                 /* survey |r|^2 */
   if (NEED_S) cp += 8 * FK_CH;
   double *cw = (double *) cp;                  /* weights */
   if (NEED_W) cp += 8 * FK_CH;
   double *cb = (double *) cp;                  /* GRAD: gradient share of each B object */
   if (GRAD) cp += 8 * FK_CH;
+  double *cx = (double *) cp, *cy = cx + FK_CH, *cz = cy + FK_CH;
+  float *fx = (float *) cp, *fy = fx + FK_CH, *fz = fy + FK_CH;
+  cp += (F32 ? 12 : 24) * FK_CH;
   int *cj = (int *) cp;                        /* sorted index */
-  cp += 4 * FK_CH;
-  int *cc = (int *) cp;                        /* periodic image code */
-  __shared__ int s_tile;
+  /* FP32 re-evaluation queue of this wavefront: sorted index of the B
+   * object, A slot in the run << 5 | periodic image code */
+  unsigned *wqj = (unsigned *) (lds + a.off_queue + wave * (FK_QCAP * 6));
+  uint16_t *wqs = (uint16_t *) (wqj + FK_QCAP);
+  __shared__ int s_next[FK_NW];
+  __shared__ double s_box[FK_NW][6];           /* bounding boxes of the runs */
+  double *box = s_box[wave];
 
   /* ---- stage tables ---- */
   const int hist_elems = a.nh * bn.ntoh;
@@ -1070,9 +1078,11 @@ k_count(const FkArgs a) {
     if (BIN == FCFC_BIN_SPI) for (int i = tid; i <= bn.np; i += FK_NT) pe[i] = bn.pbin[i];
   }
 
-  double evals = 0;
+  unsigned long long evals = 0;               /* uniform: candidate pairs */
   unsigned int nrecheck = 0, ncensus = 0;
-  double since_flush = 0;
+  /* pairs this wavefront may have added to 32-bit counters since the
+   * workgroup's last flush (FK_NW such budgets stay below 2^32) */
+  unsigned since = 0;
   unsigned int *myhist_u = hist_u + (wave % a.nh) * bn.ntoh;
   double *myhist_d = hist_d + (wave % a.nh) * bn.ntoh;
   /* byte offsets in lds of these histograms, minus the pair functions'
@@ -1082,143 +1092,180 @@ k_count(const FkArgs a) {
   const unsigned ohist_u = (unsigned) a.off_hist + 4u * ((unsigned) (wave % a.nh) * ntot - ioff);
   const unsigned ohist_d = (unsigned) a.off_hist + 8u * ((unsigned) (wave % a.nh) * ntot - ioff);
   const unsigned ohist_g = (unsigned) a.off_hist - 8u * ioff;
-  __shared__ FkJob sJ;
-  const FkJob &J = sJ;
-  int cur = -1;
+  const int lane = tid & 63;
 
-  /* add the LDS histograms of the current job to its global histogram */
-  auto flush = [&]() {
+  /* The wavefronts of a workgroup run on their own and meet only here: at
+   * the start, when the job changes, at the end of the queue (want = FK_END)
+   * and when a wavefront has used up its budget of 32-bit counts (want =
+   * cur).  Each round every wavefront posts the job it wants; the LDS
+   * histograms are added to the global one of the job counted so far, and
+   * the smallest wanted job comes next.  The queue hands out items in job
+   * order, so a wavefront that wants a later job waits in the next round for
+   * those that still count this one; every round sees all wavefronts, and
+   * the last one (all want FK_END) ends them all. */
+#define FK_END 0x7fffffff
+#define FK_BUDGET 500000000u
+  int cur = -1;
+  auto job_round = [&](int want) -> int {
+    if (lane == 0) s_next[wave] = want;
     __syncthreads();
-    if (cur >= 0) {
-      const bool w = WT && J.wt;
+    int nx = s_next[0];
+    for (int q = 1; q < FK_NW; q++) nx = min(nx, s_next[q]);
+    nx = __builtin_amdgcn_readfirstlane(nx);
+    if (!GRAD && cur >= 0) {
+      const FkJob *pj = a.jobs + cur;
+      const bool w = WT && pj->wt;
+      const long long ho = pj->hist_off;
       for (int i = tid; i < bn.ntoh; i += FK_NT) {
         const int g = fk_hslot(i, bn.ns, bn.nsh);    /* padding slots stay 0 */
         if (g < 0) continue;
         if (w) {
           double v = 0;
           for (int c = 0; c < a.nh; c++) { v += hist_d[c * bn.ntoh + i]; hist_d[c * bn.ntoh + i] = 0.0; }
-          if (v != 0) unsafeAtomicAdd(a.gcnt_d + J.hist_off + g, v);
+          if (v != 0) unsafeAtomicAdd(a.gcnt_d + ho + g, v);
         }
         else {
           unsigned long long v = 0;
           for (int c = 0; c < a.nh; c++) { v += hist_u[c * bn.ntoh + i]; hist_u[c * bn.ntoh + i] = 0u; }
-          if (v) atomicAdd(a.gcnt_u + J.hist_off + g, v);
+          if (v) atomicAdd(a.gcnt_u + ho + g, v);
         }
       }
     }
+    since = 0;
     __syncthreads();
+    return nx;
   };
 
-  for (;;) {
-    __syncthreads();
-    if (tid == 0) s_tile = (int) atomicAdd(a.queue, 1u);
-    __syncthreads();
-    const int tix = s_tile;
-    if (tix >= a.ntiles) break;
-    const FkTile t = a.tiles[tix];
-    if (t.job != cur) {
-      /* switch job: flush the histogram of the previous one, stage the new
-       * job descriptor in LDS */
-      if (!GRAD) flush();
-      __syncthreads();
-      {
-        const int *src = (const int *) (a.jobs + t.job);
-        int *dst = (int *) &sJ;
-        for (int i = tid; i < (int) (sizeof(FkJob) / sizeof(int)); i += FK_NT) dst[i] = src[i];
-      }
-      __syncthreads();
-      cur = t.job;
-      since_flush = 0;
+  /* the first item of a wavefront is its own index, the others follow from
+   * the queue */
+  const int nwaves = (int) gridDim.x * FK_NW;
+  int it = (int) blockIdx.x * FK_NW + wave;
+  for (bool first = true;; first = false) {
+    if (!first) {
+      if (lane == 0) it = nwaves + (int) atomicAdd(a.queue, 1u);
+      it = __builtin_amdgcn_readfirstlane(it);
     }
-    const int ix = t.row / J.g.ncy, iy = t.row - ix * J.g.ncy;
+    /* work item -> run and share of its strips */
+    int part = 0, S = 1;
+    FkRun t = {0, 0, 0, FK_END};
+    if (it < a.nitems) {
+      int ri;
+      const int h = a.sp.S * a.sp.tt;
+      if (it < h) { S = a.sp.S; ri = it / S; part = it - ri * S; }
+      else { S = a.sp.St; ri = (it - h) / S; part = it - h - ri * S; ri += a.sp.tt; }
+      const int grp = ri / a.sp.run;
+      t = fk_cld(a.runs + (grp * a.sp.G + (ri - grp * a.sp.run)));
+    }
+    while (t.job != cur) cur = job_round(t.job);
+    if (cur == FK_END) break;
+
+    const FkJob J = fk_cld(a.jobs + cur);
+    const int s0 = (int) ((long long) J.nstrips * part / S);
+    const int s1 = (int) ((long long) J.nstrips * (part + 1) / S);
     /* weights exist for this job (a weighted-capable kernel may run
      * unweighted jobs of a batch, whose catalogues carry no weights) */
     const bool jw = GRAD || (WT && J.wt);
+    const bool jwt = WT && J.wt;
+    const bool hasB = GRAD && J.gB != nullptr;
 
-    /* A objects of this lane; idle lanes sit far away, so that every pair
-     * they form is out of range */
+    /* A objects of this lane (a wavefront holds one run) and the bounding box
+     * of the run; idle lanes sit far away, so that every pair they form is
+     * out of range */
     double ax[R], ay[R], az[R], as[R], aw[R], gacc[R];
     float fax[R], fay[R], faz[R];
     int ai[R];
-    const double tcx = J.g.ox + (ix + 0.5) * J.g.wx;
-    const double tcy = J.g.oy + (iy + 0.5) * J.g.wy;
-    const double tcz = J.g.oz + 0.5 * (t.iz0 + t.iz1 + 1) * J.g.wz;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int p = t.p0 + tid * R + r;     /* a wavefront holds one run of 64 R objects */
-      const bool v = p < t.p1;
-      ai[r] = v ? p : 0x7fffffff;
-      ax[r] = v ? J.A.x[p] : FK_FAR;
-      ay[r] = v ? J.A.y[p] : FK_FAR;
-      az[r] = v ? J.A.z[p] : FK_FAR;
-      as[r] = NEED_S ? (v ? J.A.s[p] : 3.0 * FK_FAR * FK_FAR) : 0.0;
-      aw[r] = (jw && v) ? J.A.w[p] : 1.0;
-      gacc[r] = 0.0;
-      /* idle lanes: |a| = 1e18 and |dz| / s = 1 / (2 nmu), so that the mu
-       * estimate of their pairs is 1/2, clear of the windows */
-      fax[r] = v ? (float) (ax[r] - tcx) : J.win.idle_x;
-      fay[r] = v ? (float) (ay[r] - tcy) : 0.0f;
-      faz[r] = v ? (float) (az[r] - tcz) : J.win.idle_z;
-    }
-    /* survey FP32: m = a + b = 2 a' + d + 2 c (a' = a - c, c = tile centre).
-     * Idle lanes (a' = (10^6, 0, 0): s^2 and pi^2 far out of range) may
-     * look ambiguous in mu: their queue bits are masked off */
-    const float c2x = fk_uni((float) (2.0 * tcx)), c2y = fk_uni((float) (2.0 * tcy)),
-                c2z = fk_uni((float) (2.0 * tcz));
-    /* the FP32 windows of the job, in scalar registers for the pair loop */
-    const FkWin wn = F32 ? fk_uni(J.win) : J.win;
+    double lox = 1e300, loy = 1e300, loz = 1e300, hix = -1e300, hiy = -1e300, hiz = -1e300;
     unsigned long long actm[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) actm[r] = __builtin_amdgcn_ballot_w64(t.p0 + tid * R + r < t.p1);
-    const int nva = min(t.p1 - t.p0, R * FK_NT);
-    const bool jwt = WT && J.wt;
+    for (int r = 0; r < R; r++) {
+      const int p = t.p0 + r * 64 + lane;
+      const bool v = p < t.p1;
+      const int pc = v ? p : t.p0;
+      const double x = fk_gld(J.A.x, pc), y = fk_gld(J.A.y, pc), z = fk_gld(J.A.z, pc);
+      lox = __builtin_fmin(lox, x); hix = __builtin_fmax(hix, x);
+      loy = __builtin_fmin(loy, y); hiy = __builtin_fmax(hiy, y);
+      loz = __builtin_fmin(loz, z); hiz = __builtin_fmax(hiz, z);
+      ai[r] = v ? p : 0x7fffffff;
+      ax[r] = v ? x : FK_FAR;
+      ay[r] = v ? y : FK_FAR;
+      az[r] = v ? z : FK_FAR;
+      as[r] = NEED_S ? (v ? fk_gld(J.A.s, pc) : 3.0 * FK_FAR * FK_FAR) : 0.0;
+      aw[r] = (jw && v) ? fk_gld(J.A.w, pc) : 1.0;
+      gacc[r] = 0.0;
+      actm[r] = __builtin_amdgcn_ballot_w64(v);
+    }
+    lox = fk_wave_min(lox); hix = -fk_wave_min(-hix);
+    loy = fk_wave_min(loy); hiy = -fk_wave_min(-hiy);
+    loz = fk_wave_min(loz); hiz = -fk_wave_min(-hiz);
+    fk_wave_sync();
+    if (lane == 0) { box[0] = lox; box[1] = hix; box[2] = loy; box[3] = hiy; box[4] = loz; box[5] = hiz; }
+    fk_wave_sync();
+    /* FP32 coordinates are relative to the centre of the box */
+    const double tcx = 0.5 * (lox + hix), tcy = 0.5 * (loy + hiy), tcz = 0.5 * (loz + hiz);
+    /* idle lanes: |a| = 1e18 and |dz| / s = 1 / (2 nmu), so that the mu
+     * estimate of their pairs is 1/2, clear of the windows */
+    const FkWin wn = J.win;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const bool v = ai[r] != 0x7fffffff;
+      fax[r] = v ? (float) (ax[r] - tcx) : wn.idle_x;
+      fay[r] = v ? (float) (ay[r] - tcy) : 0.0f;
+      faz[r] = v ? (float) (az[r] - tcz) : wn.idle_z;
+    }
+    /* survey FP32: m = a + b = 2 a' + d + 2 c (a' = a - c, c = the centre).
+     * Idle lanes (a' = (10^6, 0, 0): s^2 and pi^2 far out of range) may
+     * look ambiguous in mu: their queue bits are masked off */
+    const float c2x = (float) (2.0 * tcx), c2y = (float) (2.0 * tcy), c2z = (float) (2.0 * tcz);
+    const int nva = t.p1 - t.p0;
 
-    /* FP32: FP64 re-evaluation of the n queued pairs of this wavefront
-     * (entries: A slot << 8 | chunk index), while the chunk is staged */
-    const int lane = tid & 63;
-    auto drain = [&](int n) {
-      for (int e0 = 0; e0 < n; e0 += 64) {
-        const unsigned v = (e0 + lane < n) ? (unsigned) wq[e0 + lane] : 0xFFFFu;
-        const int p = t.p0 + wave * 64 * R + (int) (v >> 8);
-        /* entries of idle lanes (possible only when the windows cover
-         * everything) are dropped */
-        if (e0 + lane < n && p < t.p1) {
-          const int j = (int) (v & 255u);
+    /* FP32: FP64 re-evaluation of the n queued pairs of this wavefront */
+    int qn = 0;
+    auto drain = [&]() __attribute__((always_inline)) {
+      fk_wave_sync();
+      const FkJob J = fk_cld(fk_again(a.jobs, cur));
+      for (int e0 = 0; e0 < qn; e0 += 64) {
+        if (e0 + lane < qn) {
+          const int jg = (int) wqj[e0 + lane];
+          const unsigned v = wqs[e0 + lane];
+          const int p = t.p0 + (int) (v >> 5);
           unsigned idx;
           if (GEOM == FCFC_GEOM_SURVEY)
-            idx = fk_recheck_sv<BIN, HYB>(bn, J, p, cj[j], stab, ptab, s2e, pe);
+            idx = fk_recheck_sv<BIN, HYB>(bn, J, p, jg, stab, ptab, s2e, pe);
           else
-            idx = fk_recheck<BIN, HYB, CENS>(bn, J, J.A.x[p], J.A.y[p], J.A.z[p], cj[j], cc[j],
-                                             stab, ptab, s2e, pe, &ncensus);
+            idx = fk_recheck<BIN, HYB, CENS>(bn, J, fk_gld(J.A.x, p), fk_gld(J.A.y, p),
+                                             fk_gld(J.A.z, p), jg, (int) (v & 31u), stab, ptab,
+                                             s2e, pe, &ncensus);
           nrecheck++;
           if (idx < ntot) {
-            if (WT && jwt) atomicAdd(myhist_d + idx, J.A.w[p] * cw[j]);
+            if (WT && jwt) atomicAdd(myhist_d + idx, fk_gld(J.A.w, p) * fk_gld(J.B.w, jg));
             else atomicAdd(myhist_u + idx, 1u);
           }
         }
       }
+      qn = 0;
+      fk_wave_sync();
     };
 
-    /* one staged chunk of cnt B objects against the lane's A objects */
-    auto run_chunk = [&](auto selfc, int cnt) {
+    /* staged B objects [j, cnt) of a chunk against the lane's A objects; FP32:
+     * only while the queue has room for one more (64 R pairs at most).
+     * Returns the next B object */
+    auto run_chunk = [&](auto selfc, int j, int cnt, int code) __attribute__((always_inline)) -> int {
       constexpr bool SELF = decltype(selfc)::value;
-      int qn = 0;                 /* queued pairs of this wavefront */
 #pragma unroll 2
-      for (int j = 0; j < cnt; j++) {
+      for (; j < cnt; j++) {
+        if (F32 && qn > FK_QCAP - 64 * R) break;
         double bx = 0, by = 0, bz = 0, bs = 0;
         float gx = 0, gy = 0, gz = 0;
         if (F32) { gx = fx[j]; gy = fy[j]; gz = fz[j]; }
         else { bx = cx[j]; by = cy[j]; bz = cz[j]; }
         if (NEED_S) bs = cs_[j];
         const double wj = NEED_W ? cw[j] : 1.0;
-        const int jj = (SELF || F32) ? cj[j] : 0;
+        const int jj = SELF ? cj[j] : 0;
         if (GEOM == FCFC_GEOM_BOX) {
-          /* the wavefront's A objects are one run of consecutive objects
-           * of one cell column: when this B object is out of range of all
-           * of them, skip the binning (same expressions as the pair
-           * functions, so the compiler shares them).  Every form skips, so
-           * the plain form differs from the FP64 one in the per-pair mu
-           * arithmetic only */
+          /* when this B object is out of range of every A object of the run,
+           * skip the binning (same expressions as the pair functions, so the
+           * compiler shares them).  Every form skips, so the plain form
+           * differs from the FP64 one in the per-pair mu arithmetic only */
           bool any = false;
 #pragma unroll
           for (int r = 0; r < R; r++) {
@@ -1282,22 +1329,22 @@ k_count(const FkArgs a) {
               const bool keep = jj > ai[r];
               amb = amb & keep; ambm = ambm & keep; idx = keep ? idx : FK_NONE;
             }
-            /* pairs near an edge: queue (A slot, chunk entry) for FP64.  The
-             * two conditions are balloted apart (each ballot is its compare's
+            /* pairs near an edge: queue (B object, A slot, image) for FP64.
+             * The conditions are balloted apart (each ballot is its compare's
              * own mask) and the lane's bit is read back from the mask inside
              * the rare branch, so no lane value is kept across it */
             if (SELF) ambx = ambx & (jj > ai[r]);
             unsigned long long m = __builtin_amdgcn_ballot_w64(amb) |
                 __builtin_amdgcn_ballot_w64(ambm) | __builtin_amdgcn_ballot_w64(ambx);
-            if (SV32) m &= actm[r];
-            if (m) {
+            m &= actm[r];
+            if (__builtin_expect(m != 0, 0)) {
               if ((m >> lane) & 1ull) {
                 const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
                                            __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-                wq[pos] = (uint16_t) (((unsigned) (lane * R + r) << 8) | (unsigned) j);
+                wqj[pos] = (unsigned) cj[j];
+                wqs[pos] = (uint16_t) (((unsigned) (r * 64 + lane) << 5) | (unsigned) code);
               }
               qn += __popcll(m);
-              if (qn > FK_QCAP - 64) { drain(qn); qn = 0; }
             }
             queued = amb | ambm | ambx;
           }
@@ -1319,121 +1366,138 @@ k_count(const FkArgs a) {
             else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
           }
         }
-        if (GRAD && J.gB) {
+        if (GRAD && hasB) {
           /* the B object's share over the wavefront's pairs: one sum per
            * row of 16 lanes, added into the chunk's LDS accumulator */
           const double v = fk_row_sum(bsum);
           if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
         }
       }
-      if (F32 && qn) drain(qn);
+      return j;
     };
 
-    /* GRAD: after a chunk, the B objects' shares go to the output */
-    auto grad_flush = [&](int cnt) {
-      if (!GRAD || !J.gB) return;
-      __syncthreads();
-      for (int q = tid; q < cnt; q += FK_NT) {
-        const double v = cb[q];
-        if (v != 0.0) unsafeAtomicAdd(J.gB + J.B.idx[cj[q]], v);
-      }
-    };
-
-    auto guard = [&](int cnt) {
-      if (GRAD || jwt) return;
-      since_flush += (double) cnt * nva;
-      if (since_flush > 2.0e9) { flush(); since_flush = 0; }
-    };
-
-    /* ---- auto counts: pairs inside the tile (j > i), first item only ---- */
-    if (J.autoc && t.s0 == 0) {
-      for (int c0 = t.p0; c0 < t.p1; c0 += FK_CH) {
-        const int cnt = min(FK_CH, t.p1 - c0);
-        __syncthreads();
-        for (int q = tid; q < cnt; q += FK_NT) {
-          const int jg = c0 + q;
-          const double x = J.A.x[jg], y = J.A.y[jg], z = J.A.z[jg];
-          if (F32) { fx[q] = (float) (x - tcx); fy[q] = (float) (y - tcy); fz[q] = (float) (z - tcz); cc[q] = 13; }
-          else { cx[q] = x; cy[q] = y; cz[q] = z; }
-          if (NEED_S) cs_[q] = J.A.s[jg];
-          if (NEED_W) cw[q] = jw ? J.A.w[jg] : 1.0;
-          if (GRAD) cb[q] = 0.0;
-          cj[q] = jg;
+    /* B objects [b0, b0 + n) of the other catalogue (SELF: of the run itself),
+     * at the periodic image of code */
+    auto segment = [&](auto selfc, int b0, int n, int code) {
+      constexpr bool SELF = decltype(selfc)::value;
+      for (int c0 = 0; c0 < n; c0 += FK_CH) {
+        const FkJob *pj = fk_again(a.jobs, cur);
+        const FkCat B = fk_cld(SELF ? &pj->A : &pj->B);
+        const FkGrid g = fk_cld(&pj->g);
+        const bool in = c0 + lane < n;
+        const int jg = b0 + (in ? c0 + lane : 0);
+        double x = fk_gld(B.x, jg), y = fk_gld(B.y, jg), z = fk_gld(B.z, jg);
+        if (GEOM == FCFC_GEOM_BOX && code != 13) {
+          x = x + (double) (code % 3 - 1) * g.Lx;
+          y = y + (double) ((code / 3) % 3 - 1) * g.Ly;
+          z = z + (double) (code / 9 - 1) * g.Lz;
         }
-        __syncthreads();
-        run_chunk(std::integral_constant<bool, true>(), cnt);
-        grad_flush(cnt);
-        evals += (double) cnt * nva * 0.5;
-        guard(cnt);
-      }
-    }
-
-    /* ---- strips in batches of one wavefront ---- */
-    for (int sb0 = t.s0; sb0 < t.s1; sb0 += FK_NSB) {
-      __syncthreads();
-      if (wave == 0) {
-        const int l = tid;
-        int tot = 0;
-        int b0[3], len[3], code[3];
-        if (sb0 + l < t.s1) {
-          const int *sp = J.strips + 3 * (sb0 + l);
-          fk_strip_segments(J, t, sp[0], sp[1], sp[2], b0, len, code);
-          tot = len[0] + len[1] + len[2];
+        /* drop the objects beyond the maximum separation from the run's
+         * bounding box (the grid's padded ranges) */
+        bool keep = in;
+        const double lx = box[0], hx = box[1], ly = box[2], hy = box[3], lz = box[4], hz = box[5];
+        if (!SELF) {
+          const double ex = __builtin_fmax(__builtin_fmax(lx - x, x - hx), 0.0);
+          const double ey = __builtin_fmax(__builtin_fmax(ly - y, y - hy), 0.0);
+          const double ez = __builtin_fmax(__builtin_fmax(lz - z, z - hz), 0.0);
+          const double exy = __builtin_fma(ey, ey, ex * ex);
+          if (g.hz_const >= 0) keep &= (exy < g.Rxy2) & (ez < g.hz_const);
+          else keep &= __builtin_fma(ez, ez, exy) < g.R2;
         }
-        else { b0[0] = b0[1] = b0[2] = 0; len[0] = len[1] = len[2] = 0; code[0] = code[1] = code[2] = 13; }
-        for (int k = 0; k < 3; k++) { st->b0[3 * l + k] = b0[k]; st->len[3 * l + k] = len[k]; st->code[3 * l + k] = code[k]; }
-        int inc = tot;
-        for (int o = 1; o < 64; o <<= 1) {
-          int v = __shfl_up(inc, o, 64);
-          if (l >= o) inc += v;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+        evals += (unsigned long long) ((unsigned) min(FK_CH, n - c0) * (unsigned) nva);
+        if (m == 0) continue;
+        const int cnt = __popcll(m);
+        if (!GRAD && !jwt) {
+          if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) (void) job_round(cur);
+          since += (unsigned) cnt * (unsigned) nva;
         }
-        st->off[l] = inc - tot;
-        if (l == 63) st->off[64] = inc;
-      }
-      __syncthreads();
-      const int total = st->off[FK_NSB];
-      for (int c0 = 0; c0 < total; c0 += FK_CH) {
-        const int cnt = min(FK_CH, total - c0);
-        if (c0 > 0) __syncthreads();
-        for (int q = tid; q < cnt; q += FK_NT) {
-          const int pos = c0 + q;
-          int lo = 0, hi = FK_NSB;          /* off[lo] <= pos < off[hi] */
-          while (hi - lo > 1) { int mid = (lo + hi) >> 1; if (st->off[mid] <= pos) lo = mid; else hi = mid; }
-          int rem = pos - st->off[lo];
-          int sgi = 3 * lo;
-          if (rem >= st->len[sgi]) { rem -= st->len[sgi]; sgi++; if (rem >= st->len[sgi]) { rem -= st->len[sgi]; sgi++; } }
-          const int jg = st->b0[sgi] + rem;
-          const int code = st->code[sgi];
-          double x = J.B.x[jg], y = J.B.y[jg], z = J.B.z[jg];
-          if (GEOM == FCFC_GEOM_BOX && code != 13) {
-            x = x + (double) (code % 3 - 1) * J.g.Lx;
-            y = y + (double) ((code / 3) % 3 - 1) * J.g.Ly;
-            z = z + (double) (code / 9 - 1) * J.g.Lz;
+        fk_wave_sync();
+        if (keep) {
+          const int q = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                    __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+          if (F32) {
+            fx[q] = (float) (x - 0.5 * (lx + hx));
+            fy[q] = (float) (y - 0.5 * (ly + hy));
+            fz[q] = (float) (z - 0.5 * (lz + hz));
           }
-          if (F32) { fx[q] = (float) (x - tcx); fy[q] = (float) (y - tcy); fz[q] = (float) (z - tcz); cc[q] = code; }
           else { cx[q] = x; cy[q] = y; cz[q] = z; }
-          if (NEED_S) cs_[q] = J.B.s[jg];
-          if (NEED_W) cw[q] = jw ? J.B.w[jg] : 1.0;
+          if (NEED_S) cs_[q] = fk_gld(B.s, jg);
+          if (NEED_W) cw[q] = jw ? fk_gld(B.w, jg) : 1.0;
           if (GRAD) cb[q] = 0.0;
           cj[q] = jg;
         }
-        __syncthreads();
-        run_chunk(std::integral_constant<bool, false>(), cnt);
-        grad_flush(cnt);
-        evals += (double) cnt * nva;
-        guard(cnt);
+        fk_wave_sync();
+        for (int j = 0;;) {
+          j = run_chunk(selfc, j, cnt, code);
+          if (F32 && qn > FK_QCAP - 64 * R) drain();
+          if (j >= cnt) break;
+        }
+        /* GRAD: the B objects' shares go to the output */
+        if (GRAD && hasB) {
+          fk_wave_sync();
+          if (lane < cnt) {
+            const FkJob *pk = fk_again(a.jobs, cur);
+            const double v = cb[lane];
+            if (v != 0.0)
+              unsafeAtomicAdd(fk_cld(&pk->gB) + fk_gld(fk_cld(SELF ? &pk->A.idx : &pk->B.idx), cj[lane]), v);
+          }
+        }
       }
+    };
+
+    /* ---- auto counts: pairs inside the run (j > i), first item only ---- */
+    if (J.autoc && part == 0) {
+      evals -= (unsigned long long) nva * (unsigned) nva / 2;
+      segment(std::integral_constant<bool, true>(), t.p0, nva, 13);
     }
 
-    if (GRAD && J.gA) {
+    /* ---- strips, one per lane at a time ---- */
+    for (int sb0 = s0; sb0 < s1; sb0 += 64) {
+      int b0[FK_MAXSEG], len[FK_MAXSEG], code[FK_MAXSEG];
+      {
+        const int l = min(sb0 + lane, s1 - 1);
+        const FkJob *pj = fk_again(a.jobs, cur);
+        const int *sp = fk_cld(&pj->strips);
+        fk_strip_segments(fk_cld(&pj->g), fk_cld(&pj->B.cell_start), t, box[4], box[5],
+                          fk_gld(sp, 3 * l), fk_gld(sp, 3 * l + 1), fk_gld(sp, 3 * l + 2), b0, len, code);
+        if (sb0 + lane >= s1) len[0] = len[1] = len[2] = 0;
+      }
+      unsigned long long m0 = __builtin_amdgcn_ballot_w64(len[0] > 0),
+                         m1 = __builtin_amdgcn_ballot_w64(len[1] > 0),
+                         m2 = __builtin_amdgcn_ballot_w64(len[2] > 0);
+      while (m0 | m1 | m2) {
+        int b, n, cd, q;
+        if (m1) {
+          q = __builtin_ctzll(m1); m1 &= m1 - 1;
+          b = fk_lane_of(b0[1], q); n = fk_lane_of(len[1], q); cd = fk_lane_of(code[1], q);
+        }
+        else if (m0) {
+          q = __builtin_ctzll(m0); m0 &= m0 - 1;
+          b = fk_lane_of(b0[0], q); n = fk_lane_of(len[0], q); cd = fk_lane_of(code[0], q);
+        }
+        else {
+          q = __builtin_ctzll(m2); m2 &= m2 - 1;
+          b = fk_lane_of(b0[2], q); n = fk_lane_of(len[2], q); cd = fk_lane_of(code[2], q);
+        }
+        segment(std::integral_constant<bool, false>(), b, n, cd);
+      }
+    }
+    if (F32 && qn) drain();
+
+    if (GRAD) {
+      const FkJob *pj = fk_again(a.jobs, cur);
+      double *gA = fk_cld(&pj->gA);
+      const int *idx = fk_cld(&pj->A.idx);
+      if (gA)
 #pragma unroll
-      for (int r = 0; r < R; r++)
-        if (ai[r] != 0x7fffffff && gacc[r] != 0.0) unsafeAtomicAdd(J.gA + J.A.idx[ai[r]], gacc[r]);
+        for (int r = 0; r < R; r++)
+          if (ai[r] != 0x7fffffff && gacc[r] != 0.0)
+            unsafeAtomicAdd(gA + fk_gld(idx, ai[r]), gacc[r]);
     }
   }
 
-  if (!GRAD) flush();
-  if (tid == 0) atomicAdd(a.stats + 0, (unsigned long long) evals);
+  if (lane == 0) atomicAdd(a.stats + 0, evals);
   if (F32) {
     if (nrecheck) atomicAdd(a.stats + 1, (unsigned long long) nrecheck);
     if (ncensus) atomicAdd(a.stats + 2, (unsigned long long) ncensus);
@@ -1602,8 +1666,9 @@ extern "C" int fcfc_gpu_set_tuning(fcfc_gpu_ctx *c, int cell_div, int tile,
 struct JobPlan {
   int bucket;       /* density bucket for the autotuner cache */
   FkGrid g;
-  int T;            /* objects per tile */
-  int zmaxc;        /* max z-cells per tile */
+  int T;            /* objects per tile (the FK_NW runs of a workgroup) */
+  int zmaxc;        /* z-cells per block of a row: no run crosses blocks */
+  int nblk;         /* blocks per row */
   int R;            /* objects per lane */
   int T_auto;       /* T chosen by the plan (not by the caller's tuning) */
   std::vector<int> strips;
@@ -1675,14 +1740,19 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
       }
   }
   P->bucket = bucket;
-  if (cd <= 0) {
-    /* three cells per maximum separation (measured best for dense boxes);
-     * fewer for sparse catalogues, so that columns keep enough objects */
-    double objs_per_col = nden * Rxy * Rxy;   /* per unit z, for cd = 1 */
-    cd = 3;
-    while (cd > 1 && objs_per_col / (cd * cd) < 4.0) cd--;
-  }
-  if (zd <= 0) zd = 8;
+  /* Runs as compact as their object number allows: the objects of B within
+   * the maximum separation of a run's bounding box are evaluated, and a cube
+   * has the least of them.  The side of the cube that holds 128 objects of A
+   * is the cell width in x and y (rounded to cells per separation, one at
+   * least: thinner columns of a sparse catalogue would only lengthen its
+   * runs), four z-cells per width.  Measured (kernel ms at cd = 2, 3, 4, 6,
+   * 8): (s, mu) RR of 4e6 objects in the unit box 296, 245, 232, 231, 230
+   * (rule: 6); weighted DD of 5e5 9.1, 8.7, 8.9, 10.1, 12 (3); iso DD of
+   * 1e5 0.36, 0.36, 0.55, 0.82, 1.2 (2); survey (s, mu) RR of 1.2e6 16.6,
+   * 15.5, 16.4, 19.9, 25 (3). */
+  const double cube = cbrt(128.0 / std::max(ndenA, 1e-300));
+  if (cd <= 0) cd = (int) std::min(std::max(floor(Rxy / cube + 0.6), 1.0), 12.0);
+  if (zd <= 0) zd = 4;
   /* cells of Rxy / cd, but never more cells than about 4 per object
    * (between 2^18 and 2^25): a sparse catalogue in a large volume gets
    * larger cells instead of a grid of mostly empty ones */
@@ -1715,9 +1785,6 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
     g.ncz = std::max(1, (int) floor(ext[2] / wzt));
     g.wz = ext[2] / g.ncz;
     g.ox = g.oy = g.oz = 0;
-    P->zmaxc = (int) floor(zroom / g.wz) - 4;
-    if (P->zmaxc < 1) P->zmaxc = 1;
-    P->zmaxc = std::min(P->zmaxc, std::max(1, (int) ceil(2 * zd * 1.0)));
   }
   else {
     g.periodic = 0;
@@ -1727,23 +1794,28 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
     g.wz = w / zd;
     g.ncz = std::max(1, (int) ceil(ext[2] / g.wz) + 1);
     g.ox = lo[0]; g.oy = lo[1]; g.oz = lo[2];
-    P->zmaxc = std::max(1, 2 * zd);
     if ((double) g.ncx * g.ncy * g.ncz > 2.0e8) {
       set_err(c, "grid too large (%d x %d x %d cells)", g.ncx, g.ncy, g.ncz);
       return FCFC_ERR_CFG;
     }
   }
-  /* objects per tile: two per lane when the rows are long enough to fill
-   * such tiles, one per lane otherwise (and always for the gradient) */
+  /* Objects per tile: two per lane, which halves the B objects read from LDS
+   * per pair, unless a run of 128 objects is about as wide as the separations
+   * it is counted to (sparse catalogues): then 64, whose boxes reach fewer B
+   * objects (w_p of 1e6 objects to 40 Mpc/h: 3.0 against 3.9 ms; iso DD of
+   * 1e5 to 200 Mpc/h, whose cube is half the separation: 0.39 against 0.36). */
   P->T_auto = (tT <= 0);
   if (tT > 0) P->T = std::min(tT, 4 * FK_NT);
-  else {
-    /* two objects per lane only when the z extent allowed to a tile holds
-     * enough objects to fill such tiles (idle lanes cost full issue slots) */
-    const double per_window = (double) nA / ((double) g.ncx * g.ncy) * P->zmaxc / g.ncz;
-    P->T = (per_window >= 2.5 * FK_NT) ? 2 * FK_NT : FK_NT;
-  }
+  else P->T = cube > 0.75 * R ? FK_NT : 2 * FK_NT;
   P->R = (P->T + FK_NT - 1) / FK_NT;
+  /* blocks of about four runs, at least two cells wide: the z extent of a
+   * run (and with it the FP32 windows) stays bounded in sparse rows */
+  {
+    const double per_cell = (double) nA / ((double) g.ncx * g.ncy * g.ncz);
+    const double zc = std::max(2.0 * zd, ceil(4.0 * 64 * P->R / std::max(per_cell, 1e-9)));
+    P->zmaxc = (int) std::min((double) g.ncz, zc);
+    P->nblk = (g.ncz + P->zmaxc - 1) / P->zmaxc;
+  }
   /* strips */
   P->strips.clear();
   const int kx = (int) ceil(Rxy / g.wx), ky = (int) ceil(Rxy / g.wy);
@@ -1996,7 +2068,7 @@ static int hist_slots(const fcfc_bins *b) {
   return hist_stride(b) * (b->ntot / b->ns);
 }
 
-struct LdsPlan { int off_hist, off_stab, off_ptab, off_edges, off_strip, off_chunk, off_queue, total, nh, stab_c0, ptab_c0; };
+struct LdsPlan { int off_hist, off_stab, off_ptab, off_edges, off_chunk, off_queue, total, nh, stab_c0, ptab_c0; };
 
 static int align16(int v) { return (v + 15) & ~15; }
 
@@ -2023,18 +2095,11 @@ static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh
   o = align16(o);
   L.off_edges = o;
   if (hyb) o = align16(o + 8 * (b->ns + 1 + (b->bintype == FCFC_BIN_SPI ? b->np + 1 : 0)));
-  L.off_strip = o; o = align16(o + (int) sizeof(FkStripLds));
   L.off_chunk = o;
-  /* per staged B object: coordinates, |r|^2 (survey), weight, index, image code */
-  int per = (mode == MODE_C32) ? 12 : 24;
-  if (need_s && mode != MODE_C32) per += 8;
-  if (wt || mode == MODE_GRAD) per += 8;
-  if (mode == MODE_GRAD) per += 8;             /* gradient share of each B object */
-  per += 4;
-  if (mode == MODE_C32) per += 4;
-  o = align16(o + FK_CH * per);
+  const bool f32 = (mode == MODE_C32), grad = (mode == MODE_GRAD);
+  o = align16(o + FK_NW * FK_CH * fk_chunk_bytes(f32, need_s && !f32, wt || grad, grad));
   L.off_queue = o;
-  if (mode == MODE_C32) o += (FK_NT / 64) * FK_QCAP * 2;
+  if (f32) o += FK_NW * FK_QCAP * 6;
   o = align16(o);
   const int zero_based = (!hyb || mode == MODE_C32);
   L.stab_c0 = zero_based ? b->soff : 1;
@@ -2053,14 +2118,15 @@ typedef void (*kfn_t)(const FkArgs);
 
 /* Kernel variants: binning x geometry x weights x mode x table type x A
  * objects per lane (R = 1: tiles of FK_NT objects, R = 2: 2 FK_NT, R = 4:
- * 4 FK_NT).  Hybrid tables use one R (2; the gradient 1); R = 4 exists for
+ * 4 FK_NT).  The gradient with hybrid tables uses R = 1; R = 4 exists for
  * the weighted FP64 box counts with integer tables only, whose LDS-bound
  * histogram updates gain from reading each staged B object for more A
  * objects (fk_lanes_max gives the largest R of a kernel family).  The
  * survey kernels hold four more FP64 values per object and spill at R = 4
  * (weighted (s_perp, pi) DR: 950 ms against 830 at R = 2). */
 static int fk_lanes_max(int geom, int mode, int wt, int hyb) {
-  if (hyb) return mode == MODE_GRAD ? 1 : 2;
+  if (hyb && mode == MODE_GRAD) return 1;
+  if (hyb) return 2;
   return (wt && mode == MODE_C64 && geom == FCFC_GEOM_BOX) ? 4 : 2;
 }
 
@@ -2071,7 +2137,7 @@ static kfn_t pick5(int hyb, int R) {
     return R == 1 ? k_count<BIN, GEOM, WT, MODE, false, 1> : k_count<BIN, GEOM, WT, MODE, false, 2>;
   }
   else {
-    if (hyb) return k_count<BIN, GEOM, WT, MODE, true, 2>;
+    if (hyb) return R == 1 ? k_count<BIN, GEOM, WT, MODE, true, 1> : k_count<BIN, GEOM, WT, MODE, true, 2>;
     if constexpr (WT && MODE == MODE_C64 && GEOM == FCFC_GEOM_BOX)
       if (R == 4) return k_count<BIN, GEOM, WT, MODE, false, 4>;
     return R == 1 ? k_count<BIN, GEOM, WT, MODE, false, 1> : k_count<BIN, GEOM, WT, MODE, false, 2>;
@@ -2324,13 +2390,13 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
  * depend on how the runtime stages pageable host memory. */
 struct Launch {
   kfn_t fn = nullptr;
-  int nblock = 0, lds = 0, ntiles = 0;
+  int nblock = 0, lds = 0, nitems = 0;
   FkArgs a;
   std::vector<int> hstr;
   std::vector<FkJob> hj;
 };
 
-/* Tile all jobs and prepare the persistent launch that counts (or
+/* List the runs of all jobs and prepare the persistent launch that counts (or
  * differentiates) them; every buffer comes from al. */
 static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     std::vector<PJob> &jobs, int mode, const double *G, void *dhist,
@@ -2413,64 +2479,66 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     }
   }
   HIPCHK(c, hipFuncSetAttribute((const void *) fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.total));
-  /* ---- tiles of all jobs ---- */
-  std::vector<int> rowoff(jobs.size() + 1, 0);
-  for (size_t k = 0; k < jobs.size(); k++) rowoff[k + 1] = rowoff[k] + jobs[k].P.g.ncx * jobs[k].P.g.ncy;
-  const int nrow = rowoff.back();
-  int *rown = (int *) al.get(WS_ROWN, sizeof(int) * (size_t) nrow);
-  int *rowscan = (int *) al.get(WS_ROWOFF, sizeof(int) * ((size_t) nrow + 1));
-  FkTileJob *dtj = (FkTileJob *) al.get(WS_TJOBS, sizeof(FkTileJob) * jobs.size());
-  if (al.err) return al.err;
+  /* ---- runs of all jobs ---- */
   std::vector<FkTileJob> htj(jobs.size());
+  long long nunit_l = 0;
   for (size_t k = 0; k < jobs.size(); k++) {
     const PJob &J = jobs[k];
-    htj[k] = FkTileJob{rowoff[k], J.P.g.ncz, J.P.T, J.P.zmaxc, J.P.nstrips, J.A.cs};
+    htj[k] = FkTileJob{(int) nunit_l, J.P.nblk, J.P.zmaxc, J.P.g.ncz, std::min(J.P.T, 64 * J.P.R), J.A.cs};
+    nunit_l += (long long) J.P.g.ncx * J.P.g.ncy * J.P.nblk;
+    if (nunit_l > INT_MAX / 2) { set_err(c, "catalogues of one call too large"); return FCFC_ERR_CFG; }
   }
+  const int nunit = (int) nunit_l;
+  int *unitn = (int *) al.get(WS_ROWN, sizeof(int) * (size_t) nunit);
+  int *unitoff = (int *) al.get(WS_ROWOFF, sizeof(int) * ((size_t) nunit + 1));
+  FkTileJob *dtj = (FkTileJob *) al.get(WS_TJOBS, sizeof(FkTileJob) * jobs.size());
+  if (al.err) return al.err;
   HIPCHK(c, hipMemcpyAsync(dtj, htj.data(), sizeof(FkTileJob) * jobs.size(), hipMemcpyHostToDevice, c->stream));
   const int njob = (int) jobs.size();
-  if (nrow > 0)
-    hipLaunchKernelGGL(k_tile_count, dim3(nblk(nrow, 64)), dim3(64), 0, c->stream, nrow, njob, dtj, rown);
-  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, rown, rowscan, nrow);
-  int ntile0 = 0;
-  HIPCHK(c, hipMemcpyAsync(&ntile0, rowscan + nrow, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  if (nunit > 0)
+    hipLaunchKernelGGL(k_run_count, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj, unitn);
+  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, unitn, unitoff, nunit);
+  int nrun = 0;
+  HIPCHK(c, hipMemcpyAsync(&nrun, unitoff + nunit, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  /* persistent workgroups, and work items per tile: enough items that the
-   * last ones are short against the whole (16 per workgroup) */
+  /* persistent workgroups, and work items per run: enough items that the
+   * last ones are short against the whole (16 per wavefront) */
   int occ = 0;
   HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *) fn, FK_NT, L.total));
   if (occ < 1) occ = 1;
   const int nwg = c->t_nblock > 0 ? c->t_nblock : occ * c->ncu;
-  /* the autotuner's samples count about 1/tile_frac of the tiles, in 16
-   * runs of consecutive tiles spread evenly over the list, split into work
-   * items by the same rule as a full count (about 16 per workgroup), so
+  const long long nwave = (long long) nwg * FK_NW;
+  /* the autotuner's samples count about 1/tile_frac of the runs, in 16
+   * stretches of consecutive runs spread evenly over the list, split into
+   * work items by the same rule as a full count (about 16 per wavefront), so
    * that a sample ends as evenly */
-  int grp = std::max(ntile0, 1), run = grp;
-  if (c->tile_frac > 1 && ntile0 > 0) {
-    grp = (ntile0 + 15) / 16;
+  int grp = std::max(nrun, 1), run = grp;
+  if (c->tile_frac > 1 && nrun > 0) {
+    grp = (nrun + 15) / 16;
     run = std::max(1, grp / c->tile_frac);
   }
-  const int glast = ntile0 > 0 ? (ntile0 - 1) / grp : 0;
-  const int ncap = ntile0 > 0 ? glast * run + std::min(run, ntile0 - glast * grp) : 0;
+  const int glast = nrun > 0 ? (nrun - 1) / grp : 0;
+  const int ncap = nrun > 0 ? glast * run + std::min(run, nrun - glast * grp) : 0;
   FkSplit sp{1, ncap, 1, ncap, grp, run};
-  if (ntile0 > 0) {
+  if (nrun > 0) {
     int minstr = 1 << 30;
     for (auto &j : jobs) minstr = std::min(minstr, std::max(j.P.nstrips, 1));
     const int smax = std::min(minstr, 64);
-    sp.S = (int) std::min<long long>(std::max<long long>(1, (16LL * nwg + ncap - 1) / ncap),
+    sp.S = (int) std::min<long long>(std::max<long long>(1, (16LL * nwave + ncap - 1) / ncap),
                                      smax);
-    /* the tiles of about two items per workgroup at the end of the list
+    /* the runs of about two items per wavefront at the end of the list
      * are split four times finer */
     sp.St = std::min(4 * sp.S, smax);
-    sp.tt = (int) std::max<long long>(0, ncap - (2LL * nwg + sp.S - 1) / sp.S);
+    sp.tt = (int) std::max<long long>(0, ncap - (2LL * nwave + sp.S - 1) / sp.S);
     if (sp.St <= sp.S) { sp.St = sp.S; sp.tt = ncap; }
     if (split_pos(sp, ncap) > (1LL << 30)) sp = FkSplit{1, ncap, 1, ncap, grp, run};
   }
-  const int ntiles = (int) split_pos(sp, ncap);
-  FkTile *tiles = (FkTile *) al.get(WS_TILES, sizeof(FkTile) * (size_t) (ntiles > 0 ? ntiles : 1));
+  const int nitems = (int) split_pos(sp, ncap);
+  FkRun *runs = (FkRun *) al.get(WS_TILES, sizeof(FkRun) * (size_t) (nrun > 0 ? nrun : 1));
   if (al.err) return al.err;
-  if (nrow > 0)
-    hipLaunchKernelGGL(k_tile_emit, dim3(nblk(nrow, 64)), dim3(64), 0, c->stream, nrow, njob, dtj,
-                       rowscan, sp, tiles);
+  if (nunit > 0)
+    hipLaunchKernelGGL(k_run_emit, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj,
+                       unitoff, runs);
   /* ---- tables, strips, job descriptors ---- */
   size_t nstr = 0;
   for (auto &j : jobs) nstr += j.P.strips.size();
@@ -2582,24 +2650,24 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     fb.q_pad = 0;
   }
   fb.stab = dstab; fb.ptab = dptab; fb.s2bin = ds2e; fb.pbin = dpe;
-  a.tiles = tiles; a.ntiles = ntiles;
+  a.runs = runs; a.sp = sp; a.nitems = nitems;
   a.queue = dqueue;
   a.gcnt_u = (unsigned long long *) dhist; a.gcnt_d = (double *) dhist;
   a.stats = dstats;
   a.nh = L.nh;
   a.off_hist = L.off_hist; a.off_stab = L.off_stab; a.off_ptab = L.off_ptab;
   a.stab_c0 = L.stab_c0; a.ptab_c0 = L.ptab_c0;
-  a.off_edges = L.off_edges; a.off_strip = L.off_strip;
+  a.off_edges = L.off_edges;
   a.off_chunk = L.off_chunk; a.off_queue = L.off_queue;
   a.census = c->census;
   a.G = G;
   int nblock = nwg;
-  if (nblock > a.ntiles) nblock = std::max(a.ntiles, 1);
-  c->last_ntiles = ntile0;
+  if (nblock > (nitems + FK_NW - 1) / FK_NW) nblock = std::max((nitems + FK_NW - 1) / FK_NW, 1);
+  c->last_ntiles = nrun;
   c->last_nsampled = ncap;
   c->stats.tile = jobs.empty() ? 0 : jobs[0].P.T;
   c->stats.cell_div = jobs.empty() ? 0 : (int) lround(sqrt(jobs[0].P.g.Rxy2) / jobs[0].P.g.wx);
-  out->fn = fn; out->nblock = nblock; out->lds = L.total; out->ntiles = a.ntiles; out->a = a;
+  out->fn = fn; out->nblock = nblock; out->lds = L.total; out->nitems = a.nitems; out->a = a;
   return 0;
 }
 
@@ -2612,13 +2680,13 @@ struct StreamDrain {
 };
 
 static int launch(fcfc_gpu_ctx *c, const Launch &Lc) {
-  if (Lc.ntiles > 0)
+  if (Lc.nitems > 0)
     hipLaunchKernelGGL(Lc.fn, dim3(Lc.nblock), dim3(FK_NT), Lc.lds, c->stream, Lc.a);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
 
-/* Tile all jobs, then count (or differentiate) them in one persistent launch. */
+/* List the runs of all jobs, then count (or differentiate) them in one launch. */
 static int run_jobs(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     std::vector<PJob> &jobs, int mode, const double *G, void *dhist,
     unsigned long long *dstats, unsigned int *dqueue, float *kms) {
@@ -3030,7 +3098,7 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
     const int nt = c->last_ntiles;
     /* small counts (a few thousand tiles, milliseconds) are timed whole: an
      * eighth of them is too few tiles to rank shapes */
-    c->tile_frac = (nt <= 4096) ? 1 : (nt > 16384 ? 16 : 8);
+    c->tile_frac = (nt <= 4096 * FK_NW) ? 1 : (nt > 16384 * FK_NW ? 16 : 8);
     e = run();
     if (e) return e;
     *est = c->stats.kernel_ms * (double) nt / (double) std::max(1, c->last_nsampled);

@@ -9,12 +9,15 @@
  * A "row" is the set of cells sharing (ix, iy): its objects are contiguous and
  * ordered by z-cell, so every z-window of a row is one contiguous range.
  *
- * Work unit: an A tile = up to NT*R consecutive objects of one row whose
- * z-cells span a bounded range.  For each xy offset (a "strip") the B objects
- * that can be within the maximum separation form at most three contiguous
- * segments (three periodic images in z).  A persistent workgroup takes tiles
- * from a global queue, packs the segments of a batch of strips into LDS
- * chunks, and every lane evaluates its A objects against each staged B object.
+ * Work unit: a run = up to 64 R consecutive A objects of one row (R per lane
+ * of one wavefront) inside a bounded z range, against a share of the strips.
+ * For each xy offset (a "strip") the B objects that can be within the maximum
+ * separation form at most three contiguous segments (three periodic images in
+ * z).  Every wavefront of the persistent workgroups takes its own runs from a
+ * global queue: its lanes load 64 B objects, drop those farther than the
+ * maximum separation from the bounding box of the run, pack the others into
+ * the wavefront's LDS chunk, and every lane evaluates its A objects against
+ * each packed B object.  The histograms are shared by the workgroup.
  *
  * Arithmetic contract (FP64 path), after FCFC's AVX-512 leaf kernels
  * (src/fcfc/2pt_box/metric_common.c:377-534):  B objects are staged as
@@ -31,11 +34,11 @@
 #include <stdint.h>
 
 #define FK_NT        512       /* threads per workgroup (8 wave64)          */
-#define FK_NSB       64        /* strips per batch = one wavefront          */
+#define FK_NW        8         /* wavefronts per workgroup                  */
 #define FK_MAXSEG    3         /* z images per strip                        */
-#define FK_CH        256       /* B objects per LDS chunk                   */
+#define FK_CH        64        /* B objects per wavefront's LDS chunk       */
 #define FK_OUT       0xFFFFu   /* table sentinel: outside [s2min, s2max)    */
-#define FK_QCAP      128       /* FP32 re-evaluation queue per wavefront    */
+#define FK_QCAP      160       /* FP32 re-evaluation queue per wavefront    */
 
 /* Binning constants passed by value to the kernels. */
 struct FkBins {
@@ -90,12 +93,11 @@ struct FkCat {
   const int *cell_start;
 };
 
-/* A work item: the A objects [p0, p1) of one row (z-cells iz0..iz1) against
- * the strips [s0, s1) of its job; a tile with many strips is split into
- * several items so that the queue stays long (items of one tile add into
- * the same histogram; only the item with s0 == 0 counts the pairs inside
- * the tile). */
-struct FkTile { int row, p0, p1, iz0, iz1, job, s0, s1; };
+/* A run: the A objects [p0, p1) of one row, counted against the strips of
+ * its job.  A work item is a run with a share of the strip list, so that the
+ * queue stays long (items of one run add into the same histograms; only the
+ * item of the first share counts the pairs inside the run). */
+struct FkRun { int row, p0, p1, job; };
 
 /* Floor of the exact quotient a / b for a >= 0, b > 0 (b not tiny):
  * approximate quotient from the hardware reciprocal, then one-step
