@@ -47,9 +47,10 @@ __global__ void k_zero_u64(unsigned long long *p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
 }
 
-/* Exclusive scan of n ints into out[0..n] (out[n] = total), one workgroup
- * of 1024 threads, each scanning a contiguous slice. */
-__global__ void __launch_bounds__(1024) k_scan1(const int *__restrict__ in,
+/* Exclusive scan of n ints into out[0..n] (out[n] = total) and in place into
+ * in[0..n-1], one workgroup of 1024 threads, each scanning a contiguous
+ * slice. */
+__global__ void __launch_bounds__(1024) k_scan1(int *__restrict__ in,
     int *__restrict__ out, int n) {
   __shared__ int part[1024];
   const int t = threadIdx.x;
@@ -66,7 +67,7 @@ __global__ void __launch_bounds__(1024) k_scan1(const int *__restrict__ in,
     __syncthreads();
   }
   int run = part[t] - s;
-  for (int i = b; i < e; i++) { int v = in[i]; out[i] = run; run += v; }
+  for (int i = b; i < e; i++) { int v = in[i]; out[i] = run; in[i] = run; run += v; }
   if (t == 1023) out[n] = part[1023];
 }
 
@@ -74,13 +75,15 @@ __global__ void __launch_bounds__(1024) k_scan1(const int *__restrict__ in,
  * in one pass per stage (cell counting sort), so that a batch of hundreds
  * of small catalogues costs a handful of launches ---- */
 struct FkStage {
-  int n, obj0, cell0, cs0;    /* objects; offsets in the concatenated object,
-                                 count and cell-start index spaces */
+  int n, obj0, cell0;         /* objects; offsets in the concatenated object
+                                 and cell spaces */
   int need_s;                 /* survey |r|^2 wanted (computed when s is null) */
   FkGrid g;
   const double *x, *y, *z, *s, *w;      /* inputs; s, w may be null */
-  double *ox, *oy, *oz, *os, *ow;       /* sorted copies; os, ow null when unused */
-  int *oidx, *ocs;                      /* original index, cell starts [ncell + 1] */
+  FkRec *rec;                 /* sorted copies, from the catalogue's first object */
+  double *ow;                 /* sorted weights beside |r|^2 (else null) */
+  int wt;                     /* weights wanted */
+  int *oidx;                  /* original index */
 };
 
 /* request owning index v of the concatenated space whose starts are off */
@@ -94,52 +97,45 @@ __device__ __forceinline__ int fk_stage_find(const FkStage *__restrict__ st, int
   return lo;
 }
 
+__device__ __forceinline__ int fk_cell(const FkGrid &g, double x, double y, double z) {
+  const int ix = fk_cell1(x, g.ox, g.wx, g.ncx);
+  const int iy = fk_cell1(y, g.oy, g.wy, g.ncy);
+  const int iz = fk_cell1(z, g.oz, g.wz, g.ncz);
+  return (ix * g.ncy + iy) * g.ncz + iz;
+}
+
 __global__ void k_stage_assign(int nobj, int nst, const FkStage *__restrict__ st,
-    int *__restrict__ cid, int *__restrict__ rank, int *__restrict__ count, int *bad) {
+    int *__restrict__ count, int *bad) {
   for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < nobj; o += gridDim.x * blockDim.x) {
     const FkStage &q = st[fk_stage_find(st, nst, o, &FkStage::obj0)];
     const int i = o - q.obj0;
+    const double x = q.x[i], y = q.y[i], z = q.z[i];
     /* a non-finite coordinate has no cell and no bin: the call fails */
-    if (!(__builtin_isfinite(q.x[i]) && __builtin_isfinite(q.y[i]) && __builtin_isfinite(q.z[i])))
-      atomicOr(bad, 1);
-    const int ix = fk_cell1(q.x[i], q.g.ox, q.g.wx, q.g.ncx);
-    const int iy = fk_cell1(q.y[i], q.g.oy, q.g.wy, q.g.ncy);
-    const int iz = fk_cell1(q.z[i], q.g.oz, q.g.wz, q.g.ncz);
-    const int c = (ix * q.g.ncy + iy) * q.g.ncz + iz;
-    cid[o] = c;
-    rank[o] = atomicAdd(count + q.cell0 + c, 1);
+    if (!(__builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z))) atomicOr(bad, 1);
+    atomicAdd(count + q.cell0 + fk_cell(q.g, x, y, z), 1);
   }
 }
 
-/* cell starts of each catalogue from the scan of all counts */
-__global__ void k_stage_starts(int ncs, int nst, const FkStage *__restrict__ st,
-    const int *__restrict__ gstart) {
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < ncs; t += gridDim.x * blockDim.x) {
-    const FkStage &q = st[fk_stage_find(st, nst, t, &FkStage::cs0)];
-    q.ocs[t - q.cs0] = gstart[q.cell0 + (t - q.cs0)] - gstart[q.cell0];
-  }
-}
-
-/* sorted copies; |r|^2 with FCFC's data_preprocess lane rule
- * (2pt/build_tree.c:59-92: FMA for the first floor(n/8)*8 objects, unfused
- * for the tail), unit weights where a weighted count has none
- * (build_tree.c:143-156) */
+/* sorted copies (cursor: the next free place of each cell); |r|^2 with
+ * FCFC's data_preprocess lane rule (2pt/build_tree.c:59-92: FMA for the first
+ * floor(n/8)*8 objects, unfused for the tail), unit weights where a weighted
+ * count has none (build_tree.c:143-156) */
 __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ st,
-    const int *__restrict__ cid, const int *__restrict__ rank, const int *__restrict__ gstart) {
+    int *__restrict__ cursor) {
   for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < nobj; o += gridDim.x * blockDim.x) {
     const FkStage &q = st[fk_stage_find(st, nst, o, &FkStage::obj0)];
     const int i = o - q.obj0;
-    const int d = gstart[q.cell0 + cid[o]] - gstart[q.cell0] + rank[o];
     const double a = q.x[i], b = q.y[i], c = q.z[i];
-    q.ox[d] = a; q.oy[d] = b; q.oz[d] = c;
-    if (q.os) {
-      double v;
+    const int d = atomicAdd(cursor + q.cell0 + fk_cell(q.g, a, b, c), 1) - q.obj0;
+    const double w = q.wt ? (q.w ? q.w[i] : 1.0) : 0.0;
+    double v = w;
+    if (q.need_s) {
       if (q.s) v = q.s[i];
       else if (i < (q.n / 8) * 8) v = __builtin_fma(c, c, __builtin_fma(b, b, a * a));
       else { double t = a * a; t = t + b * b; v = t + c * c; }
-      q.os[d] = v;
+      if (q.ow) q.ow[d] = w;
     }
-    if (q.ow) q.ow[d] = q.w ? q.w[i] : 1.0;
+    q.rec[d] = FkRec{a, b, c, v};
     q.oidx[d] = i;
   }
 }
@@ -212,6 +208,12 @@ __global__ void k_run_emit(int nunit, int njob, const FkTileJob *__restrict__ tj
 template <class T>
 __device__ __forceinline__ T fk_gld(const T *p, int i) {
   return ((const __attribute__((address_space(1))) T *) p)[i];
+}
+__device__ __forceinline__ FkRec fk_gld(const FkRec *p, int i) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  const __attribute__((address_space(1))) d2 *q = (const __attribute__((address_space(1))) d2 *) (p + i);
+  const d2 a = q[0], b = q[1];
+  return FkRec{a.x, a.y, b.x, b.y};
 }
 /* a descriptor at a uniform address, read with scalar loads (only the fields
  * in use are kept) */
@@ -879,7 +881,8 @@ __device__ __forceinline__ unsigned fk_recheck(const FkBins &bn, const FkJob &J,
     double ax, double ay, double az, int jg, int code, const unsigned *stab,
     const unsigned *ptab, const double *s2e, const double *pe, unsigned int *ncensus) {
   const int c3[3] = {code % 3 - 1, (code / 3) % 3 - 1, code / 9 - 1};
-  const double bo[3] = {fk_gld(J.B.x, jg), fk_gld(J.B.y, jg), fk_gld(J.B.z, jg)};
+  const FkRec b = fk_gld(J.B.rec, jg);
+  const double bo[3] = {b.x, b.y, b.z};
   const double ex = bo[0] + c3[0] * J.g.Lx;
   const double ey = bo[1] + c3[1] * J.g.Ly;
   const double ez = bo[2] + c3[2] * J.g.Lz;
@@ -896,21 +899,20 @@ __device__ __forceinline__ unsigned fk_recheck(const FkBins &bn, const FkJob &J,
 template <int BIN, bool HYB>
 __device__ __forceinline__ unsigned fk_recheck_sv(const FkBins &bn, const FkJob &J, int p,
     int jg, const unsigned *stab, const unsigned *ptab, const double *s2e, const double *pe) {
-  const double as = (BIN == FCFC_BIN_ISO) ? 0.0 : fk_gld(J.A.s, p);
-  const double bs = (BIN == FCFC_BIN_ISO) ? 0.0 : fk_gld(J.B.s, jg);
-  unsigned idx = fk_sv64<BIN, HYB, false, true>(fk_gld(J.A.x, p), fk_gld(J.A.y, p), fk_gld(J.A.z, p),
-                                                as, fk_gld(J.B.x, jg), fk_gld(J.B.y, jg),
-                                                fk_gld(J.B.z, jg), bs, bn, stab, ptab, s2e, pe);
+  const FkRec a = fk_gld(J.A.rec, p), b = fk_gld(J.B.rec, jg);
+  unsigned idx = fk_sv64<BIN, HYB, false, true>(a.x, a.y, a.z, a.q, b.x, b.y, b.z, b.q, bn, stab,
+                                                ptab, s2e, pe);
   if (BIN == FCFC_BIN_SMU) idx -= (unsigned) bn.nsh;
   return idx >= (unsigned) bn.ntoh ? FK_NONE : idx;
 }
 
 /* ---------------------------- the kernel --------------------------------- */
 
-/* LDS bytes of one staged B object: coordinates (relative to the run's
- * centre in FP32), |r|^2, weight, gradient share, sorted index */
-__host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool need_s, bool need_w, bool grad) {
-  return (f32 ? 12 : 24) + (need_s ? 8 : 0) + (need_w ? 8 : 0) + (grad ? 8 : 0) + 4;
+/* LDS bytes of one staged B object: FP32 coordinates relative to the run's
+ * centre, weight and sorted index; the gradient form keeps the gradient share
+ * and the sorted index of each B object, the FP64 counts nothing */
+__host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool wt, bool grad) {
+  return f32 ? 12 + (wt ? 8 : 0) + 4 : (grad ? 8 : 0);
 }
 
 /* One persistent kernel for counts (FP64 or FP32 + recheck) and for the
@@ -929,7 +931,19 @@ __host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool need_s, bool nee
  * Against tiles of 512 R objects that shared their B chunks (same data, ms of
  * the whole call): (s, mu) RR of 4e6 objects 331 -> 232, weighted DD of 5e5
  * 16.9 -> 9.1, w_p of 1e6 to 40 Mpc/h (128 objects in tiles of 1024) 11.8 ->
- * 4.6, survey (s, mu) RR of 1.2e6 27.1 -> 16.1. */
+ * 4.6, survey (s, mu) RR of 1.2e6 27.1 -> 16.1.
+ *
+ * The weighted FP64 counts are bound by the LDS next: a table entry and an
+ * FP64 atomic per lane and pair, and with the B objects in LDS four more
+ * 8-byte reads per object, about half of the LDS's cycles (LDS 81 % busy,
+ * VALU 65 %, and room for 2 workgroups per CU).  The FP64 forms therefore
+ * read each kept B object from its sorted record into scalar registers (one
+ * 32-byte line per object, mostly hits of the scalar cache, as the wavefront
+ * has just loaded the line to test the object): weighted DD of 5e5 9.1 -> 7.5
+ * ms, DR of 2e5 x 2e6 20.9 -> 16.6, the hybrid w_p count 3.5 -> 3.0; the
+ * unweighted RR, bound by the VALU, is unchanged (232).  The FP32 forms keep
+ * the chunk: their coordinates are converted once for 64 R pairs there, and
+ * its 4-byte reads cost the LDS half as much. */
 template <int BIN, int GEOM, bool WT, int MODE, bool HYB, int R>
 __global__ void __launch_bounds__(FK_NT, WT ? 6 : 8)
 k_count(const FkArgs a) {
@@ -942,8 +956,8 @@ k_count(const FkArgs a) {
   /* |r|^2 of the objects: survey (s, mu) and (s_perp, pi) in FP64 (the FP32
    * form reads them from the catalogue when it re-evaluates a pair) */
   constexpr bool NEED_S = (GEOM == FCFC_GEOM_SURVEY && BIN != FCFC_BIN_ISO && !SV32);
-  constexpr bool NEED_W = WT || GRAD;
-  constexpr bool NEED_C = F32;
+  /* weights beside the records (which then hold |r|^2) */
+  constexpr bool WSEP = (GEOM == FCFC_GEOM_SURVEY && BIN != FCFC_BIN_ISO);
   const int tid = threadIdx.x;
   /* the wavefront index, in a scalar register (with everything derived
    * from it: the wavefront's histogram copy and queue) */
@@ -979,17 +993,12 @@ k_count(const FkArgs a) {
   double *s2e = (double *) (lds + a.off_edges);
   double *pe = s2e + (bn.ns + 1);
   /* the wavefront's chunk of B objects */
-  char *cp = lds + a.off_chunk + wave * (FK_CH * fk_chunk_bytes(F32, NEED_S, NEED_W, GRAD));
-  double *cs_ = (double *) cp;                 /* survey |r|^2 */
-  if (NEED_S) cp += 8 * FK_CH;
-  double *cw = (double *) cp;                  /* weights */
-  if (NEED_W) cp += 8 * FK_CH;
+  char *cp = lds + a.off_chunk + wave * (FK_CH * fk_chunk_bytes(F32, WT, GRAD));
+  double *cw = (double *) cp;                  /* FP32: weights */
   double *cb = (double *) cp;                  /* GRAD: gradient share of each B object */
-  if (GRAD) cp += 8 * FK_CH;
-  double *cx = (double *) cp, *cy = cx + FK_CH, *cz = cy + FK_CH;
+  if (F32 && WT) cp += 8 * FK_CH;
   float *fx = (float *) cp, *fy = fx + FK_CH, *fz = fy + FK_CH;
-  cp += (F32 ? 12 : 24) * FK_CH;
-  int *cj = (int *) cp;                        /* sorted index */
+  int *cj = (int *) (fz + FK_CH);              /* sorted index */
   /* FP32 re-evaluation queue of this wavefront: sorted index of the B
    * object, A slot in the run << 5 | periodic image code */
   unsigned *wqj = (unsigned *) (lds + a.off_queue + wave * (FK_QCAP * 6));
@@ -1181,7 +1190,8 @@ k_count(const FkArgs a) {
       const int p = t.p0 + r * 64 + lane;
       const bool v = p < t.p1;
       const int pc = v ? p : t.p0;
-      const double x = fk_gld(J.A.x, pc), y = fk_gld(J.A.y, pc), z = fk_gld(J.A.z, pc);
+      const FkRec ra = fk_gld(J.A.rec, pc);
+      const double x = ra.x, y = ra.y, z = ra.z;
       lox = __builtin_fmin(lox, x); hix = __builtin_fmax(hix, x);
       loy = __builtin_fmin(loy, y); hiy = __builtin_fmax(hiy, y);
       loz = __builtin_fmin(loz, z); hiz = __builtin_fmax(hiz, z);
@@ -1189,8 +1199,8 @@ k_count(const FkArgs a) {
       ax[r] = v ? x : FK_FAR;
       ay[r] = v ? y : FK_FAR;
       az[r] = v ? z : FK_FAR;
-      as[r] = NEED_S ? (v ? fk_gld(J.A.s, pc) : 3.0 * FK_FAR * FK_FAR) : 0.0;
-      aw[r] = (jw && v) ? fk_gld(J.A.w, pc) : 1.0;
+      as[r] = NEED_S ? (v ? ra.q : 3.0 * FK_FAR * FK_FAR) : 0.0;
+      aw[r] = (jw && v) ? (WSEP ? fk_gld(J.A.w, pc) : ra.q) : 1.0;
       gacc[r] = 0.0;
       actm[r] = __builtin_amdgcn_ballot_w64(v);
     }
@@ -1231,13 +1241,16 @@ k_count(const FkArgs a) {
           unsigned idx;
           if (GEOM == FCFC_GEOM_SURVEY)
             idx = fk_recheck_sv<BIN, HYB>(bn, J, p, jg, stab, ptab, s2e, pe);
-          else
-            idx = fk_recheck<BIN, HYB, CENS>(bn, J, fk_gld(J.A.x, p), fk_gld(J.A.y, p),
-                                             fk_gld(J.A.z, p), jg, (int) (v & 31u), stab, ptab,
-                                             s2e, pe, &ncensus);
+          else {
+            const FkRec ra = fk_gld(J.A.rec, p);
+            idx = fk_recheck<BIN, HYB, CENS>(bn, J, ra.x, ra.y, ra.z, jg, (int) (v & 31u), stab,
+                                             ptab, s2e, pe, &ncensus);
+          }
           nrecheck++;
           if (idx < ntot) {
-            if (WT && jwt) atomicAdd(myhist_d + idx, fk_gld(J.A.w, p) * fk_gld(J.B.w, jg));
+            if (WT && jwt)
+              atomicAdd(myhist_d + idx, WSEP ? fk_gld(J.A.w, p) * fk_gld(J.B.w, jg)
+                                             : fk_gld(J.A.rec, p).q * fk_gld(J.B.rec, jg).q);
             else atomicAdd(myhist_u + idx, 1u);
           }
         }
@@ -1246,152 +1259,143 @@ k_count(const FkArgs a) {
       fk_wave_sync();
     };
 
-    /* staged B objects [j, cnt) of a chunk against the lane's A objects; FP32:
-     * only while the queue has room for one more (64 R pairs at most).
-     * Returns the next B object */
-    auto run_chunk = [&](auto selfc, int j, int cnt, int code) __attribute__((always_inline)) -> int {
+    /* one B object against the lane's A objects: FP64 coordinates, |r|^2 and
+     * weight, or FP32 coordinates relative to the run's centre; jj its sorted
+     * index, j its place in the chunk, code its periodic image */
+    auto step = [&](auto selfc, double bx, double by, double bz, double bs, double wj, float gx,
+                    float gy, float gz, int jj, int j, int code) __attribute__((always_inline)) {
       constexpr bool SELF = decltype(selfc)::value;
-#pragma unroll 2
-      for (; j < cnt; j++) {
-        if (F32 && qn > FK_QCAP - 64 * R) break;
-        double bx = 0, by = 0, bz = 0, bs = 0;
-        float gx = 0, gy = 0, gz = 0;
-        if (F32) { gx = fx[j]; gy = fy[j]; gz = fz[j]; }
-        else { bx = cx[j]; by = cy[j]; bz = cz[j]; }
-        if (NEED_S) bs = cs_[j];
-        const double wj = NEED_W ? cw[j] : 1.0;
-        const int jj = SELF ? cj[j] : 0;
-        if (GEOM == FCFC_GEOM_BOX) {
-          /* when this B object is out of range of every A object of the run,
-           * skip the binning (same expressions as the pair functions, so the
-           * compiler shares them).  Every form skips, so the plain form
-           * differs from the FP64 one in the per-pair mu arithmetic only */
-          bool any = false;
-#pragma unroll
-          for (int r = 0; r < R; r++) {
-            if (F32) {
-              const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-              if (BIN == FCFC_BIN_SPI)
-                any |= (__builtin_fmaf(ey, ey, ex * ex) < bn.s2skip32) &
-                       (__builtin_fabsf(ez) < bn.pskip32);
-              else any |= __builtin_fmaf(ey, ey, __builtin_fmaf(ex, ex, ez * ez)) < bn.s2skip32;
-            }
-            else {
-              const double ex = bx - ax[r], ey = by - ay[r], ez = bz - az[r];
-              if (BIN == FCFC_BIN_SPI)
-                any |= (__builtin_fma(ey, ey, ex * ex) < bn.s2skip) &
-                       (__builtin_fabs(ez) < bn.pskip);
-              else any |= __builtin_fma(ey, ey, __builtin_fma(ex, ex, ez * ez)) < bn.s2skip;
-            }
-          }
-          if (__builtin_amdgcn_ballot_w64(any) == 0) continue;
-        }
-        if (GEOM == FCFC_GEOM_SURVEY) {
-          /* the same skip for survey pairs: |a - b|^2 (iso) or s - t
-           * (= s^2 = s_perp^2 + pi^2) beyond the largest counted value */
-          bool any = false;
-#pragma unroll
-          for (int r = 0; r < R; r++) {
-            if (SV32) {
-              const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-              any |= __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) < bn.s2skip32;
-            }
-            else if (BIN == FCFC_BIN_ISO) {
-              const double ex = ax[r] - bx, ey = ay[r] - by, ez = az[r] - bz;
-              any |= __builtin_fma(ez, ez, __builtin_fma(ey, ey, ex * ex)) < bn.s2skip;
-            }
-            else {
-              const double tt = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
-              any |= (as[r] + bs) - tt < bn.s2skip;
-            }
-          }
-          if (__builtin_amdgcn_ballot_w64(any) == 0) continue;
-        }
-        double bsum = 0.0;          /* GRAD: sum of G[bin] w_a over this lane's pairs */
+      if (GEOM == FCFC_GEOM_BOX) {
+        /* when this B object is out of range of every A object of the run,
+         * skip the binning (same expressions as the pair functions, so the
+         * compiler shares them).  Every form skips, so the plain form
+         * differs from the FP64 one in the per-pair mu arithmetic only */
+        bool any = false;
 #pragma unroll
         for (int r = 0; r < R; r++) {
-          unsigned idx;
-          bool queued = false;      /* FP32: left to the FP64 re-evaluation */
           if (F32) {
-            bool amb, ambm;
-            bool ambx = false;
-            if (SV32) {
-              const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-              idx = fk_sv32<BIN>(ex, ey, ez, __builtin_fmaf(2.0f, fax[r], ex) + c2x,
-                                 __builtin_fmaf(2.0f, fay[r], ey) + c2y,
-                                 __builtin_fmaf(2.0f, faz[r], ez) + c2z, bn, wn, stab_raw,
-                                 ptab_raw, amb, ambm, ambx);
-            }
-            else
-              idx = fk_box32<BIN>(gx - fax[r], gy - fay[r], gz - faz[r], bn, wn, stab_raw,
-                                  ptab_raw, amb, ambm);
-            if (SELF) {
-              const bool keep = jj > ai[r];
-              amb = amb & keep; ambm = ambm & keep; idx = keep ? idx : FK_NONE;
-            }
-            /* pairs near an edge: queue (B object, A slot, image) for FP64.
-             * The conditions are balloted apart (each ballot is its compare's
-             * own mask) and the lane's bit is read back from the mask inside
-             * the rare branch, so no lane value is kept across it */
-            if (SELF) ambx = ambx & (jj > ai[r]);
-            unsigned long long m = __builtin_amdgcn_ballot_w64(amb) |
-                __builtin_amdgcn_ballot_w64(ambm) | __builtin_amdgcn_ballot_w64(ambx);
-            m &= actm[r];
-            if (__builtin_expect(m != 0, 0)) {
-              if ((m >> lane) & 1ull) {
-                const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-                wqj[pos] = (unsigned) cj[j];
-                wqs[pos] = (uint16_t) (((unsigned) (r * 64 + lane) << 5) | (unsigned) code);
-              }
-              qn += __popcll(m);
-            }
-            queued = amb | ambm | ambx;
+            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
+            if (BIN == FCFC_BIN_SPI)
+              any |= (__builtin_fmaf(ey, ey, ex * ex) < bn.s2skip32) &
+                     (__builtin_fabsf(ez) < bn.pskip32);
+            else any |= __builtin_fmaf(ey, ey, __builtin_fmaf(ex, ex, ez * ez)) < bn.s2skip32;
           }
-          else if (GEOM == FCFC_GEOM_BOX)
-            idx = fk_box64<BIN, HYB, false, PLAIN, MUT>(bx - ax[r], by - ay[r], bz - az[r], bn,
-                                                         stab, ptab, s2e, pe);
-          else
-            idx = fk_sv64<BIN, HYB, PLAIN, false, MUT || QT>(ax[r], ay[r], az[r], as[r], bx, by,
-                                                             bz, bs, bn, stab, ptab, s2e, pe,
-                                                             os_lds, op_lds);
-          if (!F32 && SELF && !(jj > ai[r])) idx = FK_NONE;
-          if (idx < ntot_o && !queued) {
-            if (GRAD) {
-              const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
-              gacc[r] += gk * wj;
-              bsum += gk * aw[r];
-            }
-            else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
-            else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
+          else {
+            const double ex = bx - ax[r], ey = by - ay[r], ez = bz - az[r];
+            if (BIN == FCFC_BIN_SPI)
+              any |= (__builtin_fma(ey, ey, ex * ex) < bn.s2skip) &
+                     (__builtin_fabs(ez) < bn.pskip);
+            else any |= __builtin_fma(ey, ey, __builtin_fma(ex, ex, ez * ez)) < bn.s2skip;
           }
         }
-        if (GRAD && hasB) {
-          /* the B object's share over the wavefront's pairs: one sum per
-           * row of 16 lanes, added into the chunk's LDS accumulator */
-          const double v = fk_row_sum(bsum);
-          if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
+        if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+      }
+      if (GEOM == FCFC_GEOM_SURVEY) {
+        /* the same skip for survey pairs: |a - b|^2 (iso) or s - t
+         * (= s^2 = s_perp^2 + pi^2) beyond the largest counted value */
+        bool any = false;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          if (SV32) {
+            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
+            any |= __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) < bn.s2skip32;
+          }
+          else if (BIN == FCFC_BIN_ISO) {
+            const double ex = ax[r] - bx, ey = ay[r] - by, ez = az[r] - bz;
+            any |= __builtin_fma(ez, ez, __builtin_fma(ey, ey, ex * ex)) < bn.s2skip;
+          }
+          else {
+            const double tt = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
+            any |= (as[r] + bs) - tt < bn.s2skip;
+          }
+        }
+        if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+      }
+      double bsum = 0.0;          /* GRAD: sum of G[bin] w_a over this lane's pairs */
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        unsigned idx;
+        bool queued = false;      /* FP32: left to the FP64 re-evaluation */
+        if (F32) {
+          bool amb, ambm;
+          bool ambx = false;
+          if (SV32) {
+            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
+            idx = fk_sv32<BIN>(ex, ey, ez, __builtin_fmaf(2.0f, fax[r], ex) + c2x,
+                               __builtin_fmaf(2.0f, fay[r], ey) + c2y,
+                               __builtin_fmaf(2.0f, faz[r], ez) + c2z, bn, wn, stab_raw,
+                               ptab_raw, amb, ambm, ambx);
+          }
+          else
+            idx = fk_box32<BIN>(gx - fax[r], gy - fay[r], gz - faz[r], bn, wn, stab_raw,
+                                ptab_raw, amb, ambm);
+          if (SELF) {
+            const bool keep = jj > ai[r];
+            amb = amb & keep; ambm = ambm & keep; idx = keep ? idx : FK_NONE;
+          }
+          /* pairs near an edge: queue (B object, A slot, image) for FP64.
+           * The conditions are balloted apart (each ballot is its compare's
+           * own mask) and the lane's bit is read back from the mask inside
+           * the rare branch, so no lane value is kept across it */
+          if (SELF) ambx = ambx & (jj > ai[r]);
+          unsigned long long m = __builtin_amdgcn_ballot_w64(amb) |
+              __builtin_amdgcn_ballot_w64(ambm) | __builtin_amdgcn_ballot_w64(ambx);
+          m &= actm[r];
+          if (__builtin_expect(m != 0, 0)) {
+            if ((m >> lane) & 1ull) {
+              const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                         __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+              wqj[pos] = (unsigned) (SELF ? jj : cj[j]);
+              wqs[pos] = (uint16_t) (((unsigned) (r * 64 + lane) << 5) | (unsigned) code);
+            }
+            qn += __popcll(m);
+          }
+          queued = amb | ambm | ambx;
+        }
+        else if (GEOM == FCFC_GEOM_BOX)
+          idx = fk_box64<BIN, HYB, false, PLAIN, MUT>(bx - ax[r], by - ay[r], bz - az[r], bn,
+                                                       stab, ptab, s2e, pe);
+        else
+          idx = fk_sv64<BIN, HYB, PLAIN, false, MUT || QT>(ax[r], ay[r], az[r], as[r], bx, by,
+                                                           bz, bs, bn, stab, ptab, s2e, pe,
+                                                           os_lds, op_lds);
+        if (!F32 && SELF && !(jj > ai[r])) idx = FK_NONE;
+        if (idx < ntot_o && !queued) {
+          if (GRAD) {
+            const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
+            gacc[r] += gk * wj;
+            bsum += gk * aw[r];
+          }
+          else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
+          else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
         }
       }
-      return j;
+      if (GRAD && hasB) {
+        /* the B object's share over the wavefront's pairs: one sum per
+         * row of 16 lanes, added into the chunk's LDS accumulator */
+        const double v = fk_row_sum(bsum);
+        if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
+      }
     };
 
+
     /* B objects [b0, b0 + n) of the other catalogue (SELF: of the run itself),
-     * at the periodic image of code */
-    auto segment = [&](auto selfc, int b0, int n, int code) {
+     * at the periodic image of code (IMG: not the object's own place) */
+    auto segment = [&](auto selfc, auto imgc, int b0, int n, int code) __attribute__((always_inline)) {
       constexpr bool SELF = decltype(selfc)::value;
+      constexpr bool IMG = decltype(imgc)::value;
       for (int c0 = 0; c0 < n; c0 += FK_CH) {
         const FkJob *pj = fk_again(a.jobs, cur);
         const FkCat B = fk_cld(SELF ? &pj->A : &pj->B);
         const FkGrid g = fk_cld(&pj->g);
+        const double Dx = IMG ? (double) (code % 3 - 1) * g.Lx : 0.0;
+        const double Dy = IMG ? (double) ((code / 3) % 3 - 1) * g.Ly : 0.0;
+        const double Dz = IMG ? (double) (code / 9 - 1) * g.Lz : 0.0;
         const bool in = c0 + lane < n;
         const int jg = b0 + (in ? c0 + lane : 0);
-        double x = fk_gld(B.x, jg), y = fk_gld(B.y, jg), z = fk_gld(B.z, jg);
-        if (GEOM == FCFC_GEOM_BOX && code != 13) {
-          x = x + (double) (code % 3 - 1) * g.Lx;
-          y = y + (double) ((code / 3) % 3 - 1) * g.Ly;
-          z = z + (double) (code / 9 - 1) * g.Lz;
-        }
+        const FkRec rb = fk_gld(B.rec, jg);
+        double x = rb.x, y = rb.y, z = rb.z;
+        if (IMG) { x = x + Dx; y = y + Dy; z = z + Dz; }
         /* drop the objects beyond the maximum separation from the run's
          * bounding box (the grid's padded ranges) */
         bool keep = in;
@@ -1404,7 +1408,7 @@ k_count(const FkArgs a) {
           if (g.hz_const >= 0) keep &= (exy < g.Rxy2) & (ez < g.hz_const);
           else keep &= __builtin_fma(ez, ez, exy) < g.R2;
         }
-        const unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+        unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
         evals += (unsigned long long) ((unsigned) min(FK_CH, n - c0) * (unsigned) nva);
         if (m == 0) continue;
         const int cnt = __popcll(m);
@@ -1412,35 +1416,56 @@ k_count(const FkArgs a) {
           if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) (void) job_round(cur);
           since += (unsigned) cnt * (unsigned) nva;
         }
-        fk_wave_sync();
-        if (keep) {
-          const int q = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
-                                    __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-          if (F32) {
+        if (F32) {
+          /* pack the kept objects into the wavefront's chunk */
+          fk_wave_sync();
+          if (keep) {
+            const int q = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                      __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
             fx[q] = (float) (x - 0.5 * (lx + hx));
             fy[q] = (float) (y - 0.5 * (ly + hy));
             fz[q] = (float) (z - 0.5 * (lz + hz));
+            if (WT) cw[q] = jw ? (WSEP ? fk_gld(B.w, jg) : rb.q) : 1.0;
+            cj[q] = jg;
           }
-          else { cx[q] = x; cy[q] = y; cz[q] = z; }
-          if (NEED_S) cs_[q] = fk_gld(B.s, jg);
-          if (NEED_W) cw[q] = jw ? fk_gld(B.w, jg) : 1.0;
-          if (GRAD) cb[q] = 0.0;
-          cj[q] = jg;
-        }
-        fk_wave_sync();
-        for (int j = 0;;) {
-          j = run_chunk(selfc, j, cnt, code);
-          if (F32 && qn > FK_QCAP - 64 * R) drain();
-          if (j >= cnt) break;
-        }
-        /* GRAD: the B objects' shares go to the output */
-        if (GRAD && hasB) {
           fk_wave_sync();
-          if (lane < cnt) {
-            const FkJob *pk = fk_again(a.jobs, cur);
-            const double v = cb[lane];
-            if (v != 0.0)
-              unsafeAtomicAdd(fk_cld(&pk->gB) + fk_gld(fk_cld(SELF ? &pk->A.idx : &pk->B.idx), cj[lane]), v);
+          for (int j = 0; j < cnt;) {
+            /* while the queue has room for the pairs of one more object */
+#pragma unroll 2
+            for (; j < cnt; j++) {
+              if (qn > FK_QCAP - 64 * R) break;
+              step(selfc, 0.0, 0.0, 0.0, 0.0, WT ? cw[j] : 1.0, fx[j], fy[j], fz[j],
+                   SELF ? cj[j] : 0, j, code);
+            }
+            if (qn > FK_QCAP - 64 * R) drain();
+          }
+        }
+        else {
+          if (GRAD && hasB) { fk_wave_sync(); cb[lane] = 0.0; fk_wave_sync(); }
+          /* the kept objects, one at a time, into scalar registers */
+          typedef const __attribute__((address_space(4))) double cdouble;
+          cdouble *rp = (cdouble *) (B.rec + b0 + c0);
+          cdouble *wp = (cdouble *) (B.w + b0 + c0);
+          unsigned long long k = m;
+          while (k) {
+            const int j = __builtin_ctzll(k);
+            k &= k - 1;
+            const double px = rp[4 * j], py = rp[4 * j + 1], pz = rp[4 * j + 2], pq = rp[4 * j + 3];
+            double wj = 1.0;
+            if (WSEP && (WT || GRAD)) { if (jw) wj = wp[j]; }
+            else if (WT || GRAD) wj = jw ? pq : 1.0;
+            step(selfc, IMG ? px + Dx : px, IMG ? py + Dy : py, IMG ? pz + Dz : pz,
+                 NEED_S ? pq : 0.0, wj, 0.0f, 0.0f, 0.0f, SELF ? b0 + c0 + j : 0, j, code);
+          }
+          /* GRAD: the B objects' shares go to the output */
+          if (GRAD && hasB) {
+            fk_wave_sync();
+            if (keep) {
+              const FkJob *pk = fk_again(a.jobs, cur);
+              const double v = cb[lane];
+              if (v != 0.0)
+                unsafeAtomicAdd(fk_cld(&pk->gB) + fk_gld(fk_cld(SELF ? &pk->A.idx : &pk->B.idx), jg), v);
+            }
           }
         }
       }
@@ -1449,7 +1474,7 @@ k_count(const FkArgs a) {
     /* ---- auto counts: pairs inside the run (j > i), first item only ---- */
     if (J.autoc && part == 0) {
       evals -= (unsigned long long) nva * (unsigned) nva / 2;
-      segment(std::integral_constant<bool, true>(), t.p0, nva, 13);
+      segment(std::true_type(), std::false_type(), t.p0, nva, 13);
     }
 
     /* ---- strips, one per lane at a time ---- */
@@ -1480,7 +1505,9 @@ k_count(const FkArgs a) {
           q = __builtin_ctzll(m2); m2 &= m2 - 1;
           b = fk_lane_of(b0[2], q); n = fk_lane_of(len[2], q); cd = fk_lane_of(code[2], q);
         }
-        segment(std::integral_constant<bool, false>(), b, n, cd);
+        if (GEOM == FCFC_GEOM_SURVEY || (!F32 && cd == 13))
+          segment(std::false_type(), std::false_type(), b, n, cd);
+        else segment(std::false_type(), std::true_type(), b, n, cd);
       }
     }
     if (F32 && qn) drain();
@@ -1570,9 +1597,7 @@ static void set_err(fcfc_gpu_ctx *c, const char *fmt, ...) {
 enum {
   WS_IN_X, WS_IN_Y, WS_IN_Z, WS_IN_S, WS_IN_W,          /* uploads, catalogue A */
   WS_IN2_X, WS_IN2_Y, WS_IN2_Z, WS_IN2_S, WS_IN2_W,     /* uploads, catalogue B */
-  WS_A_X, WS_A_Y, WS_A_Z, WS_A_S, WS_A_W, WS_A_IDX, WS_A_CS,
-  WS_B_X, WS_B_Y, WS_B_Z, WS_B_S, WS_B_W, WS_B_IDX, WS_B_CS,
-  WS_CID, WS_RANK, WS_COUNT, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES,
+  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES,
   WS_STRIPS, WS_STAB, WS_PTAB, WS_S2E, WS_PE, WS_HIST, WS_MISC, WS_G, WS_GA, WS_GB, WS_JOBS,
   WS_NSLOT
 };
@@ -1837,11 +1862,26 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
   return 0;
 }
 
-/* sorted catalogue on the device */
+/* sorted catalogue on the device: records, weights beside them (survey bins
+ * with |r|^2) and original indices from its first object; obj0, cell0: its
+ * place in the objects and cells of the call, cs: its cell starts, which
+ * count objects of the call (set once the call's sort is queued) */
 struct DevCat {
-  int n = 0;
-  double *x = nullptr, *y = nullptr, *z = nullptr, *s = nullptr, *w = nullptr;
-  int *idx = nullptr, *cs = nullptr;
+  int n = 0, obj0 = 0, cell0 = 0;
+  FkRec *rec = nullptr;
+  double *w = nullptr;
+  int *idx = nullptr;
+  const int *cs = nullptr;
+  FkCat dev() const { return FkCat{n, 0, rec - obj0, w ? w - obj0 : nullptr, idx - obj0, cs}; }
+};
+
+/* A job ready to count: plan, sorted catalogues, output. */
+struct PJob {
+  JobPlan P;
+  DevCat A, B;
+  int autoc = 0, wt = 0;
+  double *gA = nullptr, *gB = nullptr;
+  long long hist_off = 0;
 };
 
 static inline int nblk(int64_t n, int bs) {
@@ -1912,8 +1952,9 @@ struct Alloc {
 };
 
 __global__ void k_gather(int n, const int *__restrict__ idx, const double *__restrict__ src,
-    double *__restrict__ dst) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[i] = src[idx[i]];
+    double *__restrict__ dst, int stride) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    dst[(size_t) stride * i] = src[idx[i]];
 }
 
 __global__ void k_fill_f64(double *p, int64_t n, double v) {
@@ -1970,13 +2011,12 @@ static int bbox(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, double lo[3], dou
 
 /* Prepare the sort of one catalogue into the grid of a job: upload host
  * inputs, allocate the sorted copies (so the job's descriptors can point
- * at them at once) and queue the work for stage_run.  slot: first of 7
+ * at them at once) and queue the work for stage_run.  slot: first of 3
  * consecutive workspace slots (single-job calls). */
 static int stage_prep(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, int need_s,
     int wt, const FkGrid &g, int slot, int upslot, DevCat *out, std::vector<FkStage> &st) {
   const int n = (int) k->n;
   const size_t nb = sizeof(double) * (size_t) (n > 0 ? n : 1);
-  const int ncell = g.ncx * g.ncy * g.ncz;
   /* inputs on the device */
   const double *x = k->x, *y = k->y, *z = k->z, *s = need_s ? k->s : nullptr, *w = wt ? k->w : nullptr;
   if (!k->on_device && n > 0) {
@@ -2000,54 +2040,60 @@ static int stage_prep(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, int need_s,
       w = dw;
     }
   }
+  const size_t no = (size_t) (n > 0 ? n : 1);
   out->n = n;
-  out->x = (double *) al.get(slot + 0, nb);
-  out->y = (double *) al.get(slot + 1, nb);
-  out->z = (double *) al.get(slot + 2, nb);
-  out->s = need_s ? (double *) al.get(slot + 3, nb) : nullptr;
-  out->w = wt ? (double *) al.get(slot + 4, nb) : nullptr;
-  out->idx = (int *) al.get(slot + 5, sizeof(int) * (size_t) (n > 0 ? n : 1));
-  out->cs = (int *) al.get(slot + 6, sizeof(int) * ((size_t) ncell + 1));
+  out->rec = (FkRec *) al.get(slot + 0, sizeof(FkRec) * no);
+  out->w = (need_s && wt) ? (double *) al.get(slot + 1, nb) : nullptr;
+  out->idx = (int *) al.get(slot + 2, sizeof(int) * no);
   if (al.err) return al.err;
   FkStage q;
   memset(&q, 0, sizeof q);
-  q.n = n; q.need_s = need_s; q.g = g;
+  q.n = n; q.need_s = need_s; q.wt = wt; q.g = g;
   q.x = x; q.y = y; q.z = z; q.s = s; q.w = w;
-  q.ox = out->x; q.oy = out->y; q.oz = out->z; q.os = out->s; q.ow = out->w;
-  q.oidx = out->idx; q.ocs = out->cs;
+  q.rec = out->rec; q.ow = out->w; q.oidx = out->idx;
+  if (!st.empty()) {
+    const FkStage &p = st.back();
+    const long long nc = p.cell0 + (long long) p.g.ncx * p.g.ncy * p.g.ncz;
+    const long long nobj = (long long) p.obj0 + p.n;
+    if (nobj + n > INT_MAX / 2 || nc + (long long) g.ncx * g.ncy * g.ncz > INT_MAX / 2) {
+      set_err(c, "catalogues of one call too large");
+      return FCFC_ERR_CFG;
+    }
+    q.obj0 = (int) nobj;
+    q.cell0 = (int) nc;
+  }
+  out->obj0 = q.obj0;
+  out->cell0 = q.cell0;
   st.push_back(q);
   return 0;
 }
 
-/* Run the queued sorts of a call: one launch per stage for all of them. */
-static int stage_run(fcfc_gpu_ctx *c, Alloc &al, std::vector<FkStage> &st) {
+/* Run the queued sorts of a call: one launch per stage for all of them.  The
+ * cell starts of all catalogues come from one scan and stay where it leaves
+ * them (cs of every job). */
+static int stage_run(fcfc_gpu_ctx *c, Alloc &al, std::vector<FkStage> &st, std::vector<PJob> &jobs) {
   if (st.empty()) return 0;
-  long long nobj = 0, ncell = 0, ncs = 0;
-  for (FkStage &q : st) {
-    q.obj0 = (int) nobj; q.cell0 = (int) ncell; q.cs0 = (int) ncs;
-    const long long nc = (long long) q.g.ncx * q.g.ncy * q.g.ncz;
-    nobj += q.n; ncell += nc; ncs += nc + 1;
-    if (nobj > INT_MAX / 2 || ncs > INT_MAX / 2) { set_err(c, "catalogues of one call too large"); return FCFC_ERR_CFG; }
-  }
+  const FkStage &last = st.back();
+  const int nobj = last.obj0 + last.n;
+  const long long ncl = last.cell0 + (long long) last.g.ncx * last.g.ncy * last.g.ncz;
+  if (nobj > INT_MAX / 2 || ncl > INT_MAX / 2) { set_err(c, "catalogues of one call too large"); return FCFC_ERR_CFG; }
+  const int ncell = (int) ncl;
   const int nst = (int) st.size();
   FkStage *dst = (FkStage *) al.tmp(WS_STAGE, sizeof(FkStage) * st.size());
-  int *cid = (int *) al.tmp(WS_CID, sizeof(int) * (size_t) (nobj > 0 ? nobj : 1));
-  int *rank = (int *) al.tmp(WS_RANK, sizeof(int) * (size_t) (nobj > 0 ? nobj : 1));
   /* count[ncell]: set when an object has a non-finite coordinate */
   int *count = (int *) al.tmp(WS_COUNT, sizeof(int) * ((size_t) ncell + 1));
-  int *gstart = (int *) al.tmp(WS_GSTART, sizeof(int) * ((size_t) ncell + 1));
+  int *gstart = (int *) al.get(WS_GSTART, sizeof(int) * ((size_t) ncell + 1));
   if (al.err) return al.err;
+  for (PJob &J : jobs) { J.A.cs = gstart + J.A.cell0; J.B.cs = gstart + J.B.cell0; }
   HIPCHK(c, hipMemcpyAsync(dst, st.data(), sizeof(FkStage) * st.size(), hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_fill_int, dim3(nblk(ncell + 1, 256)), dim3(256), 0, c->stream, count,
-                     (int) ncell + 1, 0);
+  hipLaunchKernelGGL(k_fill_int, dim3(nblk(ncell + 1, 256)), dim3(256), 0, c->stream, count, ncell + 1, 0);
   if (nobj > 0)
-    hipLaunchKernelGGL(k_stage_assign, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, (int) nobj, nst, dst,
-                       cid, rank, count, count + ncell);
-  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, count, gstart, (int) ncell);
-  hipLaunchKernelGGL(k_stage_starts, dim3(nblk(ncs, 256)), dim3(256), 0, c->stream, (int) ncs, nst, dst, gstart);
+    hipLaunchKernelGGL(k_stage_assign, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, nobj, nst, dst,
+                       count, count + ncell);
+  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, count, gstart, ncell);
   if (nobj > 0)
-    hipLaunchKernelGGL(k_stage_scatter, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, (int) nobj, nst, dst,
-                       cid, rank, gstart);
+    hipLaunchKernelGGL(k_stage_scatter, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, nobj, nst, dst,
+                       count);
   HIPCHK(c, hipGetLastError());
   int bad = 0;
   HIPCHK(c, hipMemcpyAsync(&bad, count + ncell, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -2097,7 +2143,7 @@ static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh
   if (hyb) o = align16(o + 8 * (b->ns + 1 + (b->bintype == FCFC_BIN_SPI ? b->np + 1 : 0)));
   L.off_chunk = o;
   const bool f32 = (mode == MODE_C32), grad = (mode == MODE_GRAD);
-  o = align16(o + FK_NW * FK_CH * fk_chunk_bytes(f32, need_s && !f32, wt || grad, grad));
+  o = align16(o + FK_NW * FK_CH * fk_chunk_bytes(f32, wt, grad));
   L.off_queue = o;
   if (f32) o += FK_NW * FK_QCAP * 6;
   o = align16(o);
@@ -2302,17 +2348,6 @@ static void fp32_windows(const fcfc_bins *b, const FkGrid &g, int zmaxc, double 
   w.m2_floor = (float) m2f;
 }
 
-/* One counting (or gradient) job on device-resident, sorted catalogues. */
-
-/* A job ready to count: plan, sorted catalogues, output. */
-struct PJob {
-  JobPlan P;
-  DevCat A, B;
-  int autoc = 0, wt = 0;
-  double *gA = nullptr, *gB = nullptr;
-  long long hist_off = 0;
-};
-
 static int cat_ok(const fcfc_cat *k) {
   return k && k->n >= 0 && k->n < 0x7fffffff && (k->n == 0 || (k->x && k->y && k->z));
 }
@@ -2343,7 +2378,7 @@ bool CopyKey::same(const fcfc_cat *k, int wt_, int need_s, const FkGrid &g_) con
 }
 
 /* weights of a sorted catalogue re-read from the caller's device array */
-struct Gather { const double *src; const int *idx; double *dst; int n; };
+struct Gather { const double *src; const int *idx; double *dst; int n, stride; };
 
 static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
     const fcfc_cat *a, const fcfc_cat *b, const fcfc_bins *bins, const double *bsize,
@@ -2373,12 +2408,13 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
     for (auto &cp : copies)
       if (cp.same(k, wt, need_s, J->P.g)) { *dst[q] = cp.d; found = true; break; }
     if (found) continue;
-    const int slot = (q == 0) ? WS_A_X : WS_B_X;
+    const int slot = (q == 0) ? WS_A_REC : WS_B_REC;
     const int upslot = (q == 0) ? WS_IN_X : WS_IN2_X;
     if ((e = stage_prep(c, al, k, need_s, wt, J->P.g, slot, upslot, dst[q], stages))) return e;
     if (al.own) copies.push_back(CopyKey{k->x, k->y, k->z, k->s, k->w, k->n, wt, J->P.g, *dst[q]});
     if (gathers && wt && k->w && k->on_device && k->n > 0)
-      gathers->push_back(Gather{k->w, dst[q]->idx, dst[q]->w, (int) k->n});
+      gathers->push_back(need_s ? Gather{k->w, dst[q]->idx, dst[q]->w, (int) k->n, 1}
+                                : Gather{k->w, dst[q]->idx, &dst[q]->rec->q, (int) k->n, 4});
   }
   if (autoc) J->B = J->A;
   return 0;
@@ -2562,8 +2598,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     const PJob &J = jobs[k];
     FkJob &f = hj[k];
     memset(&f, 0, sizeof f);
-    f.A = FkCat{J.A.n, J.A.x, J.A.y, J.A.z, J.A.s, J.A.w, J.A.idx, J.A.cs};
-    f.B = FkCat{J.B.n, J.B.x, J.B.y, J.B.z, J.B.s, J.B.w, J.B.idx, J.B.cs};
+    f.A = J.A.dev();
+    f.B = J.B.dev();
     f.g = J.P.g;
     f.strips = dstrips + hstr.size();
     f.nstrips = J.P.nstrips;
@@ -2781,7 +2817,7 @@ static int count_jobs(fcfc_gpu_ctx *c, int njob, const fcfc_cat *const *as,
     if (e) return e;
     jobs[k].hist_off = (long long) k * bins->ntot;
   }
-  if (int e = stage_run(c, al, stages)) return e;
+  if (int e = stage_run(c, al, stages, jobs)) return e;
   const size_t hbytes = 8 * (size_t) bins->ntot * njob;
   void *dh = al.tmp(WS_HIST, hbytes);
   unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 64 * 8);
@@ -2824,12 +2860,12 @@ extern "C" int fcfc_gpu_count(fcfc_gpu_ctx *c, const fcfc_cat *a,
   return count_jobs(c, 1, as, bs, bz, fl, bins, flags, cnt);
 }
 
-/* Device bytes a no-allocation count needs at least (uploads, sorted copies,
- * per-object sort scratch); cells, tiles and histograms come on top. */
+/* Device bytes a no-allocation count needs at least (uploads, sorted copies);
+ * cells, runs and histograms come on top. */
 static size_t noalloc_floor(const fcfc_cat *k, const fcfc_bins *bins, int wt) {
   if (!k || k->n <= 0) return 0;
   const int need_s = (bins->geometry == FCFC_GEOM_SURVEY && bins->bintype != FCFC_BIN_ISO);
-  size_t per = 24 + 4 + 8 + (wt ? 8 : 0) + (need_s ? 8 : 0);     /* sorted copy + sort */
+  size_t per = sizeof(FkRec) + 4 + (wt && need_s ? 8 : 0);       /* sorted copy */
   if (!k->on_device) per += 24 + (wt && k->w ? 8 : 0) + (need_s && k->s ? 8 : 0);
   return per * (size_t) k->n;
 }
@@ -2912,7 +2948,7 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
     hipLaunchKernelGGL(k_fill_f64, dim3(nblk(b->n, 256)), dim3(256), 0, c->stream, dgb, (int64_t) b->n, 0.0);
   jobs[0].gA = sw ? dgb : dga;
   jobs[0].gB = autoc ? dga : (sw ? dga : dgb);
-  if (int e = stage_run(c, al, stages)) return e;
+  if (int e = stage_run(c, al, stages, jobs)) return e;
   double *dG = (double *) al.tmp(WS_G, sizeof(double) * bins->ntot);
   unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 64 * 8);
   if (al.err) return al.err;
@@ -2996,7 +3032,7 @@ extern "C" int fcfc_gpu_plan_create(fcfc_gpu_ctx *c, int njob, const fcfc_batch_
     if (e) return e;
     P->jobs[k].hist_off = (long long) k * bins->ntot;
   }
-  if (int e = stage_run(c, P->al, stages)) return e;
+  if (int e = stage_run(c, P->al, stages, P->jobs)) return e;
   P->dh = P->al.get(WS_HIST, 8 * (size_t) bins->ntot * njob);
   P->misc = (unsigned long long *) P->al.get(WS_MISC, 64 * 8);
   if (P->al.err) return P->al.err;
@@ -3009,7 +3045,7 @@ extern "C" int fcfc_gpu_plan_create(fcfc_gpu_ctx *c, int njob, const fcfc_batch_
   HIPCHK(c, hipStreamSynchronize(c->stream));
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   for (const Gather &g : P->gathers)
-    hipLaunchKernelGGL(k_gather, dim3(nblk(g.n, 256)), dim3(256), 0, c->stream, g.n, g.idx, g.src, g.dst);
+    hipLaunchKernelGGL(k_gather, dim3(nblk(g.n, 256)), dim3(256), 0, c->stream, g.n, g.idx, g.src, g.dst, g.stride);
   hipLaunchKernelGGL(k_zero_u64, dim3(nblk((int64_t) bins->ntot * njob, 256)), dim3(256), 0, c->stream,
       (unsigned long long *) P->dh, bins->ntot * njob);
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, P->misc, 64);

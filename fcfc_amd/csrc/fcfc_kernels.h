@@ -4,8 +4,9 @@
  *
  * Layout in HBM (one catalogue, after the grid build):
  *   objects sorted by cell id  cid = (ix * ncy + iy) * ncz + iz,
- *   FP64 SoA x[], y[], z[] (+ s[] = |r|^2 for survey (s,mu)/(s_perp,pi),
- *   + w[] weights), idx[] = original object index, cell_start[ncell + 1].
+ *   records of four FP64 values (x, y, z and |r|^2 for survey (s,mu) and
+ *   (s_perp,pi), else the weight), w[] the weights where |r|^2 is in the
+ *   record, idx[] = original object index, cell_start[ncell + 1].
  * A "row" is the set of cells sharing (ix, iy): its objects are contiguous and
  * ordered by z-cell, so every z-window of a row is one contiguous range.
  *
@@ -15,9 +16,11 @@
  * separation form at most three contiguous segments (three periodic images in
  * z).  Every wavefront of the persistent workgroups takes its own runs from a
  * global queue: its lanes load 64 B objects, drop those farther than the
- * maximum separation from the bounding box of the run, pack the others into
- * the wavefront's LDS chunk, and every lane evaluates its A objects against
- * each packed B object.  The histograms are shared by the workgroup.
+ * maximum separation from the bounding box of the run, and every lane
+ * evaluates its A objects against each of the others, which the FP64 forms
+ * read into scalar registers and the FP32 ones pack, relative to the run's
+ * centre, into the wavefront's LDS chunk.  The histograms are shared by the
+ * workgroup.
  *
  * Arithmetic contract (FP64 path), after FCFC's AVX-512 leaf kernels
  * (src/fcfc/2pt_box/metric_common.c:377-534):  B objects are staged as
@@ -86,9 +89,16 @@ struct FkGrid {
   double hz_const;           /* >= 0: fixed z half-window (box s_perp,pi)   */
 };
 
+/* One sorted object, read as a whole by scalar and vector loads.  q: |r|^2
+ * for survey (s,mu) and (s_perp,pi) bins, else the weight (weighted jobs). */
+struct alignas(32) FkRec { double x, y, z, q; };
+
+/* rec, w and idx are indexed as cell_start counts: from the first object of
+ * the call's first catalogue */
 struct FkCat {
-  int n;
-  const double *x, *y, *z, *s, *w;
+  int n, pad;
+  const FkRec *rec;
+  const double *w;           /* weights that are not in the records          */
   const int *idx;
   const int *cell_start;
 };
