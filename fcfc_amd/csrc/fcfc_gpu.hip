@@ -140,7 +140,7 @@ __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ s
   }
 }
 
-/* Work items of the run list: run ti becomes S items (each a share of the
+/* Work items of a job's runs: run ti becomes S items (each a share of the
  * strip list) for ti < tt and St > S finer items from tt on, so that the
  * items the wavefronts take last are short and the launch ends evenly.
  * ncap runs in all: of each group of G consecutive runs of the list, its
@@ -148,17 +148,44 @@ __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ s
  * runs); the autotuner's samples take stretches spread over the whole
  * catalogue, each keeping the neighbourhood, and so the cache reuse, of a
  * full count. */
-struct FkSplit { int S, tt, St, ncap, G, run; };
+struct FkSplit { int S, tt, St, ncap, G, run, nitems, run0; };   /* run0: its first run */
 
-__host__ __device__ inline long long split_pos(const FkSplit &s, int ti) {
-  return ti < s.tt ? (long long) s.S * ti
-                   : (long long) s.S * s.tt + (long long) s.St * (ti - s.tt);
+/* The split of nrun runs of smax strips at most and of about `chunks` chunks
+ * of 64 candidate B objects each, for nw wavefronts: 16 items per wavefront,
+ * but none of fewer than 8 chunks (an item loads its A objects and searches
+ * its strips first, about the work of a chunk: survey (s_perp, pi) DR of 3e4 x
+ * 1e6 1.95 -> 1.61 ms, small-scale cross count 1.61 -> 1.11 ms against 16 items
+ * whatever their size; large counts unchanged); where that leaves wavefronts
+ * without an item, one each, of 2 chunks at least. */
+__host__ __device__ inline FkSplit fk_split(int nrun, int nw, int chunks, int smax, int frac) {
+  FkSplit sp = {1, 0, 1, 0, nrun > 1 ? nrun : 1, nrun > 1 ? nrun : 1, 0, 0};
+  if (nrun <= 0) return sp;
+  if (frac > 1) {
+    sp.G = (nrun + 15) / 16;
+    sp.run = sp.G / frac > 1 ? sp.G / frac : 1;
+  }
+  const int last = (nrun - 1) / sp.G, rest = nrun - last * sp.G;
+  sp.ncap = last * sp.run + (sp.run < rest ? sp.run : rest);
+  auto lim = [](long long v, int most) -> int { return (int) (v < most ? v : most); };
+  auto one = [](int v) -> int { return v > 1 ? v : 1; };
+  const int s16 = lim((16LL * nw + sp.ncap - 1) / sp.ncap, one(chunks / 8));
+  const int s1 = lim(((long long) nw + sp.ncap - 1) / sp.ncap, one(chunks / 2));
+  sp.S = one(lim(s16 > s1 ? s16 : s1, smax));
+  /* the runs of about two items per wavefront at the end of the list are
+   * split four times finer */
+  sp.St = one(lim(4LL * sp.S, smax));
+  const long long tail = (2LL * nw + sp.S - 1) / sp.S;
+  sp.tt = tail < sp.ncap ? sp.ncap - (int) tail : 0;
+  if (sp.St <= sp.S) { sp.St = sp.S; sp.tt = sp.ncap; }
+  if ((long long) sp.St * sp.ncap > (1LL << 30)) { sp.S = sp.St = 1; sp.tt = sp.ncap; }
+  sp.nitems = sp.S * sp.tt + sp.St * (sp.ncap - sp.tt);
+  return sp;
 }
 
-/* Runs of all jobs of a launch: job k owns the units unit0 .. unit0 + nrow
- * nblk - 1 (unit0 ascending); a unit is one block of zm z-cells of one row,
- * cut into runs of T consecutive objects. */
-struct FkTileJob { int unit0, nblk, zm, ncz, T; const int *cs; };
+/* Runs of all jobs of a launch: job k owns nunit units from unit0 (ascending);
+ * a unit is one block of zm z-cells of one row, cut into runs of T consecutive
+ * objects.  nw, chunks, smax, frac: its split (fk_split). */
+struct FkTileJob { int unit0, nunit, nblk, zm, ncz, T, nw, chunks, smax, frac; const int *cs; };
 
 __device__ __forceinline__ int fk_tile_job(const FkTileJob *__restrict__ tj, int njob, int u) {
   int lo = 0, hi = njob - 1;                  /* last job with unit0 <= u */
@@ -186,16 +213,22 @@ __global__ void k_run_count(int nunit, int njob, const FkTileJob *__restrict__ t
     nrun[u] = (p1 - p0 + t.T - 1) / t.T;
   }
 }
-/* the runs of unit u are numbered from roff[u] */
+/* the runs of unit u are numbered from roff[u]; the split of every job */
 __global__ void k_run_emit(int nunit, int njob, const FkTileJob *__restrict__ tj,
-    const int *__restrict__ roff, FkRun *__restrict__ runs) {
-  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nunit; u += gridDim.x * blockDim.x) {
-    const int k = fk_tile_job(tj, njob, u);
+    const int *__restrict__ roff, FkRun *__restrict__ runs, FkSplit *__restrict__ splits) {
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < njob; k += gridDim.x * blockDim.x) {
     const FkTileJob t = tj[k];
+    FkSplit sp = fk_split(roff[t.unit0 + t.nunit] - roff[t.unit0], max(t.nw, FK_NW), t.chunks, t.smax,
+                          t.frac);
+    sp.run0 = roff[t.unit0];
+    splits[k] = sp;
+  }
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nunit; u += gridDim.x * blockDim.x) {
+    const FkTileJob t = tj[fk_tile_job(tj, njob, u)];
     int p0, p1;
     const int row = fk_unit(t, u, p0, p1);
     FkRun *o = runs + roff[u];
-    for (int p = p0; p < p1; p += t.T) *o++ = FkRun{row, p, min(p + t.T, p1), k};
+    for (int p = p0; p < p1; p += t.T) *o++ = FkRun{row, p, min(p + t.T, p1), 0};
   }
 }
 
@@ -316,6 +349,8 @@ struct FkJob {
   int autoc;                  /* COUNT: A == B, half shell + self tile;
                                  GRAD: A == B, exclude j == i          */
   int wt;                     /* weighted histogram (double)          */
+  int wg0, wg1;               /* workgroups that start with it        */
+  int qi;                     /* its counter in the queue             */
   long long hist_off;         /* histogram of this job: gcnt + hist_off */
   double *gA;                 /* GRAD: output for A objects, original order (or null) */
   double *gB;                 /* GRAD: output for B objects, original order (or null;
@@ -328,9 +363,8 @@ struct FkArgs {
   int njobs;
   FkBins bins;
   const FkRun *runs;
-  FkSplit sp;                 /* work items of the runs              */
-  int nitems;
-  unsigned int *queue;
+  const FkSplit *splits;      /* work items of each job              */
+  unsigned int *queue;        /* work items taken, per job            */
   unsigned long long *gcnt_u;
   double *gcnt_d;
   unsigned long long *stats;  /* evals, rechecked, census */
@@ -1003,7 +1037,7 @@ k_count(const FkArgs a) {
    * object, A slot in the run << 5 | periodic image code */
   unsigned *wqj = (unsigned *) (lds + a.off_queue + wave * (FK_QCAP * 6));
   uint16_t *wqs = (uint16_t *) (wqj + FK_QCAP);
-  __shared__ int s_next[FK_NW];
+  __shared__ int s_job;
   __shared__ double s_box[FK_NW][6];           /* bounding boxes of the runs */
   double *box = s_box[wave];
 
@@ -1103,28 +1137,35 @@ k_count(const FkArgs a) {
   const unsigned ohist_g = (unsigned) a.off_hist - 8u * ioff;
   const int lane = tid & 63;
 
-  /* The wavefronts of a workgroup run on their own and meet only here: at
-   * the start, when the job changes, at the end of the queue (want = FK_END)
-   * and when a wavefront has used up its budget of 32-bit counts (want =
-   * cur).  Each round every wavefront posts the job it wants; the LDS
-   * histograms are added to the global one of the job counted so far, and
-   * the smallest wanted job comes next.  The queue hands out items in job
-   * order, so a wavefront that wants a later job waits in the next round for
-   * those that still count this one; every round sees all wavefronts, and
-   * the last one (all want FK_END) ends them all. */
-#define FK_END 0x7fffffff
+  /* 32-bit counters: a wavefront that may have added FK_BUDGET pairs since
+   * it last did so adds the workgroup's counters to the job's global histogram
+   * (the others go on counting meanwhile), so that FK_NW budgets bound every
+   * counter below 2^32 */
 #define FK_BUDGET 500000000u
   int cur = -1;
-  auto job_round = [&](int want) -> int {
-    if (lane == 0) s_next[wave] = want;
+  auto spill_counts = [&]() {
+    unsigned long long *g0 = a.gcnt_u + fk_cld(&fk_again(a.jobs, cur)->hist_off);
+    for (int i = lane; i < hist_elems; i += 64) {
+      const int g = fk_hslot(i % bn.ntoh, bn.ns, bn.nsh);
+      const unsigned v = atomicExch(hist_u + i, 0u);
+      if (g >= 0 && v) atomicAdd(g0 + g, (unsigned long long) v);
+    }
+    since = 0;
+  };
+
+  /* Each workgroup counts one job at a time; its wavefronts take the job's
+   * items on their own and meet when it has none left.  Then the LDS
+   * histograms are added to the job's global one and the workgroup goes on to
+   * a job that has some: in a batch the workgroups start dealt out to the jobs
+   * in proportion to their expected work, so that most count one job and
+   * flush once (with one queue for all jobs every workgroup visited every job:
+   * 16 mocks, 48 jobs, 8.7 -> 5.9 ms). */
+  for (;;) {
     __syncthreads();
-    int nx = s_next[0];
-    for (int q = 1; q < FK_NW; q++) nx = min(nx, s_next[q]);
-    nx = __builtin_amdgcn_readfirstlane(nx);
     if (!GRAD && cur >= 0) {
-      const FkJob *pj = a.jobs + cur;
-      const bool w = WT && pj->wt;
-      const long long ho = pj->hist_off;
+      const FkJob *pj = fk_again(a.jobs, cur);
+      const bool w = WT && fk_cld(&pj->wt);
+      const long long ho = fk_cld(&pj->hist_off);
       for (int i = tid; i < bn.ntoh; i += FK_NT) {
         const int g = fk_hslot(i, bn.ns, bn.nsh);    /* padding slots stay 0 */
         if (g < 0) continue;
@@ -1141,32 +1182,57 @@ k_count(const FkArgs a) {
       }
     }
     since = 0;
+    bool first = cur < 0;
+    if (wave == 0) {
+      int nx = -1;
+      if (first) {
+        int hi = a.njobs - 1;                 /* last job with wg0 <= this workgroup */
+        nx = 0;
+        while (nx < hi) {
+          const int mid = (nx + hi + 1) >> 1;
+          if (a.jobs[mid].wg0 <= (int) blockIdx.x) nx = mid; else hi = mid - 1;
+        }
+      }
+      /* the next job (in turn from this one) with items for every wavefront */
+      else for (int k0 = 1; k0 < a.njobs && nx < 0; k0 += 64) {
+        bool has = false;
+        if (k0 + lane < a.njobs) {
+          int q = cur + k0 + lane;
+          if (q >= a.njobs) q -= a.njobs;
+          const int nw = (a.jobs[q].wg1 - a.jobs[q].wg0) * FK_NW;
+          const long long taken = nw + (long long) __hip_atomic_load(a.queue + a.jobs[q].qi,
+              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          has = taken + (nw ? FK_NW - 1 : 0) < a.splits[q].nitems;
+        }
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(has);
+        if (m) { nx = cur + k0 + (int) __builtin_ctzll(m); if (nx >= a.njobs) nx -= a.njobs; }
+      }
+      if (lane == 0) s_job = nx;
+    }
     __syncthreads();
-    return nx;
-  };
+    cur = __builtin_amdgcn_readfirstlane(s_job);
+    if (cur < 0) break;
 
-  /* the first item of a wavefront is its own index, the others follow from
-   * the queue */
-  const int nwaves = (int) gridDim.x * FK_NW;
-  int it = (int) blockIdx.x * FK_NW + wave;
-  for (bool first = true;; first = false) {
+  /* the job's items: the first one of each wavefront that starts with the
+   * job is its own index, the others follow from the queue */
+  for (;; first = false) {
+    const FkSplit sp = fk_cld(a.splits + cur);
+    const FkJob *pq = fk_again(a.jobs, cur);
+    const int wg0 = fk_cld(&pq->wg0), nw = (fk_cld(&pq->wg1) - wg0) * FK_NW;
+    int it = ((int) blockIdx.x - wg0) * FK_NW + wave;
     if (!first) {
-      if (lane == 0) it = nwaves + (int) atomicAdd(a.queue, 1u);
+      if (lane == 0) it = nw + (int) atomicAdd(a.queue + fk_cld(&pq->qi), 1u);
       it = __builtin_amdgcn_readfirstlane(it);
     }
+    if (it >= sp.nitems) break;
     /* work item -> run and share of its strips */
-    int part = 0, S = 1;
-    FkRun t = {0, 0, 0, FK_END};
-    if (it < a.nitems) {
-      int ri;
-      const int h = a.sp.S * a.sp.tt;
-      if (it < h) { S = a.sp.S; ri = it / S; part = it - ri * S; }
-      else { S = a.sp.St; ri = (it - h) / S; part = it - h - ri * S; ri += a.sp.tt; }
-      const int grp = ri / a.sp.run;
-      t = fk_cld(a.runs + (grp * a.sp.G + (ri - grp * a.sp.run)));
-    }
-    while (t.job != cur) cur = job_round(t.job);
-    if (cur == FK_END) break;
+    int part, S, ri;
+    const int h = sp.S * sp.tt;
+    if (it < h) { S = sp.S; ri = it / S; part = it - ri * S; }
+    else { S = sp.St; ri = (it - h) / S; part = it - h - ri * S; ri += sp.tt; }
+    const int grp = ri / sp.run;
+    const FkRun t = fk_cld(a.runs + __builtin_amdgcn_readfirstlane(
+        sp.run0 + grp * sp.G + (ri - grp * sp.run)));
 
     const FkJob J = fk_cld(a.jobs + cur);
     const int s0 = (int) ((long long) J.nstrips * part / S);
@@ -1413,7 +1479,7 @@ k_count(const FkArgs a) {
         if (m == 0) continue;
         const int cnt = __popcll(m);
         if (!GRAD && !jwt) {
-          if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) (void) job_round(cur);
+          if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) spill_counts();
           since += (unsigned) cnt * (unsigned) nva;
         }
         if (F32) {
@@ -1523,6 +1589,7 @@ k_count(const FkArgs a) {
             unsafeAtomicAdd(gA + fk_gld(idx, ai[r]), gacc[r]);
     }
   }
+  }
 
   if (lane == 0) atomicAdd(a.stats + 0, evals);
   if (F32) {
@@ -1572,9 +1639,7 @@ struct fcfc_gpu_ctx {
   int census = 0;
   int tile_frac = 0;           /* autotuner: count about 1/tile_frac of the
                                   tiles (16 runs spread over the list) */
-  /* tiles (before their split into work items) of the last launch built */
-  int last_ntiles = 0;
-  int last_nsampled = 0;       /* ... and how many of them it counted */
+  const int *last_nrun = nullptr;  /* device: runs of the last launch built */
   struct Tuned { int geom, bintype, mode, autoc, wt, bucket, cd, zd, T; };
   std::vector<Tuned> tuned;    /* autotuner results per density bucket */
   std::vector<DevBuf> bufs;
@@ -1597,7 +1662,7 @@ static void set_err(fcfc_gpu_ctx *c, const char *fmt, ...) {
 enum {
   WS_IN_X, WS_IN_Y, WS_IN_Z, WS_IN_S, WS_IN_W,          /* uploads, catalogue A */
   WS_IN2_X, WS_IN2_Y, WS_IN2_Z, WS_IN2_S, WS_IN2_W,     /* uploads, catalogue B */
-  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES,
+  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES, WS_SPLITS,
   WS_STRIPS, WS_STAB, WS_PTAB, WS_S2E, WS_PE, WS_HIST, WS_MISC, WS_G, WS_GA, WS_GB, WS_JOBS,
   WS_NSLOT
 };
@@ -1694,6 +1759,7 @@ struct JobPlan {
   int T;            /* objects per tile (the FK_NW runs of a workgroup) */
   int zmaxc;        /* z-cells per block of a row: no run crosses blocks */
   int nblk;         /* blocks per row */
+  double cand;      /* candidate B objects of one run in a uniform catalogue */
   int R;            /* objects per lane */
   int T_auto;       /* T chosen by the plan (not by the caller's tuning) */
   std::vector<int> strips;
@@ -1833,11 +1899,15 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
   if (tT > 0) P->T = std::min(tT, 4 * FK_NT);
   else P->T = cube > 0.75 * R ? FK_NT : 2 * FK_NT;
   P->R = (P->T + FK_NT - 1) / FK_NT;
-  /* blocks of about four runs, at least two cells wide: the z extent of a
-   * run (and with it the FP32 windows) stays bounded in sparse rows */
+  /* blocks of about sixteen runs (the last run of a block is half empty on
+   * average: four runs, (s, mu) DR 15.9 -> 15.1 ms), at least two cells wide:
+   * the z extent of a run, and with it the FP32 windows, stays bounded in
+   * sparse rows.  Four for the survey FP32 form, whose windows grow most
+   * (more pairs re-evaluated: (s, mu) RR 15.6 against 16.5 ms). */
+  const double nrb = (mode == MODE_C32 && b->geometry == FCFC_GEOM_SURVEY) ? 4.0 : 16.0;
   {
     const double per_cell = (double) nA / ((double) g.ncx * g.ncy * g.ncz);
-    const double zc = std::max(2.0 * zd, ceil(4.0 * 64 * P->R / std::max(per_cell, 1e-9)));
+    const double zc = std::max(2.0 * zd, ceil(nrb * 64 * P->R / std::max(per_cell, 1e-9)));
     P->zmaxc = (int) std::min((double) g.ncz, zc);
     P->nblk = (g.ncz + P->zmaxc - 1) / P->zmaxc;
   }
@@ -1859,6 +1929,14 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
     }
   }
   P->nstrips = (int) P->strips.size() / 3;
+  P->cand = 0;
+  const double rlen = std::min(64.0 * P->R / std::max(ndenA * g.wx * g.wy, 1e-300), ext[2]);
+  for (int q = 0; q < P->nstrips; q++) {
+    const double gx = std::max(abs(P->strips[3 * q]) - 1, 0) * g.wx;
+    const double gy = std::max(abs(P->strips[3 * q + 1]) - 1, 0) * g.wy;
+    const double hz = (hzc >= 0) ? hzc : sqrt(std::max(r2 - gx * gx - gy * gy, 0.0));
+    P->cand += nden * g.wx * g.wy * std::min(2 * hz + rlen, ext[2]);
+  }
   return 0;
 }
 
@@ -1882,6 +1960,7 @@ struct PJob {
   int autoc = 0, wt = 0;
   double *gA = nullptr, *gB = nullptr;
   long long hist_off = 0;
+  int qi = 0;                   /* counter of its work items */
 };
 
 static inline int nblk(int64_t n, int bs) {
@@ -2426,7 +2505,7 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
  * depend on how the runtime stages pageable host memory. */
 struct Launch {
   kfn_t fn = nullptr;
-  int nblock = 0, lds = 0, nitems = 0;
+  int nblock = 0, lds = 0;
   FkArgs a;
   std::vector<int> hstr;
   std::vector<FkJob> hj;
@@ -2516,13 +2595,43 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
   }
   HIPCHK(c, hipFuncSetAttribute((const void *) fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.total));
   /* ---- runs of all jobs ---- */
+  /* persistent workgroups, dealt out to the jobs in proportion to the
+   * candidate pairs of their runs (each run at least one chunk) */
+  int occ = 0;
+  HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *) fn, FK_NT, L.total));
+  if (occ < 1) occ = 1;
+  int nwg = c->t_nblock > 0 ? c->t_nblock : occ * c->ncu;
+  const int njob = (int) jobs.size();
   std::vector<FkTileJob> htj(jobs.size());
-  long long nunit_l = 0;
-  for (size_t k = 0; k < jobs.size(); k++) {
+  std::vector<int> wg0(jobs.size() + 1, 0);
+  long long nunit_l = 0, maxrun = 0, maxitem = 0;
+  double work = 0, done = 0;
+  for (int k = 0; k < njob; k++) {
     const PJob &J = jobs[k];
-    htj[k] = FkTileJob{(int) nunit_l, J.P.nblk, J.P.zmaxc, J.P.g.ncz, std::min(J.P.T, 64 * J.P.R), J.A.cs};
-    nunit_l += (long long) J.P.g.ncx * J.P.g.ncy * J.P.nblk;
+    FkTileJob &t = htj[k];
+    memset(&t, 0, sizeof t);
+    const long long nu = (long long) J.P.g.ncx * J.P.g.ncy * J.P.nblk;
+    t.unit0 = (int) nunit_l;
+    t.nunit = (int) nu;
+    t.nblk = J.P.nblk; t.zm = J.P.zmaxc; t.ncz = J.P.g.ncz;
+    t.T = std::min(J.P.T, 64 * J.P.R);
+    t.chunks = (int) std::min(J.P.cand / 64, 1e9);
+    t.smax = std::min(std::max(J.P.nstrips, 1), 64);
+    t.frac = c->tile_frac;
+    t.cs = J.A.cs;
+    nunit_l += nu;
     if (nunit_l > INT_MAX / 2) { set_err(c, "catalogues of one call too large"); return FCFC_ERR_CFG; }
+    /* at most as many runs as full ones and one remainder per non-empty unit */
+    const long long nr = J.A.n / t.T + std::min<long long>(nu, J.A.n);
+    maxrun += nr;
+    maxitem += nr * t.smax;
+    work += (double) J.A.n * std::max(J.P.cand, 64.0);
+  }
+  nwg = (int) std::max<long long>(1, std::min<long long>(nwg, (maxitem + FK_NW - 1) / FK_NW));
+  for (int k = 0; k < njob; k++) {
+    done += (double) jobs[k].A.n * std::max(jobs[k].P.cand, 64.0);
+    wg0[k + 1] = k + 1 == njob ? nwg : (int) (work > 0 ? nwg * std::min(done / work, 1.0) : 0.0);
+    htj[k].nw = (wg0[k + 1] - wg0[k]) * FK_NW;
   }
   const int nunit = (int) nunit_l;
   int *unitn = (int *) al.get(WS_ROWN, sizeof(int) * (size_t) nunit);
@@ -2530,51 +2639,15 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
   FkTileJob *dtj = (FkTileJob *) al.get(WS_TJOBS, sizeof(FkTileJob) * jobs.size());
   if (al.err) return al.err;
   HIPCHK(c, hipMemcpyAsync(dtj, htj.data(), sizeof(FkTileJob) * jobs.size(), hipMemcpyHostToDevice, c->stream));
-  const int njob = (int) jobs.size();
   if (nunit > 0)
     hipLaunchKernelGGL(k_run_count, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj, unitn);
   hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, unitn, unitoff, nunit);
-  int nrun = 0;
-  HIPCHK(c, hipMemcpyAsync(&nrun, unitoff + nunit, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  /* persistent workgroups, and work items per run: enough items that the
-   * last ones are short against the whole (16 per wavefront) */
-  int occ = 0;
-  HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *) fn, FK_NT, L.total));
-  if (occ < 1) occ = 1;
-  const int nwg = c->t_nblock > 0 ? c->t_nblock : occ * c->ncu;
-  const long long nwave = (long long) nwg * FK_NW;
-  /* the autotuner's samples count about 1/tile_frac of the runs, in 16
-   * stretches of consecutive runs spread evenly over the list, split into
-   * work items by the same rule as a full count (about 16 per wavefront), so
-   * that a sample ends as evenly */
-  int grp = std::max(nrun, 1), run = grp;
-  if (c->tile_frac > 1 && nrun > 0) {
-    grp = (nrun + 15) / 16;
-    run = std::max(1, grp / c->tile_frac);
-  }
-  const int glast = nrun > 0 ? (nrun - 1) / grp : 0;
-  const int ncap = nrun > 0 ? glast * run + std::min(run, nrun - glast * grp) : 0;
-  FkSplit sp{1, ncap, 1, ncap, grp, run};
-  if (nrun > 0) {
-    int minstr = 1 << 30;
-    for (auto &j : jobs) minstr = std::min(minstr, std::max(j.P.nstrips, 1));
-    const int smax = std::min(minstr, 64);
-    sp.S = (int) std::min<long long>(std::max<long long>(1, (16LL * nwave + ncap - 1) / ncap),
-                                     smax);
-    /* the runs of about two items per wavefront at the end of the list
-     * are split four times finer */
-    sp.St = std::min(4 * sp.S, smax);
-    sp.tt = (int) std::max<long long>(0, ncap - (2LL * nwave + sp.S - 1) / sp.S);
-    if (sp.St <= sp.S) { sp.St = sp.S; sp.tt = ncap; }
-    if (split_pos(sp, ncap) > (1LL << 30)) sp = FkSplit{1, ncap, 1, ncap, grp, run};
-  }
-  const int nitems = (int) split_pos(sp, ncap);
-  FkRun *runs = (FkRun *) al.get(WS_TILES, sizeof(FkRun) * (size_t) (nrun > 0 ? nrun : 1));
+  FkRun *runs = (FkRun *) al.get(WS_TILES, sizeof(FkRun) * (size_t) (maxrun > 0 ? maxrun : 1));
+  FkSplit *splits = (FkSplit *) al.get(WS_SPLITS, sizeof(FkSplit) * jobs.size());
   if (al.err) return al.err;
   if (nunit > 0)
     hipLaunchKernelGGL(k_run_emit, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj,
-                       unitoff, runs);
+                       unitoff, runs, splits);
   /* ---- tables, strips, job descriptors ---- */
   size_t nstr = 0;
   for (auto &j : jobs) nstr += j.P.strips.size();
@@ -2606,6 +2679,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     f.autoc = J.autoc;
     f.wt = J.wt;
     f.hist_off = J.hist_off;
+    f.wg0 = wg0[k];
+    f.wg1 = wg0[k + 1];
+    f.qi = J.qi;
     f.gA = J.gA;
     f.gB = J.gB;
     if (m == MODE_C32) {
@@ -2686,7 +2762,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     fb.q_pad = 0;
   }
   fb.stab = dstab; fb.ptab = dptab; fb.s2bin = ds2e; fb.pbin = dpe;
-  a.runs = runs; a.sp = sp; a.nitems = nitems;
+  a.runs = runs; a.splits = splits;
   a.queue = dqueue;
   a.gcnt_u = (unsigned long long *) dhist; a.gcnt_d = (double *) dhist;
   a.stats = dstats;
@@ -2697,15 +2773,16 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
   a.off_chunk = L.off_chunk; a.off_queue = L.off_queue;
   a.census = c->census;
   a.G = G;
-  int nblock = nwg;
-  if (nblock > (nitems + FK_NW - 1) / FK_NW) nblock = std::max((nitems + FK_NW - 1) / FK_NW, 1);
-  c->last_ntiles = nrun;
-  c->last_nsampled = ncap;
+  c->last_nrun = unitoff + nunit;
   c->stats.tile = jobs.empty() ? 0 : jobs[0].P.T;
   c->stats.cell_div = jobs.empty() ? 0 : (int) lround(sqrt(jobs[0].P.g.Rxy2) / jobs[0].P.g.wx);
-  out->fn = fn; out->nblock = nblock; out->lds = L.total; out->nitems = a.nitems; out->a = a;
+  out->fn = fn; out->nblock = nwg; out->lds = L.total; out->a = a;
   return 0;
 }
+
+/* Counters of a call, zeroed before its launches: 8 words of statistics and
+ * the queue, one 32-bit word per job. */
+static int misc_words(int njob) { return 8 + (njob + 1) / 2; }
 
 /* Waits for the stream when it goes out of scope: declared after the
  * launches of a call (destroyed before them), it keeps their host copies
@@ -2716,7 +2793,7 @@ struct StreamDrain {
 };
 
 static int launch(fcfc_gpu_ctx *c, const Launch &Lc) {
-  if (Lc.nitems > 0)
+  if (Lc.nblock > 0)
     hipLaunchKernelGGL(Lc.fn, dim3(Lc.nblock), dim3(FK_NT), Lc.lds, c->stream, Lc.a);
   HIPCHK(c, hipGetLastError());
   return 0;
@@ -2816,22 +2893,24 @@ static int count_jobs(fcfc_gpu_ctx *c, int njob, const fcfc_cat *const *as,
     int e = setup_job(c, al, copies, as[k], bs[k], bins, bsz[k], autoc, wt, mode, &jobs[k], stages);
     if (e) return e;
     jobs[k].hist_off = (long long) k * bins->ntot;
+    jobs[k].qi = k;
   }
   if (int e = stage_run(c, al, stages, jobs)) return e;
   const size_t hbytes = 8 * (size_t) bins->ntot * njob;
   void *dh = al.tmp(WS_HIST, hbytes);
-  unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 64 * 8);
+  const int nmisc = misc_words((int) jobs.size());
+  unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 8 * (size_t) nmisc);
   if (al.err) return al.err;
   hipLaunchKernelGGL(k_zero_u64, dim3(nblk((int64_t) bins->ntot * njob, 256)), dim3(256), 0, c->stream,
       (unsigned long long *) dh, bins->ntot * njob);
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, misc, 64);
+  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nmisc, 256)), dim3(256), 0, c->stream, misc, nmisc);
   /* one persistent launch per group (each with its own queue word) */
   std::vector<std::vector<PJob>> groups = launch_groups(jobs);
   std::vector<Launch> L(groups.size());
   StreamDrain drain{c};
   for (size_t q = 0; q < groups.size(); q++) {
-    int e = build_launch(c, al, bins, groups[q], mode, nullptr, dh, misc + 8,
-                         (unsigned int *) misc + q, &L[q]);
+    int e = build_launch(c, al, bins, groups[q], mode, nullptr, dh, misc,
+                         (unsigned int *) (misc + 8), &L[q]);
     if (e) return e;
   }
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -2842,7 +2921,7 @@ static int count_jobs(fcfc_gpu_ctx *c, int njob, const fcfc_cat *const *as,
   HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   int e = deliver(c, jobs, bins->ntot, dh, flags, cnt);
   if (e) return e;
-  if ((e = stats_from(c, misc + 8))) return e;
+  if ((e = stats_from(c, misc))) return e;
   c->stats.kernel_ms = ms;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->stats.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -2950,13 +3029,14 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
   jobs[0].gB = autoc ? dga : (sw ? dga : dgb);
   if (int e = stage_run(c, al, stages, jobs)) return e;
   double *dG = (double *) al.tmp(WS_G, sizeof(double) * bins->ntot);
-  unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 64 * 8);
+  const int nmisc = misc_words((int) jobs.size());
+  unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 8 * (size_t) nmisc);
   if (al.err) return al.err;
   HIPCHK(c, hipMemcpyAsync(dG, grad_cnt, sizeof(double) * bins->ntot,
       dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, misc, 64);
+  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nmisc, 256)), dim3(256), 0, c->stream, misc, nmisc);
   float ms = 0;
-  int e = run_jobs(c, al, bins, jobs, MODE_GRAD, dG, nullptr, misc + 8, (unsigned int *) misc, &ms);
+  int e = run_jobs(c, al, bins, jobs, MODE_GRAD, dG, nullptr, misc, (unsigned int *) (misc + 8), &ms);
   if (e) return e;
   for (int p = 0; p < 2; p++) {
     const fcfc_cat *k = p ? b : a;
@@ -2973,7 +3053,7 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
       for (int64_t i = 0; i < k->n; i++) gout[i] += h[(size_t) i];
     }
   }
-  if ((e = stats_from(c, misc + 8))) return e;
+  if ((e = stats_from(c, misc))) return e;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->stats.kernel_ms = ms;
   c->stats.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -3031,24 +3111,26 @@ extern "C" int fcfc_gpu_plan_create(fcfc_gpu_ctx *c, int njob, const fcfc_batch_
                       &P->gathers);
     if (e) return e;
     P->jobs[k].hist_off = (long long) k * bins->ntot;
+    P->jobs[k].qi = k;
   }
   if (int e = stage_run(c, P->al, stages, P->jobs)) return e;
   P->dh = P->al.get(WS_HIST, 8 * (size_t) bins->ntot * njob);
-  P->misc = (unsigned long long *) P->al.get(WS_MISC, 64 * 8);
+  const int nmisc = misc_words(njob);
+  P->misc = (unsigned long long *) P->al.get(WS_MISC, 8 * (size_t) nmisc);
   if (P->al.err) return P->al.err;
   std::vector<std::vector<PJob>> groups = launch_groups(P->jobs);
   P->L.resize(groups.size());
   int e = 0;
   for (size_t q = 0; q < groups.size(); q++)
-    if ((e = build_launch(c, P->al, bins, groups[q], mode, nullptr, P->dh, P->misc + 8,
-                          (unsigned int *) P->misc + q, &P->L[q]))) return e;
+    if ((e = build_launch(c, P->al, bins, groups[q], mode, nullptr, P->dh, P->misc,
+                          (unsigned int *) (P->misc + 8), &P->L[q]))) return e;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   for (const Gather &g : P->gathers)
     hipLaunchKernelGGL(k_gather, dim3(nblk(g.n, 256)), dim3(256), 0, c->stream, g.n, g.idx, g.src, g.dst, g.stride);
   hipLaunchKernelGGL(k_zero_u64, dim3(nblk((int64_t) bins->ntot * njob, 256)), dim3(256), 0, c->stream,
       (unsigned long long *) P->dh, bins->ntot * njob);
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, P->misc, 64);
+  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nmisc, 256)), dim3(256), 0, c->stream, P->misc, nmisc);
   for (const Launch &Lq : P->L) if ((e = launch(c, Lq))) break;
   hipGraph_t graph = nullptr;
   const hipError_t ce = hipStreamEndCapture(c->stream, &graph);
@@ -3072,7 +3154,7 @@ extern "C" int fcfc_gpu_plan_run(fcfc_gpu_plan *P, void *cnt) {
   HIPCHK(c, hipEventRecord(c->ev1, c->stream));
   int e = deliver(c, P->jobs, P->ntot, P->dh, P->flags, cnt);
   if (e) return e;
-  if ((e = stats_from(c, P->misc + 8))) return e;
+  if ((e = stats_from(c, P->misc))) return e;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   float ms = 0;
   HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
@@ -3131,17 +3213,20 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
     c->tile_frac = 1 << 30;
     int e = run();
     if (e) return e;
-    const int nt = c->last_ntiles;
+    int nt = 0;
+    HIPCHK(c, hipMemcpyAsync(&nt, c->last_nrun, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     /* small counts (a few thousand tiles, milliseconds) are timed whole: an
      * eighth of them is too few tiles to rank shapes */
     c->tile_frac = (nt <= 4096 * FK_NW) ? 1 : (nt > 16384 * FK_NW ? 16 : 8);
     e = run();
     if (e) return e;
-    *est = c->stats.kernel_ms * (double) nt / (double) std::max(1, c->last_nsampled);
+    const int ns = fk_split(nt, 1, 1, 1, c->tile_frac).ncap;     /* runs counted */
+    *est = c->stats.kernel_ms * (double) nt / (double) std::max(1, ns);
     last_T = c->stats.tile;
     if (tune_log)
-      fprintf(stderr, "fcfc_gpu_autotune: cell_div %d zcell_div %d tile %d: %d of %d tiles "
-              "in %.3f ms, estimate %.3f ms\n", cd, zd, last_T, c->last_nsampled, nt,
+      fprintf(stderr, "fcfc_gpu_autotune: cell_div %d zcell_div %d tile %d: %d of %d runs "
+              "in %.3f ms, estimate %.3f ms\n", cd, zd, last_T, ns, nt,
               c->stats.kernel_ms, *est);
     return 0;
   };

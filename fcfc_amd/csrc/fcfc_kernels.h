@@ -107,7 +107,7 @@ struct FkCat {
  * its job.  A work item is a run with a share of the strip list, so that the
  * queue stays long (items of one run add into the same histograms; only the
  * item of the first share counts the pairs inside the run). */
-struct FkRun { int row, p0, p1, job; };
+struct FkRun { int row, p0, p1, pad; };
 
 /* Floor of the exact quotient a / b for a >= 0, b > 0 (b not tiny):
  * approximate quotient from the hardware reciprocal, then one-step
