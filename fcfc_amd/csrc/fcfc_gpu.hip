@@ -47,28 +47,56 @@ __global__ void k_zero_u64(unsigned long long *p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
 }
 
-/* Exclusive scan of n ints into out[0..n] (out[n] = total) and in place into
- * in[0..n-1], one workgroup of 1024 threads, each scanning a contiguous
- * slice. */
-__global__ void __launch_bounds__(1024) k_scan1(int *__restrict__ in,
-    int *__restrict__ out, int n) {
-  __shared__ int part[1024];
-  const int t = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int b = t * per, e = min(n, b + per);
+/* Exclusive scan of n ints into out[0..n] (out[n] = total).  Workgroups of
+ * 1024 threads scan FK_SCAN consecutive ints each; with more than one, k_scan_sum
+ * has written the workgroups' totals before, and each adds up those of the
+ * workgroups ahead of it (a chain between the workgroups would serialize
+ * them).  One workgroup walking all cells took 190 us for 1.1e5 and 1.1 ms for
+ * 5.8e5 cells, these two launches 4.8 + 4.9 us for 2.9e5. */
+#define FK_SCAN 4096
+__device__ __forceinline__ int fk_scan_load(const int *in, int n, int i, int v[4]) {
   int s = 0;
-  for (int i = b; i < e; i++) s += in[i];
-  part[t] = s;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    int v = (t >= off) ? part[t - off] : 0;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; q++) { v[q] = i + q < n ? in[i + q] : 0; s += v[q]; }
+  return s;
+}
+/* sum of v over the workgroup's threads before this one (and of all) */
+__device__ __forceinline__ int fk_scan_block(int v, int *all) {
+  __shared__ int part[16];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int inc = v;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
   }
-  int run = part[t] - s;
-  for (int i = b; i < e; i++) { int v = in[i]; out[i] = run; in[i] = run; run += v; }
-  if (t == 1023) out[n] = part[1023];
+  if (lane == 63) part[w] = inc;
+  __syncthreads();
+  int base = 0, tot = 0;
+  for (int q = 0; q < 16; q++) { if (q < w) base += part[q]; tot += part[q]; }
+  __syncthreads();
+  *all = tot;
+  return base + inc - v;
+}
+__global__ void __launch_bounds__(1024) k_scan_sum(const int *__restrict__ in, int n,
+    int *__restrict__ sums) {
+  int v[4], all;
+  const int s = fk_scan_load(in, n, blockIdx.x * FK_SCAN + threadIdx.x * 4, v);
+  (void) fk_scan_block(s, &all);
+  if (threadIdx.x == 0) sums[blockIdx.x] = all;
+}
+__global__ void __launch_bounds__(1024) k_scan_out(const int *__restrict__ in,
+    int *__restrict__ out, int n, const int *__restrict__ sums) {
+  int v[4], all, ahead = 0, base = 0;
+  if (gridDim.x > 1) {
+    for (int q = threadIdx.x; q < (int) blockIdx.x; q += 1024) ahead += sums[q];
+    (void) fk_scan_block(ahead, &base);
+  }
+  const int i = blockIdx.x * FK_SCAN + threadIdx.x * 4;
+  const int s = fk_scan_load(in, n, i, v);
+  int run = base + fk_scan_block(s, &all);
+#pragma unroll
+  for (int q = 0; q < 4; q++) if (i + q < n) { out[i + q] = run; run += v[q]; }
+  if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) out[n] = base + all;
 }
 
 /* ---- grid build: every catalogue of a call sorted into its job's grid
@@ -83,7 +111,7 @@ struct FkStage {
   FkRec *rec;                 /* sorted copies, from the catalogue's first object */
   double *ow;                 /* sorted weights beside |r|^2 (else null) */
   int wt;                     /* weights wanted */
-  int *oidx;                  /* original index */
+  int *oidx;                  /* original index (null when unused) */
 };
 
 /* request owning index v of the concatenated space whose starts are off */
@@ -105,28 +133,30 @@ __device__ __forceinline__ int fk_cell(const FkGrid &g, double x, double y, doub
 }
 
 __global__ void k_stage_assign(int nobj, int nst, const FkStage *__restrict__ st,
-    int *__restrict__ count, int *bad) {
+    int *__restrict__ count, int *__restrict__ rank, int *bad) {
   for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < nobj; o += gridDim.x * blockDim.x) {
     const FkStage &q = st[fk_stage_find(st, nst, o, &FkStage::obj0)];
     const int i = o - q.obj0;
     const double x = q.x[i], y = q.y[i], z = q.z[i];
     /* a non-finite coordinate has no cell and no bin: the call fails */
     if (!(__builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z))) atomicOr(bad, 1);
-    atomicAdd(count + q.cell0 + fk_cell(q.g, x, y, z), 1);
+    rank[o] = atomicAdd(count + q.cell0 + fk_cell(q.g, x, y, z), 1);
   }
 }
 
-/* sorted copies (cursor: the next free place of each cell); |r|^2 with
- * FCFC's data_preprocess lane rule (2pt/build_tree.c:59-92: FMA for the first
- * floor(n/8)*8 objects, unfused for the tail), unit weights where a weighted
- * count has none (build_tree.c:143-156) */
+/* sorted copies; |r|^2 with FCFC's data_preprocess lane rule
+ * (2pt/build_tree.c:59-92: FMA for the first floor(n/8)*8 objects, unfused
+ * for the tail), unit weights where a weighted count has none
+ * (build_tree.c:143-156).  The cell is found again, which costs less than
+ * storing it; its place in the cell comes from k_stage_assign (a second atomic
+ * per object here took 85 us for 5e5 clustered objects, the rank 12). */
 __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ st,
-    int *__restrict__ cursor) {
+    const int *__restrict__ gstart, const int *__restrict__ rank) {
   for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < nobj; o += gridDim.x * blockDim.x) {
     const FkStage &q = st[fk_stage_find(st, nst, o, &FkStage::obj0)];
     const int i = o - q.obj0;
     const double a = q.x[i], b = q.y[i], c = q.z[i];
-    const int d = atomicAdd(cursor + q.cell0 + fk_cell(q.g, a, b, c), 1) - q.obj0;
+    const int d = gstart[q.cell0 + fk_cell(q.g, a, b, c)] + rank[o] - q.obj0;
     const double w = q.wt ? (q.w ? q.w[i] : 1.0) : 0.0;
     double v = w;
     if (q.need_s) {
@@ -136,7 +166,7 @@ __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ s
       if (q.ow) q.ow[d] = w;
     }
     q.rec[d] = FkRec{a, b, c, v};
-    q.oidx[d] = i;
+    if (q.oidx) q.oidx[d] = i;
   }
 }
 
@@ -1662,7 +1692,7 @@ static void set_err(fcfc_gpu_ctx *c, const char *fmt, ...) {
 enum {
   WS_IN_X, WS_IN_Y, WS_IN_Z, WS_IN_S, WS_IN_W,          /* uploads, catalogue A */
   WS_IN2_X, WS_IN2_Y, WS_IN2_Z, WS_IN2_S, WS_IN2_W,     /* uploads, catalogue B */
-  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES, WS_SPLITS,
+  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_RANK, WS_SUMS, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES, WS_SPLITS,
   WS_STRIPS, WS_STAB, WS_PTAB, WS_S2E, WS_PE, WS_HIST, WS_MISC, WS_G, WS_GA, WS_GB, WS_JOBS,
   WS_NSLOT
 };
@@ -1950,7 +1980,8 @@ struct DevCat {
   double *w = nullptr;
   int *idx = nullptr;
   const int *cs = nullptr;
-  FkCat dev() const { return FkCat{n, 0, rec - obj0, w ? w - obj0 : nullptr, idx - obj0, cs}; }
+  FkCat dev() const { return FkCat{n, 0, rec - obj0, w ? w - obj0 : nullptr,
+                                   idx ? idx - obj0 : nullptr, cs}; }
 };
 
 /* A job ready to count: plan, sorted catalogues, output. */
@@ -2093,7 +2124,7 @@ static int bbox(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, double lo[3], dou
  * at them at once) and queue the work for stage_run.  slot: first of 3
  * consecutive workspace slots (single-job calls). */
 static int stage_prep(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, int need_s,
-    int wt, const FkGrid &g, int slot, int upslot, DevCat *out, std::vector<FkStage> &st) {
+    int wt, int need_idx, const FkGrid &g, int slot, int upslot, DevCat *out, std::vector<FkStage> &st) {
   const int n = (int) k->n;
   const size_t nb = sizeof(double) * (size_t) (n > 0 ? n : 1);
   /* inputs on the device */
@@ -2123,7 +2154,7 @@ static int stage_prep(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, int need_s,
   out->n = n;
   out->rec = (FkRec *) al.get(slot + 0, sizeof(FkRec) * no);
   out->w = (need_s && wt) ? (double *) al.get(slot + 1, nb) : nullptr;
-  out->idx = (int *) al.get(slot + 2, sizeof(int) * no);
+  out->idx = need_idx ? (int *) al.get(slot + 2, sizeof(int) * no) : nullptr;
   if (al.err) return al.err;
   FkStage q;
   memset(&q, 0, sizeof q);
@@ -2147,6 +2178,16 @@ static int stage_prep(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, int need_s,
   return 0;
 }
 
+/* exclusive scan of in[0..n-1] into out[0..n] */
+static int scan(fcfc_gpu_ctx *c, Alloc &al, const int *in, int *out, int n) {
+  const int nb = std::max(1, (n + FK_SCAN - 1) / FK_SCAN);
+  int *sums = nb > 1 ? (int *) al.tmp(WS_SUMS, sizeof(int) * (size_t) nb) : nullptr;
+  if (al.err) return al.err;
+  if (nb > 1) hipLaunchKernelGGL(k_scan_sum, dim3(nb), dim3(1024), 0, c->stream, in, n, sums);
+  hipLaunchKernelGGL(k_scan_out, dim3(nb), dim3(1024), 0, c->stream, in, out, n, sums);
+  return 0;
+}
+
 /* Run the queued sorts of a call: one launch per stage for all of them.  The
  * cell starts of all catalogues come from one scan and stay where it leaves
  * them (cs of every job). */
@@ -2162,17 +2203,18 @@ static int stage_run(fcfc_gpu_ctx *c, Alloc &al, std::vector<FkStage> &st, std::
   /* count[ncell]: set when an object has a non-finite coordinate */
   int *count = (int *) al.tmp(WS_COUNT, sizeof(int) * ((size_t) ncell + 1));
   int *gstart = (int *) al.get(WS_GSTART, sizeof(int) * ((size_t) ncell + 1));
+  int *rank = (int *) al.tmp(WS_RANK, sizeof(int) * (size_t) (nobj > 0 ? nobj : 1));
   if (al.err) return al.err;
   for (PJob &J : jobs) { J.A.cs = gstart + J.A.cell0; J.B.cs = gstart + J.B.cell0; }
   HIPCHK(c, hipMemcpyAsync(dst, st.data(), sizeof(FkStage) * st.size(), hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL(k_fill_int, dim3(nblk(ncell + 1, 256)), dim3(256), 0, c->stream, count, ncell + 1, 0);
   if (nobj > 0)
     hipLaunchKernelGGL(k_stage_assign, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, nobj, nst, dst,
-                       count, count + ncell);
-  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, count, gstart, ncell);
+                       count, rank, count + ncell);
+  if (int e = scan(c, al, count, gstart, ncell)) return e;
   if (nobj > 0)
     hipLaunchKernelGGL(k_stage_scatter, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, nobj, nst, dst,
-                       count);
+                       gstart, rank);
   HIPCHK(c, hipGetLastError());
   int bad = 0;
   HIPCHK(c, hipMemcpyAsync(&bad, count + ncell, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -2489,7 +2531,7 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
     if (found) continue;
     const int slot = (q == 0) ? WS_A_REC : WS_B_REC;
     const int upslot = (q == 0) ? WS_IN_X : WS_IN2_X;
-    if ((e = stage_prep(c, al, k, need_s, wt, J->P.g, slot, upslot, dst[q], stages))) return e;
+    if ((e = stage_prep(c, al, k, need_s, wt, gathers || mode == MODE_GRAD, J->P.g, slot, upslot, dst[q], stages))) return e;
     if (al.own) copies.push_back(CopyKey{k->x, k->y, k->z, k->s, k->w, k->n, wt, J->P.g, *dst[q]});
     if (gathers && wt && k->w && k->on_device && k->n > 0)
       gathers->push_back(need_s ? Gather{k->w, dst[q]->idx, dst[q]->w, (int) k->n, 1}
@@ -2641,7 +2683,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
   HIPCHK(c, hipMemcpyAsync(dtj, htj.data(), sizeof(FkTileJob) * jobs.size(), hipMemcpyHostToDevice, c->stream));
   if (nunit > 0)
     hipLaunchKernelGGL(k_run_count, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj, unitn);
-  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, c->stream, unitn, unitoff, nunit);
+  if (int e = scan(c, al, unitn, unitoff, nunit)) return e;
   FkRun *runs = (FkRun *) al.get(WS_TILES, sizeof(FkRun) * (size_t) (maxrun > 0 ? maxrun : 1));
   FkSplit *splits = (FkSplit *) al.get(WS_SPLITS, sizeof(FkSplit) * jobs.size());
   if (al.err) return al.err;
@@ -2944,7 +2986,7 @@ extern "C" int fcfc_gpu_count(fcfc_gpu_ctx *c, const fcfc_cat *a,
 static size_t noalloc_floor(const fcfc_cat *k, const fcfc_bins *bins, int wt) {
   if (!k || k->n <= 0) return 0;
   const int need_s = (bins->geometry == FCFC_GEOM_SURVEY && bins->bintype != FCFC_BIN_ISO);
-  size_t per = sizeof(FkRec) + 4 + (wt && need_s ? 8 : 0);       /* sorted copy */
+  size_t per = sizeof(FkRec) + 4 + (wt && need_s ? 8 : 0);       /* sorted copy, rank */
   if (!k->on_device) per += 24 + (wt && k->w ? 8 : 0) + (need_s && k->s ? 8 : 0);
   return per * (size_t) k->n;
 }
