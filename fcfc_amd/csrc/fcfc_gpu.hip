@@ -40,11 +40,14 @@ __device__ __forceinline__ int fk_cell1(double v, double o, double w, int nc) {
   return q < 0 ? 0 : (q >= nc ? nc - 1 : q);
 }
 
-__global__ void k_fill_int(int *p, int n, int v) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
 __global__ void k_zero_u64(unsigned long long *p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
+}
+/* the counters and histograms of a call and the cell counts of its sort */
+__global__ void k_zero_call(unsigned long long *p, int n, int *q, int m) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, st = gridDim.x * blockDim.x;
+  for (int i = t; i < n; i += st) p[i] = 0ull;
+  for (int i = t; i < m; i += st) q[i] = 0;
 }
 
 /* Exclusive scan of n ints into out[0..n] (out[n] = total).  Workgroups of
@@ -133,13 +136,13 @@ __device__ __forceinline__ int fk_cell(const FkGrid &g, double x, double y, doub
 }
 
 __global__ void k_stage_assign(int nobj, int nst, const FkStage *__restrict__ st,
-    int *__restrict__ count, int *__restrict__ rank, int *bad) {
+    int *__restrict__ count, int *__restrict__ rank, unsigned long long *bad) {
   for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < nobj; o += gridDim.x * blockDim.x) {
     const FkStage &q = st[fk_stage_find(st, nst, o, &FkStage::obj0)];
     const int i = o - q.obj0;
     const double x = q.x[i], y = q.y[i], z = q.z[i];
     /* a non-finite coordinate has no cell and no bin: the call fails */
-    if (!(__builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z))) atomicOr(bad, 1);
+    if (!(__builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z))) atomicOr(bad, 1ull);
     rank[o] = atomicAdd(count + q.cell0 + fk_cell(q.g, x, y, z), 1);
   }
 }
@@ -243,14 +246,17 @@ __global__ void k_run_count(int nunit, int njob, const FkTileJob *__restrict__ t
     nrun[u] = (p1 - p0 + t.T - 1) / t.T;
   }
 }
-/* the runs of unit u are numbered from roff[u]; the split of every job */
+/* the runs of unit u are numbered from roff[u]; the split of every job (no
+ * work item when the sort has met a non-finite coordinate) */
 __global__ void k_run_emit(int nunit, int njob, const FkTileJob *__restrict__ tj,
-    const int *__restrict__ roff, FkRun *__restrict__ runs, FkSplit *__restrict__ splits) {
+    const int *__restrict__ roff, FkRun *__restrict__ runs, FkSplit *__restrict__ splits,
+    const unsigned long long *__restrict__ bad) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < njob; k += gridDim.x * blockDim.x) {
     const FkTileJob t = tj[k];
     FkSplit sp = fk_split(roff[t.unit0 + t.nunit] - roff[t.unit0], max(t.nw, FK_NW), t.chunks, t.smax,
                           t.frac);
     sp.run0 = roff[t.unit0];
+    if (*bad) sp.nitems = 0;                  /* a non-finite coordinate: nothing is counted */
     splits[k] = sp;
   }
   for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nunit; u += gridDim.x * blockDim.x) {
@@ -1651,6 +1657,8 @@ __global__ void k_add_f64(double *dst, const double *src, int n) {
  * (once per device) and every host use goes through that address. */
 #define FK_SCRATCH_BYTES ((size_t) 128 << 20)
 #define FK_MAXDEV 64
+#define FK_PIN_BYTES ((size_t) 1 << 20)     /* pinned at the start; grown up to */
+#define FK_PIN_MOST ((size_t) 64 << 20)     /* this for large batches           */
 static __device__ __align__(256) unsigned char scratch[FK_SCRATCH_BYTES];
 static void *g_scratch_ptr[FK_MAXDEV];
 static std::mutex g_scratch_mu;
@@ -1673,6 +1681,11 @@ struct fcfc_gpu_ctx {
   struct Tuned { int geom, bintype, mode, autoc, wt, bucket, cd, zd, T; };
   std::vector<Tuned> tuned;    /* autotuner results per density bucket */
   std::vector<DevBuf> bufs;
+  char *pin = nullptr;         /* pinned host memory: a call's upload, then its results */
+  size_t pin_cap = 0;
+  /* histogram copies and workgroups per CU of a kernel at an LDS size */
+  struct Occ { const void *fn; int lds1, nh, lds, occ; };
+  std::vector<Occ> occs;
   void *scratch = nullptr;     /* device address of this GPU's scratch array */
   char scratch_err[128] = {0};
 };
@@ -1688,12 +1701,18 @@ static void set_err(fcfc_gpu_ctx *c, const char *fmt, ...) {
     set_err(ctx, "%s failed: %s (%s:%d)", #call, hipGetErrorString(_e), __FILE__, __LINE__); \
     return FCFC_ERR_GPU; } } while (0)
 
+/* Words of a call's results, zeroed before its launches: pairs evaluated,
+ * re-evaluated, of the census, the flag of non-finite coordinates, then the
+ * queue (one 32-bit word per job) and the histograms. */
+enum { RES_EVALS, RES_RECHECKED, RES_CENSUS, RES_BAD, RES_QUEUE };
+static int res_hist(int njob) { return RES_QUEUE + (njob + 1) / 2; }
+
 /* workspace slots */
 enum {
   WS_IN_X, WS_IN_Y, WS_IN_Z, WS_IN_S, WS_IN_W,          /* uploads, catalogue A */
   WS_IN2_X, WS_IN2_Y, WS_IN2_Z, WS_IN2_S, WS_IN2_W,     /* uploads, catalogue B */
-  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_RANK, WS_SUMS, WS_GSTART, WS_STAGE, WS_TJOBS, WS_ROWN, WS_ROWOFF, WS_TILES, WS_SPLITS,
-  WS_STRIPS, WS_STAB, WS_PTAB, WS_S2E, WS_PE, WS_HIST, WS_MISC, WS_G, WS_GA, WS_GB, WS_JOBS,
+  WS_A_REC, WS_A_W, WS_A_IDX, WS_B_REC, WS_B_W, WS_B_IDX, WS_COUNT, WS_RANK, WS_SUMS, WS_GSTART, WS_ROWN, WS_ROWOFF, WS_TILES, WS_SPLITS,
+  WS_RES, WS_UP, WS_BOX, WS_GA, WS_GB,
   WS_NSLOT
 };
 
@@ -1746,6 +1765,8 @@ extern "C" int fcfc_gpu_init(fcfc_gpu_ctx **out, int device) {
     c->scratch = g_scratch_ptr[device];
   }
   else snprintf(c->scratch_err, sizeof c->scratch_err, "device index beyond %d", FK_MAXDEV - 1);
+  if (hipHostMalloc((void **) &c->pin, FK_PIN_BYTES, hipHostMallocDefault) == hipSuccess) c->pin_cap = FK_PIN_BYTES;
+  else { c->pin = nullptr; (void) hipGetLastError(); }
   *out = c;
   return 0;
 }
@@ -1755,6 +1776,7 @@ extern "C" int fcfc_gpu_destroy(fcfc_gpu_ctx *c) {
   (void) hipSetDevice(c->device);
   if (c->stream) (void) hipStreamSynchronize(c->stream);
   for (auto &b : c->bufs) if (b.p) (void) hipFree(b.p);
+  if (c->pin) (void) hipHostFree(c->pin);
   if (c->ev0) (void) hipEventDestroy(c->ev0);
   if (c->ev1) (void) hipEventDestroy(c->ev1);
   if (c->stream) (void) hipStreamDestroy(c->stream);
@@ -2095,29 +2117,86 @@ __global__ void k_minmax(int n, const double *__restrict__ x, const double *__re
 
 
 
-static int bbox(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *k, double lo[3], double hi[3]) {
-  if (k->n <= 0) return 0;
-  if (!k->on_device) {
-    for (int64_t i = 0; i < k->n; i++) {
-      const double v[3] = {k->x[i], k->y[i], k->z[i]};
-      for (int d = 0; d < 3; d++) { lo[d] = fmin(lo[d], v[d]); hi[d] = fmax(hi[d], v[d]); }
+/* Bounding box of one or two catalogues. */
+static int bbox(fcfc_gpu_ctx *c, Alloc &al, const fcfc_cat *const *ks, int nk, double lo[3], double hi[3]) {
+  const int nbk = 64, nd = 8 + 6 * nbk;
+  double *d = nullptr;
+  for (int q = 0; q < nk; q++) {
+    const fcfc_cat *k = ks[q];
+    if (k->n <= 0) continue;
+    if (!k->on_device) {
+      for (int64_t i = 0; i < k->n; i++) {
+        const double v[3] = {k->x[i], k->y[i], k->z[i]};
+        for (int m = 0; m < 3; m++) { lo[m] = fmin(lo[m], v[m]); hi[m] = fmax(hi[m], v[m]); }
+      }
+      continue;
     }
-    return 0;
+    if (!d) d = (double *) al.tmp(WS_BOX, sizeof(double) * 2 * nd);
+    if (al.err) return al.err;
+    hipLaunchKernelGGL(k_minmax, dim3(nbk), dim3(256), 0, c->stream, (int) k->n, k->x, k->y, k->z, d + q * nd);
   }
-  const int nbk = 64;
-  double *d = (double *) al.tmp(WS_MISC, sizeof(double) * (8 + 6 * nbk));
-  if (al.err) return al.err;
-  hipLaunchKernelGGL(k_minmax, dim3(nbk), dim3(256), 0, c->stream, (int) k->n, k->x, k->y, k->z, d);
-  std::vector<double> h(8 + 6 * nbk);
-  HIPCHK(c, hipMemcpyAsync(h.data(), d, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
+  if (!d) return 0;
+  std::vector<double> hv;
+  double *h = (double *) c->pin;
+  if (c->pin_cap < sizeof(double) * 2 * nd) { hv.resize(2 * nd); h = hv.data(); }
+  HIPCHK(c, hipMemcpyAsync(h, d, sizeof(double) * 2 * nd, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int bk = 0; bk < nbk; bk++)
-    for (int q = 0; q < 3; q++) {
-      lo[q] = fmin(lo[q], h[8 + bk * 6 + q]);
-      hi[q] = fmax(hi[q], h[8 + bk * 6 + 3 + q]);
-    }
+  for (int q = 0; q < nk; q++) {
+    if (ks[q]->n <= 0 || !ks[q]->on_device) continue;
+    for (int bk = 0; bk < nbk; bk++)
+      for (int m = 0; m < 3; m++) {
+        lo[m] = fmin(lo[m], h[q * nd + 8 + bk * 6 + m]);
+        hi[m] = fmax(hi[m], h[q * nd + 8 + bk * 6 + 3 + m]);
+      }
+  }
   return 0;
 }
+
+/* What a call uploads besides catalogues -- sort requests, tables, strips,
+ * job descriptors -- gathered in (pinned) host memory and copied at once.  The
+ * device addresses are known as soon as something is put. */
+struct Upload {
+  fcfc_gpu_ctx *c;
+  char *h = nullptr, *d = nullptr;
+  size_t cap = 0, used = 0;
+  std::vector<char> own;
+  explicit Upload(fcfc_gpu_ctx *c_) : c(c_) {}
+  int reserve(Alloc &al, size_t bytes, bool plan) {
+    cap = (bytes + 255) & ~(size_t) 255;
+    d = (char *) al.get(WS_UP, cap);
+    if (al.err) return al.err;
+    if (!plan && pin_fit(c, cap, al.arena != nullptr)) h = c->pin;
+    else { own.resize(cap); h = own.data(); }
+    return 0;
+  }
+  /* room for bytes of pinned memory in the context (grown when allowed) */
+  static bool pin_fit(fcfc_gpu_ctx *c, size_t bytes, bool fixed) {
+    if (bytes <= c->pin_cap) return true;
+    if (fixed || bytes > FK_PIN_MOST) return false;
+    char *p = nullptr;
+    if (hipStreamSynchronize(c->stream) != hipSuccess ||
+        hipHostMalloc((void **) &p, 2 * bytes, hipHostMallocDefault) != hipSuccess) {
+      (void) hipGetLastError();
+      return false;
+    }
+    if (c->pin) (void) hipHostFree(c->pin);
+    c->pin = p;
+    c->pin_cap = 2 * bytes;
+    return true;
+  }
+  template <class T> T *put(const T *src, size_t n) {
+    const size_t bytes = (sizeof(T) * n + 15) & ~(size_t) 15;
+    if (used + bytes > cap) return nullptr;
+    memcpy(h + used, src, sizeof(T) * n);
+    T *r = (T *) (d + used);
+    used += bytes;
+    return r;
+  }
+  int flush() {
+    if (used) HIPCHK(c, hipMemcpyAsync(d, h, used, hipMemcpyHostToDevice, c->stream));
+    return 0;
+  }
+};
 
 /* Prepare the sort of one catalogue into the grid of a job: upload host
  * inputs, allocate the sorted copies (so the job's descriptors can point
@@ -2188,41 +2267,47 @@ static int scan(fcfc_gpu_ctx *c, Alloc &al, const int *in, int *out, int n) {
   return 0;
 }
 
-/* Run the queued sorts of a call: one launch per stage for all of them.  The
+/* The queued sorts of a call: one launch per stage for all of them.  The
  * cell starts of all catalogues come from one scan and stay where it leaves
  * them (cs of every job). */
-static int stage_run(fcfc_gpu_ctx *c, Alloc &al, std::vector<FkStage> &st, std::vector<PJob> &jobs) {
+struct Sort {
+  int nobj = 0, ncell = 0, nst = 0;
+  FkStage *st = nullptr;             /* uploaded requests */
+  int *count = nullptr, *gstart = nullptr, *rank = nullptr;
+};
+
+static int sort_alloc(fcfc_gpu_ctx *c, Alloc &al, const std::vector<FkStage> &st,
+    std::vector<PJob> &jobs, Sort *so) {
   if (st.empty()) return 0;
   const FkStage &last = st.back();
-  const int nobj = last.obj0 + last.n;
   const long long ncl = last.cell0 + (long long) last.g.ncx * last.g.ncy * last.g.ncz;
-  if (nobj > INT_MAX / 2 || ncl > INT_MAX / 2) { set_err(c, "catalogues of one call too large"); return FCFC_ERR_CFG; }
-  const int ncell = (int) ncl;
-  const int nst = (int) st.size();
-  FkStage *dst = (FkStage *) al.tmp(WS_STAGE, sizeof(FkStage) * st.size());
-  /* count[ncell]: set when an object has a non-finite coordinate */
-  int *count = (int *) al.tmp(WS_COUNT, sizeof(int) * ((size_t) ncell + 1));
-  int *gstart = (int *) al.get(WS_GSTART, sizeof(int) * ((size_t) ncell + 1));
-  int *rank = (int *) al.tmp(WS_RANK, sizeof(int) * (size_t) (nobj > 0 ? nobj : 1));
+  if ((long long) last.obj0 + last.n > INT_MAX / 2 || ncl > INT_MAX / 2) {
+    set_err(c, "catalogues of one call too large");
+    return FCFC_ERR_CFG;
+  }
+  so->nobj = last.obj0 + last.n;
+  so->ncell = (int) ncl;
+  so->nst = (int) st.size();
+  so->count = (int *) al.tmp(WS_COUNT, sizeof(int) * (size_t) so->ncell);
+  so->gstart = (int *) al.get(WS_GSTART, sizeof(int) * ((size_t) so->ncell + 1));
+  so->rank = (int *) al.tmp(WS_RANK, sizeof(int) * (size_t) std::max(so->nobj, 1));
   if (al.err) return al.err;
-  for (PJob &J : jobs) { J.A.cs = gstart + J.A.cell0; J.B.cs = gstart + J.B.cell0; }
-  HIPCHK(c, hipMemcpyAsync(dst, st.data(), sizeof(FkStage) * st.size(), hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_fill_int, dim3(nblk(ncell + 1, 256)), dim3(256), 0, c->stream, count, ncell + 1, 0);
-  if (nobj > 0)
-    hipLaunchKernelGGL(k_stage_assign, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, nobj, nst, dst,
-                       count, rank, count + ncell);
-  if (int e = scan(c, al, count, gstart, ncell)) return e;
-  if (nobj > 0)
-    hipLaunchKernelGGL(k_stage_scatter, dim3(nblk(nobj, 256)), dim3(256), 0, c->stream, nobj, nst, dst,
-                       gstart, rank);
+  for (PJob &J : jobs) { J.A.cs = so->gstart + J.A.cell0; J.B.cs = so->gstart + J.B.cell0; }
+  return 0;
+}
+
+/* zero the call's result words and sort its catalogues */
+static int sort_run(fcfc_gpu_ctx *c, Alloc &al, const Sort &so, unsigned long long *res, int nres) {
+  hipLaunchKernelGGL(k_zero_call, dim3(nblk(std::max(nres, so.ncell), 256)), dim3(256), 0, c->stream,
+                     res, nres, so.count, so.ncell);
+  if (so.nobj > 0)
+    hipLaunchKernelGGL(k_stage_assign, dim3(nblk(so.nobj, 256)), dim3(256), 0, c->stream, so.nobj,
+                       so.nst, so.st, so.count, so.rank, res + RES_BAD);
+  if (int e = scan(c, al, so.count, so.gstart, so.ncell)) return e;
+  if (so.nobj > 0)
+    hipLaunchKernelGGL(k_stage_scatter, dim3(nblk(so.nobj, 256)), dim3(256), 0, c->stream, so.nobj,
+                       so.nst, so.st, so.gstart, so.rank);
   HIPCHK(c, hipGetLastError());
-  int bad = 0;
-  HIPCHK(c, hipMemcpyAsync(&bad, count + ncell, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  /* the descriptors are read by the kernels above: keep the host copy until
-   * the copy has completed */
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  st.clear();
-  if (bad) { set_err(c, "a catalogue has a non-finite coordinate"); return FCFC_ERR_DATA; }
   return 0;
 }
 
@@ -2514,8 +2599,8 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
   int e;
   if (bins->geometry == FCFC_GEOM_SURVEY) {
-    if ((e = bbox(c, al, a, lo, hi))) return e;
-    if (!autoc && (e = bbox(c, al, b, lo, hi))) return e;
+    const fcfc_cat *ks[2] = {a, b};
+    if ((e = bbox(c, al, ks, autoc ? 1 : 2, lo, hi))) return e;
     if (!(lo[0] <= hi[0])) { for (int k = 0; k < 3; k++) { lo[k] = 0; hi[k] = 1; } }
   }
   if ((e = make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, a->n, autoc ? a->n : b->n, &J->P))) return e;
@@ -2542,22 +2627,44 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
 }
 
 /* A recorded count launch: kernel, grid, LDS bytes and arguments, and the
- * host copies of the strip triples and job descriptors its uploads read.
- * They live as long as the launch, so that the asynchronous uploads do not
- * depend on how the runtime stages pageable host memory. */
+ * arrays of its run list. */
 struct Launch {
   kfn_t fn = nullptr;
   int nblock = 0, lds = 0;
   FkArgs a;
-  std::vector<int> hstr;
-  std::vector<FkJob> hj;
+  int nunit = 0, njob = 0;
+  const FkTileJob *tj = nullptr;
+  int *unitn = nullptr, *unitoff = nullptr;
+  FkRun *runs = nullptr;
+  FkSplit *splits = nullptr;
 };
 
-/* List the runs of all jobs and prepare the persistent launch that counts (or
- * differentiates) them; every buffer comes from al. */
-static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
-    std::vector<PJob> &jobs, int mode, const double *G, void *dhist,
-    unsigned long long *dstats, unsigned int *dqueue, Launch *out) {
+/* binning tables of a call on the device */
+struct DevTabs { const uint16_t *stab = nullptr, *ptab = nullptr; const double *s2e = nullptr, *pe = nullptr, *G = nullptr; };
+
+/* bytes to reserve for the uploads of a call */
+static size_t upload_bytes(const fcfc_bins *b, const std::vector<PJob> &jobs, size_t nst, bool grad) {
+  size_t n = 64 * 16 + sizeof(FkStage) * nst + 2 * (b->stab_len + 1) + 8 * (b->ns + 1);
+  if (b->bintype == FCFC_BIN_SPI) n += 2 * (b->ptab_len + 1) + 8 * (b->np + 1);
+  if (grad) n += 8 * (size_t) b->ntot;
+  for (const PJob &J : jobs) n += sizeof(FkJob) + sizeof(FkTileJob) + 4 * J.P.strips.size() + 64;
+  return n;
+}
+
+static void put_tables(Upload &up, const fcfc_bins *b, DevTabs *t) {
+  t->stab = up.put(b->stab, b->stab_len);
+  t->s2e = up.put(b->s2bin, b->ns + 1);
+  if (b->bintype == FCFC_BIN_SPI) {
+    t->ptab = up.put(b->ptab, b->ptab_len);
+    t->pe = up.put(b->pbin, b->np + 1);
+  }
+}
+
+/* Prepare the run list and the persistent launch that counts (or
+ * differentiates) the jobs; every buffer comes from al, descriptors go to up,
+ * res are the result words and dhist the histograms. */
+static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &tabs, const fcfc_bins *b,
+    std::vector<PJob> &jobs, int mode, unsigned long long *res, void *dhist, Launch *out) {
   const int geom = b->geometry;
   int m = mode;
   const bool zb = zb_fits(b);
@@ -2622,26 +2729,41 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     set_err(c, "binning tables need %d bytes of LDS (limit %d)", L.total, lds_max);
     return FCFC_ERR_CFG;
   }
-  if (m != MODE_GRAD) {
+  /* (the choice depends on the kernel and the LDS size of one copy alone, and
+   * is kept: it takes several queries) */
+  int occ = 0;
+  const int lds1 = L.total;
+  for (const auto &o : c->occs)
+    if (o.fn == (const void *) fn && o.lds1 == lds1 && c->t_nh <= 0) {
+      L = lds_plan(b, m, anywt, need_s, o.nh, hyb, ssearch, psearch);
+      if (L.total == o.lds) occ = o.occ;
+      else L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch);
+      break;
+    }
+  if (!occ) {
     int occ1 = 0;
     if (int e = occ_of(fn, L, &occ1)) return e;
-    const int nhmax = c->t_nh > 0 ? c->t_nh : 8;
-    for (int nh = 2; nh <= nhmax; nh *= 2) {
-      LdsPlan L2 = lds_plan(b, m, anywt, need_s, nh, hyb, ssearch, psearch);
-      int occ = 0;
-      if (L2.total > lds_max) break;
-      if (int e = occ_of(fn, L2, &occ)) return e;
-      if (occ < occ1 && c->t_nh <= 0) break;
-      L = L2;
+    if (m != MODE_GRAD) {
+      const int nhmax = c->t_nh > 0 ? c->t_nh : 8;
+      for (int nh = 2; nh <= nhmax; nh *= 2) {
+        LdsPlan L2 = lds_plan(b, m, anywt, need_s, nh, hyb, ssearch, psearch);
+        int o2 = 0;
+        if (L2.total > lds_max) break;
+        if (int e = occ_of(fn, L2, &o2)) return e;
+        if (o2 < occ1 && c->t_nh <= 0) break;
+        L = L2;
+      }
+    }
+    if (int e = occ_of(fn, L, &occ)) return e;
+    if (occ < 1) occ = 1;
+    if (c->t_nh <= 0) {
+      if (c->occs.size() >= 256) c->occs.clear();
+      c->occs.push_back({(const void *) fn, lds1, L.nh, L.total, occ});
     }
   }
-  HIPCHK(c, hipFuncSetAttribute((const void *) fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.total));
   /* ---- runs of all jobs ---- */
   /* persistent workgroups, dealt out to the jobs in proportion to the
    * candidate pairs of their runs (each run at least one chunk) */
-  int occ = 0;
-  HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *) fn, FK_NT, L.total));
-  if (occ < 1) occ = 1;
   int nwg = c->t_nblock > 0 ? c->t_nblock : occ * c->ncu;
   const int njob = (int) jobs.size();
   std::vector<FkTileJob> htj(jobs.size());
@@ -2678,33 +2800,16 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
   const int nunit = (int) nunit_l;
   int *unitn = (int *) al.get(WS_ROWN, sizeof(int) * (size_t) nunit);
   int *unitoff = (int *) al.get(WS_ROWOFF, sizeof(int) * ((size_t) nunit + 1));
-  FkTileJob *dtj = (FkTileJob *) al.get(WS_TJOBS, sizeof(FkTileJob) * jobs.size());
-  if (al.err) return al.err;
-  HIPCHK(c, hipMemcpyAsync(dtj, htj.data(), sizeof(FkTileJob) * jobs.size(), hipMemcpyHostToDevice, c->stream));
-  if (nunit > 0)
-    hipLaunchKernelGGL(k_run_count, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj, unitn);
-  if (int e = scan(c, al, unitn, unitoff, nunit)) return e;
+  const FkTileJob *dtj = up.put(htj.data(), htj.size());
   FkRun *runs = (FkRun *) al.get(WS_TILES, sizeof(FkRun) * (size_t) (maxrun > 0 ? maxrun : 1));
   FkSplit *splits = (FkSplit *) al.get(WS_SPLITS, sizeof(FkSplit) * jobs.size());
   if (al.err) return al.err;
-  if (nunit > 0)
-    hipLaunchKernelGGL(k_run_emit, dim3(nblk(nunit, 64)), dim3(64), 0, c->stream, nunit, njob, dtj,
-                       unitoff, runs, splits);
-  /* ---- tables, strips, job descriptors ---- */
-  size_t nstr = 0;
-  for (auto &j : jobs) nstr += j.P.strips.size();
-  uint16_t *dstab = (uint16_t *) al.get(WS_STAB, sizeof(uint16_t) * (b->stab_len + 1));
-  uint16_t *dptab = (uint16_t *) al.get(WS_PTAB, sizeof(uint16_t) * (b->ptab_len + 1));
-  double *ds2e = (double *) al.get(WS_S2E, sizeof(double) * (b->ns + 1));
-  double *dpe = (double *) al.get(WS_PE, sizeof(double) * (b->np + 1));
-  int *dstrips = (int *) al.get(WS_STRIPS, sizeof(int) * (nstr ? nstr : 1));
-  FkJob *djobs = nullptr;
-  if (al.err) return al.err;
-  std::vector<int> &hstr = out->hstr;
-  hstr.clear();
-  hstr.reserve(nstr);
-  std::vector<FkJob> &hj = out->hj;
-  hj.assign(jobs.size(), FkJob{});
+  /* ---- strips, job descriptors ---- */
+  std::vector<int> hstr;
+  for (auto &j : jobs) hstr.insert(hstr.end(), j.P.strips.begin(), j.P.strips.end());
+  const int *dstrips = up.put(hstr.data(), hstr.size());
+  std::vector<FkJob> hj(jobs.size(), FkJob{});
+  size_t str0 = 0;
   double s2f = 0;
   float win2s = 0.0f, win2p = 0.0f;
   if (m == MODE_C32)
@@ -2716,7 +2821,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     f.A = J.A.dev();
     f.B = J.B.dev();
     f.g = J.P.g;
-    f.strips = dstrips + hstr.size();
+    f.strips = dstrips + str0;
+    str0 += J.P.strips.size();
     f.nstrips = J.P.nstrips;
     f.autoc = J.autoc;
     f.wt = J.wt;
@@ -2731,18 +2837,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
       win2s = std::max(win2s, f.win.e_s2x2);
       win2p = std::max(win2p, f.win.e_pix2);
     }
-    hstr.insert(hstr.end(), J.P.strips.begin(), J.P.strips.end());
   }
-  djobs = (FkJob *) al.get(WS_JOBS, sizeof(FkJob) * jobs.size());
-  if (al.err) return al.err;
-  HIPCHK(c, hipMemcpyAsync(dstab, b->stab, sizeof(uint16_t) * b->stab_len, hipMemcpyHostToDevice, c->stream));
-  if (b->bintype == FCFC_BIN_SPI)
-    HIPCHK(c, hipMemcpyAsync(dptab, b->ptab, sizeof(uint16_t) * b->ptab_len, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(ds2e, b->s2bin, sizeof(double) * (b->ns + 1), hipMemcpyHostToDevice, c->stream));
-  if (b->bintype == FCFC_BIN_SPI)
-    HIPCHK(c, hipMemcpyAsync(dpe, b->pbin, sizeof(double) * (b->np + 1), hipMemcpyHostToDevice, c->stream));
-  if (nstr) HIPCHK(c, hipMemcpyAsync(dstrips, hstr.data(), sizeof(int) * nstr, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(djobs, hj.data(), sizeof(FkJob) * jobs.size(), hipMemcpyHostToDevice, c->stream));
+  const FkJob *djobs = up.put(hj.data(), hj.size());
+  if (!dtj || !dstrips || !djobs) { set_err(c, "upload buffer too small"); return FCFC_ERR_UNKNOWN; }
 
   FkArgs a;
   memset(&a, 0, sizeof a);
@@ -2803,28 +2900,26 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
     fb.q_t16 = 65532u;
     fb.q_pad = 0;
   }
-  fb.stab = dstab; fb.ptab = dptab; fb.s2bin = ds2e; fb.pbin = dpe;
+  fb.stab = tabs.stab; fb.ptab = tabs.ptab; fb.s2bin = tabs.s2e; fb.pbin = tabs.pe;
   a.runs = runs; a.splits = splits;
-  a.queue = dqueue;
+  a.queue = (unsigned int *) (res + RES_QUEUE);
   a.gcnt_u = (unsigned long long *) dhist; a.gcnt_d = (double *) dhist;
-  a.stats = dstats;
+  a.stats = res;
   a.nh = L.nh;
   a.off_hist = L.off_hist; a.off_stab = L.off_stab; a.off_ptab = L.off_ptab;
   a.stab_c0 = L.stab_c0; a.ptab_c0 = L.ptab_c0;
   a.off_edges = L.off_edges;
   a.off_chunk = L.off_chunk; a.off_queue = L.off_queue;
   a.census = c->census;
-  a.G = G;
+  a.G = tabs.G;
   c->last_nrun = unitoff + nunit;
   c->stats.tile = jobs.empty() ? 0 : jobs[0].P.T;
   c->stats.cell_div = jobs.empty() ? 0 : (int) lround(sqrt(jobs[0].P.g.Rxy2) / jobs[0].P.g.wx);
   out->fn = fn; out->nblock = nwg; out->lds = L.total; out->a = a;
+  out->nunit = nunit; out->njob = njob; out->tj = dtj;
+  out->unitn = unitn; out->unitoff = unitoff; out->runs = runs; out->splits = splits;
   return 0;
 }
-
-/* Counters of a call, zeroed before its launches: 8 words of statistics and
- * the queue, one 32-bit word per job. */
-static int misc_words(int njob) { return 8 + (njob + 1) / 2; }
 
 /* Waits for the stream when it goes out of scope: declared after the
  * launches of a call (destroyed before them), it keeps their host copies
@@ -2834,26 +2929,19 @@ struct StreamDrain {
   ~StreamDrain() { (void) hipStreamSynchronize(c->stream); }
 };
 
-static int launch(fcfc_gpu_ctx *c, const Launch &Lc) {
-  if (Lc.nblock > 0)
-    hipLaunchKernelGGL(Lc.fn, dim3(Lc.nblock), dim3(FK_NT), Lc.lds, c->stream, Lc.a);
+/* the run list of a launch, on its sorted catalogues */
+static int list_runs(fcfc_gpu_ctx *c, Alloc &al, const Launch &L, const unsigned long long *res) {
+  hipLaunchKernelGGL(k_run_count, dim3(nblk(L.nunit, 64)), dim3(64), 0, c->stream, L.nunit, L.njob, L.tj, L.unitn);
+  if (int e = scan(c, al, L.unitn, L.unitoff, L.nunit)) return e;
+  hipLaunchKernelGGL(k_run_emit, dim3(nblk(L.nunit, 64)), dim3(64), 0, c->stream, L.nunit, L.njob, L.tj,
+                     L.unitoff, L.runs, L.splits, res + RES_BAD);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
 
-/* List the runs of all jobs, then count (or differentiate) them in one launch. */
-static int run_jobs(fcfc_gpu_ctx *c, Alloc &al, const fcfc_bins *b,
-    std::vector<PJob> &jobs, int mode, const double *G, void *dhist,
-    unsigned long long *dstats, unsigned int *dqueue, float *kms) {
-  Launch Lc;
-  StreamDrain drain{c};
-  int e = build_launch(c, al, b, jobs, mode, G, dhist, dstats, dqueue, &Lc);
-  if (e) return e;
-  HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-  if ((e = launch(c, Lc))) return e;
-  HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  HIPCHK(c, hipEventElapsedTime(kms, c->ev0, c->ev1));
+static int launch(fcfc_gpu_ctx *c, const Launch &Lc) {
+  hipLaunchKernelGGL(Lc.fn, dim3(Lc.nblock), dim3(FK_NT), Lc.lds, c->stream, Lc.a);
+  HIPCHK(c, hipGetLastError());
   return 0;
 }
 
@@ -2873,40 +2961,41 @@ static std::vector<std::vector<PJob>> launch_groups(const std::vector<PJob> &job
   return g;
 }
 
-static int stats_from(fcfc_gpu_ctx *c, unsigned long long *dstats) {
-  unsigned long long st[3] = {0, 0, 0};
-  HIPCHK(c, hipMemcpyAsync(st, dstats, sizeof st, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->stats.evals = (double) st[0];
-  c->stats.rechecked = (double) st[1];
-  c->stats.census = (double) st[2];
-  return 0;
-}
-
-/* add the device histograms of the jobs (8 bytes per bin: int64 or
- * double) into the caller's cnt (device or host) */
+/* Wait for a call and take its results: statistics, the check for
+ * non-finite coordinates, and (nhist words from the histograms on) the
+ * histograms of its jobs added into the caller's cnt, 8 bytes per bin (int64
+ * or double), in device or host memory. */
 static int deliver(fcfc_gpu_ctx *c, const std::vector<PJob> &jobs, int ntot,
-    const void *dh, uint32_t flags, void *cnt) {
-  const int njob = (int) jobs.size();
-  const int n = ntot * njob;
-  if (flags & FCFC_GPU_CNT_DEVICE) {
-    for (int k = 0; k < njob; k++) {
-      char *dst = (char *) cnt + (size_t) k * ntot * 8;
-      const char *src = (const char *) dh + (size_t) k * ntot * 8;
-      if (jobs[k].wt) hipLaunchKernelGGL(k_add_f64, dim3(nblk(ntot, 256)), dim3(256), 0, c->stream, (double *) dst, (const double *) src, ntot);
-      else hipLaunchKernelGGL(k_add_u64, dim3(nblk(ntot, 256)), dim3(256), 0, c->stream, (long long *) dst, (const unsigned long long *) src, ntot);
+    const unsigned long long *res, int nhist, uint32_t flags, void *cnt, bool fixed) {
+  const int njob = (int) jobs.size(), off = res_hist(njob);
+  const bool dev = (flags & FCFC_GPU_CNT_DEVICE) != 0;
+  const size_t n = dev ? (size_t) RES_QUEUE : (size_t) off + nhist;
+  std::vector<unsigned long long> hv;
+  unsigned long long *h;
+  /* (pinned memory that the call's upload used is free: the device has read
+   * it before anything this copy waits for) */
+  if (Upload::pin_fit(c, 8 * n, fixed)) h = (unsigned long long *) c->pin;
+  else { hv.resize(n); h = hv.data(); }
+  HIPCHK(c, hipMemcpyAsync(h, res, 8 * n, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->stats.evals = (double) h[RES_EVALS];
+  c->stats.rechecked = (double) h[RES_RECHECKED];
+  c->stats.census = (double) h[RES_CENSUS];
+  if (h[RES_BAD]) { set_err(c, "a catalogue has a non-finite coordinate"); return FCFC_ERR_DATA; }
+  if (!nhist) return 0;
+  for (int k = 0; k < njob; k++) {
+    const size_t o = (size_t) k * ntot;
+    if (dev) {
+      const unsigned long long *src = res + off + o;
+      if (jobs[k].wt) hipLaunchKernelGGL(k_add_f64, dim3(nblk(ntot, 256)), dim3(256), 0, c->stream, (double *) cnt + o, (const double *) src, ntot);
+      else hipLaunchKernelGGL(k_add_u64, dim3(nblk(ntot, 256)), dim3(256), 0, c->stream, (long long *) cnt + o, src, ntot);
     }
-    HIPCHK(c, hipGetLastError());
+    else if (jobs[k].wt) { double *dst = (double *) cnt + o; const double *hd = (const double *) (h + off) + o; for (int i = 0; i < ntot; i++) dst[i] += hd[i]; }
+    else { int64_t *dst = (int64_t *) cnt + o; for (int i = 0; i < ntot; i++) dst[i] += (int64_t) h[off + o + i]; }
   }
-  else {
-    std::vector<unsigned long long> h(n);
-    HIPCHK(c, hipMemcpyAsync(h.data(), dh, 8 * (size_t) n, hipMemcpyDeviceToHost, c->stream));
+  if (dev) {
+    HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int k = 0; k < njob; k++) {
-      const size_t o = (size_t) k * ntot;
-      if (jobs[k].wt) { double *dst = (double *) cnt + o; const double *hd = (const double *) h.data() + o; for (int i = 0; i < ntot; i++) dst[i] += hd[i]; }
-      else { int64_t *dst = (int64_t *) cnt + o; for (int i = 0; i < ntot; i++) dst[i] += (int64_t) h[o + i]; }
-    }
   }
   return 0;
 }
@@ -2937,35 +3026,33 @@ static int count_jobs(fcfc_gpu_ctx *c, int njob, const fcfc_cat *const *as,
     jobs[k].hist_off = (long long) k * bins->ntot;
     jobs[k].qi = k;
   }
-  if (int e = stage_run(c, al, stages, jobs)) return e;
-  const size_t hbytes = 8 * (size_t) bins->ntot * njob;
-  void *dh = al.tmp(WS_HIST, hbytes);
-  const int nmisc = misc_words((int) jobs.size());
-  unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 8 * (size_t) nmisc);
+  Sort so;
+  if (int e = sort_alloc(c, al, stages, jobs, &so)) return e;
+  const int nhist = bins->ntot * njob, nres = res_hist(njob) + nhist;
+  unsigned long long *res = (unsigned long long *) al.tmp(WS_RES, 8 * (size_t) nres);
   if (al.err) return al.err;
-  hipLaunchKernelGGL(k_zero_u64, dim3(nblk((int64_t) bins->ntot * njob, 256)), dim3(256), 0, c->stream,
-      (unsigned long long *) dh, bins->ntot * njob);
-  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nmisc, 256)), dim3(256), 0, c->stream, misc, nmisc);
-  /* one persistent launch per group (each with its own queue word) */
+  /* one persistent launch per group */
   std::vector<std::vector<PJob>> groups = launch_groups(jobs);
   std::vector<Launch> L(groups.size());
+  Upload up(c);
   StreamDrain drain{c};
-  for (size_t q = 0; q < groups.size(); q++) {
-    int e = build_launch(c, al, bins, groups[q], mode, nullptr, dh, misc,
-                         (unsigned int *) (misc + 8), &L[q]);
-    if (e) return e;
-  }
+  if (int e = up.reserve(al, upload_bytes(bins, jobs, stages.size(), false), false)) return e;
+  DevTabs tabs;
+  put_tables(up, bins, &tabs);
+  so.st = up.put(stages.data(), stages.size());
+  for (size_t q = 0; q < groups.size(); q++)
+    if (int e = build_launch(c, al, up, tabs, bins, groups[q], mode, res, res + res_hist(njob), &L[q]))
+      return e;
+  if (int e = up.flush()) return e;
+  if (int e = sort_run(c, al, so, res, nres)) return e;
+  for (const Launch &Lq : L) if (int e = list_runs(c, al, Lq, res)) return e;
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-  for (const Launch &Lq : L) { int e = launch(c, Lq); if (e) return e; }
+  for (const Launch &Lq : L) if (int e = launch(c, Lq)) return e;
   HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (int e = deliver(c, jobs, bins->ntot, res, nhist, flags, cnt, arena != nullptr)) return e;
   float ms = 0;
   HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
-  int e = deliver(c, jobs, bins->ntot, dh, flags, cnt);
-  if (e) return e;
-  if ((e = stats_from(c, misc))) return e;
   c->stats.kernel_ms = ms;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->stats.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return 0;
 }
@@ -3069,17 +3156,30 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
     hipLaunchKernelGGL(k_fill_f64, dim3(nblk(b->n, 256)), dim3(256), 0, c->stream, dgb, (int64_t) b->n, 0.0);
   jobs[0].gA = sw ? dgb : dga;
   jobs[0].gB = autoc ? dga : (sw ? dga : dgb);
-  if (int e = stage_run(c, al, stages, jobs)) return e;
-  double *dG = (double *) al.tmp(WS_G, sizeof(double) * bins->ntot);
-  const int nmisc = misc_words((int) jobs.size());
-  unsigned long long *misc = (unsigned long long *) al.tmp(WS_MISC, 8 * (size_t) nmisc);
+  Sort so;
+  if (int e = sort_alloc(c, al, stages, jobs, &so)) return e;
+  const int nres = res_hist(1);
+  unsigned long long *res = (unsigned long long *) al.tmp(WS_RES, 8 * (size_t) nres);
   if (al.err) return al.err;
-  HIPCHK(c, hipMemcpyAsync(dG, grad_cnt, sizeof(double) * bins->ntot,
-      dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nmisc, 256)), dim3(256), 0, c->stream, misc, nmisc);
+  Launch L;
+  Upload up(c);
+  StreamDrain drain2{c};
+  if (int e = up.reserve(al, upload_bytes(bins, jobs, stages.size(), true), false)) return e;
+  DevTabs tabs;
+  put_tables(up, bins, &tabs);
+  if (dev) tabs.G = grad_cnt;
+  else tabs.G = up.put(grad_cnt, bins->ntot);
+  so.st = up.put(stages.data(), stages.size());
+  if (int e = build_launch(c, al, up, tabs, bins, jobs, MODE_GRAD, res, nullptr, &L)) return e;
+  if (int e = up.flush()) return e;
+  if (int e = sort_run(c, al, so, res, nres)) return e;
+  if (int e = list_runs(c, al, L, res)) return e;
+  HIPCHK(c, hipEventRecord(c->ev0, c->stream));
+  if (int e = launch(c, L)) return e;
+  HIPCHK(c, hipEventRecord(c->ev1, c->stream));
+  if (int e = deliver(c, jobs, 0, res, 0, 0, nullptr, false)) return e;
   float ms = 0;
-  int e = run_jobs(c, al, bins, jobs, MODE_GRAD, dG, nullptr, misc, (unsigned int *) (misc + 8), &ms);
-  if (e) return e;
+  HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   for (int p = 0; p < 2; p++) {
     const fcfc_cat *k = p ? b : a;
     double *gout = p ? gb : ga, *gdev = p ? dgb : dga;
@@ -3088,14 +3188,17 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
       hipLaunchKernelGGL(k_add_f64, dim3(nblk(k->n, 256)), dim3(256), 0, c->stream, gout, gdev, (int) k->n);
       HIPCHK(c, hipGetLastError());
     }
-    else {
-      std::vector<double> h((size_t) k->n);
-      HIPCHK(c, hipMemcpyAsync(h.data(), gdev, sizeof(double) * (size_t) k->n, hipMemcpyDeviceToHost, c->stream));
+    else if (k->n > 0) {
+      std::vector<double> hv;
+      const size_t nb = sizeof(double) * (size_t) k->n;
+      double *h = (double *) c->pin;
+      if (!Upload::pin_fit(c, nb, false)) { hv.resize((size_t) k->n); h = hv.data(); }
+      else h = (double *) c->pin;
+      HIPCHK(c, hipMemcpyAsync(h, gdev, nb, hipMemcpyDeviceToHost, c->stream));
       HIPCHK(c, hipStreamSynchronize(c->stream));
-      for (int64_t i = 0; i < k->n; i++) gout[i] += h[(size_t) i];
+      for (int64_t i = 0; i < k->n; i++) gout[i] += h[i];
     }
   }
-  if ((e = stats_from(c, misc))) return e;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->stats.kernel_ms = ms;
   c->stats.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -3112,8 +3215,7 @@ struct fcfc_gpu_plan {
   int ntot = 0;
   uint32_t flags = 0;
   std::vector<Launch> L;             /* one per launch group */
-  void *dh = nullptr;                /* njob x ntot histograms (8 bytes per bin) */
-  unsigned long long *misc = nullptr;
+  unsigned long long *res = nullptr; /* result words: counters, njob x ntot histograms */
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   explicit fcfc_gpu_plan(fcfc_gpu_ctx *c_) : c(c_), al(c_, true) {}
@@ -3155,24 +3257,34 @@ extern "C" int fcfc_gpu_plan_create(fcfc_gpu_ctx *c, int njob, const fcfc_batch_
     P->jobs[k].hist_off = (long long) k * bins->ntot;
     P->jobs[k].qi = k;
   }
-  if (int e = stage_run(c, P->al, stages, P->jobs)) return e;
-  P->dh = P->al.get(WS_HIST, 8 * (size_t) bins->ntot * njob);
-  const int nmisc = misc_words(njob);
-  P->misc = (unsigned long long *) P->al.get(WS_MISC, 8 * (size_t) nmisc);
+  Sort so;
+  if (int e = sort_alloc(c, P->al, stages, P->jobs, &so)) return e;
+  const int nres = res_hist(njob) + bins->ntot * njob;
+  P->res = (unsigned long long *) P->al.get(WS_RES, 8 * (size_t) nres);
   if (P->al.err) return P->al.err;
   std::vector<std::vector<PJob>> groups = launch_groups(P->jobs);
   P->L.resize(groups.size());
-  int e = 0;
+  Upload up(c);
+  StreamDrain drain2{c};
+  int e = up.reserve(P->al, upload_bytes(bins, P->jobs, stages.size(), false), true);
+  if (e) return e;
+  DevTabs tabs;
+  put_tables(up, bins, &tabs);
+  so.st = up.put(stages.data(), stages.size());
   for (size_t q = 0; q < groups.size(); q++)
-    if ((e = build_launch(c, P->al, bins, groups[q], mode, nullptr, P->dh, P->misc,
-                          (unsigned int *) (P->misc + 8), &P->L[q]))) return e;
+    if ((e = build_launch(c, P->al, up, tabs, bins, groups[q], mode, P->res, P->res + res_hist(njob),
+                          &P->L[q]))) return e;
+  if ((e = up.flush())) return e;
+  if ((e = sort_run(c, P->al, so, P->res, nres))) return e;
+  for (const Launch &Lq : P->L) if ((e = list_runs(c, P->al, Lq, P->res))) return e;
+  unsigned long long bad = 0;
+  HIPCHK(c, hipMemcpyAsync(&bad, P->res + RES_BAD, 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (bad) { set_err(c, "a catalogue has a non-finite coordinate"); return FCFC_ERR_DATA; }
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   for (const Gather &g : P->gathers)
     hipLaunchKernelGGL(k_gather, dim3(nblk(g.n, 256)), dim3(256), 0, c->stream, g.n, g.idx, g.src, g.dst, g.stride);
-  hipLaunchKernelGGL(k_zero_u64, dim3(nblk((int64_t) bins->ntot * njob, 256)), dim3(256), 0, c->stream,
-      (unsigned long long *) P->dh, bins->ntot * njob);
-  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nmisc, 256)), dim3(256), 0, c->stream, P->misc, nmisc);
+  hipLaunchKernelGGL(k_zero_u64, dim3(nblk(nres, 256)), dim3(256), 0, c->stream, P->res, nres);
   for (const Launch &Lq : P->L) if ((e = launch(c, Lq))) break;
   hipGraph_t graph = nullptr;
   const hipError_t ce = hipStreamEndCapture(c->stream, &graph);
@@ -3194,10 +3306,7 @@ extern "C" int fcfc_gpu_plan_run(fcfc_gpu_plan *P, void *cnt) {
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   HIPCHK(c, hipGraphLaunch(P->exec, c->stream));
   HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-  int e = deliver(c, P->jobs, P->ntot, P->dh, P->flags, cnt);
-  if (e) return e;
-  if ((e = stats_from(c, P->misc))) return e;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (int e = deliver(c, P->jobs, P->ntot, P->res, P->ntot * (int) P->jobs.size(), P->flags, cnt, false)) return e;
   float ms = 0;
   HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   c->stats.kernel_ms = ms;
@@ -3286,14 +3395,15 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
     }
     if (e) break;
   }
-  /* the grid runs each shape at its automatic tile size (FK_NT objects for
-   * small cells); the best three shapes are also timed at the other sizes
-   * the kernel family holds (fk_lanes_max: 4 FK_NT for weighted FP64 box
-   * counts with integer tables, FK_NT for the hybrid gradient kernel) */
+  /* the grid runs each shape at its automatic tile size; the best three
+   * shapes are also timed at the other size the kernel family holds (FK_NT
+   * for the hybrid gradient kernel).  4 FK_NT is left to the caller: since B
+   * objects are read by scalar loads it loses (weighted DR of 2e5 x 2e6 15.6
+   * against 15.1 ms, DD of 5e5 7.6 against 6.9) */
   std::sort(grid.begin(), grid.end(), [](const Cand &x, const Cand &y) { return x.est < y.est; });
   const int lmax = fk_lanes_max(bins->geometry, mode, grad || (flags & FCFC_GPU_WEIGHTED) ? 1 : 0,
                                 (bins->tabtype || !zb_fits(bins)) ? 1 : 0);
-  const int Ts[] = {FK_NT, 2 * FK_NT, 4 * FK_NT};
+  const int Ts[] = {FK_NT, 2 * FK_NT};
   for (size_t k = 0; k < grid.size() && k < 3 && !e; k++) {
     for (int T : Ts) {
       double est;
@@ -3315,8 +3425,8 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
     if (bins->geometry == FCFC_GEOM_SURVEY) {
       for (int k = 0; k < 3; k++) { lo[k] = 1e300; hi[k] = -1e300; }
       Alloc tal(c, false);
-      bbox(c, tal, ka, lo, hi);
-      if (!autoc) bbox(c, tal, kb, lo, hi);
+      const fcfc_cat *ks[2] = {ka, kb};
+      if ((e = bbox(c, tal, ks, autoc ? 1 : 2, lo, hi))) return e;
     }
     const int wt = (grad || (flags & FCFC_GPU_WEIGHTED)) ? 1 : 0;
     make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, ka->n, kb->n, &P);

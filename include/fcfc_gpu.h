@@ -188,7 +188,10 @@ int fcfc_gpu_count_noalloc(fcfc_gpu_ctx *ctx, const fcfc_cat *a,
 
 /* Per-call statistics of the last fcfc_gpu_count / _batch / _backward. */
 typedef struct {
-  double evals;          /* candidate pair distances evaluated              */
+  double evals;          /* candidate pairs of the grid's cell windows (each
+                            settled by its distance, or with the 64 pairs or
+                            more of a B object beyond the separation from the
+                            bounding box of a wavefront's A objects)        */
   double rechecked;      /* pairs re-evaluated in FP64 (FP32 mode)          */
   double census;         /* rounding-path ambiguous pairs (FCFC_GPU_CENSUS) */
   double kernel_ms;      /* device time of the count kernel(s)              */
@@ -249,25 +252,24 @@ int fcfc_gpu_count_backward(fcfc_gpu_ctx *ctx, const fcfc_cat *a,
 /* ---- tuning ------------------------------------------------------------- */
 /* Override the grid and launch shape (0 = automatic / autotuned):
  * cell_div = cells per maximum separation in x and y, tile = A objects per
- * tile (at most 2048; above 1024 only the weighted FP64 box counts with
- * integer tables hold such tiles, four objects per lane, other counts cut
- * them to 1024), zcell_div = z-cells per x-cell, nblock = persistent workgroups. */
+ * tile, the runs of a workgroup's 8 wavefronts (at most 2048; above 1024 only
+ * the weighted FP64 box counts with integer tables hold such tiles, four
+ * objects per lane, other counts cut them to 1024), zcell_div = z-cells per
+ * x-cell, nblock = persistent workgroups. */
 int fcfc_gpu_set_tuning(fcfc_gpu_ctx *ctx, int cell_div, int tile,
     int zcell_div, int nblock);
 
 /* Autotuner (no counterpart in the reference): times candidate grid / tile
  * shapes for counts like (a, b, bins, flags) on an eighth (beyond 16384
- * tiles: a sixteenth) of their tile list, taken as 16 runs of consecutive
- * tiles spread over the whole list (counts of at most 4096 tiles whole):
+ * tiles: a sixteenth) of their runs, taken as 16 stretches of consecutive
+ * runs spread over the whole list (counts of at most 4096 tiles whole):
  * every pair of cell_div {2, 3, 4, 6} and zcell_div {1, 2, 4, 8, 16} at its
- * automatic tile size, then the best three pairs at the other tile sizes of
- * {512, 1024} (and 2048 for weighted FP64 box counts with integer tables), and
- * keeps the fastest in the
- * context for this geometry, binning, precision and density bucket; later
- * counts whose shape is automatic use it.  With FCFC_GPU_GRADIENT in flags
- * it tunes fcfc_gpu_count_backward for such counts instead.  best (may be
- * NULL) receives {cell_div, zcell_div, tile, estimated full-count
- * microseconds}. */
+ * automatic tile size, then the best three pairs at the other tile size of
+ * {512, 1024}, and keeps the fastest in the context for this geometry,
+ * binning, precision and density bucket; later counts whose shape is
+ * automatic use it.  With FCFC_GPU_GRADIENT in flags it tunes
+ * fcfc_gpu_count_backward for such counts instead.  best (may be NULL)
+ * receives {cell_div, zcell_div, tile, estimated full-count microseconds}. */
 int fcfc_gpu_autotune(fcfc_gpu_ctx *ctx, const fcfc_cat *a, const fcfc_cat *b,
     const fcfc_bins *bins, const double *bsize, uint32_t flags, int *best);
 
