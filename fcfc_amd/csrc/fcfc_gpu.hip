@@ -40,14 +40,14 @@ __device__ __forceinline__ int fk_cell1(double v, double o, double w, int nc) {
   return q < 0 ? 0 : (q >= nc ? nc - 1 : q);
 }
 
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
+__global__ void k_zero_u64(unsigned long long *p, size_t n) {
+  for (size_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
 }
 /* the counters and histograms of a call and the cell counts of its sort */
-__global__ void k_zero_call(unsigned long long *p, int n, int *q, int m) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x, st = gridDim.x * blockDim.x;
-  for (int i = t; i < n; i += st) p[i] = 0ull;
-  for (int i = t; i < m; i += st) q[i] = 0;
+__global__ void k_zero_call(unsigned long long *p, size_t n, int *q, size_t m) {
+  const size_t t = blockIdx.x * blockDim.x + threadIdx.x, st = gridDim.x * blockDim.x;
+  for (size_t i = t; i < n; i += st) p[i] = 0ull;
+  for (size_t i = t; i < m; i += st) q[i] = 0;
 }
 
 /* Exclusive scan of n ints into out[0..n] (out[n] = total).  Workgroups of
@@ -173,25 +173,30 @@ __global__ void k_stage_scatter(int nobj, int nst, const FkStage *__restrict__ s
   }
 }
 
-/* Work items of a job's runs: run ti becomes S items (each a share of the
- * strip list) for ti < tt and St > S finer items from tt on, so that the
- * items the wavefronts take last are short and the launch ends evenly.
- * ncap runs in all: of each group of G consecutive runs of the list, its
- * first `run` runs.  A full count has one group (G = run = the number of
- * runs); the autotuner's samples take stretches spread over the whole
- * catalogue, each keeping the neighbourhood, and so the cache reuse, of a
- * full count. */
-struct FkSplit { int S, tt, St, ncap, G, run, nitems, run0; };   /* run0: its first run */
+/* Work items of a job's runs: run ti becomes S items for ti < tt and St > S
+ * finer items from tt on, so that the items the wavefronts take last are short
+ * and the launch ends evenly.  An item is a share of the strip list and, of
+ * each segment there, every SQ-th (StQ-th) chunk of 64 B objects: S / SQ
+ * shares, SQ items each.  ncap runs in all: of each group of G consecutive
+ * runs of the list, its first `run` runs.  A full count has one group (G = run
+ * = the number of runs); the autotuner's samples take stretches spread over
+ * the whole catalogue, each keeping the neighbourhood, and so the cache reuse,
+ * of a full count. */
+struct FkSplit { int S, SQ, tt, St, StQ, ncap, G, run, nitems, run0; };   /* run0: first run */
 
 /* The split of nrun runs of smax strips at most and of about `chunks` chunks
- * of 64 candidate B objects each, for nw wavefronts: 16 items per wavefront,
- * but none of fewer than 8 chunks (an item loads its A objects and searches
- * its strips first, about the work of a chunk: survey (s_perp, pi) DR of 3e4 x
- * 1e6 1.95 -> 1.61 ms, small-scale cross count 1.61 -> 1.11 ms against 16 items
- * whatever their size; large counts unchanged); where that leaves wavefronts
- * without an item, one each, of 2 chunks at least. */
-__host__ __device__ inline FkSplit fk_split(int nrun, int nw, int chunks, int smax, int frac) {
-  FkSplit sp = {1, 0, 1, 0, nrun > 1 ? nrun : 1, nrun > 1 ? nrun : 1, 0, 0};
+ * of candidate B objects each, for nw wavefronts: ipw items per wavefront, but
+ * none of fewer than 4 chunks (an item loads its A objects and searches its
+ * strips first, about the work of a chunk); where that leaves wavefronts
+ * without an item, one each, of 2 chunks at least.  More items than strips
+ * share the chunks of a strip: sparse catalogues have few strips (weight
+ * gradient of DD of 4e4 objects, 5 strips: 1.29 -> 0.40 ms).  ipw = 16 for a
+ * single job (8: DR of 2e5 x 2e6 16.7 against 15.2 ms, survey (s, mu) RR 16.8
+ * against 16.1); 2 for the jobs of a batch, whose workgroups move on to other
+ * jobs (16: 16 mocks 5.1 against 4.2 ms, DD + DR of a fit 1.52 against 1.23).
+ * At least 8 chunks: small-scale cross count 1.12 against 1.00 ms. */
+__host__ __device__ inline FkSplit fk_split(int nrun, int nw, int ipw, int chunks, int smax, int frac) {
+  FkSplit sp = {1, 1, 0, 1, 1, 0, nrun > 1 ? nrun : 1, nrun > 1 ? nrun : 1, 0, 0};
   if (nrun <= 0) return sp;
   if (frac > 1) {
     sp.G = (nrun + 15) / 16;
@@ -201,24 +206,28 @@ __host__ __device__ inline FkSplit fk_split(int nrun, int nw, int chunks, int sm
   sp.ncap = last * sp.run + (sp.run < rest ? sp.run : rest);
   auto lim = [](long long v, int most) -> int { return (int) (v < most ? v : most); };
   auto one = [](int v) -> int { return v > 1 ? v : 1; };
-  const int s16 = lim((16LL * nw + sp.ncap - 1) / sp.ncap, one(chunks / 8));
+  /* n items of at most smax shares: q per share */
+  auto parts = [&](int n, int *q) -> int { *q = (n + smax - 1) / smax; return (n + *q - 1) / *q * *q; };
+  const int s16 = lim(((long long) ipw * nw + sp.ncap - 1) / sp.ncap, one(chunks / 4));
   const int s1 = lim(((long long) nw + sp.ncap - 1) / sp.ncap, one(chunks / 2));
-  sp.S = one(lim(s16 > s1 ? s16 : s1, smax));
+  const int S = one(lim(s16 > s1 ? s16 : s1, 1024));
+  sp.S = parts(S, &sp.SQ);
   /* the runs of about two items per wavefront at the end of the list are
-   * split four times finer */
-  sp.St = one(lim(4LL * sp.S, smax));
+   * split up to four times finer, into items of 2 chunks at least */
+  const int St = lim(4LL * S, chunks / 2 > S ? chunks / 2 : S);
+  sp.St = parts(lim(St, 1024), &sp.StQ);
   const long long tail = (2LL * nw + sp.S - 1) / sp.S;
   sp.tt = tail < sp.ncap ? sp.ncap - (int) tail : 0;
-  if (sp.St <= sp.S) { sp.St = sp.S; sp.tt = sp.ncap; }
-  if ((long long) sp.St * sp.ncap > (1LL << 30)) { sp.S = sp.St = 1; sp.tt = sp.ncap; }
+  if (sp.St <= sp.S) { sp.St = sp.S; sp.StQ = sp.SQ; sp.tt = sp.ncap; }
+  if ((long long) sp.St * sp.ncap > (1LL << 30)) { sp.S = sp.St = sp.SQ = sp.StQ = 1; sp.tt = sp.ncap; }
   sp.nitems = sp.S * sp.tt + sp.St * (sp.ncap - sp.tt);
   return sp;
 }
 
 /* Runs of all jobs of a launch: job k owns nunit units from unit0 (ascending);
  * a unit is one block of zm z-cells of one row, cut into runs of T consecutive
- * objects.  nw, chunks, smax, frac: its split (fk_split). */
-struct FkTileJob { int unit0, nunit, nblk, zm, ncz, T, nw, chunks, smax, frac; const int *cs; };
+ * objects.  nw, ipw, chunks, smax, frac: its split (fk_split). */
+struct FkTileJob { int unit0, nunit, nblk, zm, ncz, T, nw, ipw, chunks, smax, frac; const int *cs; };
 
 __device__ __forceinline__ int fk_tile_job(const FkTileJob *__restrict__ tj, int njob, int u) {
   int lo = 0, hi = njob - 1;                  /* last job with unit0 <= u */
@@ -253,7 +262,7 @@ __global__ void k_run_emit(int nunit, int njob, const FkTileJob *__restrict__ tj
     const unsigned long long *__restrict__ bad) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < njob; k += gridDim.x * blockDim.x) {
     const FkTileJob t = tj[k];
-    FkSplit sp = fk_split(roff[t.unit0 + t.nunit] - roff[t.unit0], max(t.nw, FK_NW), t.chunks, t.smax,
+    FkSplit sp = fk_split(roff[t.unit0 + t.nunit] - roff[t.unit0], max(t.nw, FK_NW), t.ipw, t.chunks, t.smax,
                           t.frac);
     sp.run0 = roff[t.unit0];
     if (*bad) sp.nitems = 0;                  /* a non-finite coordinate: nothing is counted */
@@ -375,6 +384,14 @@ struct FkWin {
 #define FK_F_ALWAYS 0x4000u   /* FP32 threshold (high half) of FK_F_ALW cells: 2 */
 #define FK_F_NEVER  0xBF80u   /* ... of cells without flags: -1                  */
 
+/* Atomics on one address take 11.4 ns each, wherever they come from (8192
+ * wavefronts: 93 us); spread over 64 lines 0.25 to 0.4 ns.  So the statistics
+ * of a call are summed in FK_STATS lines, and a job's work items are dealt to
+ * up to FK_GROUPS groups of workgroups with a counter each. */
+#define FK_LINE 64
+#define FK_STATS 64
+#define FK_GROUPS 64
+
 /* One counting job: a catalogue pair and its histogram.  A launch counts the
  * runs of one or many jobs (batched mocks); runs carry their job index. */
 struct FkJob {
@@ -386,11 +403,10 @@ struct FkJob {
                                  GRAD: A == B, exclude j == i          */
   int wt;                     /* weighted histogram (double)          */
   int wg0, wg1;               /* workgroups that start with it        */
-  int qi;                     /* its counter in the queue             */
+  int q0, G;                  /* its counters: line q0 of the queue, G of them */
   long long hist_off;         /* histogram of this job: gcnt + hist_off */
-  double *gA;                 /* GRAD: output for A objects, original order (or null) */
-  double *gB;                 /* GRAD: output for B objects, original order (or null;
-                                 auto counts: the same array as gA)   */
+  double *gA;                 /* GRAD: output for A objects, indexed as the records (or null) */
+  double *gB;                 /* GRAD: output for B objects (or null; auto counts: gA) */
   FkWin win;                  /* FP32 error model (MODE_C32)          */
 };
 
@@ -400,10 +416,10 @@ struct FkArgs {
   FkBins bins;
   const FkRun *runs;
   const FkSplit *splits;      /* work items of each job              */
-  unsigned int *queue;        /* work items taken, per job            */
+  unsigned int *queue;        /* work items taken: counters of FK_LINE bytes */
   unsigned long long *gcnt_u;
   double *gcnt_d;
-  unsigned long long *stats;  /* evals, rechecked, census */
+  unsigned long long *stats;  /* FK_STATS lines of evals, rechecked, census  */
   int nh;                     /* LDS histogram copies */
   /* LDS byte offsets */
   int off_hist, off_stab, off_ptab, off_edges, off_chunk, off_queue;
@@ -1189,6 +1205,13 @@ k_count(const FkArgs a) {
     since = 0;
   };
 
+  /* wavefronts of the workgroups of group g (of G) of a job that nwg
+   * workgroups start with, and the counter of line q of the queue */
+  auto group_waves = [](int nwg, int G, int g) -> int { return FK_NW * ((nwg - g + G - 1) / G); };
+  auto queue_load = [&](int q) -> unsigned {
+    return __hip_atomic_load(a.queue + (size_t) q * (FK_LINE / 4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+
   /* Each workgroup counts one job at a time; its wavefronts take the job's
    * items on their own and meet when it has none left.  Then the LDS
    * histograms are added to the job's global one and the workgroup goes on to
@@ -1235,10 +1258,14 @@ k_count(const FkArgs a) {
         if (k0 + lane < a.njobs) {
           int q = cur + k0 + lane;
           if (q >= a.njobs) q -= a.njobs;
-          const int nw = (a.jobs[q].wg1 - a.jobs[q].wg0) * FK_NW;
-          const long long taken = nw + (long long) __hip_atomic_load(a.queue + a.jobs[q].qi,
-              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          has = taken + (nw ? FK_NW - 1 : 0) < a.splits[q].nitems;
+          const FkJob *pj = a.jobs + q;
+          const int n = a.splits[q].nitems, nwg = pj->wg1 - pj->wg0;
+          long long left = 0;
+          for (int g = 0; g < pj->G; g++) {
+            const int taken = group_waves(nwg, pj->G, g) + (int) queue_load(pj->q0 + g);
+            left += max((n - g + pj->G - 1) / pj->G - taken, 0);
+          }
+          has = left >= (nwg ? FK_NW : 1);
         }
         const unsigned long long m = __builtin_amdgcn_ballot_w64(has);
         if (m) { nx = cur + k0 + (int) __builtin_ctzll(m); if (nx >= a.njobs) nx -= a.njobs; }
@@ -1249,26 +1276,43 @@ k_count(const FkArgs a) {
     cur = __builtin_amdgcn_readfirstlane(s_job);
     if (cur < 0) break;
 
-  /* the job's items: the first one of each wavefront that starts with the
-   * job is its own index, the others follow from the queue */
-  for (;; first = false) {
+  /* The job's items: item i belongs to group i % G.  The first one of each
+   * wavefront that starts with the job follows from its place among the
+   * group's wavefronts, the others from the group's counter; when the group
+   * has none left, another one's (every wavefront ends when no group has any). */
+  int grp = first ? ((int) blockIdx.x - fk_cld(&fk_again(a.jobs, cur)->wg0)) % fk_cld(&fk_again(a.jobs, cur)->G)
+                  : (int) blockIdx.x % fk_cld(&fk_again(a.jobs, cur)->G);
+  for (;;) {
     const FkSplit sp = fk_cld(a.splits + cur);
     const FkJob *pq = fk_again(a.jobs, cur);
-    const int wg0 = fk_cld(&pq->wg0), nw = (fk_cld(&pq->wg1) - wg0) * FK_NW;
-    int it = ((int) blockIdx.x - wg0) * FK_NW + wave;
+    const int wg0 = fk_cld(&pq->wg0), nwg = fk_cld(&pq->wg1) - wg0, G = fk_cld(&pq->G), q0 = fk_cld(&pq->q0);
+    int it = ((int) blockIdx.x - wg0) / G * FK_NW + wave;
     if (!first) {
-      if (lane == 0) it = nw + (int) atomicAdd(a.queue + fk_cld(&pq->qi), 1u);
+      if (lane == 0)
+        it = group_waves(nwg, G, grp) + (int) atomicAdd(a.queue + (size_t) (q0 + grp) * (FK_LINE / 4), 1u);
       it = __builtin_amdgcn_readfirstlane(it);
     }
-    if (it >= sp.nitems) break;
-    /* work item -> run and share of its strips */
-    int part, S, ri;
+    first = false;
+    it = grp + G * it;
+    if (it >= sp.nitems) {
+      bool has = false;
+      if (lane < G) has = lane + (long long) G * (group_waves(nwg, G, lane) + (int) queue_load(q0 + lane)) < sp.nitems;
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(has), mn = m >> grp >> 1;
+      if (m == 0) break;
+      grp = mn ? grp + 1 + (int) __builtin_ctzll(mn) : (int) __builtin_ctzll(m);
+      continue;
+    }
+    /* work item -> run, share of its strips, chunks of their segments */
+    int part, S, SQ, ri;
     const int h = sp.S * sp.tt;
-    if (it < h) { S = sp.S; ri = it / S; part = it - ri * S; }
-    else { S = sp.St; ri = (it - h) / S; part = it - h - ri * S; ri += sp.tt; }
-    const int grp = ri / sp.run;
+    if (it < h) { S = sp.S; SQ = sp.SQ; ri = it / S; part = it - ri * S; }
+    else { S = sp.St; SQ = sp.StQ; ri = (it - h) / S; part = it - h - ri * S; ri += sp.tt; }
+    const int sq = part % SQ;
+    S /= SQ;
+    part /= SQ;
+    const int smp = ri / sp.run;
     const FkRun t = fk_cld(a.runs + __builtin_amdgcn_readfirstlane(
-        sp.run0 + grp * sp.G + (ri - grp * sp.run)));
+        sp.run0 + smp * sp.G + (ri - smp * sp.run)));
 
     const FkJob J = fk_cld(a.jobs + cur);
     const int s0 = (int) ((long long) J.nstrips * part / S);
@@ -1465,8 +1509,8 @@ k_count(const FkArgs a) {
         if (idx < ntot_o && !queued) {
           if (GRAD) {
             const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
-            gacc[r] += gk * wj;
-            bsum += gk * aw[r];
+            gacc[r] = __builtin_fma(gk, wj, gacc[r]);
+            bsum = __builtin_fma(gk, aw[r], bsum);
           }
           else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
           else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
@@ -1486,7 +1530,7 @@ k_count(const FkArgs a) {
     auto segment = [&](auto selfc, auto imgc, int b0, int n, int code) __attribute__((always_inline)) {
       constexpr bool SELF = decltype(selfc)::value;
       constexpr bool IMG = decltype(imgc)::value;
-      for (int c0 = 0; c0 < n; c0 += FK_CH) {
+      for (int c0 = SELF ? 0 : sq * FK_CH; c0 < n; c0 += SELF ? FK_CH : SQ * FK_CH) {
         const FkJob *pj = fk_again(a.jobs, cur);
         const FkCat B = fk_cld(SELF ? &pj->A : &pj->B);
         const FkGrid g = fk_cld(&pj->g);
@@ -1563,10 +1607,8 @@ k_count(const FkArgs a) {
           if (GRAD && hasB) {
             fk_wave_sync();
             if (keep) {
-              const FkJob *pk = fk_again(a.jobs, cur);
               const double v = cb[lane];
-              if (v != 0.0)
-                unsafeAtomicAdd(fk_cld(&pk->gB) + fk_gld(fk_cld(SELF ? &pk->A.idx : &pk->B.idx), jg), v);
+              if (v != 0.0) unsafeAtomicAdd(fk_cld(&fk_again(a.jobs, cur)->gB) + jg, v);
             }
           }
         }
@@ -1574,7 +1616,7 @@ k_count(const FkArgs a) {
     };
 
     /* ---- auto counts: pairs inside the run (j > i), first item only ---- */
-    if (J.autoc && part == 0) {
+    if (J.autoc && part == 0 && sq == 0) {
       evals -= (unsigned long long) nva * (unsigned) nva / 2;
       segment(std::true_type(), std::false_type(), t.p0, nva, 13);
     }
@@ -1615,23 +1657,26 @@ k_count(const FkArgs a) {
     if (F32 && qn) drain();
 
     if (GRAD) {
-      const FkJob *pj = fk_again(a.jobs, cur);
-      double *gA = fk_cld(&pj->gA);
-      const int *idx = fk_cld(&pj->A.idx);
+      double *gA = fk_cld(&fk_again(a.jobs, cur)->gA);
       if (gA)
 #pragma unroll
         for (int r = 0; r < R; r++)
-          if (ai[r] != 0x7fffffff && gacc[r] != 0.0)
-            unsafeAtomicAdd(gA + fk_gld(idx, ai[r]), gacc[r]);
+          if (ai[r] != 0x7fffffff && gacc[r] != 0.0) unsafeAtomicAdd(gA + ai[r], gacc[r]);
     }
   }
   }
 
-  if (lane == 0) atomicAdd(a.stats + 0, evals);
+  /* statistics: summed over the workgroup, then in one of FK_STATS lines */
+  __shared__ unsigned long long s_stat[3];
+  if (tid < 3) s_stat[tid] = 0ull;
+  __syncthreads();
+  if (lane == 0) atomicAdd(&s_stat[0], evals);
   if (F32) {
-    if (nrecheck) atomicAdd(a.stats + 1, (unsigned long long) nrecheck);
-    if (ncensus) atomicAdd(a.stats + 2, (unsigned long long) ncensus);
+    if (nrecheck) atomicAdd(&s_stat[1], (unsigned long long) nrecheck);
+    if (ncensus) atomicAdd(&s_stat[2], (unsigned long long) ncensus);
   }
+  __syncthreads();
+  if (tid < 3 && s_stat[tid]) atomicAdd(a.stats + blockIdx.x % FK_STATS * (FK_LINE / 8) + tid, s_stat[tid]);
 }
 
 /* add a device histogram into the caller's device array */
@@ -1701,11 +1746,14 @@ static void set_err(fcfc_gpu_ctx *c, const char *fmt, ...) {
     set_err(ctx, "%s failed: %s (%s:%d)", #call, hipGetErrorString(_e), __FILE__, __LINE__); \
     return FCFC_ERR_GPU; } } while (0)
 
-/* Words of a call's results, zeroed before its launches: pairs evaluated,
- * re-evaluated, of the census, the flag of non-finite coordinates, then the
- * queue (one 32-bit word per job) and the histograms. */
-enum { RES_EVALS, RES_RECHECKED, RES_CENSUS, RES_BAD, RES_QUEUE };
-static int res_hist(int njob) { return RES_QUEUE + (njob + 1) / 2; }
+/* Words of a call's results, zeroed before its launches: FK_STATS lines of
+ * statistics (pairs evaluated, re-evaluated, of the census; the first line
+ * also holds the flag of non-finite coordinates), the histograms, and after
+ * them the queue. */
+enum { RES_EVALS, RES_RECHECKED, RES_CENSUS, RES_BAD, RES_HIST = FK_STATS * (FK_LINE / 8) };
+/* counters per job of a call */
+static int queue_lines(int njob) { return njob <= 64 ? FK_GROUPS : 16; }
+static size_t queue_words(int njob) { return (size_t) njob * queue_lines(njob) * (FK_LINE / 8); }
 
 /* workspace slots */
 enum {
@@ -2013,7 +2061,7 @@ struct PJob {
   int autoc = 0, wt = 0;
   double *gA = nullptr, *gB = nullptr;
   long long hist_off = 0;
-  int qi = 0;                   /* counter of its work items */
+  int qi = 0;                   /* its place in the call's queue */
 };
 
 static inline int nblk(int64_t n, int bs) {
@@ -2087,6 +2135,16 @@ __global__ void k_gather(int n, const int *__restrict__ idx, const double *__res
     double *__restrict__ dst, int stride) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     dst[(size_t) stride * i] = src[idx[i]];
+}
+
+/* sorted values into the original order.  The gradient kernel adds each B
+ * object's share once per chunk and run, 64 neighbours of the sorted order at
+ * a time: 8 lines where the original order has up to 64 (weight gradient of
+ * DR, 4e4 x 2e5: 1.66 -> 1.54 ms). */
+__global__ void k_unsort(int n, const int *__restrict__ idx, const double *__restrict__ src,
+    double *__restrict__ dst) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    dst[idx[i]] = src[i];
 }
 
 __global__ void k_fill_f64(double *p, int64_t n, double v) {
@@ -2297,9 +2355,9 @@ static int sort_alloc(fcfc_gpu_ctx *c, Alloc &al, const std::vector<FkStage> &st
 }
 
 /* zero the call's result words and sort its catalogues */
-static int sort_run(fcfc_gpu_ctx *c, Alloc &al, const Sort &so, unsigned long long *res, int nres) {
-  hipLaunchKernelGGL(k_zero_call, dim3(nblk(std::max(nres, so.ncell), 256)), dim3(256), 0, c->stream,
-                     res, nres, so.count, so.ncell);
+static int sort_run(fcfc_gpu_ctx *c, Alloc &al, const Sort &so, unsigned long long *res, size_t nres) {
+  hipLaunchKernelGGL(k_zero_call, dim3(nblk(std::max<int64_t>(nres, so.ncell), 256)), dim3(256), 0,
+                     c->stream, res, nres, so.count, (size_t) so.ncell);
   if (so.nobj > 0)
     hipLaunchKernelGGL(k_stage_assign, dim3(nblk(so.nobj, 256)), dim3(256), 0, c->stream, so.nobj,
                        so.nst, so.st, so.count, so.rank, res + RES_BAD);
@@ -2662,9 +2720,9 @@ static void put_tables(Upload &up, const fcfc_bins *b, DevTabs *t) {
 
 /* Prepare the run list and the persistent launch that counts (or
  * differentiates) the jobs; every buffer comes from al, descriptors go to up,
- * res are the result words and dhist the histograms. */
+ * res are the result words of the call and ncall its jobs. */
 static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &tabs, const fcfc_bins *b,
-    std::vector<PJob> &jobs, int mode, unsigned long long *res, void *dhist, Launch *out) {
+    std::vector<PJob> &jobs, int mode, unsigned long long *res, int ncall, Launch *out) {
   const int geom = b->geometry;
   int m = mode;
   const bool zb = zb_fits(b);
@@ -2781,6 +2839,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     t.T = std::min(J.P.T, 64 * J.P.R);
     t.chunks = (int) std::min(J.P.cand / 64, 1e9);
     t.smax = std::min(std::max(J.P.nstrips, 1), 64);
+    t.ipw = njob > 1 ? 2 : 16;
     t.frac = c->tile_frac;
     t.cs = J.A.cs;
     nunit_l += nu;
@@ -2788,7 +2847,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     /* at most as many runs as full ones and one remainder per non-empty unit */
     const long long nr = J.A.n / t.T + std::min<long long>(nu, J.A.n);
     maxrun += nr;
-    maxitem += nr * t.smax;
+    maxitem += nr * std::min<long long>(std::max(1, t.chunks / 2), 1024);
     work += (double) J.A.n * std::max(J.P.cand, 64.0);
   }
   nwg = (int) std::max<long long>(1, std::min<long long>(nwg, (maxitem + FK_NW - 1) / FK_NW));
@@ -2829,9 +2888,10 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     f.hist_off = J.hist_off;
     f.wg0 = wg0[k];
     f.wg1 = wg0[k + 1];
-    f.qi = J.qi;
-    f.gA = J.gA;
-    f.gB = J.gB;
+    f.q0 = J.qi * queue_lines(ncall);
+    f.G = std::min(std::max((wg0[k + 1] - wg0[k]) / 8, 1), queue_lines(ncall));
+    f.gA = J.gA ? J.gA - J.A.obj0 : nullptr;
+    f.gB = J.gB ? J.gB - J.B.obj0 : nullptr;
     if (m == MODE_C32) {
       fp32_windows(b, J.P.g, J.P.zmaxc, s2f, &f.win);
       win2s = std::max(win2s, f.win.e_s2x2);
@@ -2902,8 +2962,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   }
   fb.stab = tabs.stab; fb.ptab = tabs.ptab; fb.s2bin = tabs.s2e; fb.pbin = tabs.pe;
   a.runs = runs; a.splits = splits;
-  a.queue = (unsigned int *) (res + RES_QUEUE);
-  a.gcnt_u = (unsigned long long *) dhist; a.gcnt_d = (double *) dhist;
+  a.queue = (unsigned int *) (res + RES_HIST + (size_t) b->ntot * (m == MODE_GRAD ? 0 : ncall));
+  a.gcnt_u = res + RES_HIST; a.gcnt_d = (double *) (res + RES_HIST);
   a.stats = res;
   a.nh = L.nh;
   a.off_hist = L.off_hist; a.off_stab = L.off_stab; a.off_ptab = L.off_ptab;
@@ -2967,9 +3027,9 @@ static std::vector<std::vector<PJob>> launch_groups(const std::vector<PJob> &job
  * or double), in device or host memory. */
 static int deliver(fcfc_gpu_ctx *c, const std::vector<PJob> &jobs, int ntot,
     const unsigned long long *res, int nhist, uint32_t flags, void *cnt, bool fixed) {
-  const int njob = (int) jobs.size(), off = res_hist(njob);
+  const int njob = (int) jobs.size(), off = RES_HIST;
   const bool dev = (flags & FCFC_GPU_CNT_DEVICE) != 0;
-  const size_t n = dev ? (size_t) RES_QUEUE : (size_t) off + nhist;
+  const size_t n = (size_t) off + (dev ? 0 : nhist);
   std::vector<unsigned long long> hv;
   unsigned long long *h;
   /* (pinned memory that the call's upload used is free: the device has read
@@ -2978,9 +3038,12 @@ static int deliver(fcfc_gpu_ctx *c, const std::vector<PJob> &jobs, int ntot,
   else { hv.resize(n); h = hv.data(); }
   HIPCHK(c, hipMemcpyAsync(h, res, 8 * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->stats.evals = (double) h[RES_EVALS];
-  c->stats.rechecked = (double) h[RES_RECHECKED];
-  c->stats.census = (double) h[RES_CENSUS];
+  unsigned long long st[3] = {0, 0, 0};
+  for (int q = 0; q < FK_STATS; q++)
+    for (int k = 0; k < 3; k++) st[k] += h[q * (FK_LINE / 8) + k];
+  c->stats.evals = (double) st[RES_EVALS];
+  c->stats.rechecked = (double) st[RES_RECHECKED];
+  c->stats.census = (double) st[RES_CENSUS];
   if (h[RES_BAD]) { set_err(c, "a catalogue has a non-finite coordinate"); return FCFC_ERR_DATA; }
   if (!nhist) return 0;
   for (int k = 0; k < njob; k++) {
@@ -3028,8 +3091,9 @@ static int count_jobs(fcfc_gpu_ctx *c, int njob, const fcfc_cat *const *as,
   }
   Sort so;
   if (int e = sort_alloc(c, al, stages, jobs, &so)) return e;
-  const int nhist = bins->ntot * njob, nres = res_hist(njob) + nhist;
-  unsigned long long *res = (unsigned long long *) al.tmp(WS_RES, 8 * (size_t) nres);
+  const int nhist = bins->ntot * njob;
+  const size_t nres = RES_HIST + nhist + queue_words(njob);
+  unsigned long long *res = (unsigned long long *) al.tmp(WS_RES, 8 * nres);
   if (al.err) return al.err;
   /* one persistent launch per group */
   std::vector<std::vector<PJob>> groups = launch_groups(jobs);
@@ -3041,7 +3105,7 @@ static int count_jobs(fcfc_gpu_ctx *c, int njob, const fcfc_cat *const *as,
   put_tables(up, bins, &tabs);
   so.st = up.put(stages.data(), stages.size());
   for (size_t q = 0; q < groups.size(); q++)
-    if (int e = build_launch(c, al, up, tabs, bins, groups[q], mode, res, res + res_hist(njob), &L[q]))
+    if (int e = build_launch(c, al, up, tabs, bins, groups[q], mode, res, njob, &L[q]))
       return e;
   if (int e = up.flush()) return e;
   if (int e = sort_run(c, al, so, res, nres)) return e;
@@ -3147,19 +3211,19 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
   StreamDrain drain{c};
   if (int e = setup_job(c, al, copies, pa, pb, bins, bsize, autoc, 1, MODE_GRAD, &jobs[0], stages))
     return e;
-  double *dga = (double *) al.get(WS_GA, sizeof(double) * (size_t) (a->n > 0 ? a->n : 1));
-  double *dgb = (!autoc && gb) ? (double *) al.get(WS_GB, sizeof(double) * (size_t) (b->n > 0 ? b->n : 1))
-                               : nullptr;
+  /* gradients of the sorted objects, then in the original order */
+  const int64_t na = std::max<int64_t>(a->n, 1), nb = autoc || !gb ? 0 : std::max<int64_t>(b->n, 1);
+  double *dga = (double *) al.get(WS_GA, sizeof(double) * 2 * (size_t) na);
+  double *dgb = nb ? (double *) al.get(WS_GB, sizeof(double) * 2 * (size_t) nb) : nullptr;
   if (al.err) return al.err;
-  hipLaunchKernelGGL(k_fill_f64, dim3(nblk(a->n, 256)), dim3(256), 0, c->stream, dga, (int64_t) a->n, 0.0);
-  if (dgb)
-    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(b->n, 256)), dim3(256), 0, c->stream, dgb, (int64_t) b->n, 0.0);
+  hipLaunchKernelGGL(k_fill_f64, dim3(nblk(na, 256)), dim3(256), 0, c->stream, dga, na, 0.0);
+  if (dgb) hipLaunchKernelGGL(k_fill_f64, dim3(nblk(nb, 256)), dim3(256), 0, c->stream, dgb, nb, 0.0);
   jobs[0].gA = sw ? dgb : dga;
   jobs[0].gB = autoc ? dga : (sw ? dga : dgb);
   Sort so;
   if (int e = sort_alloc(c, al, stages, jobs, &so)) return e;
-  const int nres = res_hist(1);
-  unsigned long long *res = (unsigned long long *) al.tmp(WS_RES, 8 * (size_t) nres);
+  const size_t nres = RES_HIST + queue_words(1);
+  unsigned long long *res = (unsigned long long *) al.tmp(WS_RES, 8 * nres);
   if (al.err) return al.err;
   Launch L;
   Upload up(c);
@@ -3170,7 +3234,7 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
   if (dev) tabs.G = grad_cnt;
   else tabs.G = up.put(grad_cnt, bins->ntot);
   so.st = up.put(stages.data(), stages.size());
-  if (int e = build_launch(c, al, up, tabs, bins, jobs, MODE_GRAD, res, nullptr, &L)) return e;
+  if (int e = build_launch(c, al, up, tabs, bins, jobs, MODE_GRAD, res, 1, &L)) return e;
   if (int e = up.flush()) return e;
   if (int e = sort_run(c, al, so, res, nres)) return e;
   if (int e = list_runs(c, al, L, res)) return e;
@@ -3182,19 +3246,22 @@ extern "C" int fcfc_gpu_count_backward(fcfc_gpu_ctx *c, const fcfc_cat *a,
   HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   for (int p = 0; p < 2; p++) {
     const fcfc_cat *k = p ? b : a;
-    double *gout = p ? gb : ga, *gdev = p ? dgb : dga;
-    if (!gdev) continue;
+    double *gout = p ? gb : ga, *gsrt = p ? dgb : dga;
+    if (!gsrt) continue;
+    double *gdev = gsrt + (p ? nb : na);
+    const DevCat &dc = p == sw ? jobs[0].A : jobs[0].B;
+    hipLaunchKernelGGL(k_unsort, dim3(nblk(k->n, 256)), dim3(256), 0, c->stream, (int) k->n, dc.idx, gsrt, gdev);
     if (dev) {
       hipLaunchKernelGGL(k_add_f64, dim3(nblk(k->n, 256)), dim3(256), 0, c->stream, gout, gdev, (int) k->n);
       HIPCHK(c, hipGetLastError());
     }
     else if (k->n > 0) {
       std::vector<double> hv;
-      const size_t nb = sizeof(double) * (size_t) k->n;
-      double *h = (double *) c->pin;
-      if (!Upload::pin_fit(c, nb, false)) { hv.resize((size_t) k->n); h = hv.data(); }
-      else h = (double *) c->pin;
-      HIPCHK(c, hipMemcpyAsync(h, gdev, nb, hipMemcpyDeviceToHost, c->stream));
+      const size_t bytes = sizeof(double) * (size_t) k->n;
+      double *h;
+      if (Upload::pin_fit(c, bytes, false)) h = (double *) c->pin;
+      else { hv.resize((size_t) k->n); h = hv.data(); }
+      HIPCHK(c, hipMemcpyAsync(h, gdev, bytes, hipMemcpyDeviceToHost, c->stream));
       HIPCHK(c, hipStreamSynchronize(c->stream));
       for (int64_t i = 0; i < k->n; i++) gout[i] += h[i];
     }
@@ -3259,8 +3326,8 @@ extern "C" int fcfc_gpu_plan_create(fcfc_gpu_ctx *c, int njob, const fcfc_batch_
   }
   Sort so;
   if (int e = sort_alloc(c, P->al, stages, P->jobs, &so)) return e;
-  const int nres = res_hist(njob) + bins->ntot * njob;
-  P->res = (unsigned long long *) P->al.get(WS_RES, 8 * (size_t) nres);
+  const size_t nres = RES_HIST + (size_t) bins->ntot * njob + queue_words(njob);
+  P->res = (unsigned long long *) P->al.get(WS_RES, 8 * nres);
   if (P->al.err) return P->al.err;
   std::vector<std::vector<PJob>> groups = launch_groups(P->jobs);
   P->L.resize(groups.size());
@@ -3272,8 +3339,7 @@ extern "C" int fcfc_gpu_plan_create(fcfc_gpu_ctx *c, int njob, const fcfc_batch_
   put_tables(up, bins, &tabs);
   so.st = up.put(stages.data(), stages.size());
   for (size_t q = 0; q < groups.size(); q++)
-    if ((e = build_launch(c, P->al, up, tabs, bins, groups[q], mode, P->res, P->res + res_hist(njob),
-                          &P->L[q]))) return e;
+    if ((e = build_launch(c, P->al, up, tabs, bins, groups[q], mode, P->res, njob, &P->L[q]))) return e;
   if ((e = up.flush())) return e;
   if ((e = sort_run(c, P->al, so, P->res, nres))) return e;
   for (const Launch &Lq : P->L) if ((e = list_runs(c, P->al, Lq, P->res))) return e;
@@ -3372,7 +3438,7 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
     c->tile_frac = (nt <= 4096 * FK_NW) ? 1 : (nt > 16384 * FK_NW ? 16 : 8);
     e = run();
     if (e) return e;
-    const int ns = fk_split(nt, 1, 1, 1, c->tile_frac).ncap;     /* runs counted */
+    const int ns = fk_split(nt, 1, 1, 1, 1, c->tile_frac).ncap;     /* runs counted */
     *est = c->stats.kernel_ms * (double) nt / (double) std::max(1, ns);
     last_T = c->stats.tile;
     if (tune_log)
