@@ -480,14 +480,19 @@ __device__ __forceinline__ void fk_strip_segments(const FkGrid &g, const int *ce
 /* ---------------- FP64 pair evaluation (the arithmetic contract) -------- */
 
 /* Pair functions return an LDS histogram index sb + nsh * mb; every value
- * >= ntoh = nsh * rows means "not counted".  The row stride nsh is ns
- * rounded up to an odd number: lanes of one histogram atomic that share an
- * s bin but differ in mu (or pi) then fall on different LDS banks (an even
- * stride such as 40 folds them onto a few).  Table sentinels are FK_OUT =
- * 0xFFFF >= ntoh (the histogram lives in LDS, so ntoh < 40960), hence
- * sb + nsh * mb needs no range test of its own: an out-of-range s (or pi)
- * gives sb >= ntoh, a dropped mu gives mb = nmu and sb + nsh * nmu >= ntoh.
- * fk_hslot maps an LDS slot to the reference layout sb + ns * mb. */
+ * >= ntoh = nsh * rows means "not counted".  The row stride nsh is an odd
+ * number above ns: lanes of one histogram atomic that share an s bin but
+ * differ in mu (or pi) then fall on different LDS banks (an even stride such
+ * as 40 folds them onto a few).  Table sentinels are FK_OUT = 0xFFFF >= ntoh
+ * (the histogram lives in LDS, so ntoh < 40960), hence sb + nsh * mb needs no
+ * range test of its own: an out-of-range s (or pi) gives sb >= ntoh, a dropped
+ * mu gives mb = nmu and sb + nsh * nmu >= ntoh.
+ *
+ * The forms that mask the lanes out of range before the binning (`masked` in
+ * k_count) have neither sentinel nor test: their tables give values below the
+ * range the unused column ns (or, for pi, the dummy row after the last one),
+ * whose counts are never read.  fk_hslot maps an LDS slot to the reference
+ * layout sb + ns * mb, -1 for unused ones. */
 __device__ __forceinline__ int fk_hslot(int i, int ns, int nsh) {
   const int row = i / nsh, col = i - row * nsh;
   return col < ns ? col + ns * row : -1;
@@ -663,13 +668,14 @@ __device__ __forceinline__ unsigned fk_mu_plain(double num, double s2, const FkB
  * threshold then rides in the index too, which grows by mu_t16 << 16. */
 template <bool CAP, bool MUT, class FA>
 __device__ __forceinline__ unsigned fk_smu_index(double anmu, double r, FA fa, double s2,
-    unsigned sb, const FkBins &bn) {
+    unsigned sb, const FkBins &bn, bool *slow = nullptr) {
   double tm = __builtin_fma(anmu, r, bn.mu_c);
   if (CAP) tm = fk_min64(tm, bn.mu_cmax);
   const unsigned v = (unsigned) __builtin_bit_cast(unsigned long long, tm);
   unsigned idx = fk_mad_hi16(v, (unsigned) bn.nsh, sb);
   const bool exact = MUT ? !((v & 0xFFFFu) < (sb >> 16))
                          : (!((v & 0xFFFFu) < bn.mu_t16) || s2 < bn.s2_exact);
+  if (slow) *slow = exact;
   if (__builtin_expect(exact, 0))
     idx = (sb & 0xFFFFu) + __umul24((unsigned) bn.nsh, fk_mu_exact(fa(), s2, tm - FK_MU_C0, bn) + 1u)
           + (MUT ? bn.mu_t16 << 16 : 0u);
@@ -677,9 +683,9 @@ __device__ __forceinline__ unsigned fk_smu_index(double anmu, double r, FA fa, d
 }
 
 /* Box pair, B already at its periodic image (b' = fl(b + D)).  Returns the
- * histogram index, plus nsh (and mu_t16 << 16 with MUT) for (s, mu) bins
- * outside the plain form (fk_smu_index); >= ntot (+ that): not counted. */
-template <int BIN, bool HYB, bool MK = false, bool PLAIN = false, bool MUT = false>
+ * histogram index, plus nsh for (s, mu) bins outside the plain form
+ * (fk_smu_index); >= ntot (+ that): not counted. */
+template <int BIN, bool HYB, bool MK = false, bool PLAIN = false>
 __device__ __forceinline__ unsigned fk_box64(double dx, double dy, double dz,
     const FkBins &bn, const unsigned *stab, const unsigned *ptab,
     const double *s2e, const double *pe) {
@@ -688,25 +694,26 @@ __device__ __forceinline__ unsigned fk_box64(double dx, double dy, double dz,
     const double s2 = __builtin_fma(dy, dy, dx * dx);          /* :416-420 */
     const unsigned sb = fk_sbin<HYB, MK>(s2, bn, stab, s2e);
     const unsigned pb = fk_pbin<HYB, MK>(pi, bn, ptab, pe);
+    if (MK && (sb == (unsigned) bn.ns || pb == (unsigned) bn.np)) return FK_NONE;
     return sb + __umul24((unsigned) bn.nsh, pb);
   }
   const double dz2 = dz * dz;
   const double s2 = __builtin_fma(dy, dy, __builtin_fma(dx, dx, dz2));  /* :426-430 */
   const unsigned sb = fk_sbin<HYB, MK>(s2, bn, stab, s2e);
+  if (MK && sb == (unsigned) bn.ns) return FK_NONE;
   if (BIN == FCFC_BIN_ISO) return sb;
   if (PLAIN) return sb + __umul24((unsigned) bn.nsh, fk_mu_plain(dz2, s2, bn));
-  return fk_smu_index<false, MUT>(__builtin_fabs(dz) * bn.nmu_d, __builtin_amdgcn_rsq(s2),
+  return fk_smu_index<false, false>(__builtin_fabs(dz) * bn.nmu_d, __builtin_amdgcn_rsq(s2),
                       [&] { return dz2 * bn.nmu2; }, s2, sb, bn);
 }
 
 /* Survey pair (src/fcfc/2pt/metric_common.c:283-460, FMA vector formulas):
  * t = 2 a.b, s = |a|^2 + |b|^2, d = |a|^2 - |b|^2, pi^2 = d^2 / (t + s),
  * s^2 = s - t, s_perp^2 = (s - t) - pi^2.  (s, mu) bins need pi^2 only in
- * the exact branch of the mu bin: sqrt(pi^2) = |d| / sqrt(t + s).  MUT:
- * integer tables whose cells carry a threshold in their high half ((s, mu):
- * the mu fraction threshold; (s_perp, pi): fixed-point lookups, below);
- * os (op) is the s (pi) table's LDS byte address for those lookups. */
-template <int BIN, bool HYB, bool PLAIN = false, bool MK = false, bool MUT = false>
+ * the exact branch of the mu bin: sqrt(pi^2) = |d| / sqrt(t + s).  QT:
+ * (s_perp, pi) integer tables read in fixed point, below; os (op) is the s
+ * (pi) table's LDS byte address for those lookups. */
+template <int BIN, bool HYB, bool PLAIN = false, bool MK = false, bool QT = false>
 __device__ __forceinline__ unsigned fk_sv64(double ax, double ay, double az,
     double as, double bx, double by, double bz, double bs, const FkBins &bn,
     const unsigned *stab, const unsigned *ptab, const double *s2e, const double *pe,
@@ -714,7 +721,8 @@ __device__ __forceinline__ unsigned fk_sv64(double ax, double ay, double az,
   if (BIN == FCFC_BIN_ISO) {
     const double dx = ax - bx, dy = ay - by, dz = az - bz;
     const double s2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-    return fk_sbin<HYB, MK>(s2, bn, stab, s2e);
+    const unsigned sb = fk_sbin<HYB, MK>(s2, bn, stab, s2e);
+    return MK && sb == (unsigned) bn.ns ? FK_NONE : sb;
   }
   const double t = __builtin_fma(az, bz, __builtin_fma(ay, by, ax * bx)) * 2.0;
   const double s = as + bs;
@@ -722,14 +730,15 @@ __device__ __forceinline__ unsigned fk_sv64(double ax, double ay, double az,
   if (BIN == FCFC_BIN_SMU) {
     const double s2 = s - t;
     const unsigned sb = fk_sbin<HYB, MK>(s2, bn, stab, s2e);
+    if (MK && sb == (unsigned) bn.ns) return FK_NONE;
     if (PLAIN) return sb + __umul24((unsigned) bn.nsh, fk_mu_plain((d * d) / (t + s), s2, bn));
-    return fk_smu_index<true, MUT>(__builtin_fabs(d) * bn.nmu_d,
+    return fk_smu_index<true, false>(__builtin_fabs(d) * bn.nmu_d,
                         __builtin_amdgcn_rsq((t + s) * s2),
                         [&] { return ((d * d) / (t + s)) * bn.nmu2; }, s2, sb, bn);
   }
   /* (s_perp, pi): pbin holds pi^2 edges; with s2min == 0 the reference has
    * no lower bound on s_perp^2 (a rounding-negative value lands in bin 0) */
-  if (MUT) {
+  if (QT) {
     /* Integer tables in the FP64 forms: no division on the fast path.
      * With y = rcp(B) refined once (B = t + s, |y - 1/B| <= 2^-45.9 / B for
      * the documented 2^-23 of v_rcp_f64 and B >= q_bmin), q = n y is within
@@ -799,6 +808,7 @@ __device__ unsigned fk_box_variant(int var, const double a[3], const double bo[3
     const double s2 = scalar ? (d[0] * d[0] + d[1] * d[1]) : __builtin_fma(d[1], d[1], d[0] * d[0]);
     const unsigned sb = fk_sbin<HYB, true>(s2, bn, stab, s2e);
     const unsigned pb = fk_pbin<HYB, true>(pi, bn, ptab, pe);
+    if (sb == (unsigned) bn.ns || pb == (unsigned) bn.np) return FK_NONE;
     return sb + __umul24((unsigned) bn.nsh, pb);
   }
   const double dz2 = d[2] * d[2];
@@ -806,6 +816,7 @@ __device__ unsigned fk_box_variant(int var, const double a[3], const double bo[3
   if (scalar) { double t = d[0] * d[0]; t = t + d[1] * d[1]; s2 = t + dz2; }
   else s2 = __builtin_fma(d[1], d[1], __builtin_fma(d[0], d[0], dz2));
   const unsigned sb = fk_sbin<HYB, true>(s2, bn, stab, s2e);
+  if (sb == (unsigned) bn.ns) return FK_NONE;
   if (BIN == FCFC_BIN_ISO || sb == FK_OUT) return sb;
   int m = 0;
   if (s2 >= FK_DBL_EPS) {
@@ -824,11 +835,9 @@ __device__ unsigned fk_box_variant(int var, const double a[3], const double bo[3
 }
 
 /* ---------------- FP32 pair evaluation with exactness windows ----------- */
-/* Coordinates relative to the A tile centre in FP32.  Returns the histogram
- * index (>= ntot: not counted; (s, mu) bins: the index plus 0x4301 nsh, see
- * fk_mu32) and sets ambig when the pair lies within the
- * rounding bound of a bin edge that matters (it is then re-evaluated in
- * FP64 and the index is ignored).  Window test of s^2 (and pi): with
+/* Coordinates relative to the centre of the A run in FP32.  A pair within the
+ * rounding bound of a bin edge that matters is re-evaluated in FP64 and its
+ * index ignored.  Window test of s^2 (and pi): with
  * u = s2 + e, s2 is within e of an integer k exactly when fract(u) < 2e,
  * and then k = (int) u; otherwise (int) u = (int) s2.  So the table entry
  * at (int) u is the cell of s2 when s2 is clear of the integers, and the
@@ -840,8 +849,12 @@ __device__ unsigned fk_box_variant(int var, const double a[3], const double bo[3
  * FK_F_ALW.  Read as a float, the cell lies within 2^-7 relative of its
  * threshold, on the side away from zero (thresholds are normal numbers:
  * comparisons with subnormals are slow), so the test is one compare of the
- * cell itself: fract(u) < cell.  A pair whose s (or pi) is certainly out of
- * range reads a flagless sentinel. */
+ * cell itself: fract(u) < cell.  The zero-based FP32 tables run to (int)
+ * s2min + len + 1: the entry after the last cell flags the edge at s2max, the
+ * last one is a plain FK_OUT for pairs certainly out of range (survey
+ * (s_perp, pi), whose pairs are not masked). */
+
+
 /* FP32 mu bin floor(t) from x = anmu r (|x - t| < D above s2_floor, the
  * cells below s2_floor carry FK_F_ALW: every pair there is re-evaluated;
  * t <= nmu (1 + 2^-20) <= 126), in fixed point as in fk_mu_exact: the fma
@@ -858,40 +871,7 @@ __device__ __forceinline__ unsigned fk_mu32(float anmu, float r, unsigned sb,
   return fk_mad_hi16(v, (unsigned) bn.nsh, sb);
 }
 
-template <int BIN>
-__device__ __forceinline__ unsigned fk_box32(float dx, float dy, float dz,
-    const FkBins &bn, const FkWin &wn, const unsigned *stab,
-    const unsigned *ptab, bool &ambig, bool &ambig_mu) {
-  ambig_mu = false;
-  float s2;
-  if (BIN == FCFC_BIN_SPI) s2 = __builtin_fmaf(dy, dy, dx * dx);
-  else s2 = __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, dz * dz));
-  /* u >= 0: truncation is the floor.  The zero-based FP32 tables run to
-   * (int) s2min + len + 1: the entry after the last cell flags the edge at
-   * s2max, the last one is a plain FK_OUT for pairs certainly out of range
-   * (as are the entries below s2min) */
-  const float u = s2 + wn.e_s2;
-  const unsigned e = stab[min((int) u, bn.scap32)];
-  const bool amb = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
-  const unsigned sb = e & 0xFFFFu;
-  if (BIN == FCFC_BIN_ISO) { ambig = amb; return sb; }
-  if (BIN == FCFC_BIN_SPI) {
-    const float up = __builtin_fabsf(dz) + wn.e_pi;
-    const unsigned ep = ptab[min((int) up, bn.pcap32)];
-    const bool ambp = __builtin_amdgcn_fractf(up) < __uint_as_float(ep);
-    const unsigned pb = ep & 0xFFFFu;
-    const bool out = ((sb == FK_OUT) & !amb) | ((pb == FK_OUT) & !ambp);
-    ambig = (amb | ambp) & !out;
-    return sb + __umul24((unsigned) bn.nsh, pb);
-  }
-  /* mu bin = floor(t), t = nmu |dz| / s (fk_mu32).  A pair out of range in
-   * s whose t is near an integer is re-evaluated too (rare, and cheaper than
-   * testing sb here); idle lanes sit where t = 1/2. */
-  ambig = amb;                                 /* the caller ORs the two */
-  return fk_mu32(wn.nmu_f * __builtin_fabsf(dz), __builtin_amdgcn_rsqf(s2), sb, bn, wn, ambig_mu);
-}
-
-/* FP32 survey pair.  d = b - a from coordinates relative to the A tile
+/* FP32 survey pairs.  d = b - a from coordinates relative to the run's
  * centre (as for box pairs) and m = a + b = 2 a + d (m* = 2 a in FP32), so
  * that s^2 = |d|^2, pi = d.m / |m| and mu = pi / s carry the FP32 error of
  * differences, not the cancellation of |a|^2 + |b|^2 - 2 a.b that the
@@ -899,46 +879,27 @@ __device__ __forceinline__ unsigned fk_box32(float dx, float dy, float dz,
  * differ from the exact ones by its own rounding, which the windows include
  * (fp32_windows).  Pairs with |m|^2 below m2_floor (both objects near the
  * observer, on opposite sides) are always re-evaluated, as are pairs of
- * cells flagged for it (the three conditions come back apart, so that each
- * ballot is its compare's own mask).  (s_perp, pi): the tables hold pi^2 and s_perp^2 =
+ * cells flagged for it.  (s_perp, pi): the tables hold pi^2 and s_perp^2 =
  * s^2 - pi^2, whose FP32 value may come out slightly negative (index 0, as
  * the reference's truncation gives); lanes whose indices come out below -1
- * (pairs below m2_floor) read the "out" sentinel. */
-template <int BIN>
-__device__ __forceinline__ unsigned fk_sv32(float dx, float dy, float dz, float mx, float my,
+ * (pairs below m2_floor) read the "out" sentinel (the three conditions come
+ * back apart, so that each ballot is its compare's own mask). */
+__device__ __forceinline__ unsigned fk_sv32_spi(float dx, float dy, float dz, float mx, float my,
     float mz, const FkBins &bn, const FkWin &wn, const unsigned *stab, const unsigned *ptab,
-    bool &ambig, bool &ambig_mu, bool &ambig_m) {
-  ambig_mu = false;
-  ambig_m = false;
+    bool &ambig, bool &ambig_pi, bool &ambig_m) {
   const float s2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-  if (BIN == FCFC_BIN_ISO) {
-    const float u = s2 + wn.e_s2;
-    const unsigned e = stab[min((int) u, bn.scap32)];
-    ambig = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
-    return e & 0xFFFFu;
-  }
   const float p = __builtin_fmaf(dz, mz, __builtin_fmaf(dy, my, dx * mx));
   const float m2 = __builtin_fmaf(mz, mz, __builtin_fmaf(my, my, mx * mx));
   ambig_m = m2 < wn.m2_floor;          /* near the observer: re-evaluate */
-  if (BIN == FCFC_BIN_SPI) {
-    const float p2 = (p * p) * __builtin_amdgcn_rcpf(m2);
-    const float sp2 = s2 - p2;
-    const float u = sp2 + wn.e_s2;
-    const unsigned e = stab[min((unsigned) (int) u, (unsigned) bn.scap32)];
-    const bool amb = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
-    const float up = p2 + wn.e_pi;
-    const unsigned ep = ptab[min((unsigned) (int) up, (unsigned) bn.pcap32)];
-    const bool ambp = __builtin_amdgcn_fractf(up) < __uint_as_float(ep);
-    ambig = amb;
-    ambig_mu = ambp;
-    return (e & 0xFFFFu) + __umul24((unsigned) bn.nsh, ep & 0xFFFFu);
-  }
-  const float u = s2 + wn.e_s2;
-  const unsigned e = stab[min((int) u, bn.scap32)];
+  const float p2 = (p * p) * __builtin_amdgcn_rcpf(m2);
+  const float sp2 = s2 - p2;
+  const float u = sp2 + wn.e_s2;
+  const unsigned e = stab[min((unsigned) (int) u, (unsigned) bn.scap32)];
   ambig = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
-  return fk_mu32(wn.nmu_f * __builtin_fabsf(p),
-                 __builtin_amdgcn_rsqf(m2 * s2), e & 0xFFFFu, bn, wn,
-                 ambig_mu);
+  const float up = p2 + wn.e_pi;
+  const unsigned ep = ptab[min((unsigned) (int) up, (unsigned) bn.pcap32)];
+  ambig_pi = __builtin_amdgcn_fractf(up) < __uint_as_float(ep);
+  return (e & 0xFFFFu) + __umul24((unsigned) bn.nsh, ep & 0xFFFFu);
 }
 
 /* Exact FP64 re-evaluation of a pair flagged by the FP32 windows (rare: the
@@ -1058,6 +1019,14 @@ k_count(const FkArgs a) {
    * and s_perp^2 read in fixed point (fk_sv64); the tables start at floor
    * cell -2 and carry fraction thresholds (qt_entry below) */
   constexpr bool QT = (GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SPI && !F32 && !PLAIN && !HYB);
+  /* MASKED: the lanes out of range are masked off before the binning, so that
+   * neither the table index nor the histogram index needs a test of its own
+   * (the pair loop is bound by its VALU instructions: two of seventeen less.
+   * (s, mu) RR of 4e6 213 -> 208 ms, FP32 survey
+   * RR of 1.2e6 16.2 -> 15.5, DD of 5e5 7.0 -> 6.7).  FP64 with integer tables and
+   * FP32, except survey (s_perp, pi), whose s_perp^2 and pi^2 are found
+   * together. */
+  constexpr bool MASKED = !(GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SPI) && (F32 || (!HYB && !PLAIN));
   const unsigned ioff = (BIN != FCFC_BIN_SMU || PLAIN) ? 0u
                         : F32 ? 0x4301u * (unsigned) bn.nsh
                         : (unsigned) bn.nsh + (MUT ? bn.mu_t16 << 16 : 0u);
@@ -1094,10 +1063,10 @@ k_count(const FkArgs a) {
   double *box = s_box[wave];
 
   /* ---- stage tables ---- */
-  const int hist_elems = a.nh * bn.ntoh;
+  const int hist_elems = a.nh * bn.nslot;
   if (GRAD) {
-    for (int i = tid; i < bn.ntoh; i += FK_NT) {
-      const int g = fk_hslot(i, bn.ns, bn.nsh);
+    for (int i = tid; i < bn.nslot; i += FK_NT) {
+      const int g = i < bn.ntoh ? fk_hslot(i, bn.ns, bn.nsh) : -1;
       hist_d[i] = g >= 0 ? a.G[g] : 0.0;
     }
   }
@@ -1117,8 +1086,8 @@ k_count(const FkArgs a) {
      * well (refinement cells, v >= nb, always are). */
     auto entry = [&](const uint16_t *t, int len, int nb, int c, double off, double alw_below,
                      double lo_edge) -> unsigned {
-      const unsigned v = cell(t, len, c);
-      if (!F32) return v;
+      unsigned v = cell(t, len, c);
+      if (!F32) return MASKED && c < 0 ? (unsigned) nb : v;
       unsigned f = 0;
       if (cell(t, len, c - 1) != v) f |= FK_F_EDGE;
       /* the cell after one holding a non-integer lower edge: a value just
@@ -1128,6 +1097,10 @@ k_count(const FkArgs a) {
       if (v != FK_OUT && (v >= (unsigned) nb || (alw_below > 0 && off + c < alw_below + 1.0) ||
                           (HYB && c == 0 && off != lo_edge)))
         f |= FK_F_ALW | FK_F_EDGE;
+      /* masked lanes reach the first sentinel only within the window of the
+       * upper range edge */
+      if (MASKED && c == len) f |= FK_F_ALW | FK_F_EDGE;
+      if (MASKED && c < 0) v = (unsigned) nb;
       return v | f;
     };
     /* FP32 tables: bin and the high half of the threshold of fract(u),
@@ -1178,14 +1151,14 @@ k_count(const FkArgs a) {
   /* pairs this wavefront may have added to 32-bit counters since the
    * workgroup's last flush (FK_NW such budgets stay below 2^32) */
   unsigned since = 0;
-  unsigned int *myhist_u = hist_u + (wave % a.nh) * bn.ntoh;
-  double *myhist_d = hist_d + (wave % a.nh) * bn.ntoh;
+  unsigned int *myhist_u = hist_u + (wave % a.nh) * bn.nslot;
+  double *myhist_d = hist_d + (wave % a.nh) * bn.nslot;
   /* byte offsets in lds of these histograms, minus the pair functions'
    * index offset times the slot size: lds + (o + idx * size) is slot
    * idx - ioff (unsigned arithmetic, modulo 2^32; in range for every
    * counted index) */
-  const unsigned ohist_u = (unsigned) a.off_hist + 4u * ((unsigned) (wave % a.nh) * ntot - ioff);
-  const unsigned ohist_d = (unsigned) a.off_hist + 8u * ((unsigned) (wave % a.nh) * ntot - ioff);
+  const unsigned ohist_u = (unsigned) a.off_hist + 4u * ((unsigned) (wave % a.nh) * (unsigned) bn.nslot - ioff);
+  const unsigned ohist_d = (unsigned) a.off_hist + 8u * ((unsigned) (wave % a.nh) * (unsigned) bn.nslot - ioff);
   const unsigned ohist_g = (unsigned) a.off_hist - 8u * ioff;
   const int lane = tid & 63;
 
@@ -1198,7 +1171,7 @@ k_count(const FkArgs a) {
   auto spill_counts = [&]() {
     unsigned long long *g0 = a.gcnt_u + fk_cld(&fk_again(a.jobs, cur)->hist_off);
     for (int i = lane; i < hist_elems; i += 64) {
-      const int g = fk_hslot(i % bn.ntoh, bn.ns, bn.nsh);
+      const int slot = i % bn.nslot, g = slot < bn.ntoh ? fk_hslot(slot, bn.ns, bn.nsh) : -1;
       const unsigned v = atomicExch(hist_u + i, 0u);
       if (g >= 0 && v) atomicAdd(g0 + g, (unsigned long long) v);
     }
@@ -1226,16 +1199,16 @@ k_count(const FkArgs a) {
       const bool w = WT && fk_cld(&pj->wt);
       const long long ho = fk_cld(&pj->hist_off);
       for (int i = tid; i < bn.ntoh; i += FK_NT) {
-        const int g = fk_hslot(i, bn.ns, bn.nsh);    /* padding slots stay 0 */
+        const int g = fk_hslot(i, bn.ns, bn.nsh);    /* unused slots are left */
         if (g < 0) continue;
         if (w) {
           double v = 0;
-          for (int c = 0; c < a.nh; c++) { v += hist_d[c * bn.ntoh + i]; hist_d[c * bn.ntoh + i] = 0.0; }
+          for (int c = 0; c < a.nh; c++) { v += hist_d[c * bn.nslot + i]; hist_d[c * bn.nslot + i] = 0.0; }
           if (v != 0) unsafeAtomicAdd(a.gcnt_d + ho + g, v);
         }
         else {
           unsigned long long v = 0;
-          for (int c = 0; c < a.nh; c++) { v += hist_u[c * bn.ntoh + i]; hist_u[c * bn.ntoh + i] = 0u; }
+          for (int c = 0; c < a.nh; c++) { v += hist_u[c * bn.nslot + i]; hist_u[c * bn.nslot + i] = 0u; }
           if (v) atomicAdd(a.gcnt_u + ho + g, v);
         }
       }
@@ -1411,28 +1384,149 @@ k_count(const FkArgs a) {
     auto step = [&](auto selfc, double bx, double by, double bz, double bs, double wj, float gx,
                     float gy, float gz, int jj, int j, int code) __attribute__((always_inline)) {
       constexpr bool SELF = decltype(selfc)::value;
+      if (MASKED) {
+        double bsum = 0.0;        /* GRAD: sum of G[bin] w_a over this lane's pairs */
+        auto add = [&](unsigned idx, int r) __attribute__((always_inline)) {
+          if (GRAD) {
+            const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
+            gacc[r] = __builtin_fma(gk, wj, gacc[r]);
+            bsum = __builtin_fma(gk, aw[r], bsum);
+          }
+          else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
+          else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
+        };
+        if (F32) {
+          float ex[R], ey[R], ez[R], s2[R];
+          bool in[R], any = false;
+#pragma unroll
+          for (int r = 0; r < R; r++) {
+            ex[r] = gx - fax[r]; ey[r] = gy - fay[r]; ez[r] = gz - faz[r];
+            if (BIN == FCFC_BIN_SPI) s2[r] = __builtin_fmaf(ey[r], ey[r], ex[r] * ex[r]);
+            else if (SV32) s2[r] = __builtin_fmaf(ez[r], ez[r], __builtin_fmaf(ey[r], ey[r], ex[r] * ex[r]));
+            else s2[r] = __builtin_fmaf(ey[r], ey[r], __builtin_fmaf(ex[r], ex[r], ez[r] * ez[r]));
+            in[r] = s2[r] + wn.e_s2 < bn.m32s;
+            if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabsf(ez[r]) + wn.e_pi < bn.m32p);
+            if (SELF) in[r] = in[r] & (jj > ai[r]);
+            any |= in[r];
+          }
+          if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+#pragma unroll
+          for (int r = 0; r < R; r++) {
+            bool amb = false;
+            if (in[r]) {
+              const float u = s2[r] + wn.e_s2;
+              const unsigned e = stab_raw[(int) u];
+              amb = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
+              unsigned idx = e & 0xFFFFu;
+              if (BIN == FCFC_BIN_SPI) {
+                const float up = __builtin_fabsf(ez[r]) + wn.e_pi;
+                const unsigned ep = ptab_raw[(int) up];
+                amb |= __builtin_amdgcn_fractf(up) < __uint_as_float(ep);
+                idx += __umul24((unsigned) bn.nsh, ep & 0xFFFFu);
+              }
+              if (BIN == FCFC_BIN_SMU) {
+                bool ambm;
+                if (SV32) {
+                  const float mx = __builtin_fmaf(2.0f, fax[r], ex[r]) + c2x;
+                  const float my = __builtin_fmaf(2.0f, fay[r], ey[r]) + c2y;
+                  const float mz = __builtin_fmaf(2.0f, faz[r], ez[r]) + c2z;
+                  const float p = __builtin_fmaf(ez[r], mz, __builtin_fmaf(ey[r], my, ex[r] * mx));
+                  const float m2 = __builtin_fmaf(mz, mz, __builtin_fmaf(my, my, mx * mx));
+                  idx = fk_mu32(wn.nmu_f * __builtin_fabsf(p), __builtin_amdgcn_rsqf(m2 * s2[r]), idx,
+                                bn, wn, ambm);
+                  amb |= m2 < wn.m2_floor;         /* near the observer */
+                }
+                else
+                  idx = fk_mu32(wn.nmu_f * __builtin_fabsf(ez[r]), __builtin_amdgcn_rsqf(s2[r]), idx,
+                                bn, wn, ambm);
+                amb |= ambm;
+              }
+              if (!amb) add(idx, r);
+            }
+            /* pairs near an edge: queue (B object, A slot, image) for FP64 */
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(amb);
+            if (__builtin_expect(m != 0, 0)) {
+              if (amb) {
+                const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                           __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+                wqj[pos] = (unsigned) (SELF ? jj : cj[j]);
+                wqs[pos] = (uint16_t) (((unsigned) (r * 64 + lane) << 5) | (unsigned) code);
+              }
+              qn += __popcll(m);
+            }
+          }
+        }
+        else {
+          double s2[R], ez[R], dz2[R];
+          bool in[R], any = false;
+#pragma unroll
+          for (int r = 0; r < R; r++) {
+            if (GEOM == FCFC_GEOM_BOX) {
+              const double ex = bx - ax[r], ey = by - ay[r];
+              ez[r] = bz - az[r];
+              dz2[r] = ez[r] * ez[r];
+              if (BIN == FCFC_BIN_SPI) s2[r] = __builtin_fma(ey, ey, ex * ex);             /* :416-420 */
+              else s2[r] = __builtin_fma(ey, ey, __builtin_fma(ex, ex, dz2[r]));           /* :426-430 */
+            }
+            else if (BIN == FCFC_BIN_ISO) {
+              const double ex = ax[r] - bx, ey = ay[r] - by, e3 = az[r] - bz;
+              s2[r] = __builtin_fma(e3, e3, __builtin_fma(ey, ey, ex * ex));
+            }
+            else {
+              /* t (in dz2) and s^2 = s - t of the survey formulas (fk_sv64) */
+              dz2[r] = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
+              s2[r] = (as[r] + bs) - dz2[r];
+            }
+            in[r] = s2[r] < bn.s2max;
+            if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabs(ez[r]) < bn.pmax);
+            if (SELF) in[r] = in[r] & (jj > ai[r]);
+            any |= in[r];
+          }
+          if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+#pragma unroll
+          for (int r = 0; r < R; r++) {
+            if (!in[r]) continue;
+            const unsigned cell = stab[(int) s2[r]];
+            if (BIN == FCFC_BIN_ISO) add(cell, r);
+            else if (BIN == FCFC_BIN_SPI)
+              add(cell + __umul24((unsigned) bn.nsh, ptab[(int) __builtin_fabs(ez[r])]), r);
+            else {
+              bool slow;
+              unsigned idx;
+              if (GEOM == FCFC_GEOM_BOX)
+                idx = fk_smu_index<false, MUT>(__builtin_fabs(ez[r]) * bn.nmu_d, __builtin_amdgcn_rsq(s2[r]),
+                                               [&] { return dz2[r] * bn.nmu2; }, s2[r], cell, bn, &slow);
+              else {
+                const double d = as[r] - bs, m2 = dz2[r] + (as[r] + bs);
+                idx = fk_smu_index<true, MUT>(__builtin_fabs(d) * bn.nmu_d, __builtin_amdgcn_rsq(m2 * s2[r]),
+                                              [&] { return ((d * d) / m2) * bn.nmu2; }, s2[r], cell, bn, &slow);
+              }
+              /* a mu that the exact path drops; the fast path has none (a
+               * survey value at its cap falls on the dummy row) */
+              if (!slow || idx < ntot_o) add(idx, r);
+            }
+          }
+        }
+        if (GRAD && hasB) {
+          /* the B object's share over the wavefront's pairs: one sum per
+           * row of 16 lanes, added into the chunk's LDS accumulator */
+          const double v = fk_row_sum(bsum);
+          if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
+        }
+        return;
+      }
       if (GEOM == FCFC_GEOM_BOX) {
         /* when this B object is out of range of every A object of the run,
          * skip the binning (same expressions as the pair functions, so the
-         * compiler shares them).  Every form skips, so the plain form
-         * differs from the FP64 one in the per-pair mu arithmetic only */
+         * compiler shares them) */
         bool any = false;
 #pragma unroll
         for (int r = 0; r < R; r++) {
-          if (F32) {
-            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-            if (BIN == FCFC_BIN_SPI)
-              any |= (__builtin_fmaf(ey, ey, ex * ex) < bn.s2skip32) &
-                     (__builtin_fabsf(ez) < bn.pskip32);
-            else any |= __builtin_fmaf(ey, ey, __builtin_fmaf(ex, ex, ez * ez)) < bn.s2skip32;
-          }
-          else {
-            const double ex = bx - ax[r], ey = by - ay[r], ez = bz - az[r];
-            if (BIN == FCFC_BIN_SPI)
-              any |= (__builtin_fma(ey, ey, ex * ex) < bn.s2skip) &
-                     (__builtin_fabs(ez) < bn.pskip);
-            else any |= __builtin_fma(ey, ey, __builtin_fma(ex, ex, ez * ez)) < bn.s2skip;
-          }
+          const double ex = bx - ax[r], ey = by - ay[r], ez = bz - az[r];
+          if (BIN == FCFC_BIN_SPI)
+            any |= (__builtin_fma(ey, ey, ex * ex) < bn.s2skip) &
+                   (__builtin_fabs(ez) < bn.pskip);
+          else any |= __builtin_fma(ey, ey, __builtin_fma(ex, ex, ez * ez)) < bn.s2skip;
         }
         if (__builtin_amdgcn_ballot_w64(any) == 0) return;
       }
@@ -1463,18 +1557,12 @@ k_count(const FkArgs a) {
         unsigned idx;
         bool queued = false;      /* FP32: left to the FP64 re-evaluation */
         if (F32) {
-          bool amb, ambm;
-          bool ambx = false;
-          if (SV32) {
-            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-            idx = fk_sv32<BIN>(ex, ey, ez, __builtin_fmaf(2.0f, fax[r], ex) + c2x,
-                               __builtin_fmaf(2.0f, fay[r], ey) + c2y,
-                               __builtin_fmaf(2.0f, faz[r], ez) + c2z, bn, wn, stab_raw,
-                               ptab_raw, amb, ambm, ambx);
-          }
-          else
-            idx = fk_box32<BIN>(gx - fax[r], gy - fay[r], gz - faz[r], bn, wn, stab_raw,
-                                ptab_raw, amb, ambm);
+          bool amb, ambm, ambx;
+          const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
+          idx = fk_sv32_spi(ex, ey, ez, __builtin_fmaf(2.0f, fax[r], ex) + c2x,
+                            __builtin_fmaf(2.0f, fay[r], ey) + c2y,
+                            __builtin_fmaf(2.0f, faz[r], ez) + c2z, bn, wn, stab_raw,
+                            ptab_raw, amb, ambm, ambx);
           if (SELF) {
             const bool keep = jj > ai[r];
             amb = amb & keep; ambm = ambm & keep; idx = keep ? idx : FK_NONE;
@@ -1499,12 +1587,11 @@ k_count(const FkArgs a) {
           queued = amb | ambm | ambx;
         }
         else if (GEOM == FCFC_GEOM_BOX)
-          idx = fk_box64<BIN, HYB, false, PLAIN, MUT>(bx - ax[r], by - ay[r], bz - az[r], bn,
-                                                       stab, ptab, s2e, pe);
+          idx = fk_box64<BIN, HYB, false, PLAIN>(bx - ax[r], by - ay[r], bz - az[r], bn, stab,
+                                                 ptab, s2e, pe);
         else
-          idx = fk_sv64<BIN, HYB, PLAIN, false, MUT || QT>(ax[r], ay[r], az[r], as[r], bx, by,
-                                                           bz, bs, bn, stab, ptab, s2e, pe,
-                                                           os_lds, op_lds);
+          idx = fk_sv64<BIN, HYB, PLAIN, false, QT>(ax[r], ay[r], az[r], as[r], bx, by, bz, bs,
+                                                   bn, stab, ptab, s2e, pe, os_lds, op_lds);
         if (!F32 && SELF && !(jj > ai[r])) idx = FK_NONE;
         if (idx < ntot_o && !queued) {
           if (GRAD) {
@@ -2369,13 +2456,27 @@ static int sort_run(fcfc_gpu_ctx *c, Alloc &al, const Sort &so, unsigned long lo
   return 0;
 }
 
-/* LDS histogram geometry: row stride ns rounded up to an odd number (rows
- * of mu or pi bins), see fk_hslot */
-static int hist_stride(const fcfc_bins *b) {
-  return b->bintype == FCFC_BIN_ISO ? b->ns : (b->ns | 1);
+/* the kernels with a masked pair loop (see k_count) */
+static bool masked_form(const fcfc_bins *b, int mode, int hyb) {
+  if (b->geometry == FCFC_GEOM_SURVEY && b->bintype == FCFC_BIN_SPI) return false;
+  return mode == MODE_C32 || (!hyb && mode != MODE_P64);
 }
-static int hist_slots(const fcfc_bins *b) {
-  return hist_stride(b) * (b->ntot / b->ns);
+
+/* LDS histogram geometry: an odd row stride (rows of mu or pi bins), see
+ * fk_hslot.  Masked forms whose tables have entries below the s range need a
+ * column beyond ns for them, and a dummy row for pi below the range and for
+ * survey mu values at their ceiling. */
+struct HistDim { int nsh, ntoh, nslot; };
+static HistDim hist_dim(const fcfc_bins *b, int mode, int hyb) {
+  HistDim h;
+  const bool msk = masked_form(b, mode, hyb);
+  if (msk && b->soff > 0) h.nsh = (b->ns + 1) | 1;
+  else h.nsh = b->bintype == FCFC_BIN_ISO ? b->ns : (b->ns | 1);
+  h.ntoh = h.nsh * (b->ntot / b->ns);
+  const bool dummy = (b->bintype == FCFC_BIN_SPI && b->poff > 0) ||
+      (b->bintype == FCFC_BIN_SMU && b->geometry == FCFC_GEOM_SURVEY);
+  h.nslot = h.ntoh + (msk && dummy ? h.nsh : 0);
+  return h;
 }
 
 struct LdsPlan { int off_hist, off_stab, off_ptab, off_edges, off_chunk, off_queue, total, nh, stab_c0, ptab_c0; };
@@ -2400,8 +2501,9 @@ static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh
   int o = 0;
   L.nh = nh;
   L.off_hist = o;
-  if (mode == MODE_GRAD) o += hist_slots(b) * 8;
-  else o += nh * hist_slots(b) * (wt ? 8 : 4);
+  const int nslot = hist_dim(b, mode, hyb).nslot;
+  if (mode == MODE_GRAD) o += nslot * 8;
+  else o += nh * nslot * (wt ? 8 : 4);
   o = align16(o);
   L.off_edges = o;
   if (hyb) o = align16(o + 8 * (b->ns + 1 + (b->bintype == FCFC_BIN_SPI ? b->np + 1 : 0)));
@@ -2734,7 +2836,11 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   int anywt = 0;
   for (auto &j : jobs) anywt |= j.wt;
   if (m == MODE_GRAD) anywt = 1;
-  const int lds_max = 160 * 1024 - 2048;       /* room for the static LDS */
+  /* room for the static LDS (416 bytes); the unused slots of the masked forms
+   * come out of the margin */
+  auto fits = [&](const LdsPlan &P, int mode_, int hyb_) {
+    return P.total <= 160 * 1024 - (masked_form(b, mode_, hyb_) ? 512 : 2048);
+  };
   /* the FP32 window test reads one table cell and the edge at its lower end:
    * windows must stay well inside a cell (wide only for a few objects in a
    * huge volume, whose grid cells, and so tiles, are large) */
@@ -2750,11 +2856,11 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   /* tables too long for LDS (hybrid binnings rescaled to large integers):
    * hybrid lookups that binary-search the edges, in the FP64 forms */
   int ssearch = 0, psearch = 0;
-  if (lds_plan(b, m, anywt, need_s, 1, hyb).total > lds_max) {
+  if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb), m, hyb)) {
     if (m == MODE_C32) m = MODE_C64;
     hyb = 1;
     ssearch = 1;
-    if (lds_plan(b, m, anywt, need_s, 1, hyb, 1, 0).total > lds_max) psearch = 1;
+    if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 1, 0), m, hyb)) psearch = 1;
   }
   /* one kernel serves every job of the launch: tiles of the longest kind.
    * A lane holds R objects (1, 2 or 4), so no tile may exceed R FK_NT
@@ -2783,8 +2889,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   kfn_t fn = pick_kernel(b->bintype, geom, anywt, km, hyb, R);
   /* histogram copies: as many as keep the occupancy of a single copy */
   LdsPlan L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch);
-  if (L.total > lds_max) {
-    set_err(c, "binning tables need %d bytes of LDS (limit %d)", L.total, lds_max);
+  if (!fits(L, m, hyb)) {
+    set_err(c, "binning tables need %d bytes of LDS (limit %d)", L.total, 160 * 1024 - 2048);
     return FCFC_ERR_CFG;
   }
   /* (the choice depends on the kernel and the LDS size of one copy alone, and
@@ -2806,7 +2912,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
       for (int nh = 2; nh <= nhmax; nh *= 2) {
         LdsPlan L2 = lds_plan(b, m, anywt, need_s, nh, hyb, ssearch, psearch);
         int o2 = 0;
-        if (L2.total > lds_max) break;
+        if (!fits(L2, m, hyb)) break;
         if (int e = occ_of(fn, L2, &o2)) return e;
         if (o2 < occ1 && c->t_nh <= 0) break;
         L = L2;
@@ -2908,7 +3014,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   FkBins &fb = a.bins;
   fb.bintype = b->bintype; fb.geometry = geom;
   fb.ns = b->ns; fb.nmu = b->nmu; fb.np = b->np; fb.ntot = b->ntot;
-  fb.nsh = hist_stride(b); fb.ntoh = hist_slots(b);
+  const HistDim hd = hist_dim(b, m, hyb);
+  fb.nsh = hd.nsh; fb.ntoh = hd.ntoh; fb.nslot = hd.nslot;
   fb.scap32 = b->soff + b->stab_len + 1; fb.pcap32 = b->poff + b->ptab_len + 1;
   fb.tabtype = b->tabtype; fb.soff = b->soff; fb.poff = b->poff;
   /* searched tables are not staged to LDS (length 0: sentinels only) */
@@ -2927,10 +3034,13 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
       ? (fb.s2max + fb.pmax) * (1 + ldexp(1.0, -30)) + 1e-6 * (fb.s2max + fb.pmax + 1)
       : fb.s2max * (1 + ldexp(1.0, -30));
   fb.pskip = (b->bintype == FCFC_BIN_SPI) ? fb.pmax * (1 + ldexp(1.0, -30)) : 1e300;
-  fb.s2skip32 = (float) (fb.s2max + (geom == FCFC_GEOM_SURVEY ? fb.pmax : 0.0) + 2.0);
+  fb.s2skip32 = (float) (fb.s2max + fb.pmax + 2.0);
+  /* the upper end of the window of s2max (pmax): FP32 values at or beyond it
+   * are out of range */
+  fb.m32s = nextafterf((float) (fb.s2max + win2s), INFINITY);
+  fb.m32p = nextafterf((float) (fb.pmax + win2p), INFINITY);
   fb.win2s = win2s;
   fb.win2p = win2p;
-  fb.pskip32 = (b->bintype == FCFC_BIN_SPI) ? (float) (fb.pmax + 2.0) : 3.0e38f;
   {
     /* fixed-point mu (fk_mu_exact): sh >= nmu 2^-20 + 2^-16 on the grid
      * 2^-16, the addend 2^36 + 1 - sh exact */
@@ -2942,7 +3052,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
      * indices (fk_smu_index): keep the largest, (nmu + 1) nsh + 0xFFFF +
      * (mu_t16 << 16), below 2^32 (a lower threshold only sends more pairs
      * to the exact path) */
-    const unsigned long long room = (0xFFFF0000ull - (unsigned long long) (b->nmu + 1) * fb.nsh) >> 16;
+    const unsigned long long room = (0xFFFF0000ull - (unsigned long long) (b->nmu + 2) * fb.nsh) >> 16;
     fb.mu_t16 = (unsigned) std::min<unsigned long long>(fb.mu_t16, room);
     fb.mu_pad = 0;
   }

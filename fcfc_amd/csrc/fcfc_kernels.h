@@ -47,7 +47,8 @@
 struct FkBins {
   int bintype, geometry;
   int ns, nmu, np, ntot;
-  int nsh, ntoh;             /* LDS histogram row stride (odd) and slots    */
+  int nsh, ntoh;             /* LDS histogram row stride (odd, > ns), slots */
+  int nslot, slot_pad;       /* slots of one copy, with the dummy row       */
   int tabtype;               /* 0 integer table, 1 hybrid table             */
   int soff, poff;            /* (int) s2min, (int) pmin (or pi^2 min)       */
   int stab_len, ptab_len;    /* table lengths without sentinels             */
@@ -67,8 +68,9 @@ struct FkBins {
   double q_caps, q_capp;     /* pi^2 and s_perp^2 in fixed point (fk_sv64): */
   double q_bmin;             /* addend, ceilings, least |a+b|^2 of the fast */
   unsigned q_t16, q_pad;     /* path, fraction threshold of edge cells      */
-  double s2skip, pskip;      /* box: a pair at s^2 >= s2skip or pi >= pskip  */
-  float s2skip32, pskip32;   /* is out of range (FP64 / FP32 values)         */
+  double s2skip, pskip;      /* forms without a mask: a pair at s^2 >= s2skip */
+  float s2skip32, skip_pad;  /* or pi >= pskip is out of range (FP64 / FP32) */
+  float m32s, m32p;          /* FP32: values at or beyond are out of range   */
   float win2s, win2p;        /* FP32 tables: window 2 e of the edge cells,   */
                              /* the largest over the jobs of a launch        */
   const uint16_t *stab;      /* device tables (global), staged to LDS       */
