@@ -958,8 +958,10 @@ __device__ __forceinline__ unsigned fk_recheck_sv(const FkBins &bn, const FkJob 
 /* LDS bytes of one staged B object: FP32 coordinates relative to the run's
  * centre, weight and sorted index; the gradient form keeps the gradient share
  * and the sorted index of each B object, the FP64 counts nothing */
-__host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool wt, bool grad) {
-  return f32 ? 12 + (wt ? 8 : 0) + 4 : (grad ? 8 : 0);
+/* (wsep: the weights are not in the records; G > 1: groups of lanes, k_count) */
+__host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool wt, bool grad, bool wsep, int G) {
+  return f32 ? 12 + (wt ? 8 : 0) + 4
+             : (grad ? 8 : 0) + (G > 1 ? 36 + (wsep && (wt || grad) ? 8 : 0) : 0);
 }
 
 /* One persistent kernel for counts (FP64 or FP32 + recheck) and for the
@@ -990,8 +992,14 @@ __host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool wt, bool grad) {
  * ms, DR of 2e5 x 2e6 20.9 -> 16.6, the hybrid w_p count 3.5 -> 3.0; the
  * unweighted RR, bound by the VALU, is unchanged (232).  The FP32 forms keep
  * the chunk: their coordinates are converted once for 64 R pairs there, and
- * its 4-byte reads cost the LDS half as much. */
-template <int BIN, int GEOM, bool WT, int MODE, bool HYB, int R>
+ * its 4-byte reads cost the LDS half as much.
+ *
+ * NG > 1: NG groups of 64 / NG lanes hold the same run of 64 / NG A objects
+ * and take every NG-th kept B object each, from the chunk.  In a sparse
+ * catalogue 64 objects spread over more than the separations counted, and most
+ * pairs of a run are out of range: 16 objects have a quarter of the volume
+ * (iso cross count of 3e5 x 1e6: 1.10 -> 0.56 ms, w_p of 1e6 2.5 -> 1.7). */
+template <int BIN, int GEOM, bool WT, int MODE, bool HYB, int R, int NG = 1>
 __global__ void __launch_bounds__(FK_NT, WT ? 6 : 8)
 k_count(const FkArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -1022,11 +1030,11 @@ k_count(const FkArgs a) {
   /* MASKED: the lanes out of range are masked off before the binning, so that
    * neither the table index nor the histogram index needs a test of its own
    * (the pair loop is bound by its VALU instructions: two of seventeen less.
-   * (s, mu) RR of 4e6 213 -> 208 ms, FP32 survey
-   * RR of 1.2e6 16.2 -> 15.5, DD of 5e5 7.0 -> 6.7).  FP64 with integer tables and
-   * FP32, except survey (s_perp, pi), whose s_perp^2 and pi^2 are found
-   * together. */
-  constexpr bool MASKED = !(GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SPI) && (F32 || (!HYB && !PLAIN));
+   * (s, mu) RR of 4e6 213 -> 208 ms, FP32 survey RR of 1.2e6 16.2 -> 15.5,
+   * weighted DD of 5e5 7.0 -> 6.7).  FP64 with integer tables and FP32, except
+   * survey (s_perp, pi), whose s_perp^2 and pi^2 are found together. */
+  constexpr bool MASKED = !(GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SPI) &&
+                          (F32 || (!HYB && !PLAIN));
   const unsigned ioff = (BIN != FCFC_BIN_SMU || PLAIN) ? 0u
                         : F32 ? 0x4301u * (unsigned) bn.nsh
                         : (unsigned) bn.nsh + (MUT ? bn.mu_t16 << 16 : 0u);
@@ -1048,12 +1056,15 @@ k_count(const FkArgs a) {
   double *s2e = (double *) (lds + a.off_edges);
   double *pe = s2e + (bn.ns + 1);
   /* the wavefront's chunk of B objects */
-  char *cp = lds + a.off_chunk + wave * (FK_CH * fk_chunk_bytes(F32, WT, GRAD));
-  double *cw = (double *) cp;                  /* FP32: weights */
+  char *cp = lds + a.off_chunk + wave * (FK_CH * fk_chunk_bytes(F32, WT, GRAD, WSEP, NG));
+  FkRec *cr = (FkRec *) cp;                    /* FP64, NG > 1: records at the image of B */
+  if (!F32 && NG > 1) cp += sizeof(FkRec) * FK_CH;
   double *cb = (double *) cp;                  /* GRAD: gradient share of each B object */
-  if (F32 && WT) cp += 8 * FK_CH;
+  if (GRAD) cp += 8 * FK_CH;
+  double *cw = (double *) cp;                  /* weights: FP32, and FP64 with NG > 1 */
+  if (F32 ? WT : NG > 1 && WSEP && (WT || GRAD)) cp += 8 * FK_CH;
   float *fx = (float *) cp, *fy = fx + FK_CH, *fz = fy + FK_CH;
-  int *cj = (int *) (fz + FK_CH);              /* sorted index */
+  int *cj = F32 ? (int *) (fz + FK_CH) : (int *) cp;   /* sorted index */
   /* FP32 re-evaluation queue of this wavefront: sorted index of the B
    * object, A slot in the run << 5 | periodic image code */
   unsigned *wqj = (unsigned *) (lds + a.off_queue + wave * (FK_QCAP * 6));
@@ -1161,6 +1172,9 @@ k_count(const FkArgs a) {
   const unsigned ohist_d = (unsigned) a.off_hist + 8u * ((unsigned) (wave % a.nh) * (unsigned) bn.nslot - ioff);
   const unsigned ohist_g = (unsigned) a.off_hist - 8u * ioff;
   const int lane = tid & 63;
+  /* NG groups of NA lanes hold the same A objects, each for its own B objects */
+  constexpr int NA = 64 / NG;
+  const int slot = lane & (NA - 1), sub = NG > 1 ? lane / NA : 0;
 
   /* 32-bit counters: a wavefront that may have added FK_BUDGET pairs since
    * it last did so adds the workgroup's counters to the job's global histogram
@@ -1171,7 +1185,7 @@ k_count(const FkArgs a) {
   auto spill_counts = [&]() {
     unsigned long long *g0 = a.gcnt_u + fk_cld(&fk_again(a.jobs, cur)->hist_off);
     for (int i = lane; i < hist_elems; i += 64) {
-      const int slot = i % bn.nslot, g = slot < bn.ntoh ? fk_hslot(slot, bn.ns, bn.nsh) : -1;
+      const int k = i % bn.nslot, g = k < bn.ntoh ? fk_hslot(k, bn.ns, bn.nsh) : -1;
       const unsigned v = atomicExch(hist_u + i, 0u);
       if (g >= 0 && v) atomicAdd(g0 + g, (unsigned long long) v);
     }
@@ -1249,262 +1263,358 @@ k_count(const FkArgs a) {
     cur = __builtin_amdgcn_readfirstlane(s_job);
     if (cur < 0) break;
 
-  /* The job's items: item i belongs to group i % G.  The first one of each
-   * wavefront that starts with the job follows from its place among the
-   * group's wavefronts, the others from the group's counter; when the group
-   * has none left, another one's (every wavefront ends when no group has any). */
-  int grp = first ? ((int) blockIdx.x - fk_cld(&fk_again(a.jobs, cur)->wg0)) % fk_cld(&fk_again(a.jobs, cur)->G)
-                  : (int) blockIdx.x % fk_cld(&fk_again(a.jobs, cur)->G);
-  for (;;) {
-    const FkSplit sp = fk_cld(a.splits + cur);
-    const FkJob *pq = fk_again(a.jobs, cur);
-    const int wg0 = fk_cld(&pq->wg0), nwg = fk_cld(&pq->wg1) - wg0, G = fk_cld(&pq->G), q0 = fk_cld(&pq->q0);
-    int it = ((int) blockIdx.x - wg0) / G * FK_NW + wave;
-    if (!first) {
-      if (lane == 0)
-        it = group_waves(nwg, G, grp) + (int) atomicAdd(a.queue + (size_t) (q0 + grp) * (FK_LINE / 4), 1u);
-      it = __builtin_amdgcn_readfirstlane(it);
-    }
-    first = false;
-    it = grp + G * it;
-    if (it >= sp.nitems) {
-      bool has = false;
-      if (lane < G) has = lane + (long long) G * (group_waves(nwg, G, lane) + (int) queue_load(q0 + lane)) < sp.nitems;
-      const unsigned long long m = __builtin_amdgcn_ballot_w64(has), mn = m >> grp >> 1;
-      if (m == 0) break;
-      grp = mn ? grp + 1 + (int) __builtin_ctzll(mn) : (int) __builtin_ctzll(m);
-      continue;
-    }
-    /* work item -> run, share of its strips, chunks of their segments */
-    int part, S, SQ, ri;
-    const int h = sp.S * sp.tt;
-    if (it < h) { S = sp.S; SQ = sp.SQ; ri = it / S; part = it - ri * S; }
-    else { S = sp.St; SQ = sp.StQ; ri = (it - h) / S; part = it - h - ri * S; ri += sp.tt; }
-    const int sq = part % SQ;
-    S /= SQ;
-    part /= SQ;
-    const int smp = ri / sp.run;
-    const FkRun t = fk_cld(a.runs + __builtin_amdgcn_readfirstlane(
-        sp.run0 + smp * sp.G + (ri - smp * sp.run)));
+    /* The job's items: item i belongs to group i % G.  The first one of each
+     * wavefront that starts with the job follows from its place among the
+     * group's wavefronts, the others from the group's counter; when the group
+     * has none left, another one's (every wavefront ends when no group has any). */
+    int grp = first ? ((int) blockIdx.x - fk_cld(&fk_again(a.jobs, cur)->wg0)) % fk_cld(&fk_again(a.jobs, cur)->G)
+                    : (int) blockIdx.x % fk_cld(&fk_again(a.jobs, cur)->G);
+    for (;;) {
+      const FkSplit sp = fk_cld(a.splits + cur);
+      const FkJob *pq = fk_again(a.jobs, cur);
+      const int wg0 = fk_cld(&pq->wg0), nwg = fk_cld(&pq->wg1) - wg0, G = fk_cld(&pq->G), q0 = fk_cld(&pq->q0);
+      int it = ((int) blockIdx.x - wg0) / G * FK_NW + wave;
+      if (!first) {
+        if (lane == 0)
+          it = group_waves(nwg, G, grp) + (int) atomicAdd(a.queue + (size_t) (q0 + grp) * (FK_LINE / 4), 1u);
+        it = __builtin_amdgcn_readfirstlane(it);
+      }
+      first = false;
+      it = grp + G * it;
+      if (it >= sp.nitems) {
+        bool has = false;
+        if (lane < G) has = lane + (long long) G * (group_waves(nwg, G, lane) + (int) queue_load(q0 + lane)) < sp.nitems;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(has), mn = m >> grp >> 1;
+        if (m == 0) break;
+        grp = mn ? grp + 1 + (int) __builtin_ctzll(mn) : (int) __builtin_ctzll(m);
+        continue;
+      }
+      /* work item -> run, share of its strips, chunks of their segments */
+      int part, S, SQ, ri;
+      const int h = sp.S * sp.tt;
+      if (it < h) { S = sp.S; SQ = sp.SQ; ri = it / S; part = it - ri * S; }
+      else { S = sp.St; SQ = sp.StQ; ri = (it - h) / S; part = it - h - ri * S; ri += sp.tt; }
+      const int sq = part % SQ;
+      S /= SQ;
+      part /= SQ;
+      const int smp = ri / sp.run;
+      const FkRun t = fk_cld(a.runs + __builtin_amdgcn_readfirstlane(
+          sp.run0 + smp * sp.G + (ri - smp * sp.run)));
 
-    const FkJob J = fk_cld(a.jobs + cur);
-    const int s0 = (int) ((long long) J.nstrips * part / S);
-    const int s1 = (int) ((long long) J.nstrips * (part + 1) / S);
-    /* weights exist for this job (a weighted-capable kernel may run
-     * unweighted jobs of a batch, whose catalogues carry no weights) */
-    const bool jw = GRAD || (WT && J.wt);
-    const bool jwt = WT && J.wt;
-    const bool hasB = GRAD && J.gB != nullptr;
+      const FkJob J = fk_cld(a.jobs + cur);
+      const int s0 = (int) ((long long) J.nstrips * part / S);
+      const int s1 = (int) ((long long) J.nstrips * (part + 1) / S);
+      /* weights exist for this job (a weighted-capable kernel may run
+       * unweighted jobs of a batch, whose catalogues carry no weights) */
+      const bool jw = GRAD || (WT && J.wt);
+      const bool jwt = WT && J.wt;
+      const bool hasB = GRAD && J.gB != nullptr;
 
-    /* A objects of this lane (a wavefront holds one run) and the bounding box
-     * of the run; idle lanes sit far away, so that every pair they form is
-     * out of range */
-    double ax[R], ay[R], az[R], as[R], aw[R], gacc[R];
-    float fax[R], fay[R], faz[R];
-    int ai[R];
-    double lox = 1e300, loy = 1e300, loz = 1e300, hix = -1e300, hiy = -1e300, hiz = -1e300;
-    unsigned long long actm[R];
+      /* A objects of this lane (a wavefront holds one run) and the bounding box
+       * of the run; idle lanes sit far away, so that every pair they form is
+       * out of range */
+      double ax[R], ay[R], az[R], as[R], aw[R], gacc[R];
+      float fax[R], fay[R], faz[R];
+      int ai[R];
+      double lox = 1e300, loy = 1e300, loz = 1e300, hix = -1e300, hiy = -1e300, hiz = -1e300;
+      unsigned long long actm[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int p = t.p0 + r * 64 + lane;
-      const bool v = p < t.p1;
-      const int pc = v ? p : t.p0;
-      const FkRec ra = fk_gld(J.A.rec, pc);
-      const double x = ra.x, y = ra.y, z = ra.z;
-      lox = __builtin_fmin(lox, x); hix = __builtin_fmax(hix, x);
-      loy = __builtin_fmin(loy, y); hiy = __builtin_fmax(hiy, y);
-      loz = __builtin_fmin(loz, z); hiz = __builtin_fmax(hiz, z);
-      ai[r] = v ? p : 0x7fffffff;
-      ax[r] = v ? x : FK_FAR;
-      ay[r] = v ? y : FK_FAR;
-      az[r] = v ? z : FK_FAR;
-      as[r] = NEED_S ? (v ? ra.q : 3.0 * FK_FAR * FK_FAR) : 0.0;
-      aw[r] = (jw && v) ? (WSEP ? fk_gld(J.A.w, pc) : ra.q) : 1.0;
-      gacc[r] = 0.0;
-      actm[r] = __builtin_amdgcn_ballot_w64(v);
-    }
-    lox = fk_wave_min(lox); hix = -fk_wave_min(-hix);
-    loy = fk_wave_min(loy); hiy = -fk_wave_min(-hiy);
-    loz = fk_wave_min(loz); hiz = -fk_wave_min(-hiz);
-    fk_wave_sync();
-    if (lane == 0) { box[0] = lox; box[1] = hix; box[2] = loy; box[3] = hiy; box[4] = loz; box[5] = hiz; }
-    fk_wave_sync();
-    /* FP32 coordinates are relative to the centre of the box */
-    const double tcx = 0.5 * (lox + hix), tcy = 0.5 * (loy + hiy), tcz = 0.5 * (loz + hiz);
-    /* idle lanes: |a| = 1e18 and |dz| / s = 1 / (2 nmu), so that the mu
-     * estimate of their pairs is 1/2, clear of the windows */
-    const FkWin wn = J.win;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const bool v = ai[r] != 0x7fffffff;
-      fax[r] = v ? (float) (ax[r] - tcx) : wn.idle_x;
-      fay[r] = v ? (float) (ay[r] - tcy) : 0.0f;
-      faz[r] = v ? (float) (az[r] - tcz) : wn.idle_z;
-    }
-    /* survey FP32: m = a + b = 2 a' + d + 2 c (a' = a - c, c = the centre).
-     * Idle lanes (a' = (10^6, 0, 0): s^2 and pi^2 far out of range) may
-     * look ambiguous in mu: their queue bits are masked off */
-    const float c2x = (float) (2.0 * tcx), c2y = (float) (2.0 * tcy), c2z = (float) (2.0 * tcz);
-    const int nva = t.p1 - t.p0;
-
-    /* FP32: FP64 re-evaluation of the n queued pairs of this wavefront */
-    int qn = 0;
-    auto drain = [&]() __attribute__((always_inline)) {
+      for (int r = 0; r < R; r++) {
+        const int p = t.p0 + r * 64 + slot;
+        const bool v = p < t.p1;
+        const int pc = v ? p : t.p0;
+        const FkRec ra = fk_gld(J.A.rec, pc);
+        const double x = ra.x, y = ra.y, z = ra.z;
+        lox = __builtin_fmin(lox, x); hix = __builtin_fmax(hix, x);
+        loy = __builtin_fmin(loy, y); hiy = __builtin_fmax(hiy, y);
+        loz = __builtin_fmin(loz, z); hiz = __builtin_fmax(hiz, z);
+        ai[r] = v ? p : 0x7fffffff;
+        ax[r] = v ? x : FK_FAR;
+        ay[r] = v ? y : FK_FAR;
+        az[r] = v ? z : FK_FAR;
+        as[r] = NEED_S ? (v ? ra.q : 3.0 * FK_FAR * FK_FAR) : 0.0;
+        aw[r] = (jw && v) ? (WSEP ? fk_gld(J.A.w, pc) : ra.q) : 1.0;
+        gacc[r] = 0.0;
+        actm[r] = __builtin_amdgcn_ballot_w64(v);
+      }
+      lox = fk_wave_min(lox); hix = -fk_wave_min(-hix);
+      loy = fk_wave_min(loy); hiy = -fk_wave_min(-hiy);
+      loz = fk_wave_min(loz); hiz = -fk_wave_min(-hiz);
       fk_wave_sync();
-      const FkJob J = fk_cld(fk_again(a.jobs, cur));
-      for (int e0 = 0; e0 < qn; e0 += 64) {
-        if (e0 + lane < qn) {
-          const int jg = (int) wqj[e0 + lane];
-          const unsigned v = wqs[e0 + lane];
-          const int p = t.p0 + (int) (v >> 5);
-          unsigned idx;
-          if (GEOM == FCFC_GEOM_SURVEY)
-            idx = fk_recheck_sv<BIN, HYB>(bn, J, p, jg, stab, ptab, s2e, pe);
-          else {
-            const FkRec ra = fk_gld(J.A.rec, p);
-            idx = fk_recheck<BIN, HYB, CENS>(bn, J, ra.x, ra.y, ra.z, jg, (int) (v & 31u), stab,
-                                             ptab, s2e, pe, &ncensus);
-          }
-          nrecheck++;
-          if (idx < ntot) {
-            if (WT && jwt)
-              atomicAdd(myhist_d + idx, WSEP ? fk_gld(J.A.w, p) * fk_gld(J.B.w, jg)
-                                             : fk_gld(J.A.rec, p).q * fk_gld(J.B.rec, jg).q);
-            else atomicAdd(myhist_u + idx, 1u);
+      if (lane == 0) { box[0] = lox; box[1] = hix; box[2] = loy; box[3] = hiy; box[4] = loz; box[5] = hiz; }
+      fk_wave_sync();
+      /* FP32 coordinates are relative to the centre of the box */
+      const double tcx = 0.5 * (lox + hix), tcy = 0.5 * (loy + hiy), tcz = 0.5 * (loz + hiz);
+      /* idle lanes: |a| = 1e18 and |dz| / s = 1 / (2 nmu), so that the mu
+       * estimate of their pairs is 1/2, clear of the windows */
+      const FkWin wn = J.win;
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const bool v = ai[r] != 0x7fffffff;
+        fax[r] = v ? (float) (ax[r] - tcx) : wn.idle_x;
+        fay[r] = v ? (float) (ay[r] - tcy) : 0.0f;
+        faz[r] = v ? (float) (az[r] - tcz) : wn.idle_z;
+      }
+      /* survey FP32: m = a + b = 2 a' + d + 2 c (a' = a - c, c = the centre).
+       * Idle lanes (a' = (10^6, 0, 0): s^2 and pi^2 far out of range) may
+       * look ambiguous in mu: their queue bits are masked off */
+      const float c2x = (float) (2.0 * tcx), c2y = (float) (2.0 * tcy), c2z = (float) (2.0 * tcz);
+      const int nva = t.p1 - t.p0;
+
+      /* FP32: FP64 re-evaluation of the n queued pairs of this wavefront */
+      int qn = 0;
+      auto drain = [&]() __attribute__((always_inline)) {
+        fk_wave_sync();
+        const FkJob J = fk_cld(fk_again(a.jobs, cur));
+        for (int e0 = 0; e0 < qn; e0 += 64) {
+          if (e0 + lane < qn) {
+            const int jg = (int) wqj[e0 + lane];
+            const unsigned v = wqs[e0 + lane];
+            const int p = t.p0 + (int) (v >> 5);
+            unsigned idx;
+            if (GEOM == FCFC_GEOM_SURVEY)
+              idx = fk_recheck_sv<BIN, HYB>(bn, J, p, jg, stab, ptab, s2e, pe);
+            else {
+              const FkRec ra = fk_gld(J.A.rec, p);
+              idx = fk_recheck<BIN, HYB, CENS>(bn, J, ra.x, ra.y, ra.z, jg, (int) (v & 31u), stab,
+                                               ptab, s2e, pe, &ncensus);
+            }
+            nrecheck++;
+            if (idx < ntot) {
+              if (WT && jwt)
+                atomicAdd(myhist_d + idx, WSEP ? fk_gld(J.A.w, p) * fk_gld(J.B.w, jg)
+                                               : fk_gld(J.A.rec, p).q * fk_gld(J.B.rec, jg).q);
+              else atomicAdd(myhist_u + idx, 1u);
+            }
           }
         }
-      }
-      qn = 0;
-      fk_wave_sync();
-    };
+        qn = 0;
+        fk_wave_sync();
+      };
 
-    /* one B object against the lane's A objects: FP64 coordinates, |r|^2 and
-     * weight, or FP32 coordinates relative to the run's centre; jj its sorted
-     * index, j its place in the chunk, code its periodic image */
-    auto step = [&](auto selfc, double bx, double by, double bz, double bs, double wj, float gx,
-                    float gy, float gz, int jj, int j, int code) __attribute__((always_inline)) {
-      constexpr bool SELF = decltype(selfc)::value;
-      if (MASKED) {
-        double bsum = 0.0;        /* GRAD: sum of G[bin] w_a over this lane's pairs */
-        auto add = [&](unsigned idx, int r) __attribute__((always_inline)) {
-          if (GRAD) {
-            const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
-            gacc[r] = __builtin_fma(gk, wj, gacc[r]);
-            bsum = __builtin_fma(gk, aw[r], bsum);
+      /* one B object against the lane's A objects: FP64 coordinates, |r|^2 and
+       * weight, or FP32 coordinates relative to the run's centre; jj its sorted
+       * index, j its place in the chunk, code its periodic image */
+      auto step = [&](auto selfc, double bx, double by, double bz, double bs, double wj, float gx,
+                      float gy, float gz, int jj, int j, int code) __attribute__((always_inline)) {
+        constexpr bool SELF = decltype(selfc)::value;
+        if (MASKED) {
+          double bsum = 0.0;        /* GRAD: sum of G[bin] w_a over this lane's pairs */
+          auto add = [&](unsigned idx, int r) __attribute__((always_inline)) {
+            if (GRAD) {
+              const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
+              gacc[r] = __builtin_fma(gk, wj, gacc[r]);
+              bsum = __builtin_fma(gk, aw[r], bsum);
+            }
+            else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
+            else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
+          };
+          if (F32) {
+            float ex[R], ey[R], ez[R], s2[R];
+            bool in[R], any = false;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+              ex[r] = gx - fax[r]; ey[r] = gy - fay[r]; ez[r] = gz - faz[r];
+              if (BIN == FCFC_BIN_SPI) s2[r] = __builtin_fmaf(ey[r], ey[r], ex[r] * ex[r]);
+              else if (SV32) s2[r] = __builtin_fmaf(ez[r], ez[r], __builtin_fmaf(ey[r], ey[r], ex[r] * ex[r]));
+              else s2[r] = __builtin_fmaf(ey[r], ey[r], __builtin_fmaf(ex[r], ex[r], ez[r] * ez[r]));
+              in[r] = s2[r] + wn.e_s2 < bn.m32s;
+              if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabsf(ez[r]) + wn.e_pi < bn.m32p);
+              if (SELF) in[r] = in[r] & (jj > ai[r]);
+              any |= in[r];
+            }
+            if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+              bool amb = false;
+              if (in[r]) {
+                const float u = s2[r] + wn.e_s2;
+                const unsigned e = stab_raw[(int) u];
+                amb = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
+                unsigned idx = e & 0xFFFFu;
+                if (BIN == FCFC_BIN_SPI) {
+                  const float up = __builtin_fabsf(ez[r]) + wn.e_pi;
+                  const unsigned ep = ptab_raw[(int) up];
+                  amb |= __builtin_amdgcn_fractf(up) < __uint_as_float(ep);
+                  idx += __umul24((unsigned) bn.nsh, ep & 0xFFFFu);
+                }
+                if (BIN == FCFC_BIN_SMU) {
+                  bool ambm;
+                  if (SV32) {
+                    const float mx = __builtin_fmaf(2.0f, fax[r], ex[r]) + c2x;
+                    const float my = __builtin_fmaf(2.0f, fay[r], ey[r]) + c2y;
+                    const float mz = __builtin_fmaf(2.0f, faz[r], ez[r]) + c2z;
+                    const float p = __builtin_fmaf(ez[r], mz, __builtin_fmaf(ey[r], my, ex[r] * mx));
+                    const float m2 = __builtin_fmaf(mz, mz, __builtin_fmaf(my, my, mx * mx));
+                    idx = fk_mu32(wn.nmu_f * __builtin_fabsf(p), __builtin_amdgcn_rsqf(m2 * s2[r]), idx,
+                                  bn, wn, ambm);
+                    amb |= m2 < wn.m2_floor;         /* near the observer */
+                  }
+                  else
+                    idx = fk_mu32(wn.nmu_f * __builtin_fabsf(ez[r]), __builtin_amdgcn_rsqf(s2[r]), idx,
+                                  bn, wn, ambm);
+                  amb |= ambm;
+                }
+                if (!amb) add(idx, r);
+              }
+              /* pairs near an edge: queue (B object, A slot, image) for FP64 */
+              const unsigned long long m = __builtin_amdgcn_ballot_w64(amb);
+              if (__builtin_expect(m != 0, 0)) {
+                if (amb) {
+                  const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                             __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+                  wqj[pos] = (unsigned) (SELF ? jj : cj[j]);
+                  wqs[pos] = (uint16_t) (((unsigned) (r * 64 + slot) << 5) | (unsigned) code);
+                }
+                qn += __popcll(m);
+              }
+            }
           }
-          else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
-          else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
-        };
-        if (F32) {
-          float ex[R], ey[R], ez[R], s2[R];
-          bool in[R], any = false;
+          else {
+            double s2[R], ez[R], dz2[R];
+            bool in[R], any = false;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+              if (GEOM == FCFC_GEOM_BOX) {
+                const double ex = bx - ax[r], ey = by - ay[r];
+                ez[r] = bz - az[r];
+                dz2[r] = ez[r] * ez[r];
+                if (BIN == FCFC_BIN_SPI) s2[r] = __builtin_fma(ey, ey, ex * ex);             /* :416-420 */
+                else s2[r] = __builtin_fma(ey, ey, __builtin_fma(ex, ex, dz2[r]));           /* :426-430 */
+              }
+              else if (BIN == FCFC_BIN_ISO) {
+                const double ex = ax[r] - bx, ey = ay[r] - by, e3 = az[r] - bz;
+                s2[r] = __builtin_fma(e3, e3, __builtin_fma(ey, ey, ex * ex));
+              }
+              else {
+                /* t (in dz2) and s^2 = s - t of the survey formulas (fk_sv64) */
+                dz2[r] = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
+                s2[r] = (as[r] + bs) - dz2[r];
+              }
+              in[r] = s2[r] < bn.s2max;
+              if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabs(ez[r]) < bn.pmax);
+              if (SELF) in[r] = in[r] & (jj > ai[r]);
+              any |= in[r];
+            }
+            if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+              if (!in[r]) continue;
+              const unsigned cell = stab[(int) s2[r]];
+              if (BIN == FCFC_BIN_ISO) add(cell, r);
+              else if (BIN == FCFC_BIN_SPI)
+                add(cell + __umul24((unsigned) bn.nsh, ptab[(int) __builtin_fabs(ez[r])]), r);
+              else {
+                bool slow;
+                unsigned idx;
+                if (GEOM == FCFC_GEOM_BOX)
+                  idx = fk_smu_index<false, MUT>(__builtin_fabs(ez[r]) * bn.nmu_d, __builtin_amdgcn_rsq(s2[r]),
+                                                 [&] { return dz2[r] * bn.nmu2; }, s2[r], cell, bn, &slow);
+                else {
+                  const double d = as[r] - bs, m2 = dz2[r] + (as[r] + bs);
+                  idx = fk_smu_index<true, MUT>(__builtin_fabs(d) * bn.nmu_d, __builtin_amdgcn_rsq(m2 * s2[r]),
+                                                [&] { return ((d * d) / m2) * bn.nmu2; }, s2[r], cell, bn, &slow);
+                }
+                /* a mu that the exact path drops; the fast path has none (a
+                 * survey value at its cap falls on the dummy row) */
+                if (!slow || idx < ntot_o) add(idx, r);
+              }
+            }
+          }
+          if (GRAD && hasB) {
+            /* the B object's share over the wavefront's pairs: one sum per
+             * row of 16 lanes, added into the chunk's LDS accumulator */
+            const double v = fk_row_sum(bsum);
+            if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
+          }
+          return;
+        }
+        if (GEOM == FCFC_GEOM_BOX) {
+          /* when this B object is out of range of every A object of the run,
+           * skip the binning (same expressions as the pair functions, so the
+           * compiler shares them) */
+          bool any = false;
 #pragma unroll
           for (int r = 0; r < R; r++) {
-            ex[r] = gx - fax[r]; ey[r] = gy - fay[r]; ez[r] = gz - faz[r];
-            if (BIN == FCFC_BIN_SPI) s2[r] = __builtin_fmaf(ey[r], ey[r], ex[r] * ex[r]);
-            else if (SV32) s2[r] = __builtin_fmaf(ez[r], ez[r], __builtin_fmaf(ey[r], ey[r], ex[r] * ex[r]));
-            else s2[r] = __builtin_fmaf(ey[r], ey[r], __builtin_fmaf(ex[r], ex[r], ez[r] * ez[r]));
-            in[r] = s2[r] + wn.e_s2 < bn.m32s;
-            if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabsf(ez[r]) + wn.e_pi < bn.m32p);
-            if (SELF) in[r] = in[r] & (jj > ai[r]);
-            any |= in[r];
+            const double ex = bx - ax[r], ey = by - ay[r], ez = bz - az[r];
+            if (BIN == FCFC_BIN_SPI)
+              any |= (__builtin_fma(ey, ey, ex * ex) < bn.s2skip) &
+                     (__builtin_fabs(ez) < bn.pskip);
+            else any |= __builtin_fma(ey, ey, __builtin_fma(ex, ex, ez * ez)) < bn.s2skip;
           }
           if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+        }
+        if (GEOM == FCFC_GEOM_SURVEY) {
+          /* the same skip for survey pairs: |a - b|^2 (iso) or s - t
+           * (= s^2 = s_perp^2 + pi^2) beyond the largest counted value */
+          bool any = false;
 #pragma unroll
           for (int r = 0; r < R; r++) {
-            bool amb = false;
-            if (in[r]) {
-              const float u = s2[r] + wn.e_s2;
-              const unsigned e = stab_raw[(int) u];
-              amb = __builtin_amdgcn_fractf(u) < __uint_as_float(e);
-              unsigned idx = e & 0xFFFFu;
-              if (BIN == FCFC_BIN_SPI) {
-                const float up = __builtin_fabsf(ez[r]) + wn.e_pi;
-                const unsigned ep = ptab_raw[(int) up];
-                amb |= __builtin_amdgcn_fractf(up) < __uint_as_float(ep);
-                idx += __umul24((unsigned) bn.nsh, ep & 0xFFFFu);
-              }
-              if (BIN == FCFC_BIN_SMU) {
-                bool ambm;
-                if (SV32) {
-                  const float mx = __builtin_fmaf(2.0f, fax[r], ex[r]) + c2x;
-                  const float my = __builtin_fmaf(2.0f, fay[r], ey[r]) + c2y;
-                  const float mz = __builtin_fmaf(2.0f, faz[r], ez[r]) + c2z;
-                  const float p = __builtin_fmaf(ez[r], mz, __builtin_fmaf(ey[r], my, ex[r] * mx));
-                  const float m2 = __builtin_fmaf(mz, mz, __builtin_fmaf(my, my, mx * mx));
-                  idx = fk_mu32(wn.nmu_f * __builtin_fabsf(p), __builtin_amdgcn_rsqf(m2 * s2[r]), idx,
-                                bn, wn, ambm);
-                  amb |= m2 < wn.m2_floor;         /* near the observer */
-                }
-                else
-                  idx = fk_mu32(wn.nmu_f * __builtin_fabsf(ez[r]), __builtin_amdgcn_rsqf(s2[r]), idx,
-                                bn, wn, ambm);
-                amb |= ambm;
-              }
-              if (!amb) add(idx, r);
+            if (SV32) {
+              const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
+              any |= __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) < bn.s2skip32;
             }
-            /* pairs near an edge: queue (B object, A slot, image) for FP64 */
-            const unsigned long long m = __builtin_amdgcn_ballot_w64(amb);
+            else if (BIN == FCFC_BIN_ISO) {
+              const double ex = ax[r] - bx, ey = ay[r] - by, ez = az[r] - bz;
+              any |= __builtin_fma(ez, ez, __builtin_fma(ey, ey, ex * ex)) < bn.s2skip;
+            }
+            else {
+              const double tt = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
+              any |= (as[r] + bs) - tt < bn.s2skip;
+            }
+          }
+          if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+        }
+        double bsum = 0.0;          /* GRAD: sum of G[bin] w_a over this lane's pairs */
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          unsigned idx;
+          bool queued = false;      /* FP32: left to the FP64 re-evaluation */
+          if (F32) {
+            bool amb, ambm, ambx;
+            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
+            idx = fk_sv32_spi(ex, ey, ez, __builtin_fmaf(2.0f, fax[r], ex) + c2x,
+                              __builtin_fmaf(2.0f, fay[r], ey) + c2y,
+                              __builtin_fmaf(2.0f, faz[r], ez) + c2z, bn, wn, stab_raw,
+                              ptab_raw, amb, ambm, ambx);
+            if (SELF) {
+              const bool keep = jj > ai[r];
+              amb = amb & keep; ambm = ambm & keep; idx = keep ? idx : FK_NONE;
+            }
+            /* pairs near an edge: queue (B object, A slot, image) for FP64.
+             * The conditions are balloted apart (each ballot is its compare's
+             * own mask) and the lane's bit is read back from the mask inside
+             * the rare branch, so no lane value is kept across it */
+            if (SELF) ambx = ambx & (jj > ai[r]);
+            unsigned long long m = __builtin_amdgcn_ballot_w64(amb) |
+                __builtin_amdgcn_ballot_w64(ambm) | __builtin_amdgcn_ballot_w64(ambx);
+            m &= actm[r];
             if (__builtin_expect(m != 0, 0)) {
-              if (amb) {
+              if ((m >> lane) & 1ull) {
                 const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
                                            __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
                 wqj[pos] = (unsigned) (SELF ? jj : cj[j]);
-                wqs[pos] = (uint16_t) (((unsigned) (r * 64 + lane) << 5) | (unsigned) code);
+                wqs[pos] = (uint16_t) (((unsigned) (r * 64 + slot) << 5) | (unsigned) code);
               }
               qn += __popcll(m);
             }
+            queued = amb | ambm | ambx;
           }
-        }
-        else {
-          double s2[R], ez[R], dz2[R];
-          bool in[R], any = false;
-#pragma unroll
-          for (int r = 0; r < R; r++) {
-            if (GEOM == FCFC_GEOM_BOX) {
-              const double ex = bx - ax[r], ey = by - ay[r];
-              ez[r] = bz - az[r];
-              dz2[r] = ez[r] * ez[r];
-              if (BIN == FCFC_BIN_SPI) s2[r] = __builtin_fma(ey, ey, ex * ex);             /* :416-420 */
-              else s2[r] = __builtin_fma(ey, ey, __builtin_fma(ex, ex, dz2[r]));           /* :426-430 */
+          else if (GEOM == FCFC_GEOM_BOX)
+            idx = fk_box64<BIN, HYB, false, PLAIN>(bx - ax[r], by - ay[r], bz - az[r], bn, stab,
+                                                   ptab, s2e, pe);
+          else
+            idx = fk_sv64<BIN, HYB, PLAIN, false, QT>(ax[r], ay[r], az[r], as[r], bx, by, bz, bs,
+                                                     bn, stab, ptab, s2e, pe, os_lds, op_lds);
+          if (!F32 && SELF && !(jj > ai[r])) idx = FK_NONE;
+          if (idx < ntot_o && !queued) {
+            if (GRAD) {
+              const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
+              gacc[r] = __builtin_fma(gk, wj, gacc[r]);
+              bsum = __builtin_fma(gk, aw[r], bsum);
             }
-            else if (BIN == FCFC_BIN_ISO) {
-              const double ex = ax[r] - bx, ey = ay[r] - by, e3 = az[r] - bz;
-              s2[r] = __builtin_fma(e3, e3, __builtin_fma(ey, ey, ex * ex));
-            }
-            else {
-              /* t (in dz2) and s^2 = s - t of the survey formulas (fk_sv64) */
-              dz2[r] = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
-              s2[r] = (as[r] + bs) - dz2[r];
-            }
-            in[r] = s2[r] < bn.s2max;
-            if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabs(ez[r]) < bn.pmax);
-            if (SELF) in[r] = in[r] & (jj > ai[r]);
-            any |= in[r];
-          }
-          if (__builtin_amdgcn_ballot_w64(any) == 0) return;
-#pragma unroll
-          for (int r = 0; r < R; r++) {
-            if (!in[r]) continue;
-            const unsigned cell = stab[(int) s2[r]];
-            if (BIN == FCFC_BIN_ISO) add(cell, r);
-            else if (BIN == FCFC_BIN_SPI)
-              add(cell + __umul24((unsigned) bn.nsh, ptab[(int) __builtin_fabs(ez[r])]), r);
-            else {
-              bool slow;
-              unsigned idx;
-              if (GEOM == FCFC_GEOM_BOX)
-                idx = fk_smu_index<false, MUT>(__builtin_fabs(ez[r]) * bn.nmu_d, __builtin_amdgcn_rsq(s2[r]),
-                                               [&] { return dz2[r] * bn.nmu2; }, s2[r], cell, bn, &slow);
-              else {
-                const double d = as[r] - bs, m2 = dz2[r] + (as[r] + bs);
-                idx = fk_smu_index<true, MUT>(__builtin_fabs(d) * bn.nmu_d, __builtin_amdgcn_rsq(m2 * s2[r]),
-                                              [&] { return ((d * d) / m2) * bn.nmu2; }, s2[r], cell, bn, &slow);
-              }
-              /* a mu that the exact path drops; the fast path has none (a
-               * survey value at its cap falls on the dummy row) */
-              if (!slow || idx < ntot_o) add(idx, r);
-            }
+            else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
+            else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
           }
         }
         if (GRAD && hasB) {
@@ -1513,244 +1623,185 @@ k_count(const FkArgs a) {
           const double v = fk_row_sum(bsum);
           if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
         }
-        return;
-      }
-      if (GEOM == FCFC_GEOM_BOX) {
-        /* when this B object is out of range of every A object of the run,
-         * skip the binning (same expressions as the pair functions, so the
-         * compiler shares them) */
-        bool any = false;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const double ex = bx - ax[r], ey = by - ay[r], ez = bz - az[r];
-          if (BIN == FCFC_BIN_SPI)
-            any |= (__builtin_fma(ey, ey, ex * ex) < bn.s2skip) &
-                   (__builtin_fabs(ez) < bn.pskip);
-          else any |= __builtin_fma(ey, ey, __builtin_fma(ex, ex, ez * ez)) < bn.s2skip;
-        }
-        if (__builtin_amdgcn_ballot_w64(any) == 0) return;
-      }
-      if (GEOM == FCFC_GEOM_SURVEY) {
-        /* the same skip for survey pairs: |a - b|^2 (iso) or s - t
-         * (= s^2 = s_perp^2 + pi^2) beyond the largest counted value */
-        bool any = false;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          if (SV32) {
-            const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-            any |= __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) < bn.s2skip32;
-          }
-          else if (BIN == FCFC_BIN_ISO) {
-            const double ex = ax[r] - bx, ey = ay[r] - by, ez = az[r] - bz;
-            any |= __builtin_fma(ez, ez, __builtin_fma(ey, ey, ex * ex)) < bn.s2skip;
-          }
-          else {
-            const double tt = __builtin_fma(az[r], bz, __builtin_fma(ay[r], by, ax[r] * bx)) * 2.0;
-            any |= (as[r] + bs) - tt < bn.s2skip;
-          }
-        }
-        if (__builtin_amdgcn_ballot_w64(any) == 0) return;
-      }
-      double bsum = 0.0;          /* GRAD: sum of G[bin] w_a over this lane's pairs */
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        unsigned idx;
-        bool queued = false;      /* FP32: left to the FP64 re-evaluation */
-        if (F32) {
-          bool amb, ambm, ambx;
-          const float ex = gx - fax[r], ey = gy - fay[r], ez = gz - faz[r];
-          idx = fk_sv32_spi(ex, ey, ez, __builtin_fmaf(2.0f, fax[r], ex) + c2x,
-                            __builtin_fmaf(2.0f, fay[r], ey) + c2y,
-                            __builtin_fmaf(2.0f, faz[r], ez) + c2z, bn, wn, stab_raw,
-                            ptab_raw, amb, ambm, ambx);
-          if (SELF) {
-            const bool keep = jj > ai[r];
-            amb = amb & keep; ambm = ambm & keep; idx = keep ? idx : FK_NONE;
-          }
-          /* pairs near an edge: queue (B object, A slot, image) for FP64.
-           * The conditions are balloted apart (each ballot is its compare's
-           * own mask) and the lane's bit is read back from the mask inside
-           * the rare branch, so no lane value is kept across it */
-          if (SELF) ambx = ambx & (jj > ai[r]);
-          unsigned long long m = __builtin_amdgcn_ballot_w64(amb) |
-              __builtin_amdgcn_ballot_w64(ambm) | __builtin_amdgcn_ballot_w64(ambx);
-          m &= actm[r];
-          if (__builtin_expect(m != 0, 0)) {
-            if ((m >> lane) & 1ull) {
-              const int pos = qn + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
-                                         __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-              wqj[pos] = (unsigned) (SELF ? jj : cj[j]);
-              wqs[pos] = (uint16_t) (((unsigned) (r * 64 + lane) << 5) | (unsigned) code);
-            }
-            qn += __popcll(m);
-          }
-          queued = amb | ambm | ambx;
-        }
-        else if (GEOM == FCFC_GEOM_BOX)
-          idx = fk_box64<BIN, HYB, false, PLAIN>(bx - ax[r], by - ay[r], bz - az[r], bn, stab,
-                                                 ptab, s2e, pe);
-        else
-          idx = fk_sv64<BIN, HYB, PLAIN, false, QT>(ax[r], ay[r], az[r], as[r], bx, by, bz, bs,
-                                                   bn, stab, ptab, s2e, pe, os_lds, op_lds);
-        if (!F32 && SELF && !(jj > ai[r])) idx = FK_NONE;
-        if (idx < ntot_o && !queued) {
-          if (GRAD) {
-            const double gk = *(const double *) (lds + (ohist_g + 8u * idx));
-            gacc[r] = __builtin_fma(gk, wj, gacc[r]);
-            bsum = __builtin_fma(gk, aw[r], bsum);
-          }
-          else if (WT && jwt) atomicAdd((double *) (lds + (ohist_d + 8u * idx)), aw[r] * wj);
-          else atomicAdd((unsigned int *) (lds + (ohist_u + 4u * idx)), 1u);
-        }
-      }
-      if (GRAD && hasB) {
-        /* the B object's share over the wavefront's pairs: one sum per
-         * row of 16 lanes, added into the chunk's LDS accumulator */
-        const double v = fk_row_sum(bsum);
-        if ((lane & 15) == 0 && v != 0.0) atomicAdd(cb + j, v);
-      }
-    };
+      };
 
 
-    /* B objects [b0, b0 + n) of the other catalogue (SELF: of the run itself),
-     * at the periodic image of code (IMG: not the object's own place) */
-    auto segment = [&](auto selfc, auto imgc, int b0, int n, int code) __attribute__((always_inline)) {
-      constexpr bool SELF = decltype(selfc)::value;
-      constexpr bool IMG = decltype(imgc)::value;
-      for (int c0 = SELF ? 0 : sq * FK_CH; c0 < n; c0 += SELF ? FK_CH : SQ * FK_CH) {
-        const FkJob *pj = fk_again(a.jobs, cur);
-        const FkCat B = fk_cld(SELF ? &pj->A : &pj->B);
-        const FkGrid g = fk_cld(&pj->g);
-        const double Dx = IMG ? (double) (code % 3 - 1) * g.Lx : 0.0;
-        const double Dy = IMG ? (double) ((code / 3) % 3 - 1) * g.Ly : 0.0;
-        const double Dz = IMG ? (double) (code / 9 - 1) * g.Lz : 0.0;
-        const bool in = c0 + lane < n;
-        const int jg = b0 + (in ? c0 + lane : 0);
-        const FkRec rb = fk_gld(B.rec, jg);
-        double x = rb.x, y = rb.y, z = rb.z;
-        if (IMG) { x = x + Dx; y = y + Dy; z = z + Dz; }
-        /* drop the objects beyond the maximum separation from the run's
-         * bounding box (the grid's padded ranges) */
-        bool keep = in;
-        const double lx = box[0], hx = box[1], ly = box[2], hy = box[3], lz = box[4], hz = box[5];
-        if (!SELF) {
-          const double ex = __builtin_fmax(__builtin_fmax(lx - x, x - hx), 0.0);
-          const double ey = __builtin_fmax(__builtin_fmax(ly - y, y - hy), 0.0);
-          const double ez = __builtin_fmax(__builtin_fmax(lz - z, z - hz), 0.0);
-          const double exy = __builtin_fma(ey, ey, ex * ex);
-          if (g.hz_const >= 0) keep &= (exy < g.Rxy2) & (ez < g.hz_const);
-          else keep &= __builtin_fma(ez, ez, exy) < g.R2;
-        }
-        unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
-        evals += (unsigned long long) ((unsigned) min(FK_CH, n - c0) * (unsigned) nva);
-        if (m == 0) continue;
-        const int cnt = __popcll(m);
-        if (!GRAD && !jwt) {
-          if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) spill_counts();
-          since += (unsigned) cnt * (unsigned) nva;
-        }
-        if (F32) {
-          /* pack the kept objects into the wavefront's chunk */
-          fk_wave_sync();
-          if (keep) {
-            const int q = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
-                                      __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-            fx[q] = (float) (x - 0.5 * (lx + hx));
-            fy[q] = (float) (y - 0.5 * (ly + hy));
-            fz[q] = (float) (z - 0.5 * (lz + hz));
-            if (WT) cw[q] = jw ? (WSEP ? fk_gld(B.w, jg) : rb.q) : 1.0;
-            cj[q] = jg;
+      /* B objects [b0, b0 + n) of the other catalogue (SELF: of the run itself),
+       * at the periodic image of code (IMG: not the object's own place) */
+      auto segment = [&](auto selfc, auto imgc, int b0, int n, int code) __attribute__((always_inline)) {
+        constexpr bool SELF = decltype(selfc)::value;
+        constexpr bool IMG = decltype(imgc)::value;
+        for (int c0 = SELF ? 0 : sq * FK_CH; c0 < n; c0 += SELF ? FK_CH : SQ * FK_CH) {
+          const FkJob *pj = fk_again(a.jobs, cur);
+          const FkCat B = fk_cld(SELF ? &pj->A : &pj->B);
+          const FkGrid g = fk_cld(&pj->g);
+          const double Dx = IMG ? (double) (code % 3 - 1) * g.Lx : 0.0;
+          const double Dy = IMG ? (double) ((code / 3) % 3 - 1) * g.Ly : 0.0;
+          const double Dz = IMG ? (double) (code / 9 - 1) * g.Lz : 0.0;
+          const bool in = c0 + lane < n;
+          const int jg = b0 + (in ? c0 + lane : 0);
+          const FkRec rb = fk_gld(B.rec, jg);
+          double x = rb.x, y = rb.y, z = rb.z;
+          if (IMG) { x = x + Dx; y = y + Dy; z = z + Dz; }
+          /* drop the objects beyond the maximum separation from the run's
+           * bounding box (the grid's padded ranges) */
+          bool keep = in;
+          const double lx = box[0], hx = box[1], ly = box[2], hy = box[3], lz = box[4], hz = box[5];
+          if (!SELF) {
+            const double ex = __builtin_fmax(__builtin_fmax(lx - x, x - hx), 0.0);
+            const double ey = __builtin_fmax(__builtin_fmax(ly - y, y - hy), 0.0);
+            const double ez = __builtin_fmax(__builtin_fmax(lz - z, z - hz), 0.0);
+            const double exy = __builtin_fma(ey, ey, ex * ex);
+            if (g.hz_const >= 0) keep &= (exy < g.Rxy2) & (ez < g.hz_const);
+            else keep &= __builtin_fma(ez, ez, exy) < g.R2;
           }
-          fk_wave_sync();
-          for (int j = 0; j < cnt;) {
-            /* while the queue has room for the pairs of one more object */
-#pragma unroll 2
-            for (; j < cnt; j++) {
-              if (qn > FK_QCAP - 64 * R) break;
-              step(selfc, 0.0, 0.0, 0.0, 0.0, WT ? cw[j] : 1.0, fx[j], fy[j], fz[j],
-                   SELF ? cj[j] : 0, j, code);
-            }
-            if (qn > FK_QCAP - 64 * R) drain();
+          unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+          evals += (unsigned long long) ((unsigned) min(FK_CH, n - c0) * (unsigned) nva);
+          if (m == 0) continue;
+          const int cnt = __popcll(m);
+          if (!GRAD && !jwt) {
+            if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) spill_counts();
+            since += (unsigned) cnt * (unsigned) nva;
           }
-        }
-        else {
-          if (GRAD && hasB) { fk_wave_sync(); cb[lane] = 0.0; fk_wave_sync(); }
-          /* the kept objects, one at a time, into scalar registers */
-          typedef const __attribute__((address_space(4))) double cdouble;
-          cdouble *rp = (cdouble *) (B.rec + b0 + c0);
-          cdouble *wp = (cdouble *) (B.w + b0 + c0);
-          unsigned long long k = m;
-          while (k) {
-            const int j = __builtin_ctzll(k);
-            k &= k - 1;
-            const double px = rp[4 * j], py = rp[4 * j + 1], pz = rp[4 * j + 2], pq = rp[4 * j + 3];
-            double wj = 1.0;
-            if (WSEP && (WT || GRAD)) { if (jw) wj = wp[j]; }
-            else if (WT || GRAD) wj = jw ? pq : 1.0;
-            step(selfc, IMG ? px + Dx : px, IMG ? py + Dy : py, IMG ? pz + Dz : pz,
-                 NEED_S ? pq : 0.0, wj, 0.0f, 0.0f, 0.0f, SELF ? b0 + c0 + j : 0, j, code);
-          }
-          /* GRAD: the B objects' shares go to the output */
-          if (GRAD && hasB) {
+          /* place in the chunk of a kept object */
+          const int q = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                    __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+          if (F32) {
+            /* pack the kept objects into the wavefront's chunk */
             fk_wave_sync();
             if (keep) {
-              const double v = cb[lane];
-              if (v != 0.0) unsafeAtomicAdd(fk_cld(&fk_again(a.jobs, cur)->gB) + jg, v);
+              fx[q] = (float) (x - 0.5 * (lx + hx));
+              fy[q] = (float) (y - 0.5 * (ly + hy));
+              fz[q] = (float) (z - 0.5 * (lz + hz));
+              if (WT) cw[q] = jw ? (WSEP ? fk_gld(B.w, jg) : rb.q) : 1.0;
+              cj[q] = jg;
+            }
+            /* NG > 1: up to a multiple of NG objects, out of range of all others */
+            if (NG > 1 && lane < (-cnt & (NG - 1))) {
+              fx[cnt + lane] = -1e18f;
+              fy[cnt + lane] = fz[cnt + lane] = 0.0f;
+              if (WT) cw[cnt + lane] = 0.0;
+              cj[cnt + lane] = 0;
+            }
+            fk_wave_sync();
+            for (int j = 0; j < cnt;) {
+              /* while the queue has room for the pairs of one more object */
+#pragma unroll 2
+              for (; j < cnt; j += NG) {
+                if (qn > FK_QCAP - 64 * R) break;
+                const int q = j + sub;
+                step(selfc, 0.0, 0.0, 0.0, 0.0, WT ? cw[q] : 1.0, fx[q], fy[q], fz[q],
+                     SELF ? cj[q] : 0, q, code);
+              }
+              if (qn > FK_QCAP - 64 * R) drain();
+            }
+          }
+          else {
+            if (GRAD && hasB) { fk_wave_sync(); cb[lane] = 0.0; fk_wave_sync(); }
+            if (NG > 1) {
+              fk_wave_sync();
+              if (keep) {
+                cr[q] = FkRec{x, y, z, rb.q};
+                if (WSEP && (WT || GRAD)) cw[q] = jw ? fk_gld(B.w, jg) : 1.0;
+                cj[q] = jg;
+              }
+              if (lane < (-cnt & (NG - 1))) {
+                cr[cnt + lane] = FkRec{-FK_FAR, -FK_FAR, -FK_FAR, NEED_S ? 3.0 * FK_FAR * FK_FAR : 0.0};
+                if (WSEP && (WT || GRAD)) cw[cnt + lane] = 0.0;
+                cj[cnt + lane] = 0;
+              }
+              fk_wave_sync();
+#pragma unroll 2
+              for (int j = sub; j < cnt + sub; j += NG) {
+                const double px = cr[j].x, py = cr[j].y, pz = cr[j].z;
+                const double pq = NEED_S || ((WT || GRAD) && !WSEP) ? cr[j].q : 0.0;
+                double wj = 1.0;
+                if (WT || GRAD) wj = WSEP ? cw[j] : (jw ? pq : 1.0);
+                step(selfc, px, py, pz, pq, wj, 0.0f, 0.0f, 0.0f, SELF ? cj[j] : 0, j, code);
+              }
+            }
+            else {
+              /* the kept objects, one at a time, into scalar registers */
+              typedef const __attribute__((address_space(4))) double cdouble;
+              cdouble *rp = (cdouble *) (B.rec + b0 + c0);
+              cdouble *wp = (cdouble *) (B.w + b0 + c0);
+              unsigned long long k = m;
+              while (k) {
+                const int j = __builtin_ctzll(k);
+                k &= k - 1;
+                const double px = rp[4 * j], py = rp[4 * j + 1], pz = rp[4 * j + 2], pq = rp[4 * j + 3];
+                double wj = 1.0;
+                if (WSEP && (WT || GRAD)) { if (jw) wj = wp[j]; }
+                else if (WT || GRAD) wj = jw ? pq : 1.0;
+                step(selfc, IMG ? px + Dx : px, IMG ? py + Dy : py, IMG ? pz + Dz : pz,
+                     NEED_S ? pq : 0.0, wj, 0.0f, 0.0f, 0.0f, SELF ? b0 + c0 + j : 0, j, code);
+              }
+            }
+            /* GRAD: the B objects' shares go to the output */
+            if (GRAD && hasB) {
+              fk_wave_sync();
+              if (keep) {
+                const double v = cb[NG > 1 ? q : lane];
+                if (v != 0.0) unsafeAtomicAdd(fk_cld(&fk_again(a.jobs, cur)->gB) + jg, v);
+              }
             }
           }
         }
-      }
-    };
+      };
 
-    /* ---- auto counts: pairs inside the run (j > i), first item only ---- */
-    if (J.autoc && part == 0 && sq == 0) {
-      evals -= (unsigned long long) nva * (unsigned) nva / 2;
-      segment(std::true_type(), std::false_type(), t.p0, nva, 13);
-    }
-
-    /* ---- strips, one per lane at a time ---- */
-    for (int sb0 = s0; sb0 < s1; sb0 += 64) {
-      int b0[FK_MAXSEG], len[FK_MAXSEG], code[FK_MAXSEG];
-      {
-        const int l = min(sb0 + lane, s1 - 1);
-        const FkJob *pj = fk_again(a.jobs, cur);
-        const int *sp = fk_cld(&pj->strips);
-        fk_strip_segments(fk_cld(&pj->g), fk_cld(&pj->B.cell_start), t, box[4], box[5],
-                          fk_gld(sp, 3 * l), fk_gld(sp, 3 * l + 1), fk_gld(sp, 3 * l + 2), b0, len, code);
-        if (sb0 + lane >= s1) len[0] = len[1] = len[2] = 0;
+      /* ---- auto counts: pairs inside the run (j > i), first item only ---- */
+      if (J.autoc && part == 0 && sq == 0) {
+        evals -= (unsigned long long) nva * (unsigned) nva / 2;
+        segment(std::true_type(), std::false_type(), t.p0, nva, 13);
       }
-      unsigned long long m0 = __builtin_amdgcn_ballot_w64(len[0] > 0),
-                         m1 = __builtin_amdgcn_ballot_w64(len[1] > 0),
-                         m2 = __builtin_amdgcn_ballot_w64(len[2] > 0);
-      while (m0 | m1 | m2) {
-        int b, n, cd, q;
-        if (m1) {
-          q = __builtin_ctzll(m1); m1 &= m1 - 1;
-          b = fk_lane_of(b0[1], q); n = fk_lane_of(len[1], q); cd = fk_lane_of(code[1], q);
-        }
-        else if (m0) {
-          q = __builtin_ctzll(m0); m0 &= m0 - 1;
-          b = fk_lane_of(b0[0], q); n = fk_lane_of(len[0], q); cd = fk_lane_of(code[0], q);
-        }
-        else {
-          q = __builtin_ctzll(m2); m2 &= m2 - 1;
-          b = fk_lane_of(b0[2], q); n = fk_lane_of(len[2], q); cd = fk_lane_of(code[2], q);
-        }
-        if (GEOM == FCFC_GEOM_SURVEY || (!F32 && cd == 13))
-          segment(std::false_type(), std::false_type(), b, n, cd);
-        else segment(std::false_type(), std::true_type(), b, n, cd);
-      }
-    }
-    if (F32 && qn) drain();
 
-    if (GRAD) {
-      double *gA = fk_cld(&fk_again(a.jobs, cur)->gA);
-      if (gA)
+      /* ---- strips, one per lane at a time ---- */
+      for (int sb0 = s0; sb0 < s1; sb0 += 64) {
+        int b0[FK_MAXSEG], len[FK_MAXSEG], code[FK_MAXSEG];
+        {
+          const int l = min(sb0 + lane, s1 - 1);
+          const FkJob *pj = fk_again(a.jobs, cur);
+          const int *sp = fk_cld(&pj->strips);
+          fk_strip_segments(fk_cld(&pj->g), fk_cld(&pj->B.cell_start), t, box[4], box[5],
+                            fk_gld(sp, 3 * l), fk_gld(sp, 3 * l + 1), fk_gld(sp, 3 * l + 2), b0, len, code);
+          if (sb0 + lane >= s1) len[0] = len[1] = len[2] = 0;
+        }
+        unsigned long long m0 = __builtin_amdgcn_ballot_w64(len[0] > 0),
+                           m1 = __builtin_amdgcn_ballot_w64(len[1] > 0),
+                           m2 = __builtin_amdgcn_ballot_w64(len[2] > 0);
+        while (m0 | m1 | m2) {
+          int b, n, cd, q;
+          if (m1) {
+            q = __builtin_ctzll(m1); m1 &= m1 - 1;
+            b = fk_lane_of(b0[1], q); n = fk_lane_of(len[1], q); cd = fk_lane_of(code[1], q);
+          }
+          else if (m0) {
+            q = __builtin_ctzll(m0); m0 &= m0 - 1;
+            b = fk_lane_of(b0[0], q); n = fk_lane_of(len[0], q); cd = fk_lane_of(code[0], q);
+          }
+          else {
+            q = __builtin_ctzll(m2); m2 &= m2 - 1;
+            b = fk_lane_of(b0[2], q); n = fk_lane_of(len[2], q); cd = fk_lane_of(code[2], q);
+          }
+          if (GEOM == FCFC_GEOM_SURVEY || (!F32 && cd == 13))
+            segment(std::false_type(), std::false_type(), b, n, cd);
+          else segment(std::false_type(), std::true_type(), b, n, cd);
+        }
+      }
+      if (F32 && qn) drain();
+
+      if (GRAD) {
+        double *gA = fk_cld(&fk_again(a.jobs, cur)->gA);
+        if (gA)
 #pragma unroll
-        for (int r = 0; r < R; r++)
-          if (ai[r] != 0x7fffffff && gacc[r] != 0.0) unsafeAtomicAdd(gA + ai[r], gacc[r]);
+          for (int r = 0; r < R; r++) {
+            double v = gacc[r];
+#pragma unroll
+            for (int k = 32; k >= NA; k >>= 1) v += __shfl_xor(v, k);
+            if (sub == 0 && ai[r] != 0x7fffffff && v != 0.0) unsafeAtomicAdd(gA + ai[r], v);
+          }
+      }
     }
-  }
   }
 
   /* statistics: summed over the workgroup, then in one of FK_STATS lines */
@@ -1940,6 +1991,8 @@ extern "C" int fcfc_gpu_set_tuning(fcfc_gpu_ctx *c, int cell_div, int tile,
 
 /* ---- per-job plan ------------------------------------------------------ */
 
+/* groups of lanes of the kernels for sparse catalogues (NG of k_count) */
+#define FK_NG 4
 struct JobPlan {
   int bucket;       /* density bucket for the autotuner cache */
   FkGrid g;
@@ -1948,6 +2001,8 @@ struct JobPlan {
   int nblk;         /* blocks per row */
   double cand;      /* candidate B objects of one run in a uniform catalogue */
   int R;            /* objects per lane */
+  int G;            /* lanes per A object (k_count) */
+  int run;          /* objects of a run */
   int T_auto;       /* T chosen by the plan (not by the caller's tuning) */
   std::vector<int> strips;
   int nstrips;
@@ -2018,18 +2073,40 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
       }
   }
   P->bucket = bucket;
+  /* Objects per tile: two per lane, which halves the B objects read per pair,
+   * unless a run of 128 objects is about as wide as the separations it is
+   * counted to (sparse catalogues): then one (iso DD of 1e5 to 200 Mpc/h,
+   * whose cube is half the separation: 0.39 against 0.36 ms). */
+  P->T_auto = (tT <= 0);
+  const double cube = cbrt(128.0 / std::max(ndenA, 1e-300));
+  if (tT > 0) P->T = std::min(tT, 4 * FK_NT);
+  else P->T = cube > 0.75 * R ? FK_NT : 2 * FK_NT;
+  P->R = (P->T + FK_NT - 1) / FK_NT;
+  /* Sparser catalogues than that: runs of 16 objects, four groups of lanes
+   * (k_count), unless B is far sparser than A (its strips then hold too few
+   * objects for four groups).  Kernel ms, without and with: iso cross count
+   * of 3e5 x 1e6 to 30 Mpc/h 1.10, 0.56; w_p of 1e6 to 40 Mpc/h 2.5, 1.7; iso
+   * DD of 2e3 0.040, 0.026; box (s, mu) DD to 200 of the unit box of 1000:
+   * n = 3e4 (cube / R = 0.81) 0.136, 0.103; 6e4 (0.64) 0.207, 0.185; 1.2e5
+   * (0.51) weighted 0.55, 0.63; survey (s, mu) to 150 of 6e4 (0.86) 0.20,
+   * 0.16; iso DD of 1e5 (0.54) 0.31, 0.42; DR of 6e3 x 6e4 (0.64) 0.087,
+   * 0.12. */
+  const bool can = mode != MODE_P64 && !c->census &&
+      !(b->geometry == FCFC_GEOM_SURVEY && b->bintype == FCFC_BIN_SPI);
+  P->G = can && (P->T <= 64 / FK_NG || (P->T == FK_NT && cube > 0.75 * R && 8 * nden >= ndenA)) ? FK_NG : 1;
+  P->run = P->G > 1 ? 64 / P->G : 64 * P->R;
   /* Runs as compact as their object number allows: the objects of B within
    * the maximum separation of a run's bounding box are evaluated, and a cube
    * has the least of them.  The side of the cube that holds 128 objects of A
-   * is the cell width in x and y (rounded to cells per separation, one at
-   * least: thinner columns of a sparse catalogue would only lengthen its
-   * runs), four z-cells per width.  Measured (kernel ms at cd = 2, 3, 4, 6,
-   * 8): (s, mu) RR of 4e6 objects in the unit box 296, 245, 232, 231, 230
-   * (rule: 6); weighted DD of 5e5 9.1, 8.7, 8.9, 10.1, 12 (3); iso DD of
-   * 1e5 0.36, 0.36, 0.55, 0.82, 1.2 (2); survey (s, mu) RR of 1.2e6 16.6,
-   * 15.5, 16.4, 19.9, 25 (3). */
-  const double cube = cbrt(128.0 / std::max(ndenA, 1e-300));
-  if (cd <= 0) cd = (int) std::min(std::max(floor(Rxy / cube + 0.6), 1.0), 12.0);
+   * (32 for runs of 16) is the cell width in x and y (rounded to cells per
+   * separation, one at least: thinner columns of a sparse catalogue would
+   * only lengthen its runs), four z-cells per width.  Measured (kernel ms at
+   * cd = 2, 3, 4, 6, 8): (s, mu) RR of 4e6 objects in the unit box 296, 245,
+   * 232, 231, 230 (rule: 6); weighted DD of 5e5 9.1, 8.7, 8.9, 10.1, 12 (3);
+   * iso DD of 1e5 0.36, 0.36, 0.55, 0.82, 1.2 (2); survey (s, mu) RR of 1.2e6
+   * 16.6, 15.5, 16.4, 19.9, 25 (3). */
+  const double width = P->G > 1 ? cbrt(32.0 / std::max(ndenA, 1e-300)) : cube;
+  if (cd <= 0) cd = (int) std::min(std::max(floor(Rxy / width + 0.6), 1.0), 12.0);
   if (zd <= 0) zd = 4;
   /* cells of Rxy / cd, but never more cells than about 4 per object
    * (between 2^18 and 2^25): a sparse catalogue in a large volume gets
@@ -2082,10 +2159,6 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
    * it is counted to (sparse catalogues): then 64, whose boxes reach fewer B
    * objects (w_p of 1e6 objects to 40 Mpc/h: 3.0 against 3.9 ms; iso DD of
    * 1e5 to 200 Mpc/h, whose cube is half the separation: 0.39 against 0.36). */
-  P->T_auto = (tT <= 0);
-  if (tT > 0) P->T = std::min(tT, 4 * FK_NT);
-  else P->T = cube > 0.75 * R ? FK_NT : 2 * FK_NT;
-  P->R = (P->T + FK_NT - 1) / FK_NT;
   /* blocks of about sixteen runs (the last run of a block is half empty on
    * average: four runs, (s, mu) DR 15.9 -> 15.1 ms), at least two cells wide:
    * the z extent of a run, and with it the FP32 windows, stays bounded in
@@ -2094,7 +2167,7 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
   const double nrb = (mode == MODE_C32 && b->geometry == FCFC_GEOM_SURVEY) ? 4.0 : 16.0;
   {
     const double per_cell = (double) nA / ((double) g.ncx * g.ncy * g.ncz);
-    const double zc = std::max(2.0 * zd, ceil(nrb * 64 * P->R / std::max(per_cell, 1e-9)));
+    const double zc = std::max(2.0 * zd, ceil(nrb * P->run / std::max(per_cell, 1e-9)));
     P->zmaxc = (int) std::min((double) g.ncz, zc);
     P->nblk = (g.ncz + P->zmaxc - 1) / P->zmaxc;
   }
@@ -2117,7 +2190,7 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
   }
   P->nstrips = (int) P->strips.size() / 3;
   P->cand = 0;
-  const double rlen = std::min(64.0 * P->R / std::max(ndenA * g.wx * g.wy, 1e-300), ext[2]);
+  const double rlen = std::min(P->run / std::max(ndenA * g.wx * g.wy, 1e-300), ext[2]);
   for (int q = 0; q < P->nstrips; q++) {
     const double gx = std::max(abs(P->strips[3 * q]) - 1, 0) * g.wx;
     const double gy = std::max(abs(P->strips[3 * q + 1]) - 1, 0) * g.wy;
@@ -2496,7 +2569,7 @@ static bool zb_fits(const fcfc_bins *b) {
 }
 
 static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh, int hyb,
-    int ssearch = 0, int psearch = 0) {
+    int ssearch = 0, int psearch = 0, int G = 1) {
   LdsPlan L;
   int o = 0;
   L.nh = nh;
@@ -2509,7 +2582,7 @@ static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh
   if (hyb) o = align16(o + 8 * (b->ns + 1 + (b->bintype == FCFC_BIN_SPI ? b->np + 1 : 0)));
   L.off_chunk = o;
   const bool f32 = (mode == MODE_C32), grad = (mode == MODE_GRAD);
-  o = align16(o + FK_NW * FK_CH * fk_chunk_bytes(f32, wt, grad));
+  o = align16(o + FK_NW * FK_CH * fk_chunk_bytes(f32, wt, grad, need_s, G));
   L.off_queue = o;
   if (f32) o += FK_NW * FK_QCAP * 6;
   o = align16(o);
@@ -2543,7 +2616,11 @@ static int fk_lanes_max(int geom, int mode, int wt, int hyb) {
 }
 
 template <int BIN, int GEOM, bool WT, int MODE>
-static kfn_t pick5(int hyb, int R) {
+static kfn_t pick5(int hyb, int R, int G) {
+  if constexpr ((MODE == MODE_C64 || MODE == MODE_C32 || MODE == MODE_GRAD) &&
+                !(GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SPI))
+    if (G > 1)
+      return hyb ? k_count<BIN, GEOM, WT, MODE, true, 1, FK_NG> : k_count<BIN, GEOM, WT, MODE, false, 1, FK_NG>;
   if constexpr (MODE == MODE_GRAD) {
     if (hyb) return k_count<BIN, GEOM, WT, MODE, true, 1>;
     return R == 1 ? k_count<BIN, GEOM, WT, MODE, false, 1> : k_count<BIN, GEOM, WT, MODE, false, 2>;
@@ -2557,28 +2634,28 @@ static kfn_t pick5(int hyb, int R) {
 }
 
 template <int BIN, int GEOM>
-static kfn_t pick3(int wt, int mode, int hyb, int R) {
-  if (mode == MODE_GRAD) return pick5<BIN, GEOM, true, MODE_GRAD>(hyb, R);
+static kfn_t pick3(int wt, int mode, int hyb, int R, int G) {
+  if (mode == MODE_GRAD) return pick5<BIN, GEOM, true, MODE_GRAD>(hyb, R, G);
   if (mode == MODE_C32)
-    return wt ? pick5<BIN, GEOM, true, MODE_C32>(hyb, R) : pick5<BIN, GEOM, false, MODE_C32>(hyb, R);
+    return wt ? pick5<BIN, GEOM, true, MODE_C32>(hyb, R, G) : pick5<BIN, GEOM, false, MODE_C32>(hyb, R, G);
   if constexpr (GEOM == FCFC_GEOM_BOX) {
     if (mode == MODE_C32C)
-      return wt ? pick5<BIN, GEOM, true, MODE_C32C>(hyb, R) : pick5<BIN, GEOM, false, MODE_C32C>(hyb, R);
+      return wt ? pick5<BIN, GEOM, true, MODE_C32C>(hyb, R, G) : pick5<BIN, GEOM, false, MODE_C32C>(hyb, R, G);
   }
   if (mode == MODE_P64)
-    return wt ? pick5<BIN, GEOM, true, MODE_P64>(hyb, R) : pick5<BIN, GEOM, false, MODE_P64>(hyb, R);
-  return wt ? pick5<BIN, GEOM, true, MODE_C64>(hyb, R) : pick5<BIN, GEOM, false, MODE_C64>(hyb, R);
+    return wt ? pick5<BIN, GEOM, true, MODE_P64>(hyb, R, G) : pick5<BIN, GEOM, false, MODE_P64>(hyb, R, G);
+  return wt ? pick5<BIN, GEOM, true, MODE_C64>(hyb, R, G) : pick5<BIN, GEOM, false, MODE_C64>(hyb, R, G);
 }
 
-static kfn_t pick_kernel(int bintype, int geom, int wt, int mode, int hyb, int R) {
+static kfn_t pick_kernel(int bintype, int geom, int wt, int mode, int hyb, int R, int G) {
   if (geom == FCFC_GEOM_BOX) {
-    if (bintype == FCFC_BIN_ISO) return pick3<FCFC_BIN_ISO, FCFC_GEOM_BOX>(wt, mode, hyb, R);
-    if (bintype == FCFC_BIN_SMU) return pick3<FCFC_BIN_SMU, FCFC_GEOM_BOX>(wt, mode, hyb, R);
-    return pick3<FCFC_BIN_SPI, FCFC_GEOM_BOX>(wt, mode, hyb, R);
+    if (bintype == FCFC_BIN_ISO) return pick3<FCFC_BIN_ISO, FCFC_GEOM_BOX>(wt, mode, hyb, R, G);
+    if (bintype == FCFC_BIN_SMU) return pick3<FCFC_BIN_SMU, FCFC_GEOM_BOX>(wt, mode, hyb, R, G);
+    return pick3<FCFC_BIN_SPI, FCFC_GEOM_BOX>(wt, mode, hyb, R, G);
   }
-  if (bintype == FCFC_BIN_ISO) return pick3<FCFC_BIN_ISO, FCFC_GEOM_SURVEY>(wt, mode, hyb, R);
-  if (bintype == FCFC_BIN_SMU) return pick3<FCFC_BIN_SMU, FCFC_GEOM_SURVEY>(wt, mode, hyb, R);
-  return pick3<FCFC_BIN_SPI, FCFC_GEOM_SURVEY>(wt, mode, hyb, R);
+  if (bintype == FCFC_BIN_ISO) return pick3<FCFC_BIN_ISO, FCFC_GEOM_SURVEY>(wt, mode, hyb, R, G);
+  if (bintype == FCFC_BIN_SMU) return pick3<FCFC_BIN_SMU, FCFC_GEOM_SURVEY>(wt, mode, hyb, R, G);
+  return pick3<FCFC_BIN_SPI, FCFC_GEOM_SURVEY>(wt, mode, hyb, R, G);
 }
 
 /* FP32 exactness windows.  With coordinates relative to the A tile centre
@@ -2836,6 +2913,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   int anywt = 0;
   for (auto &j : jobs) anywt |= j.wt;
   if (m == MODE_GRAD) anywt = 1;
+  /* a launch has runs of one kind (launch_groups) */
+  const int G = jobs.empty() ? 1 : jobs[0].P.G;
   /* room for the static LDS (416 bytes); the unused slots of the masked forms
    * come out of the margin */
   auto fits = [&](const LdsPlan &P, int mode_, int hyb_) {
@@ -2856,11 +2935,11 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   /* tables too long for LDS (hybrid binnings rescaled to large integers):
    * hybrid lookups that binary-search the edges, in the FP64 forms */
   int ssearch = 0, psearch = 0;
-  if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb), m, hyb)) {
+  if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 0, 0, G), m, hyb)) {
     if (m == MODE_C32) m = MODE_C64;
     hyb = 1;
     ssearch = 1;
-    if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 1, 0), m, hyb)) psearch = 1;
+    if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 1, 0, G), m, hyb)) psearch = 1;
   }
   /* one kernel serves every job of the launch: tiles of the longest kind.
    * A lane holds R objects (1, 2 or 4), so no tile may exceed R FK_NT
@@ -2886,9 +2965,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   };
   /* the rounding census compares the box arithmetic paths */
   const int km = (m == MODE_C32 && c->census && geom == FCFC_GEOM_BOX) ? MODE_C32C : m;
-  kfn_t fn = pick_kernel(b->bintype, geom, anywt, km, hyb, R);
+  kfn_t fn = pick_kernel(b->bintype, geom, anywt, km, hyb, R, G);
   /* histogram copies: as many as keep the occupancy of a single copy */
-  LdsPlan L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch);
+  LdsPlan L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch, G);
   if (!fits(L, m, hyb)) {
     set_err(c, "binning tables need %d bytes of LDS (limit %d)", L.total, 160 * 1024 - 2048);
     return FCFC_ERR_CFG;
@@ -2899,9 +2978,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   const int lds1 = L.total;
   for (const auto &o : c->occs)
     if (o.fn == (const void *) fn && o.lds1 == lds1 && c->t_nh <= 0) {
-      L = lds_plan(b, m, anywt, need_s, o.nh, hyb, ssearch, psearch);
+      L = lds_plan(b, m, anywt, need_s, o.nh, hyb, ssearch, psearch, G);
       if (L.total == o.lds) occ = o.occ;
-      else L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch);
+      else L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch, G);
       break;
     }
   if (!occ) {
@@ -2910,7 +2989,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     if (m != MODE_GRAD) {
       const int nhmax = c->t_nh > 0 ? c->t_nh : 8;
       for (int nh = 2; nh <= nhmax; nh *= 2) {
-        LdsPlan L2 = lds_plan(b, m, anywt, need_s, nh, hyb, ssearch, psearch);
+        LdsPlan L2 = lds_plan(b, m, anywt, need_s, nh, hyb, ssearch, psearch, G);
         int o2 = 0;
         if (!fits(L2, m, hyb)) break;
         if (int e = occ_of(fn, L2, &o2)) return e;
@@ -2942,8 +3021,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     t.unit0 = (int) nunit_l;
     t.nunit = (int) nu;
     t.nblk = J.P.nblk; t.zm = J.P.zmaxc; t.ncz = J.P.g.ncz;
-    t.T = std::min(J.P.T, 64 * J.P.R);
-    t.chunks = (int) std::min(J.P.cand / 64, 1e9);
+    t.T = std::min(J.P.T, G > 1 ? 64 / G : 64 * J.P.R);
+    t.chunks = (int) std::min(J.P.cand / (64 * G), 1e9);   /* in steps of 64 pairs per lane */
     t.smax = std::min(std::max(J.P.nstrips, 1), 64);
     t.ipw = njob > 1 ? 2 : 16;
     t.frac = c->tile_frac;
@@ -3116,13 +3195,13 @@ static int launch(fcfc_gpu_ctx *c, const Launch &Lc) {
 }
 
 /* Jobs of a batch grouped for their launches: one kernel variant per
- * launch, so weighted and unweighted jobs, and jobs whose tiles want one or
- * two objects per lane, go to separate persistent launches. */
+ * launch, so weighted and unweighted jobs, and jobs whose runs want one or
+ * two objects per lane or four groups of lanes, go to separate persistent launches. */
 static std::vector<std::vector<PJob>> launch_groups(const std::vector<PJob> &jobs) {
   std::vector<std::vector<PJob>> g;
   std::vector<int> key;
   for (const PJob &j : jobs) {
-    const int k = 2 * (j.wt ? 1 : 0) + ((j.P.T > FK_NT) ? 1 : 0);
+    const int k = 2 * (j.wt ? 1 : 0) + ((j.P.T > FK_NT) ? 1 : 0) + (j.P.G > 1 ? 4 : 0);
     size_t q = 0;
     while (q < key.size() && key[q] != k) q++;
     if (q == key.size()) { key.push_back(k); g.emplace_back(); }

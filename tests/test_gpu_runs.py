@@ -1,4 +1,4 @@
-"""Runs of A objects per wavefront: remainders of 64 and 128 objects, long
+"""Runs of A objects per wavefront: remainders of 16, 64 and 128 objects, long
 sparse columns across the periodic boundary, 32-bit counters beyond 2^32 pairs
 and job changes of few workgroups -- against the oracle (counts identical,
 weighted counts within 1e-12 relative)."""
@@ -59,6 +59,39 @@ def test_run_remainders(eng, n, bt, hyb):
         for tile in (0, 40, 512, 1024, 2048):
             eng.set_tuning(tile=tile)
             _check(eng, b, A, B, f"n={n} bt={bt} tile={tile}")
+    finally:
+        eng.set_tuning()
+
+
+@pytest.mark.parametrize("geom,bt,hyb", [(g, t, h) for g in (F.GEOM_BOX, F.GEOM_SURVEY)
+                                         for t in (F.BIN_ISO, F.BIN_SMU, F.BIN_SPI)
+                                         for h in (False, True)])
+def test_groups_of_lanes(eng, geom, bt, hyb):
+    """Runs of 16 and of 5 objects, each held by four groups of lanes, with
+    numbers of objects that leave remainders of the runs and of the groups;
+    counts, and the gradient by its linearity in the weights."""
+    rng = np.random.default_rng(21)
+    ds = 7.3 if hyb else 5.0
+    box = geom == F.GEOM_BOX
+    b = F.Bins.linear(geom, bt, 0, 20 * ds, ds, nmu=10 if bt == F.BIN_SMU else 1, pmin=0,
+                      pmax=100 if bt == F.BIN_SPI else 0, dpi=5, bsize=L if box else None)
+    o = 0.0 if box else 600.0
+    A, B = (F.Catalog(b, *(rng.uniform(o, o + 400, n) for _ in range(3)), rng.uniform(0.5, 2, n))
+            for n in (203, 1501))
+    g = rng.uniform(-1, 1, b.ntot)
+    try:
+        for tile in (16, 5):
+            eng.set_tuning(tile=tile)
+            _check(eng, b, A, B, f"groups geom={geom} bt={bt} hyb={hyb} tile={tile}")
+            for X in (None, B):
+                ga, gb = eng.count_backward(A, X, b, g, isauto=X is None)
+                cnt = eng.count_pairs(A, X, b, isauto=X is None, withwt=True)
+                # each pair weight appears in both sides' gradients
+                ref = (2 if X is None else 1) * (g @ cnt)
+                mag = 2 * np.abs(g) @ cnt
+                np.testing.assert_allclose(ga @ A.w, ref, rtol=0, atol=1e-12 * mag)
+                if X is not None:
+                    np.testing.assert_allclose(gb @ B.w, ref, rtol=0, atol=1e-12 * mag)
     finally:
         eng.set_tuning()
 
