@@ -399,7 +399,7 @@ struct FkJob {
   FkGrid g;
   const int *strips;          /* (dx, dy, diag) triples */
   int nstrips;
-  int autoc;                  /* COUNT: A == B, half shell + self tile;
+  int autoc;                  /* COUNT: A == B, half shell + the run;
                                  GRAD: A == B, exclude j == i          */
   int wt;                     /* weighted histogram (double)          */
   int wg0, wg1;               /* workgroups that start with it        */
@@ -966,7 +966,8 @@ __host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool wt, bool grad, b
 
 /* One persistent kernel for counts (FP64 or FP32 + recheck) and for the
  * weight gradient.  Template parameters: binning, geometry, weighted
- * histogram support, mode, hybrid tables, A objects per lane.  Unweighted
+ * histogram support, mode, hybrid tables, A objects per lane, groups of lanes.
+ * Unweighted
  * kernels are held to 64 VGPRs (8 waves per SIMD, 4 workgroups per CU):
  * occupancy pays more than the FP32 form's spills, which sit in its rare
  * re-evaluation paths.  Weighted ones get 80 (6 waves per SIMD), as their
@@ -1859,7 +1860,7 @@ struct fcfc_gpu_ctx {
   int t_nh = 0;                /* LDS histogram copies (0: by occupancy) */
   int census = 0;
   int tile_frac = 0;           /* autotuner: count about 1/tile_frac of the
-                                  tiles (16 runs spread over the list) */
+                                  runs (16 stretches of the list) */
   const int *last_nrun = nullptr;  /* device: runs of the last launch built */
   struct Tuned { int geom, bintype, mode, autoc, wt, bucket, cd, zd, T; };
   std::vector<Tuned> tuned;    /* autotuner results per density bucket */
@@ -2154,11 +2155,6 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
       return FCFC_ERR_CFG;
     }
   }
-  /* Objects per tile: two per lane, which halves the B objects read from LDS
-   * per pair, unless a run of 128 objects is about as wide as the separations
-   * it is counted to (sparse catalogues): then 64, whose boxes reach fewer B
-   * objects (w_p of 1e6 objects to 40 Mpc/h: 3.0 against 3.9 ms; iso DD of
-   * 1e5 to 200 Mpc/h, whose cube is half the separation: 0.39 against 0.36). */
   /* blocks of about sixteen runs (the last run of a block is half empty on
    * average: four runs, (s, mu) DR 15.9 -> 15.1 ms), at least two cells wide:
    * the z extent of a run, and with it the FP32 windows, stays bounded in
@@ -2181,7 +2177,7 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
       int diag = 0;
       if (autoc) {
         /* auto counts and their gradient: half plane, and on the own row
-         * only the objects after the tile */
+         * only the objects after the run */
         if (dx < 0 || (dx == 0 && dy < 0)) continue;
         if (dx == 0 && dy == 0) diag = 1;
       }
@@ -2604,9 +2600,8 @@ typedef void (*kfn_t)(const FkArgs);
 /* Kernel variants: binning x geometry x weights x mode x table type x A
  * objects per lane (R = 1: tiles of FK_NT objects, R = 2: 2 FK_NT, R = 4:
  * 4 FK_NT).  The gradient with hybrid tables uses R = 1; R = 4 exists for
- * the weighted FP64 box counts with integer tables only, whose LDS-bound
- * histogram updates gain from reading each staged B object for more A
- * objects (fk_lanes_max gives the largest R of a kernel family).  The
+ * the weighted FP64 box counts with integer tables only and for callers that
+ * set such tiles (fk_lanes_max gives the largest R of a kernel family).  The
  * survey kernels hold four more FP64 values per object and spill at R = 4
  * (weighted (s_perp, pi) DR: 950 ms against 830 at R = 2). */
 static int fk_lanes_max(int geom, int mode, int wt, int hyb) {
@@ -2658,9 +2653,9 @@ static kfn_t pick_kernel(int bintype, int geom, int wt, int mode, int hyb, int R
   return pick3<FCFC_BIN_SPI, FCFC_GEOM_SURVEY>(wt, mode, hyb, R, G);
 }
 
-/* FP32 exactness windows.  With coordinates relative to the A tile centre
+/* FP32 exactness windows.  With coordinates relative to the A run's centre
  * c, each FP32 difference satisfies |d32 - d| <= u (2|d| + E) + tiny
- * (u = 2^-24, E = tile extent), so
+ * (u = 2^-24, E = run extent), so
  *   |s2_32 - s2| <= 7 u s2 + 2 sqrt(3) u E s + 3 (u (2 s + E))^2,
  * evaluated at the largest in-range s^2 (plus the first integer above it:
  * beyond that the table answers "outside" without a window).  The mu bin
@@ -2670,12 +2665,12 @@ static kfn_t pick_kernel(int bintype, int geom, int wt, int mode, int hyb, int R
  * All bounds are inflated by 25%; pairs below s2_floor are always
  * re-evaluated.
  *
- * Survey pairs (fk_sv32) add two things.  The reference's own values carry
+ * Survey pairs (fk_sv32_spi) add two things.  The reference's own values carry
  * the rounding of its FP64 formulas: s^2 = (|a|^2 + |b|^2) - 2 a.b is off
  * the exact value by at most about 8 eps R^2 (R = largest |r| of the grid,
  * eps = 2^-53, |r|^2 given with 2 eps), and its pi = (|a|^2 - |b|^2) / |m|
  * by 5 eps R^2 / |m| (m = a + b).  And the FP32 m = (2 a' + d) + 2 c (c the
- * tile centre, a' = a - c) has error |dm| <= 2u|c| + 2 sqrt(3) ek + 2u|m| +
+ * run's centre, a' = a - c) has error |dm| <= 2u|c| + 2 sqrt(3) ek + 2u|m| +
  * 2uE (ek = u (2 s + E) + tiny, 2|c| <= |m| + s + E), so p = d.m is off by
  * at most |m| (sqrt(3) ek + 6 u s) + s (u (s + 3E) + 2 sqrt(3) ek) and pi
  * by e_pi = sqrt(3) ek + 6 u s + s (u (s + 3E) + 2 sqrt(3) ek) / |m|.  With |m|^2 >= m2_floor (smaller |m| is re-evaluated) these are
@@ -2914,7 +2909,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   for (auto &j : jobs) anywt |= j.wt;
   if (m == MODE_GRAD) anywt = 1;
   /* a launch has runs of one kind (launch_groups) */
-  const int G = jobs.empty() ? 1 : jobs[0].P.G;
+  int G = jobs.empty() ? 1 : jobs[0].P.G;
   /* room for the static LDS (416 bytes); the unused slots of the masked forms
    * come out of the margin */
   auto fits = [&](const LdsPlan &P, int mode_, int hyb_) {
@@ -2932,6 +2927,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
       if (!(w.e_s2x2 < 0.5f) || !(w.e_pix2 < 0.5f)) { m = MODE_C64; break; }
     }
   }
+  /* (the chunks of the groups of lanes, 18 KB or more, must not cost a
+   * binning its tables: one group then, with longer runs) */
+  if (G > 1 && !fits(lds_plan(b, m, anywt, need_s, 1, hyb, 0, 0, G), m, hyb)) G = 1;
   /* tables too long for LDS (hybrid binnings rescaled to large integers):
    * hybrid lookups that binary-search the edges, in the FP64 forms */
   int ssearch = 0, psearch = 0;
@@ -2941,9 +2939,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     ssearch = 1;
     if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 1, 0, G), m, hyb)) psearch = 1;
   }
-  /* one kernel serves every job of the launch: tiles of the longest kind.
-   * A lane holds R objects (1, 2 or 4), so no tile may exceed R FK_NT
-   * objects: R is cut to what the kernel family provides (fk_lanes_max),
+  /* one kernel serves every job of the launch: runs of the longest kind.
+   * A lane holds R objects (1, 2 or 4), so no run may exceed 64 R objects
+   * (a tile is the FK_NW runs of a workgroup): R is cut to what the kernel family provides (fk_lanes_max),
    * and a tile size set by the caller or the autotuner is clamped to what
    * the kernel covers */
   {
@@ -3575,10 +3573,10 @@ extern "C" int fcfc_gpu_plan_destroy(fcfc_gpu_plan *P) {
 }
 
 /* Project-written autotuner: for jobs like (a, b, bins, flags) try grid and
- * tile shapes (cells per maximum separation, z-cells per cell, A objects
- * per tile), timing each on the first part of the tile list (a slab of the
- * box at the true density: an eighth, a sixteenth beyond 16384 tiles) and
- * extrapolating to all tiles (counts of at most 4096 tiles are timed
+ * run shapes (cells per maximum separation, z-cells per cell, A objects
+ * per tile of FK_NW runs), timing each on a part of the list of runs (16
+ * stretches spread over it: an eighth, a sixteenth beyond 16384 tiles) and
+ * extrapolating to all runs (counts of at most 4096 tiles are timed
  * whole).  Every pair of cell_div and zdiv is timed (the best zdiv depends
  * on cell_div: a descent over one, then the other, missed the best pair of
  * a cross count), then the tile size.  The winner is cached in the
