@@ -1106,12 +1106,15 @@ k_count(const FkArgs a) {
        * below that edge may land at its lower end (same bin, no edge of the
        * table there) */
       if (HYB && c == 1 && off != lo_edge) f |= FK_F_EDGE;
-      if (v != FK_OUT && (v >= (unsigned) nb || (alw_below > 0 && off + c < alw_below + 1.0) ||
-                          (HYB && c == 0 && off != lo_edge)))
+      const bool low = alw_below > 0 && off + c < alw_below + 1.0;
+      if (v != FK_OUT && (v >= (unsigned) nb || low || (HYB && c == 0 && off != lo_edge)))
         f |= FK_F_ALW | FK_F_EDGE;
       /* masked lanes reach the first sentinel only within the window of the
-       * upper range edge */
-      if (MASKED && c == len) f |= FK_F_ALW | FK_F_EDGE;
+       * upper range edge, and the cells below the range with any s^2 down to
+       * 0.  There the mu estimate is no bin: 0 * inf at zero distance, whose
+       * NaN passes the fraction test of fk_mu32, so those below s2_floor are
+       * re-evaluated like the others (and dropped) */
+      if (MASKED && (c == len || (c < 0 && low))) f |= FK_F_ALW | FK_F_EDGE;
       if (MASKED && c < 0) v = (unsigned) nb;
       return v | f;
     };
