@@ -68,6 +68,8 @@ struct FkBins {
   double q_caps, q_capp;     /* pi^2 and s_perp^2 in fixed point (fk_sv64): */
   double q_bmin;             /* addend, ceilings, least |a+b|^2 of the fast */
   unsigned q_t16, q_pad;     /* path, fraction threshold of edge cells      */
+  double s2low;              /* masked survey (s,mu): least s^2 of a counted   */
+                             /* pair (just above -1 for ranges from 0)         */
   double s2skip, pskip;      /* forms without a mask: a pair at s^2 >= s2skip */
   float s2skip32, skip_pad;  /* or pi >= pskip is out of range (FP64 / FP32) */
   float m32s, m32p;          /* FP32: values at or beyond are out of range   */
