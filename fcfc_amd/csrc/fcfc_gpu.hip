@@ -2614,6 +2614,9 @@ static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh
   return L;
 }
 
+/* dynamic LDS of a workgroup: all but the 412 bytes of k_count's own arrays */
+#define FK_LDS_MOST (160 * 1024 - 512)
+
 typedef void (*kfn_t)(const FkArgs);
 
 /* Kernel variants: binning x geometry x weights x mode x table type x A
@@ -2932,7 +2935,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   /* room for the static LDS (416 bytes); the unused slots of the masked forms
    * come out of the margin */
   auto fits = [&](const LdsPlan &P, int mode_, int hyb_) {
-    return P.total <= 160 * 1024 - (masked_form(b, mode_, hyb_) ? 512 : 2048);
+    return P.total <= (masked_form(b, mode_, hyb_) ? FK_LDS_MOST : 160 * 1024 - 2048);
   };
   /* the FP32 window test reads one table cell and the edge at its lower end:
    * windows must stay well inside a cell (wide only for a few objects in a
@@ -2975,8 +2978,10 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   }
   /* ---- kernel and LDS plan ---- */
   const int R = jobs.empty() ? 1 : jobs[0].P.R;
+  /* (the limit belongs to the kernel, whose launches of other sizes -- other
+   * contexts', replayed plans' -- share it: always the same, the most there is) */
   auto occ_of = [&](kfn_t f, const LdsPlan &P, int *occ) -> int {
-    HIPCHK(c, hipFuncSetAttribute((const void *) f, hipFuncAttributeMaxDynamicSharedMemorySize, P.total));
+    HIPCHK(c, hipFuncSetAttribute((const void *) f, hipFuncAttributeMaxDynamicSharedMemorySize, FK_LDS_MOST));
     HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, (const void *) f, FK_NT, P.total));
     return 0;
   };
