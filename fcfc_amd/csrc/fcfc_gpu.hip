@@ -1880,6 +1880,7 @@ struct fcfc_gpu_ctx {
   int census = 0;
   int tile_frac = 0;           /* autotuner: count about 1/tile_frac of the
                                   runs (16 stretches of the list) */
+  int last_T = 0;              /* tile size of the last launch built */
   const int *last_nrun = nullptr;  /* device: runs of the last launch built */
   struct Tuned { int geom, bintype, mode, autoc, wt, bucket, cd, zd, T; };
   std::vector<Tuned> tuned;    /* autotuner results per density bucket */
@@ -2028,6 +2029,8 @@ struct JobPlan {
   int nstrips;
 };
 
+static bool groups_keep_tables(const fcfc_bins *b, int mode, int wt);
+
 static double max_sep2(const fcfc_bins *b, double *rxy2, double *hzc) {
   double s2max = b->s2bin[b->ns];
   *hzc = -1;
@@ -2046,10 +2049,11 @@ static double max_sep2(const fcfc_bins *b, double *rxy2, double *hzc) {
   return s2max;
 }
 
-/* Build the grid geometry and strip list.  lo/hi: bounding box (survey). */
+/* Build the grid geometry and strip list.  lo/hi: bounding box (survey);
+ * groups: runs of 16 objects held by groups of lanes may be planned. */
 static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
     const double lo[3], const double hi[3], int autoc, int wt, int mode, int64_t nA,
-    int64_t nB, JobPlan *P) {
+    int64_t nB, bool groups, JobPlan *P) {
   double rxy2, hzc;
   double r2 = max_sep2(b, &rxy2, &hzc);
   /* pad: the survey formula carries ~1e-10 absolute rounding in s^2 */
@@ -2111,9 +2115,10 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
    * (0.51) weighted 0.55, 0.63; survey (s, mu) to 150 of 6e4 (0.86) 0.20,
    * 0.16; iso DD of 1e5 (0.54) 0.31, 0.42; DR of 6e3 x 6e4 (0.64) 0.087,
    * 0.12. */
-  const bool can = mode != MODE_P64 && !c->census &&
+  const bool can = groups && mode != MODE_P64 && !c->census &&
       !(b->geometry == FCFC_GEOM_SURVEY && b->bintype == FCFC_BIN_SPI);
-  P->G = can && (P->T <= 64 / FK_NG || (P->T == FK_NT && cube > 0.75 * R && 8 * nden >= ndenA)) ? FK_NG : 1;
+  P->G = can && (P->T <= 64 / FK_NG || (P->T == FK_NT && cube > 0.75 * R && 8 * nden >= ndenA)) &&
+      groups_keep_tables(b, mode, wt) ? FK_NG : 1;
   P->run = P->G > 1 ? 64 / P->G : 64 * P->R;
   /* Runs as compact as their object number allows: the objects of B within
    * the maximum separation of a run's bounding box are evaluated, and a cube
@@ -2617,6 +2622,50 @@ static LdsPlan lds_plan(const fcfc_bins *b, int mode, int wt, int need_s, int nh
 /* dynamic LDS of a workgroup: all but the 412 bytes of k_count's own arrays */
 #define FK_LDS_MOST (160 * 1024 - 512)
 
+/* does a plan fit?  (The unused slots of the masked forms come out of the
+ * margin.) */
+static bool lds_fits(const fcfc_bins *b, const LdsPlan &P, int mode, int hyb) {
+  return P.total <= (masked_form(b, mode, hyb) ? FK_LDS_MOST : 160 * 1024 - 2048);
+}
+
+/* Form and tables of a count of this mode, with G groups of lanes.  FP32
+ * tables are zero-based, and the fixed-point mu value of that form holds
+ * t <= nmu (1 + 2^-20) below 127: other binnings run in FP64.  Tables too long
+ * for LDS (hybrid binnings rescaled to large integers) are replaced by hybrid
+ * lookups that binary-search the edges, in the FP64 forms. */
+struct TabForm {
+  int m, hyb, ssearch, psearch;
+  bool fits;
+  bool operator==(const TabForm &o) const {
+    return m == o.m && hyb == o.hyb && ssearch == o.ssearch && psearch == o.psearch && fits == o.fits;
+  }
+};
+static TabForm table_form(const fcfc_bins *b, int mode, int wt, int G) {
+  const int need_s = (b->geometry == FCFC_GEOM_SURVEY && b->bintype != FCFC_BIN_ISO);
+  const bool zb = zb_fits(b);
+  TabForm f = {mode, (b->tabtype || !zb) ? 1 : 0, 0, 0, true};
+  if (f.m == MODE_C32 && (!zb || (b->bintype == FCFC_BIN_SMU && b->nmu > FK_NMU32))) f.m = MODE_C64;
+  auto fit = [&]() {
+    return lds_fits(b, lds_plan(b, f.m, wt, need_s, 1, f.hyb, f.ssearch, f.psearch, G), f.m, f.hyb);
+  };
+  if (!fit()) {
+    if (f.m == MODE_C32) f.m = MODE_C64;
+    f.hyb = 1;
+    f.ssearch = 1;
+    if (!fit()) f.psearch = 1;
+    f.fits = fit();
+  }
+  return f;
+}
+
+/* The chunks of the groups of lanes take 18 KB or more of LDS: they must not
+ * cost a binning its tables (tables that do not fit without them either are
+ * searched in any case, and the search needs next to no LDS: a w_p count of
+ * 1e6 objects 1.7 ms in groups and 2.5 without). */
+static bool groups_keep_tables(const fcfc_bins *b, int mode, int wt) {
+  return table_form(b, mode, wt, FK_NG) == table_form(b, mode, wt, 1);
+}
+
 typedef void (*kfn_t)(const FkArgs);
 
 /* Kernel variants: binning x geometry x weights x mode x table type x A
@@ -2808,6 +2857,15 @@ static void fp32_windows(const fcfc_bins *b, const FkGrid &g, int zmaxc, double 
   w.m2_floor = (float) m2f;
 }
 
+/* The FP32 window test reads one table cell and the edge at its lower end:
+ * windows must stay well inside a cell (wide only for a few objects in a huge
+ * volume, whose grid cells, and so runs, are large). */
+static bool fp32_ok(const fcfc_bins *b, const JobPlan &P) {
+  FkWin w;
+  fp32_windows(b, P.g, P.zmaxc, fp32_s2_floor(b, P.g, P.zmaxc), &w);
+  return w.e_s2x2 < 0.5f && w.e_pix2 < 0.5f;
+}
+
 static int cat_ok(const fcfc_cat *k) {
   return k && k->n >= 0 && k->n < 0x7fffffff && (k->n == 0 || (k->x && k->y && k->z));
 }
@@ -2857,7 +2915,12 @@ static int setup_job(fcfc_gpu_ctx *c, Alloc &al, std::vector<CopyKey> &copies,
     if ((e = bbox(c, al, ks, autoc ? 1 : 2, lo, hi))) return e;
     if (!(lo[0] <= hi[0])) { for (int k = 0; k < 3; k++) { lo[k] = 0; hi[k] = 1; } }
   }
-  if ((e = make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, a->n, autoc ? a->n : b->n, &J->P))) return e;
+  const int64_t nb = autoc ? a->n : b->n;
+  if ((e = make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, a->n, nb, true, &J->P))) return e;
+  /* a grid for longer runs where windows take a count to FP64 whose tables
+   * leave no room for groups of lanes */
+  if (J->P.G > 1 && mode == MODE_C32 && !fp32_ok(bins, J->P) && !groups_keep_tables(bins, MODE_C64, wt) &&
+      (e = make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, a->n, nb, false, &J->P))) return e;
   J->autoc = autoc;
   J->wt = wt;
   const fcfc_cat *cs[2] = {a, autoc ? a : b};
@@ -2921,46 +2984,19 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     std::vector<PJob> &jobs, int mode, unsigned long long *res, int ncall, Launch *out) {
   const int geom = b->geometry;
   int m = mode;
-  const bool zb = zb_fits(b);
-  if (m == MODE_C32 && !zb) m = MODE_C64;                      /* FP32 tables are zero-based */
-  /* the FP32 fixed-point mu value holds t <= nmu (1 + 2^-20) below 127 */
-  if (m == MODE_C32 && b->bintype == FCFC_BIN_SMU && b->nmu > FK_NMU32) m = MODE_C64;
-  int hyb = (b->tabtype || !zb) ? 1 : 0;
   const int need_s = (geom == FCFC_GEOM_SURVEY && b->bintype != FCFC_BIN_ISO);
   int anywt = 0;
   for (auto &j : jobs) anywt |= j.wt;
   if (m == MODE_GRAD) anywt = 1;
   /* a launch has runs of one kind (launch_groups) */
   int G = jobs.empty() ? 1 : jobs[0].P.G;
-  /* room for the static LDS (416 bytes); the unused slots of the masked forms
-   * come out of the margin */
-  auto fits = [&](const LdsPlan &P, int mode_, int hyb_) {
-    return P.total <= (masked_form(b, mode_, hyb_) ? FK_LDS_MOST : 160 * 1024 - 2048);
-  };
-  /* the FP32 window test reads one table cell and the edge at its lower end:
-   * windows must stay well inside a cell (wide only for a few objects in a
-   * huge volume, whose grid cells, and so tiles, are large) */
-  if (m == MODE_C32) {
-    double s2f = 0;
-    for (const PJob &J : jobs) s2f = std::max(s2f, fp32_s2_floor(b, J.P.g, J.P.zmaxc));
-    for (const PJob &J : jobs) {
-      FkWin w;
-      fp32_windows(b, J.P.g, J.P.zmaxc, s2f, &w);
-      if (!(w.e_s2x2 < 0.5f) || !(w.e_pix2 < 0.5f)) { m = MODE_C64; break; }
-    }
-  }
-  /* (the chunks of the groups of lanes, 18 KB or more, must not cost a
-   * binning its tables: one group then, with longer runs) */
-  if (G > 1 && !fits(lds_plan(b, m, anywt, need_s, 1, hyb, 0, 0, G), m, hyb)) G = 1;
-  /* tables too long for LDS (hybrid binnings rescaled to large integers):
-   * hybrid lookups that binary-search the edges, in the FP64 forms */
-  int ssearch = 0, psearch = 0;
-  if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 0, 0, G), m, hyb)) {
-    if (m == MODE_C32) m = MODE_C64;
-    hyb = 1;
-    ssearch = 1;
-    if (!fits(lds_plan(b, m, anywt, need_s, 1, hyb, 1, 0, G), m, hyb)) psearch = 1;
-  }
+  for (const PJob &J : jobs) if (m == MODE_C32 && !fp32_ok(b, J.P)) m = MODE_C64;
+  /* (only a job whose own plan did not see this launch's form: another job of
+   * the batch has taken it to FP64) */
+  if (G > 1 && !groups_keep_tables(b, m, anywt)) G = 1;
+  const TabForm tf = table_form(b, m, anywt, G);
+  m = tf.m;
+  const int hyb = tf.hyb, ssearch = tf.ssearch, psearch = tf.psearch;
   /* one kernel serves every job of the launch: runs of the longest kind.
    * A lane holds R objects (1, 2 or 4), so no run may exceed 64 R objects
    * (a tile is the FK_NW runs of a workgroup): R is cut to what the kernel family provides (fk_lanes_max),
@@ -2990,8 +3026,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   kfn_t fn = pick_kernel(b->bintype, geom, anywt, km, hyb, R, G);
   /* histogram copies: as many as keep the occupancy of a single copy */
   LdsPlan L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch, G);
-  if (!fits(L, m, hyb)) {
-    set_err(c, "binning tables need %d bytes of LDS (limit %d)", L.total, 160 * 1024 - 2048);
+  if (!tf.fits) {
+    set_err(c, "binning tables need %d bytes of LDS (limit %d)", L.total, FK_LDS_MOST);
     return FCFC_ERR_CFG;
   }
   /* (the choice depends on the kernel and the LDS size of one copy alone, and
@@ -3013,7 +3049,7 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
       for (int nh = 2; nh <= nhmax; nh *= 2) {
         LdsPlan L2 = lds_plan(b, m, anywt, need_s, nh, hyb, ssearch, psearch, G);
         int o2 = 0;
-        if (!fits(L2, m, hyb)) break;
+        if (!lds_fits(b, L2, m, hyb)) break;
         if (int e = occ_of(fn, L2, &o2)) return e;
         if (o2 < occ1 && c->t_nh <= 0) break;
         L = L2;
@@ -3185,7 +3221,8 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
   a.census = c->census;
   a.G = tabs.G;
   c->last_nrun = unitoff + nunit;
-  c->stats.tile = jobs.empty() ? 0 : jobs[0].P.T;
+  c->last_T = jobs.empty() ? 0 : jobs[0].P.T;
+  c->stats.tile = G > 1 ? std::min(c->last_T, FK_NW * 64 / G) : c->last_T;
   c->stats.cell_div = jobs.empty() ? 0 : (int) lround(sqrt(jobs[0].P.g.Rxy2) / jobs[0].P.g.wx);
   out->fn = fn; out->nblock = nwg; out->lds = L.total; out->a = a;
   out->nunit = nunit; out->njob = njob; out->tj = dtj;
@@ -3652,7 +3689,7 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
     if (e) return e;
     const int ns = fk_split(nt, 1, 1, 1, 1, c->tile_frac).ncap;     /* runs counted */
     *est = c->stats.kernel_ms * (double) nt / (double) std::max(1, ns);
-    last_T = c->stats.tile;
+    last_T = c->last_T;
     if (tune_log)
       fprintf(stderr, "fcfc_gpu_autotune: cell_div %d zcell_div %d tile %d: %d of %d runs "
               "in %.3f ms, estimate %.3f ms\n", cd, zd, last_T, ns, nt,
@@ -3707,7 +3744,7 @@ extern "C" int fcfc_gpu_autotune(fcfc_gpu_ctx *c, const fcfc_cat *a,
       if ((e = bbox(c, tal, ks, autoc ? 1 : 2, lo, hi))) return e;
     }
     const int wt = (grad || (flags & FCFC_GPU_WEIGHTED)) ? 1 : 0;
-    make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, ka->n, kb->n, &P);
+    make_plan(c, bins, bsize, lo, hi, autoc, wt, mode, ka->n, kb->n, true, &P);
     bool found = false;
     for (auto &t : c->tuned)
       if (t.geom == bins->geometry && t.bintype == bins->bintype && t.mode == mode &&

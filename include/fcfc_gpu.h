@@ -197,7 +197,8 @@ typedef struct {
   double kernel_ms;      /* device time of the count kernel(s)              */
   double total_ms;       /* wall time of the call                            */
   int    cell_div;       /* cells per max separation used                   */
-  int    tile;           /* objects per A tile                              */
+  int    tile;           /* objects per A tile, the runs of 8 wavefronts
+                            (128: runs of 16, for sparse catalogues)        */
 } fcfc_gpu_stats;
 int fcfc_gpu_last_stats(const fcfc_gpu_ctx *ctx, fcfc_gpu_stats *st);
 
