@@ -2049,6 +2049,21 @@ static double max_sep2(const fcfc_bins *b, double *rxy2, double *hzc) {
   return s2max;
 }
 
+/* Side of the box that holds m objects of a catalogue of density nden with
+ * extents ext: of a cube, where the extents have room for one, else of a slab
+ * as thick as the catalogue, or a piece of a line.  (The cube of a plane
+ * catalogue, its thickness 1e-6, is far too small: 1e6 objects in a plane to
+ * 50 Mpc/h took 14.7 ms on cells of a twelfth of that, 0.67 on cells of 50.) */
+static double box_side(double m, double nden, const double ext[3]) {
+  double e[3] = {ext[0], ext[1], ext[2]};
+  std::sort(e, e + 3);
+  const double v = m / std::max(nden, 1e-300);
+  double side = cbrt(v);
+  if (side > e[0]) side = sqrt(v / e[0]);
+  if (side > e[1]) side = v / (e[0] * e[1]);
+  return side;
+}
+
 /* Build the grid geometry and strip list.  lo/hi: bounding box (survey);
  * groups: runs of 16 objects held by groups of lanes may be planned. */
 static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
@@ -2102,7 +2117,7 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
    * counted to (sparse catalogues): then one (iso DD of 1e5 to 200 Mpc/h,
    * whose cube is half the separation: 0.39 against 0.36 ms). */
   P->T_auto = (tT <= 0);
-  const double cube = cbrt(128.0 / std::max(ndenA, 1e-300));
+  const double cube = box_side(128, ndenA, ext);
   if (tT > 0) P->T = std::min(tT, 4 * FK_NT);
   else P->T = cube > 0.75 * R ? FK_NT : 2 * FK_NT;
   P->R = (P->T + FK_NT - 1) / FK_NT;
@@ -2130,7 +2145,7 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
    * 232, 231, 230 (rule: 6); weighted DD of 5e5 9.1, 8.7, 8.9, 10.1, 12 (3);
    * iso DD of 1e5 0.36, 0.36, 0.55, 0.82, 1.2 (2); survey (s, mu) RR of 1.2e6
    * 16.6, 15.5, 16.4, 19.9, 25 (3). */
-  const double width = P->G > 1 ? cbrt(32.0 / std::max(ndenA, 1e-300)) : cube;
+  const double width = P->G > 1 ? box_side(32, ndenA, ext) : cube;
   if (cd <= 0) cd = (int) std::min(std::max(floor(Rxy / width + 0.6), 1.0), 12.0);
   if (zd <= 0) zd = 4;
   /* cells of Rxy / cd, but never more cells than about 4 per object
@@ -2193,7 +2208,8 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
   }
   /* strips */
   P->strips.clear();
-  const int kx = (int) ceil(Rxy / g.wx), ky = (int) ceil(Rxy / g.wy);
+  int kx = (int) ceil(Rxy / g.wx), ky = (int) ceil(Rxy / g.wy);
+  if (!g.periodic) { kx = std::min(kx, g.ncx - 1); ky = std::min(ky, g.ncy - 1); }   /* rows there are */
   for (int dx = -kx; dx <= kx; dx++) {
     for (int dy = -ky; dy <= ky; dy++) {
       double gx = std::max(abs(dx) - 1, 0) * g.wx, gy = std::max(abs(dy) - 1, 0) * g.wy;
