@@ -1172,7 +1172,7 @@ k_count(const FkArgs a) {
     if (BIN == FCFC_BIN_SPI) for (int i = tid; i <= bn.np; i += FK_NT) pe[i] = bn.pbin[i];
   }
 
-  unsigned long long evals = 0;               /* uniform: candidate pairs */
+  unsigned long long evals = 0;               /* uniform: distances evaluated */
   unsigned int nrecheck = 0, ncensus = 0;
   /* pairs this wavefront may have added to 32-bit counters since the
    * workgroup's last flush (FK_NW such budgets stay below 2^32) */
@@ -1676,9 +1676,9 @@ k_count(const FkArgs a) {
             else keep &= __builtin_fma(ez, ez, exy) < g.R2;
           }
           unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
-          evals += (unsigned long long) ((unsigned) min(FK_CH, n - c0) * (unsigned) nva);
           if (m == 0) continue;
           const int cnt = __popcll(m);
+          evals += (unsigned long long) ((unsigned) cnt * (unsigned) nva);
           if (!GRAD && !jwt) {
             if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) spill_counts();
             since += (unsigned) cnt * (unsigned) nva;

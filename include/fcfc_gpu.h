@@ -188,10 +188,9 @@ int fcfc_gpu_count_noalloc(fcfc_gpu_ctx *ctx, const fcfc_cat *a,
 
 /* Per-call statistics of the last fcfc_gpu_count / _batch / _backward. */
 typedef struct {
-  double evals;          /* candidate pairs of the grid's cell windows (each
-                            settled by its distance, or with the 64 pairs or
-                            more of a B object beyond the separation from the
-                            bounding box of a wavefront's A objects)        */
+  double evals;          /* pair distances evaluated: the A objects of each
+                            wavefront times the B objects within the maximum
+                            separation of their bounding box                */
   double rechecked;      /* pairs re-evaluated in FP64 (FP32 mode)          */
   double census;         /* rounding-path ambiguous pairs (FCFC_GPU_CENSUS) */
   double kernel_ms;      /* device time of the count kernel(s)              */
