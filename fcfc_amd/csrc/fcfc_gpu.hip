@@ -30,6 +30,7 @@
 #define MODE_GRAD 2   /* weight gradient (FP64 bins)                    */
 #define MODE_C32C 3   /* MODE_C32 with the rounding census of the rechecked pairs */
 #define MODE_P64  4   /* FP64, the reference's per-pair arithmetic as written */
+#define MODE_GRADL 5  /* MODE_GRAD of a masked form whose range starts above zero */
 
 /* ======================================================================== */
 /*                          grid build kernels                              */
@@ -1018,7 +1019,7 @@ k_count(const FkArgs a) {
   constexpr bool F32 = (MODE == MODE_C32 || MODE == MODE_C32C);
   constexpr bool CENS = (MODE == MODE_C32C);
   constexpr bool PLAIN = (MODE == MODE_P64);
-  constexpr bool GRAD = (MODE == MODE_GRAD);
+  constexpr bool GRAD = (MODE == MODE_GRAD || MODE == MODE_GRADL);
   constexpr bool SV32 = (GEOM == FCFC_GEOM_SURVEY && (MODE == MODE_C32 || MODE == MODE_C32C));
   /* |r|^2 of the objects: survey (s, mu) and (s_perp, pi) in FP64 (the FP32
    * form reads them from the catalogue when it re-evaluates a pair) */
@@ -1508,6 +1509,12 @@ k_count(const FkArgs a) {
               }
               in[r] = s2[r] < bn.s2max;
               if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabs(ez[r]) < bn.pmax);
+              /* the gradient reads no slot for a pair below the range: its zero
+               * would make NaN of an infinite weight */
+              if (MODE == MODE_GRADL) {
+                in[r] = in[r] & (s2[r] >= bn.s2min);
+                if (BIN == FCFC_BIN_SPI) in[r] = in[r] & (__builtin_fabs(ez[r]) >= bn.pmin);
+              }
               if (SELF) in[r] = in[r] & (jj > ai[r]);
               any |= in[r];
             }
@@ -2717,6 +2724,11 @@ static kfn_t pick5(int hyb, int R, int G) {
 
 template <int BIN, int GEOM>
 static kfn_t pick3(int wt, int mode, int hyb, int R, int G) {
+  if constexpr (!(GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SPI))
+    if (mode == MODE_GRADL) {
+      if (G > 1) return k_count<BIN, GEOM, true, MODE_GRADL, false, 1, FK_NG>;
+      return R == 1 ? k_count<BIN, GEOM, true, MODE_GRADL, false, 1> : k_count<BIN, GEOM, true, MODE_GRADL, false, 2>;
+    }
   if (mode == MODE_GRAD) return pick5<BIN, GEOM, true, MODE_GRAD>(hyb, R, G);
   if (mode == MODE_C32)
     return wt ? pick5<BIN, GEOM, true, MODE_C32>(hyb, R, G) : pick5<BIN, GEOM, false, MODE_C32>(hyb, R, G);
@@ -3038,7 +3050,9 @@ static int build_launch(fcfc_gpu_ctx *c, Alloc &al, Upload &up, const DevTabs &t
     return 0;
   };
   /* the rounding census compares the box arithmetic paths */
-  const int km = (m == MODE_C32 && c->census && geom == FCFC_GEOM_BOX) ? MODE_C32C : m;
+  const bool above0 = b->soff > 0 || (b->bintype == FCFC_BIN_SPI && b->poff > 0);
+  const int km = (m == MODE_C32 && c->census && geom == FCFC_GEOM_BOX) ? MODE_C32C
+                 : (m == MODE_GRAD && above0 && masked_form(b, m, hyb)) ? MODE_GRADL : m;
   kfn_t fn = pick_kernel(b->bintype, geom, anywt, km, hyb, R, G);
   /* histogram copies: as many as keep the occupancy of a single copy */
   LdsPlan L = lds_plan(b, m, anywt, need_s, 1, hyb, ssearch, psearch, G);

@@ -62,3 +62,35 @@ def test_coincident_pairs(eng, geom, hyb, ns, nmu):
             np.testing.assert_allclose(gotw, refw, rtol=1e-12, atol=0)
             if prec == "fp32":
                 assert min(re, rew) >= n
+
+
+@pytest.mark.parametrize("tile", [0, 16])
+@pytest.mark.parametrize("geom,bt", [(g, t) for g in (F.GEOM_BOX, F.GEOM_SURVEY)
+                                     for t in (F.BIN_ISO, F.BIN_SMU, F.BIN_SPI)])
+def test_gradient_of_infinite_weights(eng, geom, bt, tile):
+    """A clump 8 across, counted from 20 on, whose objects have infinite
+    weights: they are in no bin with anything, and neither their gradients nor
+    the others' may notice."""
+    rng = np.random.default_rng(8)
+    b = F.Bins.linear(geom, bt, 20, 60, 5, nmu=9 if bt == F.BIN_SMU else 1,
+                      pmin=10 if bt == F.BIN_SPI else 0, pmax=40 if bt == F.BIN_SPI else 0, dpi=5,
+                      bsize=L if geom == F.GEOM_BOX else None)
+    o = 0.0 if geom == F.GEOM_BOX else 600.0
+    p = o + np.concatenate([rng.uniform(100, 250, (3, 800)), 800 + rng.uniform(0, 4.6, (3, 70))], axis=1)
+    w = np.concatenate([rng.uniform(0.5, 2, 800), np.full(70, np.inf)])
+    A, N = F.Catalog(b, *p, w), F.Catalog(b, *p[:, :800], w[:800])
+    g = rng.uniform(-1, 1, b.ntot)
+    try:
+        eng.set_tuning(tile=tile)
+        for X, Y in ((None, None), (A, N)):
+            print(f"case gradient inf geom={geom} bt={bt} tile={tile} auto={X is None}", flush=True)
+            ga, gb = eng.count_backward(A, X, b, g, isauto=X is None)
+            na, nb = eng.count_backward(N, Y, b, g, isauto=Y is None)
+            assert abs(na).max() > 0
+            tol = 1e-12 * np.abs(g).max() * w[:800].sum()
+            for got, ref in ((ga, na), (gb, nb)):
+                if got is not None:
+                    assert not got[800:].any()
+                    np.testing.assert_allclose(got[:800], ref, rtol=0, atol=tol)
+    finally:
+        eng.set_tuning()
