@@ -1527,7 +1527,8 @@ k_count(const FkArgs a) {
                * |r|^2 is huge or not that of the coordinates.  Either reads cell
                * 0, whose pairs all take the exact path, which drops the latter
                * (s2low; in the mask it cost the count of 1.2e6 objects 4 %) */
-              const unsigned cell = stab[fk_trunc_u32(s2[r])];
+              const unsigned cell = stab[GEOM == FCFC_GEOM_SURVEY && BIN == FCFC_BIN_SMU
+                                         ? fk_trunc_u32(s2[r]) : (unsigned) (int) s2[r]];
               if (BIN == FCFC_BIN_ISO) add(cell, r);
               else if (BIN == FCFC_BIN_SPI)
                 add(cell + __umul24((unsigned) bn.nsh, ptab[(int) __builtin_fabs(ez[r])]), r);
