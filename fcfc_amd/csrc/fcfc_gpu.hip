@@ -1379,6 +1379,7 @@ k_count(const FkArgs a) {
 
       /* FP32: FP64 re-evaluation of the n queued pairs of this wavefront */
       int qn = 0;
+      unsigned kept = 0;          /* B objects evaluated (at most all of the call, in two images) */
       auto drain = [&]() __attribute__((always_inline)) {
         fk_wave_sync();
         const FkJob J = fk_cld(fk_again(a.jobs, cur));
@@ -1686,7 +1687,7 @@ k_count(const FkArgs a) {
           unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
           if (m == 0) continue;
           const int cnt = __popcll(m);
-          evals += (unsigned long long) ((unsigned) cnt * (unsigned) nva);
+          kept += (unsigned) cnt;
           if (!GRAD && !jwt) {
             if (__builtin_expect(since + (unsigned) cnt * (unsigned) nva > FK_BUDGET, 0)) spill_counts();
             since += (unsigned) cnt * (unsigned) nva;
@@ -1817,6 +1818,7 @@ k_count(const FkArgs a) {
         }
       }
       if (F32 && qn) drain();
+      evals += (unsigned long long) kept * (unsigned) nva;
 
       if (GRAD) {
         double *gA = fk_cld(&fk_again(a.jobs, cur)->gA);
