@@ -1011,7 +1011,7 @@ __host__ __device__ constexpr int fk_chunk_bytes(bool f32, bool wt, bool grad, b
  * and take every NG-th kept B object each, from the chunk.  In a sparse
  * catalogue 64 objects spread over more than the separations counted, and most
  * pairs of a run are out of range: 16 objects have a quarter of the volume
- * (iso cross count of 3e5 x 1e6: 1.10 -> 0.56 ms, w_p of 1e6 2.5 -> 1.7). */
+ * (iso cross count of 3e5 x 1e6: 1.10 -> 0.56 ms, w_p of 1e6 2.5 -> 1.8). */
 template <int BIN, int GEOM, bool WT, int MODE, bool HYB, int R, int NG = 1>
 __global__ void __launch_bounds__(FK_NT, WT ? 6 : 8)
 k_count(const FkArgs a) {
@@ -1870,8 +1870,8 @@ __global__ void k_add_f64(double *dst, const double *src, int n) {
  * (once per device) and every host use goes through that address. */
 #define FK_SCRATCH_BYTES ((size_t) 128 << 20)
 #define FK_MAXDEV 64
-#define FK_PIN_BYTES ((size_t) 1 << 20)     /* pinned at the start; grown up to */
-#define FK_PIN_MOST ((size_t) 64 << 20)     /* this for large batches           */
+#define FK_PIN_BYTES ((size_t) 1 << 20)     /* pinned at the start; grown to twice   */
+#define FK_PIN_MOST ((size_t) 64 << 20)     /* what a call needs, up to this much    */
 static __device__ __align__(256) unsigned char scratch[FK_SCRATCH_BYTES];
 static void *g_scratch_ptr[FK_MAXDEV];
 static std::mutex g_scratch_mu;
@@ -2134,7 +2134,7 @@ static int make_plan(fcfc_gpu_ctx *c, const fcfc_bins *b, const double *bsize,
   /* Sparser catalogues than that: runs of 16 objects, four groups of lanes
    * (k_count), unless B is far sparser than A (its strips then hold too few
    * objects for four groups).  Kernel ms, without and with: iso cross count
-   * of 3e5 x 1e6 to 30 Mpc/h 1.10, 0.56; w_p of 1e6 to 40 Mpc/h 2.5, 1.7; iso
+   * of 3e5 x 1e6 to 30 Mpc/h 1.10, 0.56; w_p of 1e6 to 40 Mpc/h 2.5, 1.8; iso
    * DD of 2e3 0.040, 0.026; box (s, mu) DD to 200 of the unit box of 1000:
    * n = 3e4 (cube / R = 0.81) 0.136, 0.103; 6e4 (0.64) 0.207, 0.185; 1.2e5
    * (0.51) weighted 0.55, 0.63; survey (s, mu) to 150 of 6e4 (0.86) 0.20,
@@ -2687,7 +2687,7 @@ static TabForm table_form(const fcfc_bins *b, int mode, int wt, int G) {
 /* The chunks of the groups of lanes take 18 KB or more of LDS: they must not
  * cost a binning its tables (tables that do not fit without them either are
  * searched in any case, and the search needs next to no LDS: a w_p count of
- * 1e6 objects 1.7 ms in groups and 2.5 without). */
+ * 1e6 objects 1.8 ms in groups and 2.5 without). */
 static bool groups_keep_tables(const fcfc_bins *b, int mode, int wt) {
   return table_form(b, mode, wt, FK_NG) == table_form(b, mode, wt, 1);
 }
